@@ -1444,6 +1444,50 @@ def test_matmul_kquant_int8_long_and_short_steps_keep_token_bits(ctx, t, k):
         assert got[first : first + count].tobytes() == run(first, count).tobytes(), "token chunking changed bits"
 
 
+@pytest.mark.parametrize("n", [90, 16390])
+@pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_matmul_kquant_int8_tiles(ctx, t, n):
+    """Both orders of the K formats' whole-k int8 multiply (four parts of k; from 16384 rows on one)
+    at every tile height its dispatch knows, ragged in tokens and rows, with the largest products
+    the scales and weights allow (blocks of all ones or all zeros bits against inputs rounded to
+    127): 1e-5 against float64 over the rounded activations (f32 sums of exact integers:
+    k / 256 additions of 2^-24 each stay far below), the same bits whatever the step's length."""
+    c = ctx
+    rows, k, stride = 300, 768, n + 3
+    x = c.random(rows * k, 1).reshape(rows, k)
+    x[5] = 1.0
+    x[6] = np.where(np.arange(k) % 2, -1.0, 1.0)
+    xs = oracle.round_like_llama(ORACLE_TYPE[t], x)
+    raw, _ = quant_rows(c, t, n, k)
+    raw = raw.reshape(n, -1)
+    e, size = K.LAYOUT[t]
+    for row, byte in ((0, 0xFF), (1, 0x00), (n - 1, 0x7F), (n - 2, 0x80)):
+        blocks = raw[row].reshape(k // e, size)
+        scales = {TensorType.q3_k: (108,), TensorType.q4_k: (0, 2), TensorType.q5_k: (0, 2), TensorType.q6_k: (208,)}[t]
+        keep = [blocks[:, o : o + 2].copy() for o in scales]
+        blocks[:] = byte
+        for o, v in zip(scales, keep):
+            blocks[:, o : o + 2] = v
+    values = oracle.dequantize(ORACLE_TYPE[t], raw.reshape(-1), n * k).reshape(n, k)
+    wa = c.gpu_weights(t, raw.reshape(-1), k)
+    init = c.random(rows * stride, 0.5).reshape(rows, stride)
+
+    def run(first, count):
+        out = c.upload(init[first : first + count])
+        launch_int8(c, t, quantize_x(c, t, c.upload(x[first : first + count]), count, k), wa, out, count, n, k, 1, None, col0=2, stride=stride)
+        return c.read(out).reshape(count, stride)
+
+    got = run(0, rows)
+    want = init[:, 2 : 2 + n] + xs.astype(np.float64) @ values.astype(np.float64).T
+    for row in range(rows):
+        assert rel_err(got[row, 2 : 2 + n], want[row]) <= 1e-5, row
+    mask = np.ones(stride, dtype=bool)
+    mask[2 : 2 + n] = False
+    assert np.array_equal(got[:, mask].view(np.uint32), init[:, mask].view(np.uint32)), "columns outside the chunk were written"
+    for first, count in ((0, 1), (1, 63), (4, 100), (100, 33)):
+        assert got[first : first + count].tobytes() == run(first, count).tobytes(), "token chunking changed bits"
+
+
 def test_matmul_q8_0_int8_whole_steps_keep_token_bits(ctx):
     """matmul_q8_0 with k a multiple of 128, unsliced, takes the kernel whose scale products
     run on the matrix cores, in 128- or 64-token tiles: a token's sums are the same bits
