@@ -350,7 +350,7 @@ def test_quant_matvec_act_prologue(ctx, t, k):
     # Steps of exactly two tokens over short rows keep both tokens' inputs in registers:
     (TensorType.q4_k, 4096, True, 2, 100),
     (TensorType.q3_k, 3072, True, 2, 21),     # 48 tasks: idle lanes
-    (TensorType.q5_k, 4096, True, 2, 40),     # (a format whose gate / up step of two tokens stays on the general kernel)
+    (TensorType.q5_k, 4096, True, 2, 40),     # (gate and up rows in turn)
     (TensorType.q8_0, 2048, False, 2, 50),    # two rows a wave pass
     (TensorType.q6_k, 1024, False, 2, 33),    # four rows a wave pass, a ragged last pass
     (TensorType.q5_k, 4096, False, 2, 64),
@@ -383,6 +383,34 @@ def test_quant_matvec_long_rows(ctx, t, k, pair, rows, n):
         single = c.upload(init[tk])
         c.launcher().launch_pipeline(pipeline, p(), [c.upload(x[tk]), wa, single, na], (K.div_ceil(n, v.group_rows()), 1, 1))
         assert got[tk].tobytes() == c.read(single).tobytes(), "a token's sums differ between a lone launch and a multi-token launch"
+
+
+@pytest.mark.parametrize("t,k,rows,n", [
+    # Two tokens' gate and up rows in turn: one, two and four rows a wave's pass, idle lanes, a
+    # single output, one output past whole passes, more outputs than a wave keeps (64 a wave).
+    (TensorType.q5_k, 4096, 2, 1),
+    (TensorType.q8_0, 4096, 2, 9),
+    (TensorType.q6_k, 2560, 2, 130),
+    (TensorType.q5_k, 2560, 2, 515),
+    (TensorType.q4_k, 2048, 2, 257),
+    (TensorType.q3_k, 1024, 2, 65),
+    (TensorType.q8_0, 64, 2, 3),
+    (TensorType.q6_k, 1024, 2, 4099),
+])
+def test_quant_matvec_pair_rows_in_turn(ctx, t, k, rows, n):
+    test_quant_matvec_long_rows(ctx, t, k, True, rows, n)
+
+
+@pytest.mark.parametrize("k,pair,rows,n", [
+    (2048, False, 3, 7501),   # an odd last pass of one token
+    (2048, False, 8, 7449),
+    (4096, True, 4, 1870),
+    (2304, True, 5, 3315),
+])
+def test_matvec_q5_k_passes_of_two(ctx, k, pair, rows, n):
+    """Q5_K steps of more than two tokens over 10 MB of rows and more."""
+    assert n * K.row_bytes(TensorType.q5_k, k) * (2 if pair else 1) >= 10 << 20
+    test_quant_matvec_long_rows(ctx, TensorType.q5_k, k, pair, rows, n)
 
 
 def test_quant_matvec_eight_rows(ctx):

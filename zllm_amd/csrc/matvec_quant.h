@@ -30,7 +30,7 @@
 // Kernels. matvec_quant_kernel (steps of one to four tokens, any row length): inputs are read
 // from a bank-conflict-free padded LDS copy kept in task order, once per task for both rows of
 // a pass (two outputs, or the gate and up rows of one output with SILU_PAIR), the next task's
-// vectors loaded before the current one is multiplied. matvec_quant_row_kernel (one token, at
+// vectors loaded before the current one is multiplied. matvec_quant_row_kernel (one or two tokens, at
 // most one task per lane, i.e. k <= 4096): the lane's 64 inputs never change from row to row,
 // so they live in registers and the loop touches nothing but the weight stream; it asks for the
 // token's inputs (and norm weights) before its first weights: loads complete in order within a
@@ -161,7 +161,8 @@ struct KQ8 {
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = false;
-    static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers leaves two waves a SIMD their registers
+    static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
+    static constexpr bool PASS2 = false;
     static const char *name() { return "matvec_q8_0"; }
     struct Raw {
         uint4 q[4];
@@ -234,7 +235,8 @@ struct KQ3 {
     static constexpr int STAGE2 = 2, STAGE4 = 2;  // tokens whose inputs are loaded at once
     static constexpr bool ALL4 = false;           // (four at once measured slower on every shape: 1024 x 4096 7.7 against 7.1 us)
     static constexpr bool DEFER = true;
-    static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers leaves two waves a SIMD their registers
+    static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
+    static constexpr bool PASS2 = false;
     static const char *name() { return "matvec_q3_k"; }
     struct Raw {
         uint4 u[2];
@@ -322,7 +324,8 @@ struct KQ4 {
     static constexpr int STAGE2 = 2, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = true;
-    static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers leaves two waves a SIMD their registers
+    static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
+    static constexpr bool PASS2 = false;
     static const char *name() { return "matvec_q4_k"; }
     struct Raw {
         uint4 h, q0, q1;
@@ -405,7 +408,15 @@ struct KQ5 {
     static constexpr int STAGE2 = 0, STAGE4 = 4;  // tokens whose inputs are loaded at once
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = true;
-    static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers leaves two waves a SIMD their registers
+    static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
+    // A step of more than two tokens over 10 MB of rows or more runs as passes of two tokens in
+    // registers: the fifth bits leave the general kernel too few registers for more tokens' sums.
+    // Four tokens, general / passes of two: 9728 x 2560 21.7 / 17.6 us, 14336 x 4096 30.0 / 23.8,
+    // 50257 x 2560 82 / 57, 8192 x 2048 (11 MB) 11.8 / 10.7; below, the second launch costs more
+    // than it gains (3072 x 1024 6.0 / 6.9, 2 x 3072 x 1024 8.1 / 10.4). The other formats'
+    // general kernels are the faster ones at three and four tokens (14336 x 4096 at four tokens
+    // against twice the two-token launch: Q4_K 18.5 / 22, Q6_K 21.7 / 29, Q8_0 21.6 / 27).
+    static constexpr bool PASS2 = true;
     static const char *name() { return "matvec_q5_k"; }
     struct Raw {
         uint4 h, b0, b1, q0, q1;
@@ -496,7 +507,8 @@ struct KQ6 {
     static constexpr int STAGE2 = 2, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = false;
-    static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers leaves two waves a SIMD their registers
+    static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
+    static constexpr bool PASS2 = false;
     static const char *name() { return "matvec_q6_k"; }
     struct Raw {
         uint4 l0, l1, hv;
@@ -865,7 +877,7 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
     }
 }
 
-// One-token steps over rows of at most 64 tasks, with the lane's inputs in registers, so that
+// One- and two-token steps over rows of at most 64 tasks, with the inputs in registers, so that
 // the loop holds nothing but the weight stream's loads and the multiply. A wave's walk is wave
 // uniform here: pass u covers rows u * RPI .. + RPI - 1 (RPI = 64 >> SEG_LOG2 rows side by side
 // in the wave), so the pass's position lives in scalar registers, a lane's byte offsets within
@@ -880,12 +892,12 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
 // two passes asked for before the inputs are staged (instead of one) 8.7 us; the first pass
 // asked for only once the inputs have arrived 8.0 us.
 constexpr int kRowDepth = 1;
-template <class P, int MT, bool PAIR, int SEG_LOG2>
+template <class P, int MT, bool PAIR, bool TURNS, int SEG_LOG2>
 __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
     const MvArgs &a = q.a;
     extern __shared__ float4 lds4[];
     __shared__ float red[4 * MT];
-    constexpr int NSUM = P::NSUM, RUN = 64 / NSUM, kRows = PAIR ? 2 : 1;
+    constexpr int NSUM = P::NSUM, RUN = 64 / NSUM, kRows = PAIR && !TURNS ? 2 : 1;
     constexpr uint32_t SEG = 1u << SEG_LOG2, RPI = 64u >> SEG_LOG2;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t tasks = q.tasks, k4 = a.k / 4u;
@@ -915,18 +927,19 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
     const typename P::Where at = tsub < tasks ? P::where(rsub * a.row_bytes, a.k, tsub) : P::nowhere();
     const uint64_t span = (uint64_t)a.rows * a.row_bytes;  // bytes of the rows covered (and of their up rows)
     const uint64_t pass_bytes = (uint64_t)RPI * a.row_bytes;
-    // Pass u's rows, and with PAIR the up rows of its outputs.
-    auto fetch = [&](uint32_t u, typename P::Raw (&dst)[kRows]) __attribute__((always_inline)) {
+    const uint64_t up_rows = PAIR ? (uint64_t)a.half * a.row_bytes : 0u;
+    // Pass u's rows, and with PAIR the up rows of its outputs (TURNS: the ones `first` bytes in).
+    auto fetch = [&](uint32_t u, uint64_t first, typename P::Raw (&dst)[kRows]) __attribute__((always_inline)) {
         const bool live = u < units;
         const uint64_t off = live ? u * pass_bytes : 0u;
         const uint32_t left = live ? (uint32_t)(span - off) : 0u;
-        dst[0] = P::fetch(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.w + off), 0, (int)left, 0x00020000), at);
-        if (PAIR) dst[kRows - 1] = P::fetch(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.w + (size_t)a.half * a.row_bytes + off), 0, (int)left, 0x00020000), at);
+        dst[0] = P::fetch(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.w + first + off), 0, (int)left, 0x00020000), at);
+        if (PAIR && !TURNS) dst[kRows - 1] = P::fetch(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.w + up_rows + off), 0, (int)left, 0x00020000), at);
         __builtin_amdgcn_sched_barrier(0);  // (the loads stay ahead of the multiply that follows them in the source)
     };
     typename P::Raw buf[kRowDepth + 1][kRows];
 #pragma unroll
-    for (int dpt = 0; dpt < kRowDepth; dpt++) fetch(gwave + dpt * nwaves, buf[dpt]);
+    for (int dpt = 0; dpt < kRowDepth; dpt++) fetch(gwave + dpt * nwaves, 0u, buf[dpt]);
 
     // stage_token's arithmetic on the vectors already loaded, the tokens' sums of squares
     // meeting in LDS together.
@@ -1026,54 +1039,81 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
         kept_first += nkept * nwaves;
         nkept = 0;
     };
-    auto multiply = [&](uint32_t u, const typename P::Raw (&rows)[kRows]) __attribute__((always_inline)) {
-        // (a row at a time: with the inputs in registers two rows share nothing, and one row's
-        // sums and words are fewer registers than two rows')
-        float v[kRows][MT];
+    // One row's sums over the wave, for every token.
+    auto row_sums = [&](const typename P::Raw &row, float (&s)[MT]) __attribute__((always_inline)) {
+        const typename P::Raw(&one)[1] = reinterpret_cast<const typename P::Raw(&)[1]>(row);
+        float v[1][MT];
+        P::template dot<MT, 1>(one, ch, nm,
+            [&](int t, int vi) { return make_float4(xr[t][4 * vi], xr[t][4 * vi + 1], xr[t][4 * vi + 2], xr[t][4 * vi + 3]); },
+            [&](int t, int i) { return xsum[t][i]; }, v);
 #pragma unroll
-        for (int j = 0; j < kRows; j++) {
-            const typename P::Raw(&one)[1] = reinterpret_cast<const typename P::Raw(&)[1]>(rows[j]);
-            float vj[1][MT];
-            P::template dot<MT, 1>(one, ch, nm,
-                [&](int t, int vi) { return make_float4(xr[t][4 * vi], xr[t][4 * vi + 1], xr[t][4 * vi + 2], xr[t][4 * vi + 3]); },
-                [&](int t, int s) { return xsum[t][s]; }, vj);
+        for (int t = 0; t < MT; t++) s[t] = v[0][t];
+    };
+    // (0 + v: matvec_quant_kernel adds a lane's tasks to a sum that starts at zero)
+    auto reduce = [&](float (&s)[MT]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < MT; t++) v[j][t] = vj[0][t];
-        }
+        for (int t = 0; t < MT; t++) s[t] = segment_sum(0.f + s[t], SEG_LOG2);
+    };
+    auto keep = [&](const float (&s)[MT], float (&kept)[MT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            // (0 + v: matvec_quant_kernel adds a lane's tasks to a sum that starts at zero)
-            const float s0 = segment_sum(0.f + v[0][t], SEG_LOG2);
-            const float s1 = PAIR ? segment_sum(0.f + v[kRows - 1][t], SEG_LOG2) : 0.f;
-            if (kKeep) {
-                const float t0 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s0), 63));
-                kept0[t] = lane == nkept ? t0 : kept0[t];
-                if (PAIR) {
-                    const float t1 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s1), 63));
-                    kept1[t] = lane == nkept ? t1 : kept1[t];
-                }
-            } else {
-                const uint32_t j = u * RPI + rsub;
-                if (tsub == SEG - 1u && j < a.rows) {
-                    float r = PAIR ? silu_f(s0) * s1 : s0;
+            const float total = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[t]), 63));
+            kept[t] = lane == nkept ? total : kept[t];
+        }
+    };
+    // The sums of pass u's rows (s0) and, with PAIR, of the up rows (s1): kept, or stored.
+    auto finish = [&](uint32_t u, const float (&s0)[MT], const float (&s1)[MT]) __attribute__((always_inline)) {
+        if (kKeep) {
+            keep(s0, kept0);
+            if (PAIR) keep(s1, kept1);
+            nkept++;
+            if (nkept == 64u) flush_kept();
+        } else {
+            const uint32_t j = u * RPI + rsub;
+            if (tsub == SEG - 1u && j < a.rows) {
+#pragma unroll
+                for (int t = 0; t < MT; t++) {
+                    float r = PAIR ? silu_f(s0[t]) * s1[t] : s0[t];
                     if (accumulate) r += a.out[out_at(t, j)];
                     a.out[out_at(t, j)] = r;
                 }
             }
         }
-        if (kKeep) {
-            nkept++;
-            if (nkept == 64u) flush_kept();
-        }
+    };
+    // (a row at a time: with the inputs in registers two rows share nothing, and one row's
+    // sums and words are fewer registers than two rows')
+    auto multiply = [&](uint32_t u, const typename P::Raw (&rows)[kRows]) __attribute__((always_inline)) {
+        float s0[MT], s1[MT] = {};
+        row_sums(rows[0], s0);
+        if (PAIR) row_sums(rows[kRows - 1], s1);
+        reduce(s0);
+        if (PAIR) reduce(s1);
+        finish(u, s0, s1);
     };
 
+    // Gate and up rows in turn: one row's loads in flight while the other is multiplied, so a
+    // pair needs the registers of a single row (and its gate's sums).
+    if (TURNS) {
+        for (uint32_t u = gwave; u < units; u += nwaves) {
+            float s0[MT], s1[MT];
+            fetch(u, up_rows, buf[1]);
+            row_sums(buf[0][0], s0);
+            reduce(s0);
+            fetch(u + nwaves, 0u, buf[0]);
+            row_sums(buf[1][0], s1);
+            reduce(s1);
+            finish(u, s0, s1);
+        }
+        if (kKeep) flush_kept();
+        return;
+    }
     // kRowDepth passes' loads stay in flight ahead of the one multiplied; a trip of
     // kRowDepth + 1 passes so that the buffers rotate by name.
     for (uint32_t u = gwave;;) {
         bool done = false;
 #pragma unroll
         for (int ph = 0; ph <= kRowDepth; ph++) {
-            fetch(u + kRowDepth * nwaves, buf[(ph + kRowDepth) % (kRowDepth + 1)]);
+            fetch(u + kRowDepth * nwaves, 0u, buf[(ph + kRowDepth) % (kRowDepth + 1)]);
             multiply(u, buf[ph]);
             u += nwaves;
             if (u >= units) {
@@ -1506,18 +1546,18 @@ static zhip_result run_slices(const Dispatch &d, const KArgs &q, uint32_t lds, u
     return check_launch(d, P::name());
 }
 
-template <class P, int MT, bool PAIR>
+template <class P, int MT, bool PAIR, bool TURNS = false>
 static zhip_result run_row(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     if (lds > 65536u) {
-        const bool ok = q.seg_log2 == 4u ? lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, 4>, 160 * 1024 - 64>()
-                      : q.seg_log2 == 5u ? lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, 5>, 160 * 1024 - 64>()
-                                         : lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, 6>, 160 * 1024 - 64>();
+        const bool ok = q.seg_log2 == 4u ? lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, TURNS, 4>, 160 * 1024 - 64>()
+                      : q.seg_log2 == 5u ? lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, TURNS, 5>, 160 * 1024 - 64>()
+                                         : lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, TURNS, 6>, 160 * 1024 - 64>();
         if (!ok) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
     }
     switch (q.seg_log2) {
-    case 4: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, 4>), dim3(blocks), dim3(256), lds, d.stream, q); break;
-    case 5: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, 5>), dim3(blocks), dim3(256), lds, d.stream, q); break;
-    default: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, 6>), dim3(blocks), dim3(256), lds, d.stream, q); break;
+    case 4: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, TURNS, 4>), dim3(blocks), dim3(256), lds, d.stream, q); break;
+    case 5: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, TURNS, 5>), dim3(blocks), dim3(256), lds, d.stream, q); break;
+    default: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, TURNS, 6>), dim3(blocks), dim3(256), lds, d.stream, q); break;
     }
     return check_launch(d, P::name());
 }
@@ -1553,7 +1593,10 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
     if (tok_lds > max_lds) return fail(d, ZHIP_E_BAD_COMMAND, "%s: k = %u does not fit workgroup memory", P::name(), a.k);
     for (uint32_t t0 = 0; t0 < a.m;) {
         uint32_t left = a.m - t0;
-        uint32_t mt = left >= 4u ? 4u : left;
+        // (PASS2: see KQ5)
+        const bool pass2 = P::PASS2 && q.tasks <= 64u && (uint64_t)a.rows * a.row_bytes * (pair ? 2u : 1u) >= 10u << 20;
+        const uint32_t most = pass2 ? 2u : 4u;
+        uint32_t mt = left >= most ? most : left;
         // A step of exactly two tokens over rows of 65 .. 256 tasks keeps both tokens' slices in
         // registers like the one-token step (Q4_K 4096 x 14336: 16.5 us tile by tile).
         if (a.m == 2u && !pair && q.tasks > 64u && q.tasks <= 256u) {
@@ -1642,8 +1685,16 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             t0 += q.mt;
             continue;
         }
-        // Steps of one or two tokens over rows of up to 64 tasks keep the lanes' inputs in registers.
-        const bool xreg = (a.m == 1u || (a.m == 2u && (!pair || P::PAIR2))) && q.tasks <= 64u;
+        // Steps of one or two tokens over rows of up to 64 tasks keep the lanes' inputs in registers,
+        // and so do Q5_K's longer steps, two tokens a pass. A two-token gate / up step takes its
+        // gate and up rows in turn (TURNS), except whole-wave rows of the formats whose two rows
+        // fit beside two tokens' inputs (PAIR2). Two tokens with the RMSNorm prologue, through the
+        // general kernel / rows in turn, 2 x 9728 x 2560: Q5_K 31.0 / 16.0 us, Q8_0 20.3 / 16.5,
+        // Q6_K 18.6 / 16.8; 2 x 14336 x 4096: 44.3 / 23.6, 30.7 / 25.5, 28.3 / 25.3; both rows
+        // in a pass / in turn, 2 x 8192 x 2048 (two rows to a wave's pass): Q4_K 12.5 / 8.8,
+        // Q3_K 13.1 / 9.3, and 2 x 14336 x 4096: Q4_K 20.2 / 20.4, Q3_K 21.7 / 21.7. One token
+        // gains nothing from it (2 x 14336 x 4096 Q4_K 15.6 / 16.3, Q5_K 19.6 / 19.8).
+        const bool xreg = (a.m <= 2u || pass2) && q.tasks <= 64u;
         const uint32_t per_unit = pair ? rpi : rpi * (xreg ? 1u : 2u);
         const uint32_t units = (a.rows + per_unit - 1u) / per_unit;
         const uint32_t want = (units + 3u) / 4u;
@@ -1668,11 +1719,11 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             // Q5_K 18.3 / 17.2; 4096 x 4096 Q4_K 4.9 / 4.2; 28672 x 2048 Q4_K 8.0 / 9.05.
             const uint32_t cus = (uint32_t)d.dev->compute_units;
             // (two tokens' inputs leave the registers for two waves a SIMD: two workgroups)
-            const bool three = a.m == 1u && !pair && (uint64_t)rpi * a.row_bytes <= 3072u && passes >= cus * 48u;
+            const bool three = mt == 1u && !pair && (uint64_t)rpi * a.row_bytes <= 3072u && passes >= cus * 48u;
             const uint32_t cap = cus * (three ? 3u : 2u), row_blocks = row_want < cap ? row_want : cap;
-            const uint32_t row_lds = a.m * q.tasks * kTaskStride * 4u;
-            if (a.m == 1u) r = pair ? run_row<P, 1, true>(d, q, row_lds, row_blocks) : run_row<P, 1, false>(d, q, row_lds, row_blocks);
-            else if (pair) r = P::PAIR2 ? run_row<P, 2, P::PAIR2>(d, q, row_lds, row_blocks) : ZHIP_E_GPU;
+            const uint32_t row_lds = mt * q.tasks * kTaskStride * 4u;
+            if (mt == 1u) r = pair ? run_row<P, 1, true>(d, q, row_lds, row_blocks) : run_row<P, 1, false>(d, q, row_lds, row_blocks);
+            else if (pair) r = P::PAIR2 && q.seg_log2 == 6u ? run_row<P, 2, P::PAIR2, !P::PAIR2>(d, q, row_lds, row_blocks) : run_row<P, 2, true, true>(d, q, row_lds, row_blocks);
             else r = run_row<P, 2, false>(d, q, row_lds, row_blocks);
         } else if (mt == 1u) r = pair ? run_quant<P, 1, true, 1>(d, q, lds, blocks) : run_quant<P, 1, false, 1>(d, q, lds, blocks);
         else if (mt == 2u) {
