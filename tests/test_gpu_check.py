@@ -187,6 +187,52 @@ def test_matvec_bf16_several_tokens_keep_token_bits(ctx, ctx_wide, wide, half):
     assert np.array_equal(run([5], 404, 4096)[0], whole[5, 404:])
 
 
+@pytest.mark.parametrize("m,n,k,half_row,accumulate,norm", [
+    # 16 MB of gate rows and more: the matrix cores, a tile of gate rows and then one of up rows,
+    # for every count of pieces in a row.
+    (8, 8192, 1024, 8192, False, True),   # a unit of eight rows or a tile on every workgroup
+    (1, 8209, 1024, 8209, True, False),   # a ragged last unit
+    (3, 5501, 1536, 5504, False, False),  # rows between the gate and the up rows
+    (11, 4101, 2048, 4101, True, True),   # two launches of tokens
+    (5, 3300, 2560, 3300, False, True),
+    (2, 2750, 3072, 2750, False, False),
+    (6, 2400, 3584, 2400, True, True),    # (bf16: the tokens' pieces do not fit workgroup memory)
+    (4, 2080, 4096, 2080, False, True),
+    (2, 41 * 32 * 256 + 50, 1024, 32, False, True),  # more than forty output tiles on a workgroup
+    (4, 600, 1024, 600, False, True),     # a small pair: the general kernel
+    (3, 2000, 4608, 2000, False, True),   # long rows: the general kernel
+])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_silu_pair(ctx_wide, half, m, n, k, half_row, accumulate, norm):
+    """SILU_PAIR steps in a context opened with ZHIP_OPTION_WIDE_DECODE: within 1e-5 of float64,
+    and a token's bits the same alone."""
+    c = ctx_wide
+    if n > 100000 and half == "f16":
+        pytest.skip("the long run of tiles is the formats' common code")
+    eps, scale = 1e-6, k ** -0.5
+    x = c.random(m * k, 3).reshape(m, k)
+    nw = c.random(k, 1)
+    bits, values = random_half(c, (half_row + n) * k, scale, half)
+    values = values.reshape(half_row + n, k)
+    init = c.random(m * n, 1 if accumulate else 0).reshape(m, n)
+    wa, na = c.upload(bits), c.upload(nw)
+
+    def run(tokens):
+        out = c.upload(init[tokens])
+        p = P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=eps, norm=norm, accumulate=accumulate, silu_pair=True, half=half_row)
+        c.launcher().launch(Kernel["matvec_" + half], p, [c.upload(x[tokens]), wa, out, na], (K.div_ceil(n, K.matvec_rows), len(tokens), 1))
+        return c.read(out).reshape(len(tokens), n)
+
+    got = run(list(range(m)))
+    v64 = values.astype(np.float64)
+    xs = np.stack([norm_row(x[t], nw if norm else None, eps) for t in range(m)])
+    prod = xs @ v64.T
+    g, u = prod[:, :n], prod[:, half_row:]
+    assert rel_err(got, init + g * sigmoid64(g) * u) <= 1e-5
+    for t in (0, m - 1):
+        assert np.array_equal(run([t])[0], got[t])
+
+
 def test_matvec_bf16_several_tokens_special_values(ctx_wide):
     """Inputs the three-way split must carry exactly: full 24-bit mantissas (integer inputs
     against weights of +-1, where every partial sum is an integer f32 holds, so the result is

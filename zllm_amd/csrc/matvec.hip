@@ -331,18 +331,23 @@ zhip_result launch_matvec_q3k_mfma_stream(const Dispatch &d, const MvArgs &a, ui
 // matvec_q8_0 over rows of 1024 weights in the same kernel: a tile's rows as one flat stretch.
 bool matvec_q8_0_mfma_flat_accepts(const MvArgs &a);
 zhip_result launch_matvec_q8_0_mfma_flat(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
-// Which matrices take it: 16 MB of weights or more (below, its fixed costs - the split of the
-// tokens, a workgroup's first tile - outweigh what it saves at every width: 8 MB, k = 1024: 6.4 /
-// 6.8 / 7.8 us at 2 / 4 / 8 tokens against 4.7 / 6.2 / 9.3) in contexts opened with
-// ZHIP_OPTION_WIDE_DECODE, and then at every width from one token on: the kernel sums in another
-// order than the general one, and a token's bits must not depend on the width of the step it
-// runs in (src/sched/sched.zig:55-58; src/plan/qwen35.zig:380-381), so the route is a property
-// of the matrix and of the context, never of the step. Its time hardly depends on the width
-// (151936 x 1024: 55 us at 1 ... 8 tokens; the general kernel 52 / 75 / 122 us at 1 / 4 / 8), so
-// a context pays ~6 % of a one-token step for verify steps at the one-token price.
+// Which matrices take it: 16 MB of weights or more, and gate / up pairs of 32 MB or more, in
+// contexts opened with ZHIP_OPTION_WIDE_DECODE, and then at every width from one token on: the
+// kernel sums in another order than the general one, and a token's bits must not depend on the
+// width of the step it runs in (src/sched/sched.zig:55-58; src/plan/qwen35.zig:380-381), so the
+// route is a property of the matrix and of the context, never of the step. Its time hardly
+// depends on the width, so a context pays a little of a one-token step for verify steps at the
+// one-token price. With the RMSNorm prologue, this kernel / the general one at 1, 2, 4, 8 tokens:
+//   4096 x 2048 (16 MB)          8.4 8.5 8.5 8.6 / 7.5 9.1 11.7 17.5 us
+//   3072 x 2048                  8.1 8.2 8.2 8.2 / 7.0 8.5 11.0 16.6
+//   4096 x 1024 (8 MB)           5.6 5.5 5.6 5.7 / 4.8 5.4 7.5 12.5
+//   2 x 4096 x 2048 (32 MB)      11.8 11.9 12.1 12.1 / 12.0 13.8 20.2 25.6
+//   2 x 8192 x 2048              17.3 17.3 17.0 17.4 / 16.1 20.5 28.5 39.2
+//   2 x 4096 x 1024 (16 MB)      7.7 7.7 7.8 7.8 / 6.9 9.7 14.3 24.9
 constexpr uint64_t kBf16StreamBytes = 16ull << 20;
 static bool bf16_stream_pays(const Dispatch &d, const MvArgs &a) {
-    return d.dev->wide_decode && (uint64_t)a.rows * a.row_bytes >= kBf16StreamBytes;
+    const uint64_t bytes = (uint64_t)a.rows * a.row_bytes;  // (of a pair: of its gate rows)
+    return d.dev->wide_decode && bytes >= kBf16StreamBytes;
 }
 // The tuned multiply (matvec_quant.h, a source file a format): type 3, 4, 5, 6 (K-quants) or 8 (Q8_0).
 zhip_result launch_matvec_quant(const Dispatch &d, const MvArgs &a, int type);

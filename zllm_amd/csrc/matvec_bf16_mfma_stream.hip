@@ -15,7 +15,8 @@
 // (steps of more than eight tokens run as launches of eight).
 //
 // Layout of the work. A 512-thread workgroup is eight waves that split k eight ways; a wave
-// builds its k range of all tokens' operand rows once, into registers (k / 32 VGPRs). Persistent
+// builds its k range of all tokens' operand rows once, into registers (k / 32 VGPRs), from the pieces that
+// the workgroup has put in LDS, a wave a token, or that a launch in front has left in memory. Persistent
 // workgroups take 32-row weight tiles b, b + G, ... and at the end a share of the rows left
 // over, in units of eight rows, so that every workgroup reads the same number of bytes within
 // one unit. A wave's part of a tile is k / 512 pieces, a piece one 128-byte line (64 positions)
@@ -56,6 +57,12 @@ constexpr uint32_t PART_BYTES = 2u * WAVES * 256u * 4u;  // [tile parity][wave][
 constexpr uint32_t KEPT = 40;                            // tiles whose outputs wait in LDS for one burst of stores
 constexpr uint32_t RING_BYTES = WAVES * DEPTH * SLOT;
 constexpr uint32_t LDS_BYTES = PART_BYTES + RING_BYTES + KEPT * 1024u + 64u;  // (the last 64: f16 tokens' inverse scales)
+// Kernels whose workgroups split their tokens themselves keep the pieces in LDS ([piece][token of
+// 8][k], rows padded by 16 bytes so that one chunk of neighbouring rows falls in different banks)
+// until the operands are read, at its end: ring slots below them take their weights meanwhile.
+template <int NP, bool F16> constexpr uint32_t piece_row() { return 1024u * NP + 16u; }
+template <int NP, bool F16> constexpr uint32_t pieces_bytes() { return (F16 ? 16u : 24u) * piece_row<NP, F16>(); }
+template <int NP, bool F16> constexpr bool pieces_fit() { return pieces_bytes<NP, F16>() <= LDS_BYTES - 64u; }
 static_assert(LDS_BYTES <= 160u * 1024u - 64u, "the rings must fit the CU's LDS");
 
 struct StreamArgs {
@@ -128,32 +135,70 @@ __device__ __forceinline__ uint32_t piece_bits(float x, uint32_t m0, uint32_t m1
 // The upper halves of two words as a pair of bf16 values, `lo` first.
 __device__ __forceinline__ uint32_t upper_halves(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
 
+// Piece p of four values.
+__device__ __forceinline__ uint2 bf16_piece(const float4 &v, uint32_t p) {
+    const uint32_t m0 = p == 0u ? ~0u : 0u, m1 = p == 1u ? ~0u : 0u, m2 = p == 2u ? ~0u : 0u;
+    uint2 w;
+    w.x = upper_halves(piece_bits(v.x, m0, m1, m2), piece_bits(v.y, m0, m1, m2));
+    w.y = upper_halves(piece_bits(v.z, m0, m1, m2), piece_bits(v.w, m0, m1, m2));
+    return w;
+}
+
+// The power of two that puts a token's largest magnitude `big` in [2^14, 2^15), and one over it.
+__device__ __forceinline__ void f16_scale(float big, float &scale, float &inverse) {
+    const int e = (int)((__float_as_uint(big) >> 23) & 0xffu);  // biased exponent; 0 for zero and subnormals
+    int se = 127 + 14 - (e - 127);                               // scale = 2^(14 - (e - 127)), kept normal both ways
+    se = se < 1 ? 1 : se > 253 ? 253 : se;
+    const bool unit = e == 0 || e == 255;
+    scale = unit ? 1.0f : __uint_as_float((uint32_t)se << 23);
+    inverse = unit ? 1.0f : __uint_as_float((uint32_t)(254 - se) << 23);
+}
+
+// Four scaled values as their f16 roundings and what those left times 2^11.
+__device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 &upper, uint2 &lower) {
+    const float x[4] = {v.x, v.y, v.z, v.w};
+    _Float16 hi[4], lo[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        // The scale is a power of two, so x * scale - hi in one fused operation is exact.
+        hi[j] = (_Float16)(x[j] * scale);
+        lo[j] = (_Float16)(fmaf(x[j], scale, -(float)hi[j]) * 2048.0f);
+    }
+    upper = __builtin_bit_cast(uint2, hf16x4{hi[0], hi[1], hi[2], hi[3]});
+    lower = __builtin_bit_cast(uint2, hf16x4{lo[0], lo[1], lo[2], lo[3]});
+}
+
 // NP: pieces of a wave's k range (k = 512 NP). SPLIT: the tokens' three pieces come ready from
-// matvec_bf16_split_kernel's planes. A workgroup that splits its tokens itself spends 12 vector
-// operations a value on it, four lanes on the same value (the lanes of the three pieces and of
-// the zero rows): 1.5 us of a launch at k = 1024, less than another launch costs, but 12 us at
-// k = 4096.
+// matvec_bf16_split_kernel's planes (long rows, and where the pieces do not fit LDS). Otherwise
+// every workgroup normalises and splits the tokens itself, a wave each, through LDS: 1 us of the
+// workgroup's time where a launch in front costs 3 (8 tokens with the RMSNorm prologue: f16 4096 x
+// 2048 11.6 -> 8.6 us, 151936 x 1024 56.7 -> 52.9, 4096 x 4096 17.9 -> 13.1; bf16 12.4 -> 8.8,
+// 56.1 -> 53.3).
 // F16 (matvec_f16: the weights are f16 and the matrix instruction v_mfma_f32_32x32x16_f16): a
 // token enters as two f16 rows, the rounding of its inputs and the rounding of what that left
 // times 2^11, after a power of two has put its largest magnitude at 2^14 (an input keeps 22
-// bits); the planes come from matvec_f16_split_kernel, and a token's sums are multiplied by one
+// bits), and a token's sums are multiplied by one
 // over its scale.
+// PAIR: a SILU_PAIR step, an output tile's gate rows and then its up rows (the general kernel's
+// time grows with the tokens: 2 x 8192 x 2048 f16 at eight 39 us, here 17).
 // LONG: k = 512 NP q.parts; workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
 // walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums.
-template <int NP, bool SPLIT, bool F16, bool LONG>
+template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
 __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(StreamArgs q) {
-    static_assert(SPLIT || !F16, "f16 tokens are always split beforehand");
+    static_assert(SPLIT || pieces_fit<NP, F16>(), "the tokens' pieces must fit LDS");
     static_assert(SPLIT || !LONG, "the stretches of a long row read the tokens from the planes");
+    static_assert(!PAIR || !LONG, "gate / up steps take whole rows");
+    constexpr uint32_t PER = PAIR ? 2u : 1u;  // weight tiles an output tile
     constexpr uint32_t PIECES = F16 ? 2u : 3u;
     const MvArgs &a = q.a;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *lds_part = reinterpret_cast<float *>(lds);
     float *lds_kept = reinterpret_cast<float *>(lds + PART_BYTES + RING_BYTES);  // [tile % KEPT][token][row]
     float *lds_inverse = lds_kept + KEPT * 256u;                                 // [token], read behind the tiles' barriers
-    if (F16 && threadIdx.x < 8u) lds_inverse[threadIdx.x] = threadIdx.x < a.m ? q.inverse[q.t0 + threadIdx.x] : 1.0f;
+    if (F16 && SPLIT && threadIdx.x < 8u) lds_inverse[threadIdx.x] = threadIdx.x < a.m ? q.inverse[q.t0 + threadIdx.x] : 1.0f;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    uint8_t *ring = lds + PART_BYTES + wave * (DEPTH * SLOT);
+    uint8_t *ring = lds + PART_BYTES + wave * SLOT;  // [slot][wave]
     const uint32_t ring0 = (uint32_t)(uintptr_t)ring;
     const __amdgpu_buffer_rsrc_t wbuf = make_buffer(a.w, q.w_bytes), nobuf = make_buffer(a.w, 0);
 
@@ -167,8 +212,8 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     const uint32_t tail_units = q.tail_base + (b < q.tail_rem ? 1u : 0u);
     const uint32_t tail_row = 32u * q.rounds * G + 8u * (b * q.tail_base + (b < q.tail_rem ? b : q.tail_rem));
     const uint32_t count = q.rounds + (tail_units ? 1u : 0u);
-    auto first_row = [&](uint32_t p) { return p < q.rounds ? 32u * (b + p * G) : tail_row; };
-    auto rows_of = [&](uint32_t p) { return p < q.rounds ? 32u : 8u * tail_units; };
+    auto first_row = [&](uint32_t o) { return o < q.rounds ? 32u * (b + o * G) : tail_row; };
+    auto rows_of = [&](uint32_t o) { return o < q.rounds ? 32u : 8u * tail_units; };
 
     // A piece's loads: load j brings rows 8 j .. 8 j + 7, lane l row 8 j + l / 8 and the chunk
     // that belongs at position l % 8 of its line. The whole address is the lane's offset, which
@@ -182,9 +227,10 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
         // (past the run's last piece the loads still run, so that the waits count the same loads
         // every step, but against an empty buffer: zeros land and nothing is fetched; the same
         // for the rows a share of the last rows does not have)
-        const __amdgpu_buffer_rsrc_t buf = load_tile < count ? wbuf : nobuf;
-        const uint32_t base = first_row(load_tile) * a.row_bytes + 128u * load_piece, rows = rows_of(load_tile);
-        const uint32_t dst = ring0 + load_slot * SLOT;
+        const uint32_t o = load_tile / PER;
+        const __amdgpu_buffer_rsrc_t buf = o < count ? wbuf : nobuf;
+        const uint32_t base = (first_row(o) + (PAIR && (load_tile & 1u) ? a.half : 0u)) * a.row_bytes + 128u * load_piece, rows = rows_of(o);
+        const uint32_t dst = ring0 + load_slot * (WAVES * SLOT);
 #pragma unroll
         for (int j = 0; j < LOADS; j++) load_lds_b128(8u * j < rows ? buf : nobuf, dst + 1024u * j, woff[j] + base);
         load_piece = load_piece + 1u == (uint32_t)NP ? 0u : load_piece + 1u;
@@ -202,10 +248,6 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     const uint32_t rho = lane & 31u, kap = lane >> 5;
     const uint32_t tok = 4u * ((rho >> 2) & 1u) + (rho & 3u), piece = rho >> 3;
     const bool live = tok < a.m && piece < PIECES;
-    // (masks, so that picking the lane's piece is two instructions a value and not a branch)
-    uint32_t m0 = live && piece == 0u ? ~0u : 0u, m1 = live && piece == 1u ? ~0u : 0u, m2 = live && piece == 2u ? ~0u : 0u;
-    asm volatile("" : "+v"(m0), "+v"(m1), "+v"(m2));
-    const float *xt = a.x + (size_t)(tok < a.m ? tok : a.m - 1u) * a.xr + 64u * NP * wave + 8u * kap;
     hu32x4 xf[4 * NP];
     if constexpr (SPLIT) {
         // Every step's operand is sixteen bytes of a plane; the lanes of absent tokens and of
@@ -215,35 +257,72 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
 #pragma unroll
         for (int s = 0; s < 4 * NP; s++) xf[s] = __builtin_bit_cast(hu32x4, __builtin_amdgcn_raw_buffer_load_b128(pbuf, live ? at + 32u * s : at, 0, 0));
         issue();
-    } else
 #pragma unroll
-    for (int s0 = 0; s0 < 4 * NP; s0 += 8) {
-        float4 raw[16];
+        for (int s = 1; s < DEPTH - 1; s++) issue();
+    } else {
+        // Wave w takes token w, lane l its vectors l, l + 64, ... (a wave without a token reads an
+        // empty buffer). A token's values depend on nothing but its inputs.
+        constexpr uint32_t ROW = piece_row<NP, F16>(), PIECES_AT = (LDS_BYTES - 64u - pieces_bytes<NP, F16>()) & ~15u;
+        constexpr uint32_t FREE = PIECES_AT < PART_BYTES ? 0u : (PIECES_AT - PART_BYTES) / (WAVES * SLOT);
+        constexpr int EARLY = FREE < DEPTH - 1 ? FREE : DEPTH - 1;  // pieces of weights asked for meanwhile
+        const __amdgpu_buffer_rsrc_t xbuf = make_buffer(a.x + (wave < a.m ? (size_t)wave * a.xr : 0u), wave < a.m ? 4u * a.k : 0u);
+        const __amdgpu_buffer_rsrc_t gbuf = make_buffer(a.norm_w, (a.flags & FLAG_NORM) && wave < a.m ? 4u * a.k : 0u);
+        float4 v[2 * NP], g[2 * NP];
 #pragma unroll
-        for (int s = 0; s < 8 && s0 + s < 4 * NP; s++) {
-            raw[2 * s] = *reinterpret_cast<const float4 *>(xt + 16 * (s0 + s));
-            raw[2 * s + 1] = *reinterpret_cast<const float4 *>(xt + 16 * (s0 + s) + 4);
+        for (int j = 0; j < 2 * NP; j++) v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, 16u * (lane + 64u * j), 0, 0));
+        if (a.flags & FLAG_NORM) {
+#pragma unroll
+            for (int j = 0; j < 2 * NP; j++) g[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(gbuf, 16u * (lane + 64u * j), 0, 0));
         }
-        // (One piece of weights behind them for now: with more, the requests of the workgroups
-        // that start first fill the memory system's queues and the inputs of the others arrive
-        // after them.)
-        if (s0 == 0) issue();
 #pragma unroll
-        for (int s = 0; s < 8 && s0 + s < 4 * NP; s++) {
-            const float x[8] = {raw[2 * s].x, raw[2 * s].y, raw[2 * s].z, raw[2 * s].w, raw[2 * s + 1].x, raw[2 * s + 1].y, raw[2 * s + 1].z, raw[2 * s + 1].w};
-            hu32x4 words;
+        for (int s = 0; s < EARLY; s++) issue();
+        if (a.flags & FLAG_NORM) {
+            float ss = 0.f;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                words[e] = upper_halves(piece_bits(x[2 * e], m0, m1, m2), piece_bits(x[2 * e + 1], m0, m1, m2));
+            for (int j = 0; j < 2 * NP; j++) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+            const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)a.k + a.eps);
+#pragma unroll
+            for (int j = 0; j < 2 * NP; j++) {
+                v[j].x = v[j].x * scale * g[j].x; v[j].y = v[j].y * scale * g[j].y;
+                v[j].z = v[j].z * scale * g[j].z; v[j].w = v[j].w * scale * g[j].w;
             }
-            xf[s0 + s] = words;
         }
-        // (a batch's loads are not to be requested before the batch before is in its operands:
-        // all of them at once would need more registers than a lane has)
-        asm volatile("" ::: "memory");
-    }
+        uint8_t *mine = lds + PIECES_AT + wave * ROW;
+        if constexpr (F16) {
+            float big = 0.f;
 #pragma unroll
-    for (int s = 1; s < DEPTH - 1; s++) issue();
+            for (int j = 0; j < 2 * NP; j++) big = fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fmaxf(fabsf(v[j].z), fabsf(v[j].w)), big));
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off, 64));
+            float scale, inverse;
+            f16_scale(big, scale, inverse);
+            if (lane == 0) lds_inverse[wave] = inverse;
+#pragma unroll
+            for (int j = 0; j < 2 * NP; j++) {
+                uint2 hi, lo;
+                f16_pieces(v[j], scale, hi, lo);
+                *reinterpret_cast<uint2 *>(mine + 8u * (lane + 64u * j)) = hi;
+                *reinterpret_cast<uint2 *>(mine + 8u * ROW + 8u * (lane + 64u * j)) = lo;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2 * NP; j++) {
+#pragma unroll
+                for (uint32_t p = 0; p < 3u; p++) *reinterpret_cast<uint2 *>(mine + 8u * p * ROW + 8u * (lane + 64u * j)) = bf16_piece(v[j], p);
+            }
+        }
+        lds_barrier();
+        const uint8_t *from = lds + PIECES_AT + ((live ? 8u * piece + tok : 0u) * ROW) + 2u * (64u * NP * wave + 8u * kap);
+#pragma unroll
+        for (int s = 0; s < 4 * NP; s++) {
+            const hu32x4 w = *reinterpret_cast<const hu32x4 *>(from + 32u * s);
+#pragma unroll
+            for (int e = 0; e < 4; e++) xf[s][e] = live ? w[e] : 0u;
+        }
+        lds_barrier();  // (the ring, the partial sums and the kept outputs lie where the pieces were)
+#pragma unroll
+        for (int s = EARLY; s < DEPTH - 1; s++) issue();
+    }
 
     // The lane's reads of a piece: row rho, chunk 2 s + kap of its line for step s.
     uint32_t r_at[4];
@@ -266,10 +345,12 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
 #pragma unroll
             for (uint32_t wv = 1; wv < WAVES; wv++) total += src[wv * 256u];
             if (F16) total *= lds_inverse[tk];
-            lds_kept[256u * (p % KEPT) + 32u * tk + row] = total;
+            // (PAIR: the gate tile's output waits here for the up tile's, a barrier later)
+            float *kept = lds_kept + 256u * (p / PER % KEPT) + 32u * tk + row;
+            *kept = PAIR && (p & 1u) ? silu_f(*kept) * total : total;
         }
     };
-    // The outputs of tiles first .. first + n - 1, from LDS to memory: 128 contiguous bytes a
+    // The outputs of output tiles first .. first + n - 1, from LDS to memory: 128 contiguous bytes a
     // token and tile. (Stored tile by tile between the loads they took 2 us of a 55 us launch
     // longer than in one burst: every isolated write turns the memory's direction around.)
     auto store_kept = [&](uint32_t first, uint32_t n) __attribute__((always_inline)) {
@@ -290,7 +371,7 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     // inside). Before a piece is read, all but the loads of the DEPTH - 1 pieces after it have
     // landed.
     uint32_t slot = 0;
-    for (uint32_t p = 0; p < count; p++) {
+    for (uint32_t p = 0; p < PER * count; p++) {
         hf32x16 sum;
 #pragma unroll
         for (int e = 0; e < 16; e++) sum[e] = 0.f;
@@ -302,7 +383,7 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             issue();
             wait_loads<(DEPTH - 1) * LOADS>();
-            const uint8_t *t = ring + slot * SLOT;
+            const uint8_t *t = ring + slot * (WAVES * SLOT);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 const hu32x4 w = *reinterpret_cast<const hu32x4 *>(t + r_at[s]);
@@ -317,7 +398,8 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
         finish(p, sum);
         // (the next tile's sums are kept only behind its barrier, which no thread passes before
         // it has stored what it stores here)
-        if ((p + 1u) % KEPT == 0u || p + 1u == count) store_kept(p - p % KEPT, p % KEPT + 1u);
+        const uint32_t o = p / PER;
+        if ((!PAIR || (p & 1u)) && ((o + 1u) % KEPT == 0u || o + 1u == count)) store_kept(o - o % KEPT, o % KEPT + 1u);
     }
     wait_loads<0>();  // nothing may still land in LDS once the workgroup is gone
 }
@@ -333,13 +415,7 @@ __global__ __launch_bounds__(256) void matvec_bf16_split_kernel(MvArgs a, uint2 
     for (uint32_t i = threadIdx.x; i < k4; i += 256u) {
         const float4 v = staged[i];
 #pragma unroll
-        for (uint32_t piece = 0; piece < 3u; piece++) {
-            const uint32_t m0 = piece == 0u ? ~0u : 0u, m1 = piece == 1u ? ~0u : 0u, m2 = piece == 2u ? ~0u : 0u;
-            uint2 w;
-            w.x = upper_halves(piece_bits(v.x, m0, m1, m2), piece_bits(v.y, m0, m1, m2));
-            w.y = upper_halves(piece_bits(v.z, m0, m1, m2), piece_bits(v.w, m0, m1, m2));
-            planes[(size_t)(piece * gridDim.x + blockIdx.x) * k4 + i] = w;
-        }
+        for (uint32_t piece = 0; piece < 3u; piece++) planes[(size_t)(piece * gridDim.x + blockIdx.x) * k4 + i] = bf16_piece(v, piece);
     }
 }
 
@@ -362,30 +438,15 @@ __global__ __launch_bounds__(256) void matvec_f16_split_kernel(MvArgs a, uint2 *
     if ((tid & 63u) == 0) red[tid >> 6] = big;
     __syncthreads();
     big = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const int e = (int)((__float_as_uint(big) >> 23) & 0xffu);  // biased exponent; 0 for zero and subnormals
-    int se = 127 + 14 - (e - 127);                               // scale = 2^(14 - (e - 127)), kept normal both ways
-    se = se < 1 ? 1 : se > 253 ? 253 : se;
-    const bool unit = e == 0 || e == 255;
-    const float scale = unit ? 1.0f : __uint_as_float((uint32_t)se << 23);
-    if (tid == 0) inverse[blockIdx.x] = unit ? 1.0f : __uint_as_float((uint32_t)(254 - se) << 23);
-    for (uint32_t i = tid; i < k4; i += 256u) {
-        const float4 v = staged[i];
-        const float x[4] = {v.x, v.y, v.z, v.w};
-        _Float16 hi[4], lo[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            // The scale is a power of two, so x * scale - hi in one fused operation is exact.
-            hi[j] = (_Float16)(x[j] * scale);
-            lo[j] = (_Float16)(fmaf(x[j], scale, -(float)hi[j]) * 2048.0f);
-        }
-        planes[(size_t)blockIdx.x * k4 + i] = __builtin_bit_cast(uint2, hf16x4{hi[0], hi[1], hi[2], hi[3]});
-        planes[(size_t)(gridDim.x + blockIdx.x) * k4 + i] = __builtin_bit_cast(uint2, hf16x4{lo[0], lo[1], lo[2], lo[3]});
-    }
+    float scale, inv;
+    f16_scale(big, scale, inv);
+    if (tid == 0) inverse[blockIdx.x] = inv;
+    for (uint32_t i = tid; i < k4; i += 256u) f16_pieces(staged[i], scale, planes[(size_t)blockIdx.x * k4 + i], planes[(size_t)(gridDim.x + blockIdx.x) * k4 + i]);
 }
 
-template <int NP, bool SPLIT, bool F16, bool LONG = false>
+template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
 zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
-    auto kernel = matvec_bf16_mfma_stream_kernel<NP, SPLIT, F16, LONG>;
+    auto kernel = matvec_bf16_mfma_stream_kernel<NP, SPLIT, F16, LONG, PAIR>;
     static bool configured = false;
     if (!configured) {
         if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) != hipSuccess) {
@@ -401,24 +462,25 @@ zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
 }  // namespace
 
 // Whether this kernel can run the (already validated) arguments: k split into whole lines a
-// wave, no pair.
+// wave; a gate / up pair only over rows that one workgroup takes whole.
 // (rows of more than 4096 weights are taken in stretches of columns: equal ones in one launch, workgroups sharing a
 // tile, with a launch for their sums; unequal ones a launch each; up to 16384: the split launch stages a token in 64 KB of LDS)
 bool matvec_bf16_mfma_stream_accepts(const MvArgs &a) {
-    return a.m >= 1 && a.k >= 1024u && a.k <= 16384u && a.k % 512u == 0 && !(a.flags & FLAG_SILU_PAIR) && a.act_div == 0.f && a.rows >= 1 &&
+    if ((a.flags & FLAG_SILU_PAIR) && (a.k > 4096u || ((uint64_t)a.half + a.rows + 64u) * a.row_bytes >= 0xfffffff0ull)) return false;
+    return a.m >= 1 && a.k >= 1024u && a.k <= 16384u && a.k % 512u == 0 && a.act_div == 0.f && a.rows >= 1 &&
            a.xr % 4u == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0 && a.row_bytes == 2u * a.k;
 }
 
-template <bool SPLIT, bool F16, bool LONG = false>
+template <bool SPLIT, bool F16, bool LONG = false, bool PAIR = false>
 static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 grid) {
     switch (q.a.k / 512u) {
-    case 2: return launch_blocks<2, SPLIT, F16, LONG>(d, q, grid);
-    case 3: return launch_blocks<3, SPLIT, F16, LONG>(d, q, grid);
-    case 4: return launch_blocks<4, SPLIT, F16, LONG>(d, q, grid);
-    case 5: return launch_blocks<5, SPLIT, F16, LONG>(d, q, grid);
-    case 6: return launch_blocks<6, SPLIT, F16, LONG>(d, q, grid);
-    case 7: return launch_blocks<7, SPLIT, F16, LONG>(d, q, grid);
-    default: return launch_blocks<8, SPLIT, F16, LONG>(d, q, grid);
+    case 2: return launch_blocks<2, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    case 3: return launch_blocks<3, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    case 4: return launch_blocks<4, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    case 5: return launch_blocks<5, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    case 6: return launch_blocks<6, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    case 7: return launch_blocks<7, SPLIT || !pieces_fit<7, F16>(), F16, LONG, PAIR>(d, q, grid);
+    default: return launch_blocks<8, SPLIT || !pieces_fit<8, F16>(), F16, LONG, PAIR>(d, q, grid);
     }
 }
 
@@ -426,7 +488,8 @@ static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 gri
 zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16) {
     const char *name = f16 ? "matvec_f16" : "matvec_bf16";
     // 32-bit byte offsets, a tile past the last row.
-    const uint64_t used = (uint64_t)a.rows * a.row_bytes;
+    const bool pair = a.flags & FLAG_SILU_PAIR;
+    const uint64_t used = ((uint64_t)a.rows + (pair ? a.half : 0u)) * a.row_bytes;
     if (used + 64ull * a.row_bytes >= 0xfffffff0ull) return fail(d, ZHIP_E_BAD_COMMAND, "%s: weights of 4 GiB or more", name);
     const uint32_t cus = (uint32_t)d.dev->compute_units;
     const uint32_t units = (a.rows + 7u) / 8u;
@@ -434,12 +497,9 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
     const uint32_t rounds = (a.rows / 32u) / groups;
     const uint32_t tail = (a.rows - 32u * rounds * groups + 7u) / 8u;
     StreamArgs q{a, (uint32_t)(used < w_bytes ? used : w_bytes), rounds, tail / groups, tail % groups, groups % 8u == 0 ? 1u : 0u, nullptr, 0u, 0u, 0u, 0u, nullptr, 1u, nullptr};
-    // The tokens are split (and normalised) by a launch of their own where that is cheaper than
-    // every workgroup splitting them again, and wherever the step carries the RMSNorm prologue
-    // (the workgroups computing the norm themselves at k = 1024 measured the same: 151936 x 1024
-    // at 2 / 4 / 8 tokens 53.3 / 54.1 / 56.3 us against 54.2 / 54.2 / 55.5 us this way). f16
-    // tokens, which need their scales first, always.
-    const bool split = f16 || (a.flags & FLAG_NORM) || a.k >= 2048u;
+    // The tokens are split (and normalised) by a launch of their own for rows taken in stretches
+    // (no workgroup sees a whole token), and for bf16 rows whose pieces do not fit LDS.
+    const bool split = a.k > (f16 ? 4096u : 3072u);
     // Rows of more than 4096 weights (the FFN-down shapes; the general kernel takes them token by
     // token) go in stretches of up to 4096 columns. Stretches of equal length (14336 = 4 x 3584,
     // 8192 = 2 x 4096 ...) go out as one launch: `launches` workgroups share a walker's tiles, a
@@ -498,10 +558,19 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
             q.a.out = a.out + (size_t)t0 * a.out_stride;
             q.a.m = a.m - t0 < 8u ? a.m - t0 : 8u;
             q.a.flags = (a.flags & ~FLAG_NORM & ~FLAG_ACCUMULATE) | ((c || (a.flags & FLAG_ACCUMULATE)) ? FLAG_ACCUMULATE : 0u);
-            if (!split) q.a.flags = a.flags;
+            if (!split) {
+                q.a.flags = a.flags;
+                q.a.norm_w = a.norm_w;
+            }
             q.t0 = t0;
             q.plane_first = first;
-            if (zhip_result r = f16 ? launch_for_k<true, true>(d, q, grid) : split ? launch_for_k<true, false>(d, q, grid) : launch_for_k<false, false>(d, q, grid)) return r;
+            zhip_result r;
+            if (pair) {
+                if (f16) r = launch_for_k<false, true, false, true>(d, q, grid);  // (a pair's rows are at most 4096 weights)
+                else r = split ? launch_for_k<true, false, false, true>(d, q, grid) : launch_for_k<false, false, false, true>(d, q, grid);
+            } else if (f16) r = split ? launch_for_k<true, true>(d, q, grid) : launch_for_k<false, true>(d, q, grid);
+            else r = split ? launch_for_k<true, false>(d, q, grid) : launch_for_k<false, false>(d, q, grid);
+            if (r != ZHIP_OK) return r;
             first += q.a.k;
         }
     }
