@@ -187,6 +187,42 @@ def test_matvec_bf16_several_tokens_keep_token_bits(ctx, ctx_wide, wide, half):
     assert np.array_equal(run([5], 404, 4096)[0], whole[5, 404:])
 
 
+# Steps of one to eight tokens over short rows keep the inputs in registers; more than eight tokens
+# run in the general kernel, which adds in the same order: each token has its bits there.
+@pytest.mark.parametrize("k,n", [
+    (8, 5), (504, 3), (512, 2051), (520, 37),         # one task, a ragged and a whole 64, one task more
+    (1016, 2049), (1024, 4099), (1032, 100),          # the longest rows for eight tokens; two rows a pass
+    (2048, 1030), (2056, 67),                         # ... for four
+    (3072, 999), (3080, 64), (4096, 2100),            # ... for two
+    (5120, 1025), (5128, 33),                         # ... for one; the general kernel
+])
+@pytest.mark.parametrize("half", HALVES)
+@pytest.mark.parametrize("pair", [False, True])
+def test_matvec_half_rows_in_registers(ctx, half, pair, k, n):
+    c, eps, most, col0 = ctx, 1e-6, 11, 3
+    stride, gap = n + 8, 2 if pair else 0
+    x, nw = c.random(most * k, 3).reshape(most, k), c.random(k, 1)
+    bits, values = random_half(c, (2 * n + gap if pair else n) * k, 1, half)
+    init = c.random(most * stride, 4).reshape(most, stride)
+    wa, na = c.upload(bits), c.upload(nw)
+
+    def run(m, norm, accumulate):
+        out = c.upload(init[:m])
+        c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=n, k=k, col0=col0, out_stride=stride, eps=eps, norm=norm, accumulate=accumulate, silu_pair=pair, half=n + gap if pair else 0),
+                            [c.upload(x[:m]), wa, out, na], (K.div_ceil(n, K.matvec_rows), m, 1))
+        return c.read(out).reshape(m, stride)
+
+    for norm, accumulate in ((False, False), (True, True)):
+        whole = run(most, norm, accumulate)
+        for m in (1, 2, 3, 4, 5, 8):
+            assert np.array_equal(run(m, norm, accumulate), whole[:m])
+        w = values.reshape(-1, k).astype(np.float64)
+        xs = np.stack([norm_row(x[t], nw if norm else None, eps) for t in range(most)])
+        want, g = init.astype(np.float64), xs @ w[:n].T
+        want[:, col0 : col0 + n] = (g * sigmoid64(g) * (xs @ w[n + gap :].T) if pair else g) + (want[:, col0 : col0 + n] if accumulate else 0.0)
+        assert rel_err(whole, want) <= 1e-5
+
+
 @pytest.mark.parametrize("m,n,k,half_row,accumulate,norm", [
     # 16 MB of gate rows and more: the matrix cores, a tile of gate rows and then one of up rows,
     # for every count of pieces in a row.

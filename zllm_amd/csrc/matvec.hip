@@ -57,8 +57,8 @@ __global__ __launch_bounds__(256) void matvec_kernel(MvArgs a) {
             // positions in flight while it multiplies the current one (past its last position
             // the loads are clamped to a valid one and their data unused).
             constexpr int TG = MT < 4 ? MT : 4;
-            // (a lone token on short rows measured no faster that way: 3072 x 1024, 4.2 against 4.5 us)
-            const bool early = a.k <= 4096u && (MT > 1 || DEPTH > 1);
+            // (a lone token gets here with longer rows only: matvec_half_row.hip takes the others)
+            const bool early = MT > 1 && a.k <= 4096u;
             const uint32_t iters = (tasks + 63u) / 64u;
             auto place = [k4](uint32_t i) { return (i & 1u) * (k4 / 2u) + (i >> 1); };
             float4 xv[TG][4], gv[4];
@@ -349,6 +349,9 @@ static bool bf16_stream_pays(const Dispatch &d, const MvArgs &a) {
     const uint64_t bytes = (uint64_t)a.rows * a.row_bytes;  // (of a pair: of its gate rows)
     return d.dev->wide_decode && bytes >= kBf16StreamBytes;
 }
+// The 16-bit formats with the inputs in registers, one to eight tokens (matvec_half_row.hip).
+bool matvec_half_row_accepts(const MvArgs &a);
+zhip_result launch_matvec_half_row(const Dispatch &d, const MvArgs &a, bool f16);
 // The tuned multiply (matvec_quant.h, a source file a format): type 3, 4, 5, 6 (K-quants) or 8 (Q8_0).
 zhip_result launch_matvec_quant(const Dispatch &d, const MvArgs &a, int type);
 
@@ -356,8 +359,8 @@ template <class D, int MT>
 static zhip_result run(const Dispatch &d, const MvArgs &a, uint32_t lds_bytes) {
     static bool configured[2] = {false, false};  // dynamic LDS above 64 KiB needs opting in once, kernel by kernel
     // Long rows of a matrix of few rows: a wave has few positions, each a trip to memory; four
-    // in flight instead of one (1024 x 3072 bf16, one token: 6.3 -> 5.1 us). Elsewhere the
-    // registers that takes cost more than it gains (151936 x 1024: 52 -> 62 us).
+    // in flight instead of one (1024 x 3072 bf16, eight tokens in passes of four: 9.0 -> 7.4 us a pass).
+    // Elsewhere the registers that takes cost more than it gains (151936 x 1024: 52 -> 62 us).
     const bool deep = kSplitInputs<D> && a.k >= 2048u && (uint64_t)a.rows * a.row_bytes <= (64ull << 20);
     auto kernel = deep ? matvec_kernel<D, MT, kSplitInputs<D> ? 4 : 1> : matvec_kernel<D, MT, 1>;
     if (lds_bytes > 65536u && !configured[deep]) {
@@ -432,6 +435,9 @@ static zhip_result launch_matvec(const Dispatch &d, bool quant) {
     // the kernel that reads the weights once for all of a step's tokens.
     if ((std::is_same<D, DecBF16>::value || std::is_same<D, DecF16>::value) && bf16_stream_pays(d, a) && matvec_bf16_mfma_stream_accepts(a))
         return launch_matvec_bf16_mfma_stream(d, a, d.bind[2].size, std::is_same<D, DecF16>::value);
+    // Everything else of a few tokens over rows that fit the registers; the general kernel, with its
+    // inputs in LDS, adds in the same order and lost on every shape measured (figures there).
+    if (kSplitInputs<D> && matvec_half_row_accepts(a)) return launch_matvec_half_row(d, a, std::is_same<D, DecF16>::value);
 
     // MatvecVariant (wg 512, lanes 64, rows 16) names the matrix-core variants: a wave per sixteen rows.
     const bool matrix_cores = quant && v.lanes == 64u && v.rows == 16u && (D::CHUNK == 4 || D::CHUNK == 8 || D::CHUNK == 6 || D::CHUNK == 5 || D::CHUNK == 3);

@@ -22,10 +22,25 @@ struct MvArgs {
     float act_div;       // > 0: inputs staged as silu(x / act_div)
 };
 
+// The sum over a wave's lanes, in every lane: pairs 32, 16, 8, 4, 2 and 1 lanes apart, in that
+// order. Nothing goes through LDS: the halves and the rows of sixteen trade places
+// (v_permlane32_swap, v_permlane16_swap), the rest are DPP operands of the additions. A rotation
+// by four reaches the lane four apart or the one four and eight apart, and after the step
+// before those two hold the same sum. Six trips to LDS one after the other (ds_bpermute, what
+// __shfl_xor compiles to) take about 0.3 us of a launch that lasts four.
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float v) {
+    return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+    v = add_dpp<0x128>(v);  // row_ror:8
+    v = add_dpp<0x124>(v);  // row_ror:4
+    v = add_dpp<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+    return add_dpp<0xB1>(v);  // quad_perm [1, 0, 3, 2]
 }
 
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
