@@ -43,6 +43,33 @@ def test_new_buffers_read_as_zero_and_round_trip(ctx):
     assert np.array_equal(got[100:110], data[:10]) and np.array_equal(got[:100], data[:100])
 
 
+@pytest.mark.parametrize("words", [1, 3, 4, 16383, 16384, 16385, 131072, 131073, 262144, 2300000])
+def test_transfers_of_every_length(ctx, words):
+    """Short writes and reads go through pinned memory and long ones otherwise (64 KB), the longest
+    reads in pieces (512 KB; a sixteenth above 8 MB): every length and alignment arrives whole,
+    overlapping writes land in their order, and a batch without a submit has landed when it returns."""
+    c = ctx
+    old, new = c.random(words, 1), c.random(words, 1)
+    buf = c.output(words + 5)
+    c.rec.write_buffer(buf.buffer, 4, old)     # (not on sixteen bytes)
+    part = new[: max(1, words // 2)]
+    c.rec.write_buffer(buf.buffer, 4, part)    # over what the write before it leaves
+    c.host.execute(c.rec.batch(), [])          # no submit
+    c.rec.clear()
+    c.rec.write_buffer(buf.buffer, 0, new[:1])
+    for i in range(40):                        # more than the pinned memory holds at once
+        c.rec.write_buffer(buf.buffer, 4, old[: min(words, 16000)] if i % 2 == 0 else part[:16000])
+    want = np.concatenate([new[:1], old, np.zeros(4, np.float32)])
+    want[1 : 1 + part.size] = part
+    want[1 : 1 + min(words, 16000)] = old[:16000]
+    want[1 : 1 + part[:16000].size] = part[:16000]
+    whole, tail = np.zeros(words + 5, np.float32), np.zeros(words, np.float32)
+    c.rec.read_buffer(901, buf.buffer, 0, whole)
+    c.rec.read_buffer(902, buf.buffer, 4, tail)
+    c.flush()
+    assert np.array_equal(whole, want) and np.array_equal(tail, want[1 : 1 + words])
+
+
 def test_writes_land_before_work_recorded_ahead_of_them(ctx):
     """write_buffer lands before the next submit's work, even work recorded
     ahead of it (src/gpu/cmd.zig:24-25, src/agility/host.zig:4-8)."""

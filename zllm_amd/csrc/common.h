@@ -166,5 +166,7 @@ zhip_result no_alloc_matmul_q8_0_float(int device, hipStream_t stream, const flo
 // Fills `words` 32-bit words at dst with `value` on the stream (clear_buffer;
 // also used instead of memset nodes so a captured stream stays replayable).
 zhip_result launch_fill(hipStream_t stream, void *dst, uint64_t words, uint32_t value);
+// Copies `bytes` (a multiple of 4; both ends 4-byte aligned) between device and pinned host memory.
+zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t bytes);
 
 }  // namespace zhip

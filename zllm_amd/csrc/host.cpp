@@ -265,6 +265,13 @@ struct zhip_context {
     std::vector<uint32_t> released;
     uint8_t *download = nullptr;  // pinned
     uint64_t download_size = 0;
+    std::vector<hipEvent_t> read_events;  // one behind each piece of a long read
+
+    // Small writes wait here, pinned, for the copy kernel queued for each on the stream;
+    // upload_used bytes of it are taken, and nothing is in flight when that is 0.
+    uint8_t *upload = nullptr;
+    uint64_t upload_used = 0;
+    bool null_stream_work = false;  // a memset or copy on the null stream since it was last waited for
 
     const uint8_t *file = nullptr;
     size_t file_len = 0;
@@ -332,9 +339,56 @@ void drop_pending(zhip_context *c) {
     c->read_bytes = 0;
 }
 
+// ---- small transfers -------------------------------------------------------------------
+// A synchronous hipMemcpy of a step's token ids or of a lone projection's input costs 13 us,
+// a third of the shortest submit. Writes of up to kStagedWrite bytes are taken into pinned memory
+// as they are decoded and copied by a small kernel on the stream, ahead of whatever is
+// launched there later (2 us of host time). They never outlast the batch: zhip_execute and
+// everything that does not order against the stream waits for them first.
+constexpr uint64_t kStagedWrite = 64u << 10, kUploadBytes = 4 * kStagedWrite;
+// Reads of up to this many bytes are a kernel's stores to pinned memory too.
+constexpr uint64_t kSmallRead = 64u << 10;
+// Longer reads than this arrive in pieces, each handed to its destination while the next ones
+// cross the bus: 8 MB (512 tokens of 4096 values) take 150 us to arrive and 285 us to hand over.
+constexpr uint64_t kReadPiece = 512u << 10, kMostPieces = 16;
+
+zhip_result finish_writes(zhip_context *c) {
+    if (c->upload_used == 0) return ZHIP_OK;
+    c->upload_used = 0;
+    return hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+}
+
+// Host memory to a buffer, before the next submit's work; `what` names the command.
+zhip_result write_device(zhip_context *c, uint8_t *dst, const void *src, uint64_t len, const char *what) {
+    if (len <= kStagedWrite && !c->upload && hipHostMalloc(reinterpret_cast<void **>(&c->upload), kUploadBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->upload = nullptr;
+    }
+    if (len > kStagedWrite || !c->upload) {
+        if (zhip_result r = finish_writes(c)) return r;
+        c->null_stream_work = true;
+        return hip_check(c, hipMemcpy(dst, src, len, hipMemcpyHostToDevice), what);
+    }
+    // A new buffer's clearing and longer writes run on the null stream, which the context's
+    // stream does not wait for.
+    if (c->null_stream_work) {
+        if (zhip_result r = hip_check(c, hipStreamSynchronize(nullptr), "hipStreamSynchronize")) return r;
+        c->null_stream_work = false;
+    }
+    const uint64_t room = (len + 15u) & ~15ull;
+    if (c->upload_used + room > kUploadBytes)
+        if (zhip_result r = finish_writes(c)) return r;
+    uint8_t *at = c->upload + c->upload_used;
+    memcpy(at, src, len);
+    c->upload_used += room;
+    if (launch_copy(c->stream, dst, at, len) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "%s: launch failed", what);
+    return ZHIP_OK;
+}
+
 zhip_result release_buffer(zhip_context *c, uint32_t id) {
     Buffer *b = get(c->buffers, id);
     if (!b) return set_error(c, ZHIP_E_BAD_ID, "destroy: buffer %u does not exist", id);
+    if (zhip_result r = finish_writes(c)) return r;
     const hipError_t e = hipFree(b->dev);
     *b = Buffer{};
     return hip_check(c, e, "hipFree");
@@ -569,6 +623,12 @@ zhip_result run_queue(zhip_context *c) {
     std::vector<TimingKey> keys;
     uint64_t dispatches = 0;
     size_t next_read = 0;
+    struct Piece {
+        uint8_t *dst;
+        const uint8_t *src;
+        uint64_t size;
+    };
+    std::vector<Piece> pieces;  // of the long reads, in order; read_events[i] is behind piece i
     // Parameter blocks the GPU wrote are read back while resolving the launches: before the
     // timed region and before any capture.
     const size_t prefix = (c->use_graphs && !c->profiling) ? replayable_prefix(c) : 0;
@@ -619,14 +679,37 @@ zhip_result run_queue(zhip_context *c) {
             Buffer *s = get(c->buffers, op.src);
             if (!s) return set_error(c, ZHIP_E_BAD_ID, "read_buffer: the buffer was destroyed before the submit");
             const Read &rd = c->reads[next_read++];
-            if (rd.size > 0)
-                if (zhip_result r = hip_check(c, hipMemcpyAsync(c->download + rd.staging_offset, s->dev + op.src_offset, rd.size, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync")) return r;
+            if (rd.size == 0) break;
+            const uint8_t *from = s->dev + op.src_offset;
+            uint8_t *to = c->download + rd.staging_offset;
+            if (rd.size <= kSmallRead) {
+                if (launch_copy(c->stream, to, from, rd.size) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "read_buffer: launch failed");
+                break;
+            }
+            const uint64_t piece = std::max<uint64_t>(kReadPiece, (rd.size / kMostPieces + 4096u) & ~4095ull);
+            for (uint64_t done = 0; done < rd.size; done += piece) {
+                const uint64_t size = std::min(piece, rd.size - done);
+                if (zhip_result r = hip_check(c, hipMemcpyAsync(to + done, from + done, size, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync")) return r;
+                if (rd.size <= piece) break;  // (in one piece: handed over at the end)
+                if (c->read_events.size() == pieces.size()) {
+                    hipEvent_t ev;
+                    if (zhip_result r = hip_check(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return r;
+                    c->read_events.push_back(ev);
+                }
+                if (zhip_result r = hip_check(c, hipEventRecord(c->read_events[pieces.size()], c->stream), "hipEventRecord")) return r;
+                pieces.push_back(Piece{rd.dst + done, to + done, size});
+            }
             break;
         }
         }
     }
     if (zhip_result r = hip_check(c, hipEventRecord(c->ev_end, c->stream), "hipEventRecord")) return r;
+    for (size_t i = 0; i < pieces.size(); i++) {
+        if (zhip_result r = hip_check(c, hipEventSynchronize(c->read_events[i]), "hipEventSynchronize")) return r;
+        memcpy(pieces[i].dst, pieces[i].src, pieces[i].size);
+    }
     if (zhip_result r = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
+    c->upload_used = 0;
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, c->ev_begin, c->ev_end) == hipSuccess) c->last_ns = (uint64_t)((double)ms * 1e6);
     c->last_dispatches = dispatches;
@@ -637,8 +720,11 @@ zhip_result run_queue(zhip_context *c) {
         t.ns += (uint64_t)((double)dms * 1e6);
         t.count++;
     }
-    for (const Read &rd : c->reads)
-        if (rd.size > 0) memcpy(rd.dst, c->download + rd.staging_offset, rd.size);
+    for (const Read &rd : c->reads) {
+        bool in_pieces = false;
+        for (const Piece &p : pieces) in_pieces |= p.src == c->download + rd.staging_offset;
+        if (rd.size > 0 && !in_pieces) memcpy(rd.dst, c->download + rd.staging_offset, rd.size);
+    }
     return ZHIP_OK;
 }
 
@@ -653,6 +739,7 @@ zhip_result submit(zhip_context *c) {
         message = c->message;
         (void)hipStreamSynchronize(c->stream);
         (void)hipGetLastError();
+        c->upload_used = 0;
     }
     c->ops.clear();
     std::vector<uint32_t> released;
@@ -738,6 +825,7 @@ zhip_result run_command(zhip_context *c, const Command &cmd, zhip_completion *ou
         const uint64_t alloc = std::max<uint64_t>((size + 255u) & ~255ull, 256u);
         if (zhip_result r = hip_check(c, hipMalloc(reinterpret_cast<void **>(&b.dev), alloc), "hipMalloc")) return r;
         // New buffers read as zero, as WebGPU's do.
+        c->null_stream_work = true;
         if (zhip_result r = hip_check(c, hipMemset(b.dev, 0, alloc), "hipMemset")) { (void)hipFree(b.dev); return r; }
         if (b.usage & kUsageUniform) {
             b.shadowed = true;
@@ -757,7 +845,7 @@ zhip_result run_command(zhip_context *c, const Command &cmd, zhip_completion *ou
         if (len == 0) return ZHIP_OK;
         const void *data = reinterpret_cast<const void *>((uintptr_t)cmd.u64(3));
         if (!data) return set_error(c, ZHIP_E_BAD_COMMAND, "write_buffer: null data");
-        if (zhip_result r = hip_check(c, hipMemcpy(b->dev + offset, data, len, hipMemcpyHostToDevice), "hipMemcpy (write_buffer)")) return r;
+        if (zhip_result r = write_device(c, b->dev + offset, data, len, "hipMemcpy (write_buffer)")) return r;
         if (b->shadowed && !b->shadow_stale) memcpy(b->shadow.data() + offset, data, len);
         return ZHIP_OK;
     }
@@ -770,7 +858,7 @@ zhip_result run_command(zhip_context *c, const Command &cmd, zhip_completion *ou
         if (file_offset > c->file_len || size > c->file_len - file_offset || offset > b->size || size > b->size - offset || (offset | size) % 4 != 0)
             return set_error(c, ZHIP_E_BAD_COMMAND, "write_file: range outside the file or the buffer");
         if (size == 0) return ZHIP_OK;
-        if (zhip_result r = hip_check(c, hipMemcpy(b->dev + offset, c->file + file_offset, size, hipMemcpyHostToDevice), "hipMemcpy (write_file)")) return r;
+        if (zhip_result r = write_device(c, b->dev + offset, c->file + file_offset, size, "hipMemcpy (write_file)")) return r;
         if (b->shadowed && !b->shadow_stale) memcpy(b->shadow.data() + offset, c->file + file_offset, size);
         return ZHIP_OK;
     }
@@ -985,7 +1073,9 @@ zhip_result zhip_destroy(zhip_context *c) {
         if (e.exec) (void)hipGraphExecDestroy(e.exec);
     c->work.release();
     for (hipEvent_t ev : c->events) (void)hipEventDestroy(ev);
+    for (hipEvent_t ev : c->read_events) (void)hipEventDestroy(ev);
     if (c->download) (void)hipHostFree(c->download);
+    if (c->upload) (void)hipHostFree(c->upload);
     if (c->ev_begin) (void)hipEventDestroy(c->ev_begin);
     if (c->ev_end) (void)hipEventDestroy(c->ev_end);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1035,17 +1125,27 @@ zhip_result zhip_execute(zhip_context *c, const uint32_t *words, size_t n_words,
     }
     if (need > capacity) return set_error(c, ZHIP_E_INVALID_ARGUMENT, "the batch completes %zu tokens, room for %zu", need, capacity);
     // src/gpu/cmd.zig:229-246: a header word carries the command's length.
-    for (size_t pos = 0; pos < n_words;) {
+    zhip_result result = ZHIP_OK;
+    for (size_t pos = 0; pos < n_words && result == ZHIP_OK;) {
         const uint32_t word = words[pos];
         const size_t n = word >> 8;
-        if (n == 0) return set_error(c, ZHIP_E_BAD_LENGTH, "command at word %zu has length 0", pos);
-        if (n > n_words - pos) return set_error(c, ZHIP_E_TRUNCATED, "command at word %zu runs past the batch", pos);
-        const Command cmd{word & 0xffu, words + pos + 1, n - 1};
-        const zhip_result r = run_command(c, cmd, out, out_count);
-        if (r != ZHIP_OK) return r;
-        pos += n;
+        if (n == 0) {
+            result = set_error(c, ZHIP_E_BAD_LENGTH, "command at word %zu has length 0", pos);
+        } else if (n > n_words - pos) {
+            result = set_error(c, ZHIP_E_TRUNCATED, "command at word %zu runs past the batch", pos);
+        } else {
+            const Command cmd{word & 0xffu, words + pos + 1, n - 1};
+            result = run_command(c, cmd, out, out_count);
+            pos += n;
+        }
     }
-    return ZHIP_OK;
+    // Writes that no submit of the batch followed have landed when the call returns.
+    std::string message;
+    if (result != ZHIP_OK) message = c->message;
+    const zhip_result landed = finish_writes(c);
+    if (result == ZHIP_OK) return landed;
+    c->message = message;
+    return result;
 }
 
 zhip_result zhip_profile_start(zhip_context *c) {
