@@ -70,6 +70,24 @@ def test_transfers_of_every_length(ctx, words):
     assert np.array_equal(whole, want) and np.array_equal(tail, want[1 : 1 + words])
 
 
+def test_reads_into_one_destination_land_in_their_order(ctx):
+    """A long read arrives in pieces while others wait for the whole submit: where destinations
+    overlap, the read recorded last is the one that stays."""
+    c = ctx
+    words = 300000
+    a, b = c.random(words, 1), c.random(words, 1)
+    first, second = c.upload(a), c.upload(b)
+    got = np.zeros(words, np.float32)
+    c.rec.read_buffer(911, first.buffer, 0, got[100:1100])
+    c.rec.read_buffer(912, second.buffer, 0, got)
+    c.flush()
+    assert np.array_equal(got, b)
+    c.rec.read_buffer(913, first.buffer, 0, got)
+    c.rec.read_buffer(914, second.buffer, 400, got[100:1100])
+    c.flush()
+    assert np.array_equal(got[100:1100], b[100:1100]) and np.array_equal(got[:100], a[:100]) and np.array_equal(got[1100:], a[1100:])
+
+
 def test_writes_land_before_work_recorded_ahead_of_them(ctx):
     """write_buffer lands before the next submit's work, even work recorded
     ahead of it (src/gpu/cmd.zig:24-25, src/agility/host.zig:4-8)."""

@@ -358,6 +358,14 @@ zhip_result finish_writes(zhip_context *c) {
     return hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 }
 
+// A new buffer's clearing and longer writes run on the null stream, which the context's stream
+// does not wait for.
+zhip_result finish_null_stream(zhip_context *c) {
+    if (!c->null_stream_work) return ZHIP_OK;
+    c->null_stream_work = false;
+    return hip_check(c, hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+}
+
 // Host memory to a buffer, before the next submit's work; `what` names the command.
 zhip_result write_device(zhip_context *c, uint8_t *dst, const void *src, uint64_t len, const char *what) {
     if (len <= kStagedWrite && !c->upload && hipHostMalloc(reinterpret_cast<void **>(&c->upload), kUploadBytes, hipHostMallocDefault) != hipSuccess) {
@@ -369,12 +377,7 @@ zhip_result write_device(zhip_context *c, uint8_t *dst, const void *src, uint64_
         c->null_stream_work = true;
         return hip_check(c, hipMemcpy(dst, src, len, hipMemcpyHostToDevice), what);
     }
-    // A new buffer's clearing and longer writes run on the null stream, which the context's
-    // stream does not wait for.
-    if (c->null_stream_work) {
-        if (zhip_result r = hip_check(c, hipStreamSynchronize(nullptr), "hipStreamSynchronize")) return r;
-        c->null_stream_work = false;
-    }
+    if (zhip_result r = finish_null_stream(c)) return r;
     const uint64_t room = (len + 15u) & ~15ull;
     if (c->upload_used + room > kUploadBytes)
         if (zhip_result r = finish_writes(c)) return r;
@@ -619,6 +622,7 @@ zhip_result run_queue(zhip_context *c) {
         if (zhip_result r = hip_check(c, hipHostMalloc(reinterpret_cast<void **>(&c->download), size, hipHostMallocDefault), "hipHostMalloc")) return r;
         c->download_size = size;
     }
+    if (zhip_result r = finish_null_stream(c)) return r;
     size_t timed = 0;
     std::vector<TimingKey> keys;
     uint64_t dispatches = 0;
@@ -686,7 +690,10 @@ zhip_result run_queue(zhip_context *c) {
                 if (launch_copy(c->stream, to, from, rd.size) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "read_buffer: launch failed");
                 break;
             }
-            const uint64_t piece = std::max<uint64_t>(kReadPiece, (rd.size / kMostPieces + 4096u) & ~4095ull);
+            // (a read over an earlier one's destination is handed over behind it)
+            bool apart = true;
+            for (size_t i = 0; i + 1 < next_read; i++) apart &= c->reads[i].size == 0 || rd.dst + rd.size <= c->reads[i].dst || c->reads[i].dst + c->reads[i].size <= rd.dst;
+            const uint64_t piece = apart ? std::max<uint64_t>(kReadPiece, (rd.size / kMostPieces + 4096u) & ~4095ull) : rd.size;
             for (uint64_t done = 0; done < rd.size; done += piece) {
                 const uint64_t size = std::min(piece, rd.size - done);
                 if (zhip_result r = hip_check(c, hipMemcpyAsync(to + done, from + done, size, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync")) return r;
