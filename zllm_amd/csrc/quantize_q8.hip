@@ -2,13 +2,13 @@
 // multiply, value for value as llama.cpp's x86 CPU backend rounds them
 // (src/kernels/quantize_q8.wgsl, src/ref/matmul.zig:197-247). A wave takes U
 // consecutive chunks of 256 values of one row, four values a lane and chunk
-// (a chunk is one Q8_K block, or eight Q8_0 blocks of eight lanes each), all
-// their loads issued before the first is rounded: a chunk's rounding is a chain
-// of dependent operations behind one 16-byte load, and a wave with one load in
-// flight spends its time waiting for memory (512 x 14336 values to Q8_K blocks
-// took 37 us with a chunk a wave, an HBM read of 29 MB). A workgroup is four
-// such waves on neighbouring chunks; with the RMSNorm prologue it first adds the
-// row's squares together and then takes all of the row's chunks. The largest magnitude of a
+// (a chunk is one Q8_K block, or eight Q8_0 blocks of eight lanes each), and a
+// workgroup is four such waves on neighbouring chunks. A chunk's rounding is a
+// chain of dependent operations behind one 16-byte load, so what hides it is
+// other waves: without the RMSNorm prologue U is one. With it a workgroup
+// first adds the row's squares together and then takes all of the row's
+// chunks, up to four a wave, all their loads issued before the first is
+// rounded. The largest magnitude of a
 // block is found with row-local DPP steps (and, for Q8_K, four lane reads),
 // the first position that holds it with a ballot. Every operation whose rounding
 // decides a value is an operation of its own (the library is compiled with
@@ -194,16 +194,17 @@ zhip_result launch_quantize_q8(const Dispatch &d) {
     const float *x = reinterpret_cast<const float *>(d.bind[1].ptr), *nw = reinterpret_cast<const float *>(d.bind[4].ptr);
     uint32_t *qx = reinterpret_cast<uint32_t *>(d.bind[2].ptr);
     float *dx = reinterpret_cast<float *>(d.bind[3].ptr);
-    // Chunks a wave takes at once: four or two where that still leaves two workgroups a CU
-    // (few rows are faster as many short waves: 64 x 4096, 2.5 against 3.4 us).
+    // One chunk a wave, whatever the size: against two and four (the choice before, where that
+    // left two workgroups a CU), inputs in the Infinity Cache, 512 x 3072 with the SiLU-pair prologue
+    // 4.7 / 5.5 / 6.3 us, 512 x 4096 without one 3.8 / 3.9 / 4.2, 512 x 14336 with the prologue 13.9 / 13.8 /
+    // 15.9, 201 x 9728 with it 5.3 / 5.9 / 7.5; only 512 x 14336 without one is faster with two, 8.9 / 8.6.
+    // With the RMSNorm prologue a workgroup takes its whole row.
     const uint32_t n_chunks = d.grid[0];
-    // (with the RMSNorm prologue a workgroup takes its whole row)
     const bool whole = p.mode == 1u;
-    const uint64_t enough = 2u * (uint64_t)d.dev->compute_units;
-    const uint32_t at_once = whole || rows * ((n_chunks + 15u) / 16u) >= enough ? 4u : rows * ((n_chunks + 7u) / 8u) >= enough ? 2u : 1u;
-    if (at_once == 4u && n_chunks > 8u) hipLaunchKernelGGL(quantize_q8_kernel<4>, dim3(whole ? 1u : (n_chunks + 15u) / 16u, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx, nw);
-    else if (at_once >= 2u && n_chunks > 4u) hipLaunchKernelGGL(quantize_q8_kernel<2>, dim3(whole ? 1u : (n_chunks + 7u) / 8u, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx, nw);
-    else hipLaunchKernelGGL(quantize_q8_kernel<1>, dim3(whole ? 1u : (n_chunks + 3u) / 4u, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx, nw);
+    const dim3 grid(whole ? 1u : (n_chunks + 3u) / 4u, d.grid[1]);
+    if (whole && n_chunks > 8u) hipLaunchKernelGGL(quantize_q8_kernel<4>, grid, dim3(256), 0, d.stream, p, x, qx, dx, nw);
+    else if (whole && n_chunks > 4u) hipLaunchKernelGGL(quantize_q8_kernel<2>, grid, dim3(256), 0, d.stream, p, x, qx, dx, nw);
+    else hipLaunchKernelGGL(quantize_q8_kernel<1>, grid, dim3(256), 0, d.stream, p, x, qx, dx, nw);
     return check_launch(d, "quantize_q8");
 }
 
