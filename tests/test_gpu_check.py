@@ -1598,6 +1598,32 @@ def test_matmul_kquant_int8_tiles(ctx, t, n):
         assert got[first : first + count].tobytes() == run(first, count).tobytes(), "token chunking changed bits"
 
 
+@pytest.mark.parametrize("k", [768, 1280, 14336])
+@pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_matmul_kquant_int8_bits_do_not_depend_on_the_rows_of_a_launch(ctx, t, k):
+    """An output is the same sum of four parts of k whether its launch has 96 rows or 16416 (a row's
+    place in the matrix does not matter either: the matrix is the 96 rows over and over), at a step
+    for each of the kernels; 1e-5 against float64 over the rounded activations. Parts of unequal length
+    and, at three blocks, an empty one."""
+    c = ctx
+    rows, n, times = 300, 96, 171
+    x = c.random(rows * k, 1).reshape(rows, k)
+    raw, values = quant_rows(c, t, n, k)
+    small, large = c.gpu_weights(t, raw, k), c.gpu_weights(t, np.tile(raw.reshape(-1), times), k)
+    xs = oracle.round_like_llama(ORACLE_TYPE[t], x)
+    init = c.random(rows * n, 1).reshape(rows, n)
+    for accumulate in (0, 1):
+        for count in (rows, 130, 64, 32, 1):
+            act = quantize_x(c, t, c.upload(x[:count]), count, k)
+            got = []
+            for w, m in ((small, 1), (large, times)):
+                out = c.upload(np.tile(init[:count], (1, m)))
+                launch_int8(c, t, act, w, out, count, n * m, k, accumulate, None)
+                got.append(c.read(out).reshape(count, n * m))
+            assert np.array_equal(np.tile(got[0], (1, times)).view(np.uint32), got[1].view(np.uint32)), (accumulate, count)
+            assert rel_err(got[0], xs[:count].astype(np.float64) @ values.astype(np.float64).T + (init[:count] if accumulate else 0.0)) <= 1e-5
+
+
 def test_matmul_q8_0_int8_whole_steps_keep_token_bits(ctx):
     """matmul_q8_0 with k a multiple of 128, unsliced, takes the kernel whose scale products
     run on the matrix cores, in 128- or 64-token tiles: a token's sums are the same bits

@@ -21,21 +21,21 @@
 // (exact, below 2048) against the minimums. With one token tile a wave (NT = 1) the converted
 // weights would serve a single tile, and those two formats scale the sums after all.
 //
-// A workgroup is S * RW waves. Wave w walks part w % S of k (S = 4: blocks p * B / 4 .. of part p of B,
-// the parts added as ((p0 + p1) + p2) + p3; S = 1: all of k in its order) for rows 32 (w / S) .. + 31
+// k is summed in four parts, blocks p * B / 4 .. of part p of B, each in its order, and the parts are
+// added as ((p0 + p1) + p2) + p3, whatever the matrix and the step: neither how a prompt is cut into
+// steps nor how a matrix is cut into launches changes an output's bits. A workgroup is S * RW waves.
+// Wave w walks part w % S of k (S = 4) or all four, closing each part's sums (S = 1), for rows 32 (w / S) .. + 31
 // and the tile's 32 NT tokens, one 32-token tile of a block after the other with the block's
 // converted weights in registers (64 VGPRs). Every part has a ring of three token tiles in LDS, filled
 // two tiles ahead by whole-line direct loads that the part's RW waves share, and a wave's rows'
 // blocks arrive in a slot of its own a block ahead. One barrier a tile where RW > 1, which leaves the
 // loads in flight; the f32 end of a tile and block (five vector operations an output) is worked off
-// between the next tile's matrix instructions. S is the matrix's, NT and RW are the step's: how a
-// prompt is cut into steps does not change a token's bits.
+// between the next tile's matrix instructions.
 //
-// Measured (us, weights from HBM, before -> after): Q4_K 512 x 4096 x 4096 32.6 -> 26.8, 512 x 28672 x 4096
-// 220 -> 152, 512 x 4096 x 14336 105 -> 82, 128 x 4096 x 4096 16.5 -> 11.3, 64 x 4096 x 4096 9.5 -> 9.3;
-// Q5_K 36.4 -> 29.4 / 253 -> 173 / 118 -> 92; Q6_K 49.8 -> 26.2 / 322 -> 161 / 158 -> 79; Q3_K
-// 51.5 -> 18.2 / 298 -> 102 / 165 -> 52. Counters at 512 x 28672 x 4096: vector issue 44 % of the time, matrix
-// cores 40 %, 1.5 waves a SIMD.
+// Measured (us, weights from HBM, against the predecessor): Q4_K 512 x 4096 x 4096 37.9 -> 28.2, 512 x 28672 x
+// 4096 232 -> 173, 512 x 4096 x 14336 115 -> 91, 128 x 4096 x 4096 17.3 -> 11.6, 64 x 4096 x 4096 9.7 -> 8.9;
+// Q5_K 41.9 -> 32.9 / 259 -> 211 / 128 -> 101; Q6_K 53.7 -> 29.7 / 328 -> 187 / 171 -> 88; Q3_K
+// 54.1 -> 19.2 / 302 -> 112 / 165 -> 60.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -339,6 +339,24 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
     for (int tt = 0; tt < NT; tt++)
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[tt][e] = 0.f;
+    // S = 1: the sums of the parts before this one, closed where a part ends. (A row of less than four
+    // blocks begins with an empty part, whose sum is a zero; -0 leaves the first part's as they are.)
+    float closed[S == 1 ? NT : 1][16];
+    if constexpr (S == 1) {
+#pragma unroll
+        for (int tt = 0; tt < NT; tt++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) closed[tt][e] = blocks < 4u ? 0.f : -0.f;
+    }
+    auto close = [&](int tt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            closed[tt][e] += acc[tt][e];
+            acc[tt][e] = 0.f;
+        }
+    };
+    uint32_t parts = 1, end = blocks / 4u;  // S = 1: where the part ends that block b is of
+    bool closes = false;                    // the block of the last step's tile was its part's last
     u32x4 high[8], low[8];
     i32x16 total = {};  // the last tile's integer sums: finished during the next tile's matrix instructions
     const i32x16 zero = {};
@@ -379,6 +397,7 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
     step_end<T, (RW > 1)>();
     uint32_t cur = 0, count = 0;  // the ring's tile of this step; the step's number
     for (uint32_t b = 0; b < most; b++) {
+        while (S == 1 && end <= b) end = ++parts * blocks / 4u;
         auto step = [&](auto tile) __attribute__((always_inline)) {
             constexpr int tt = decltype(tile)::value, prev = (tt + NT - 1) % NT;
             const uint32_t ahead = cur == 0u ? 2u : cur - 1u;  // (cur + 2) % 3: last step's
@@ -448,6 +467,8 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
                 if (RW == 2) *reinterpret_cast<uint2 *>(sums_at(count) + 8u * group) = uint2{s4.x, s4.y};
                 if (RW == 4) *reinterpret_cast<uint32_t *>(sums_at(count) + 4u * group) = s4.x;
             }
+            if (S == 1 && closes) close(prev);
+            if (S == 1 && tt == 0) closes = end == b + 1u;
             if (tt == 0) P::factors(raw, d, dmin, mins);
 #pragma unroll
             for (int e = 0; e < 16; e++) total[e] = UNIT_SCALES ? __mul24(unit_scale(sc, 7), lsum[e]) + hsum[e] : P::PLANES == 2 ? (int)((uint32_t)hsum[e] << P::SHIFT) + lsum[e] : hsum[e];
@@ -468,6 +489,7 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
         const f32x16 msum = minimum_sums(count + 1u);
 #pragma unroll
         for (int e = 0; e < 16; e++) finish(acc[NT - 1][e], e, msum, read_dx(count + 3u, e / 4));
+        if (S == 1) close(NT - 1);
     }
     step_end<0, true>();  // nothing may still land in LDS during the exchange
 
@@ -503,7 +525,7 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
         float sum[4 * NT];
 #pragma unroll
         for (int i = 0; i < 4 * NT; i++) {
-            sum[i] = acc[(base + i) / 16][(base + i) % 16];
+            sum[i] = S == 1 ? closed[S == 1 ? (base + i) / 16 : 0][(base + i) % 16] : acc[(base + i) / 16][(base + i) % 16];
             if (S == 4) {
                 float v[4];
 #pragma unroll
@@ -533,23 +555,27 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const KqArgs &a) {
     return check_launch(d, name);
 }
 
-// Which order k is summed in is the matrix's: from 16384 rows on a wave walks all of k (a step's
-// waves fill the chip from the first chunks on; Q4_K 28672 x 4096 at 512 tokens 157 us against 180 in
-// four parts, at 64 tokens 38 against 39, while 14336 x 4096 takes 25 us against 20 at 64 tokens
-// and 85 against 104 at 512), below it four waves a part each. Which tile is the step's, and
-// does not show in the bits.
+// Which launch takes the step; the bits are the same. A wave a part each (S = 4) unless a wave that
+// walks all of k is the faster one. us, all of k / a part each:
+//   Q3_K, four token tiles, from four and a half waves a CU on: 28672 x 4096 at 512 tokens 111 / 130, 18432 x
+//     2560 at 201 34 / 41, at 4096 52 / 52, at 8192 96 / 91; below, 16384 at 256 30 / 32, 44 / 42, 81 / 71
+//   Q4_K, two (the closed sums of four do not fit the registers), from five on: 28672 x 4096 at 512 168 / 192, at
+//     128 50 / 60; 14336 at 512 91 / 104, 20480 at 128 48 / 55; below, 14336 at 128 (three and a half) 35 / 30
+//   Q4_K and Q5_K, one, steps of up to 64 tokens whose parts would take a third round of workgroups:
+//     28672 x 4096 at 32 tokens Q4_K 25 / 28, Q5_K 28 / 32, at 64 36 / 38, 40 / 46; with two rounds, 14336 at 32, 23 / 16
+// Q5_K and Q6_K at two tiles gain nothing (28672 x 4096 at 512: 215 / 214, 214 / 190).
 template <class P>
 zhip_result launch_format(const Dispatch &d, const char *name, const KqArgs &a) {
     const uint64_t cus = (uint64_t)d.dev->compute_units, groups = (a.n + 31u) / 32u;
     auto tokens = [&](uint32_t nt) { return (uint64_t)((a.rows + 32u * nt - 1u) / (32u * nt)); };
-    if (a.n >= 16384u) {
-        // The tallest tile that leaves a SIMD its waves: where a block's end is dear (minimums), six
-        // waves a CU for four token tiles a wave and four for two, otherwise two and any
-        // (28672 x 4096, one / two / four tiles: Q4_K at 64 tokens 38 / 42 us, at 128 64 / 55 / 67, at 200
-        // 104 / 94 / 85; Q6_K at 64 tokens 53 / 43, at 128 89 / 64 / 60).
-        if (a.rows > 64u && groups * tokens(4) >= (P::HAS_MIN ? 6u : 2u) * cus) return launch_tile<P, 4, 4, 1>(d, name, a);
-        if (a.rows > 32u && (!P::HAS_MIN || groups * tokens(2) >= 4u * cus)) return launch_tile<P, 2, 4, 1>(d, name, a);
-        return launch_tile<P, 1, 4, 1>(d, name, a);
+    if constexpr (P::PLANES == 1) {
+        if (a.rows > 64u && 2u * groups * tokens(4) >= 9u * cus) return launch_tile<P, 4, 4, 1>(d, name, a);
+    }
+    if constexpr (P::HAS_MIN) {
+        if constexpr (P::SHIFT == 3) {
+            if (a.rows > 32u && groups * tokens(2) >= 5u * cus) return launch_tile<P, 2, 4, 1>(d, name, a);
+        }
+        if (a.rows <= 64u && groups > 2u * cus) return launch_tile<P, 1, 4, 1>(d, name, a);
     }
     // One workgroup a CU at a time: the tile whose rounds take least. A round's time in eighths of
     // the smallest tile's, measured at k = 4096 (Q4_K 9.3 / 12.6 / 11.0 / 16.8 / 24 us, Q6_K 10.2 /
