@@ -1624,6 +1624,29 @@ def test_matmul_kquant_int8_bits_do_not_depend_on_the_rows_of_a_launch(ctx, t, k
             assert rel_err(got[0], xs[:count].astype(np.float64) @ values.astype(np.float64).T + (init[:count] if accumulate else 0.0)) <= 1e-5
 
 
+@pytest.mark.parametrize("n", [1, 32, 77, 160])
+@pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_matmul_kquant_int8_lone_token_at_any_stride(ctx, t, n):
+    """A step of one token does not use its stride: none at all, ones short of the outputs and ones past
+    them give the same token, and nothing is written on either side of it."""
+    c = ctx
+    k, col0 = 768, 3
+    x, init = c.random(k, 1), c.random(n + 2 * col0, 1)
+    raw, values = quant_rows(c, t, n, k)
+    wa, act = c.gpu_weights(t, raw, k), quantize_x(c, t, c.upload(x), 1, k)
+    exact = oracle.round_like_llama(ORACLE_TYPE[t], x.reshape(1, k)).astype(np.float64) @ values.astype(np.float64).T
+    for accumulate in (0, 1):
+        want = init.astype(np.float64)
+        want[col0 : col0 + n] = exact[0] + (want[col0 : col0 + n] if accumulate else 0.0)
+        for stride in (0, 1, n // 2, n - 1, n, n + 5):
+            out = c.upload(init)
+            c.launcher().launch(K.weight_kernel("matmul", t), P.MatmulQuant(rows=1, n=n, k=k, col0=col0, out_stride=stride, accumulate=accumulate, k_slice=k), [act[0], wa, out, act[1]],
+                                (K.div_ceil(n, K.matmul_quant_tile_n), 1, 1))
+            got = c.read(out)
+            assert rel_err(got, want) <= 1e-5, (accumulate, stride)
+            assert np.array_equal(got[:col0], init[:col0]) and np.array_equal(got[col0 + n :], init[col0 + n :])
+
+
 def test_matmul_q8_0_int8_whole_steps_keep_token_bits(ctx):
     """matmul_q8_0 with k a multiple of 128, unsliced, takes the kernel whose scale products
     run on the matrix cores, in 128- or 64-token tiles: a token's sums are the same bits

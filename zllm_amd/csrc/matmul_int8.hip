@@ -586,9 +586,12 @@ static zhip_result launch_int8(const Dispatch &d, const char *name, int type) {
             a.w_bytes, a.dx_bytes);
     const dim3 grid((uint32_t)tiles_n, (uint32_t)tiles_t, (uint32_t)slices);
     const bool ragged = p.k % STEP != 0 || (p.k_slice < p.k && p.k_slice % STEP != 0);
-    // (its outputs are stored at 32-bit offsets within a tile of 128 tokens)
-    if (type != 8 && slices == 1u && p.k_slice >= p.k && 128ull * p.out_stride * 4u < kNowhere)
-        return launch_matmul_kquant_i8(d, name, type, a.qx, a.w, a.dx, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate, a.row_bytes, a.qx_bytes,
+    // (Its outputs are stored at 32-bit offsets within a tile of 128 tokens, the absent tokens' past the
+    // end of the last one's: that takes a stride that reaches over a row. A lone token has no use for its
+    // stride and may come with a shorter one.)
+    const uint32_t stride = rows == 1u && p.out_stride < n ? (uint32_t)n : p.out_stride;
+    if (type != 8 && slices == 1u && p.k_slice >= p.k && stride >= n && 128ull * stride * 4u < kNowhere)
+        return launch_matmul_kquant_i8(d, name, type, a.qx, a.w, a.dx, a.out, a.rows, a.n, a.k, a.col0, stride, a.accumulate, a.row_bytes, a.qx_bytes,
             a.w_bytes, a.dx_bytes);
     if (type == 3) {
         return launch_kquant<I8Q3>(d, name, grid, a);

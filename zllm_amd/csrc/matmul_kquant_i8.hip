@@ -511,7 +511,8 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
         asm volatile("" ::: "memory");
     }
     // Sum base + i of the lane: tile (base + i) / 16, token 8 (e / 4) + 4 h + e % 4 of it. The buffer
-    // ends with the step's last token, and lanes past the last row ask past it.
+    // ends with the step's last token (out_stride >= n: the tokens after it begin past its end), and lanes
+    // past the last row ask past it.
     const __amdgpu_buffer_rsrc_t obuf = make_buffer(reinterpret_cast<const uint8_t *>(a.out + (size_t)t0 * a.out_stride + a.col0), ((min(a.rows - t0, 32u * NT) - 1u) * a.out_stride + a.n) * 4u);
     const uint32_t j = n0 + lrow, olane = (4u * h * a.out_stride + j) * 4u | (j < a.n ? 0u : kNowhere);
     auto collect = [&](auto quarter) __attribute__((always_inline)) {
@@ -599,7 +600,7 @@ zhip_result launch_format(const Dispatch &d, const char *name, const KqArgs &a) 
 
 // Whole, unsliced k in 256-weight blocks; the caller has validated the bindings and that 32-bit
 // offsets reach every operand up to a tile past the last token and row (n + 128 rows, rows + 128
-// tokens), and the outputs of 128 tokens.
+// tokens), and the outputs of 128 tokens, and passes a stride of n or more.
 zhip_result launch_matmul_kquant_i8(const Dispatch &d, const char *name, int type, const uint8_t *qx, const uint8_t *w, const uint8_t *dx, float *out,
     uint32_t rows, uint32_t n, uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t qx_bytes, uint32_t w_bytes,
     uint32_t dx_bytes) {
