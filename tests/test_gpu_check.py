@@ -1647,6 +1647,25 @@ def test_matmul_kquant_int8_lone_token_at_any_stride(ctx, t, n):
             assert np.array_equal(got[:col0], init[:col0]) and np.array_equal(got[col0 + n :], init[col0 + n :])
 
 
+@pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_matmul_kquant_int8_wide_strides(ctx, t):
+    """Rows of outputs so far apart that a tile's last token lies more than 2^28 bytes behind its first,
+    and a row tile that the matrix does not fill: nothing but the matrix's own outputs is written."""
+    c = ctx
+    rows, n, k, stride = 32, 33, 256, 2600000
+    x = c.random(rows * k, 1).reshape(rows, k)
+    raw, values = quant_rows(c, t, n, k)
+    init = np.full((rows - 1) * stride + n, 7.0, np.float32)
+    out = c.upload(init)
+    launch_int8(c, t, quantize_x(c, t, c.upload(x), rows, k), c.gpu_weights(t, raw, k), out, rows, n, k, 0, None, stride=stride)
+    got = c.read(out)
+    mine = np.arange(rows)[:, None] * stride + np.arange(n)
+    want = oracle.round_like_llama(ORACLE_TYPE[t], x).astype(np.float64) @ values.astype(np.float64).T
+    assert rel_err(got[mine], want) <= 1e-5
+    got[mine] = 7.0
+    assert np.array_equal(got, init)
+
+
 def test_matmul_q8_0_int8_whole_steps_keep_token_bits(ctx):
     """matmul_q8_0 with k a multiple of 128, unsliced, takes the kernel whose scale products
     run on the matrix cores, in 128- or 64-token tiles: a token's sums are the same bits

@@ -514,10 +514,11 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
     // ends with the step's last token (out_stride >= n: the tokens after it begin past its end), and lanes
     // past the last row ask past it.
     const __amdgpu_buffer_rsrc_t obuf = make_buffer(reinterpret_cast<const uint8_t *>(a.out + (size_t)t0 * a.out_stride + a.col0), ((min(a.rows - t0, 32u * NT) - 1u) * a.out_stride + a.n) * 4u);
-    const uint32_t j = n0 + lrow, olane = (4u * h * a.out_stride + j) * 4u | (j < a.n ? 0u : kNowhere);
+    const uint32_t j = n0 + lrow, olane = (4u * h * a.out_stride + j) * 4u, beyond = j < a.n ? 0u : kNowhere;
     auto collect = [&](auto quarter) __attribute__((always_inline)) {
         constexpr int Q = decltype(quarter)::value, base = 4 * NT * Q;
-        auto offset = [&](int i) __attribute__((always_inline)) { return olane + (32u * ((base + i) / 16) + 8u * (((base + i) % 16) / 4) + (base + i) % 4) * a.out_stride * 4u; };
+        // (kNowhere's bits set last: added to, they would carry out of the word)
+        auto offset = [&](int i) __attribute__((always_inline)) { return (olane + (32u * ((base + i) / 16) + 8u * (((base + i) % 16) / 4) + (base + i) % 4) * a.out_stride * 4u) | beyond; };
         float held[4 * NT];
         if (a.accumulate) {  // all of them asked for before the first is waited for
 #pragma unroll
