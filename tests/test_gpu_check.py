@@ -269,6 +269,27 @@ def test_matvec_bf16_several_tokens_silu_pair(ctx_wide, half, m, n, k, half_row,
         assert np.array_equal(run([t])[0], got[t])
 
 
+@pytest.mark.parametrize("k", [1024, 1536, 2048, 2560, 3072, 3584, 4096])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_norm_is_every_kernels(ctx, ctx_wide, half, k):
+    """The RMSNorm prologue has one arithmetic: a step that normalises equals, bit for bit, the same step over
+    the tokens that another kernel normalised (read through an identity matrix: one product by 1, and zeros)."""
+    m, n, eps = 8, (16 << 20) // (2 * k) + 5, 1e-6
+    x, nw = ctx.random(m * k, 3), ctx.random(k, 1)
+    bits, _ = random_half(ctx, n * k, 1, half)
+    eye = np.eye(k, dtype=np.float16).view(np.uint16) if half == "f16" else synth.to_bf16_bits(np.eye(k, dtype=np.float32).reshape(-1))
+
+    def run(c, inputs, weights, rows, norm):
+        out = c.output(m * rows)
+        c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=rows, k=k, col0=0, out_stride=rows, eps=eps, norm=norm),
+                            [c.upload(inputs), c.upload(weights), out, c.upload(nw)], (K.div_ceil(rows, K.matvec_rows), m, 1))
+        return c.read(out)
+
+    staged = run(ctx, x, eye, k, True)
+    assert rel_err(staged, np.stack([norm_row(t, nw, eps) for t in x.reshape(m, k)])) <= 1e-6
+    assert run(ctx_wide, x, bits, n, True).tobytes() == run(ctx_wide, staged, bits, n, False).tobytes()
+
+
 def test_matvec_bf16_several_tokens_special_values(ctx_wide):
     """Inputs the three-way split must carry exactly: full 24-bit mantissas (integer inputs
     against weights of +-1, where every partial sum is an integer f32 holds, so the result is

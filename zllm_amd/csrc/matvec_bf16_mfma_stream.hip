@@ -277,10 +277,14 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
 #pragma unroll
         for (int s = 0; s < EARLY; s++) issue();
         if (a.flags & FLAG_NORM) {
-            float ss = 0.f;
+            // (stage_token's additions: its wave w takes the vectors of every fourth j from w on, so that a
+            // token is the same bits however it is staged; a single chain of all of them would be four times as long)
+            float ss[4] = {};
 #pragma unroll
-            for (int j = 0; j < 2 * NP; j++) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
-            const float scale = 1.0f / sqrtf(wave_sum(ss) / (float)a.k + a.eps);
+            for (int j = 0; j < 2 * NP; j++) ss[j & 3] += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+#pragma unroll
+            for (int w = 0; w < 4; w++) ss[w] = wave_sum(ss[w]);
+            const float scale = 1.0f / sqrtf(((ss[0] + ss[1]) + (ss[2] + ss[3])) / (float)a.k + a.eps);
 #pragma unroll
             for (int j = 0; j < 2 * NP; j++) {
                 v[j].x = v[j].x * scale * g[j].x; v[j].y = v[j].y * scale * g[j].y;
