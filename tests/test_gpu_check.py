@@ -232,7 +232,7 @@ def test_matvec_half_rows_in_registers(ctx, half, pair, k, n):
     (11, 4101, 2048, 4101, True, True),   # two launches of tokens
     (5, 3300, 2560, 3300, False, True),
     (2, 2750, 3072, 2750, False, False),
-    (6, 2400, 3584, 2400, True, True),    # (bf16: the tokens' pieces do not fit workgroup memory)
+    (6, 2400, 3584, 2400, True, True),    # (the tokens' pieces do not fit workgroup memory)
     (4, 2080, 4096, 2080, False, True),
     (2, 41 * 32 * 256 + 50, 1024, 32, False, True),  # more than forty output tiles on a workgroup
     (4, 600, 1024, 600, False, True),     # a small pair: the general kernel
@@ -288,6 +288,28 @@ def test_matvec_bf16_several_tokens_norm_is_every_kernels(ctx, ctx_wide, half, k
     staged = run(ctx, x, eye, k, True)
     assert rel_err(staged, np.stack([norm_row(t, nw, eps) for t in x.reshape(m, k)])) <= 1e-6
     assert run(ctx_wide, x, bits, n, True).tobytes() == run(ctx_wide, staged, bits, n, False).tobytes()
+
+
+@pytest.mark.parametrize("k", [1024, 3072, 4096])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_pair_takes_every_bit(ctx_wide, half, k):
+    """A gate / up step on the matrix cores takes its inputs with all their 24 bits: pairs of neighbouring integers
+    against up rows of +-1, whose partial sums f32 all holds, times a gate of 64 (its sigmoid rounds to one), are exact."""
+    c = ctx_wide
+    m, n = 3, (16 << 20) // (2 * k) + 1
+    r = np.repeat(c.rand.integers(2 ** 23, 2 ** 24 - 2000, size=(m, k // 2)), 2, axis=1)
+    r[:, ::2] += c.rand.integers(0, 2000, size=(m, k // 2))
+    x = r.astype(np.float32)
+    x[:, 0] = 64
+    w = np.zeros((2 * n, k), np.float32)
+    w[:n, 0] = 1
+    w[n:, 2:] = np.where(np.arange(2, k) % 2, -1, 1)
+    bits = w.astype(np.float16).view(np.uint16) if half == "f16" else synth.to_bf16_bits(w.reshape(-1))
+    out = c.output(m * n)
+    c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=1e-6, silu_pair=True, half=n),
+                        [c.upload(x), c.upload(bits), out, c.upload(x)], (K.div_ceil(n, K.matvec_rows), m, 1))
+    want = 64.0 * (r[:, 2::2].sum(axis=1) - r[:, 3::2].sum(axis=1))
+    assert np.array_equal(c.read(out).reshape(m, n), np.repeat(want[:, None], n, axis=1).astype(np.float32))
 
 
 def test_matvec_bf16_several_tokens_special_values(ctx_wide):

@@ -60,9 +60,11 @@ constexpr uint32_t LDS_BYTES = PART_BYTES + RING_BYTES + KEPT * 1024u + 64u;  //
 // Kernels whose workgroups split their tokens themselves keep the pieces in LDS ([piece][token of
 // 8][k], rows padded by 16 bytes so that one chunk of neighbouring rows falls in different banks)
 // until the operands are read, at its end: ring slots below them take their weights meanwhile.
-template <int NP, bool F16> constexpr uint32_t piece_row() { return 1024u * NP + 16u; }
-template <int NP, bool F16> constexpr uint32_t pieces_bytes() { return (F16 ? 16u : 24u) * piece_row<NP, F16>(); }
-template <int NP, bool F16> constexpr bool pieces_fit() { return pieces_bytes<NP, F16>() <= LDS_BYTES - 64u; }
+// An f16 token of a step without a pair enters as two pieces, every other as three.
+constexpr uint32_t pieces_of(bool f16, bool pair) { return f16 && !pair ? 2u : 3u; }
+template <int NP> constexpr uint32_t piece_row() { return 1024u * NP + 16u; }
+template <int NP, uint32_t PIECES> constexpr uint32_t pieces_bytes() { return 8u * PIECES * piece_row<NP>(); }
+template <int NP, uint32_t PIECES> constexpr bool pieces_fit() { return pieces_bytes<NP, PIECES>() <= LDS_BYTES - 64u; }
 static_assert(LDS_BYTES <= 160u * 1024u - 64u, "the rings must fit the CU's LDS");
 
 struct StreamArgs {
@@ -72,7 +74,7 @@ struct StreamArgs {
     uint32_t tail_base;  // units of eight rows after those: tail_base for every workgroup
     uint32_t tail_rem;   // and one more for each of the first tail_rem
     uint32_t by_die;     // workgroups renumbered die by die (the grid is a multiple of eight)
-    // Inputs split beforehand (SPLIT kernels): three planes [piece][token][k] of bf16.
+    // Inputs split beforehand (SPLIT kernels): planes [piece][token][k] of the weights' type.
     const uint8_t *planes;
     uint32_t plane_tokens;  // tokens a plane holds
     uint32_t plane_k;       // positions of a token in a plane (the whole row's, of which the launch may take a stretch)
@@ -154,18 +156,22 @@ __device__ __forceinline__ void f16_scale(float big, float &scale, float &invers
     inverse = unit ? 1.0f : __uint_as_float((uint32_t)(254 - se) << 23);
 }
 
-// Four scaled values as their f16 roundings and what those left times 2^11.
-__device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 &upper, uint2 &lower) {
+// Four scaled values as their f16 roundings, what those left times 2^11 and, with PIECES 3, what that left
+// times 2^22: eleven significant bits each, an f32 input's 24 in three.
+template <uint32_t PIECES>
+__device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (&w)[PIECES]) {
     const float x[4] = {v.x, v.y, v.z, v.w};
-    _Float16 hi[4], lo[4];
+    _Float16 q[PIECES][4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        // The scale is a power of two, so x * scale - hi in one fused operation is exact.
-        hi[j] = (_Float16)(x[j] * scale);
-        lo[j] = (_Float16)(fmaf(x[j], scale, -(float)hi[j]) * 2048.0f);
+        // The scale is a power of two, so x * scale - q in one fused operation is exact, and so is what the next leaves.
+        q[0][j] = (_Float16)(x[j] * scale);
+        const float rest = fmaf(x[j], scale, -(float)q[0][j]) * 2048.0f;
+        q[1][j] = (_Float16)rest;
+        if constexpr (PIECES == 3) q[2][j] = (_Float16)((rest - (float)q[1][j]) * 2048.0f);
     }
-    upper = __builtin_bit_cast(uint2, hf16x4{hi[0], hi[1], hi[2], hi[3]});
-    lower = __builtin_bit_cast(uint2, hf16x4{lo[0], lo[1], lo[2], lo[3]});
+#pragma unroll
+    for (uint32_t p = 0; p < PIECES; p++) w[p] = __builtin_bit_cast(uint2, hf16x4{q[p][0], q[p][1], q[p][2], q[p][3]});
 }
 
 // NP: pieces of a wave's k range (k = 512 NP). SPLIT: the tokens' three pieces come ready from
@@ -177,19 +183,20 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 &
 // F16 (matvec_f16: the weights are f16 and the matrix instruction v_mfma_f32_32x32x16_f16): a
 // token enters as two f16 rows, the rounding of its inputs and the rounding of what that left
 // times 2^11, after a power of two has put its largest magnitude at 2^14 (an input keeps 22
-// bits), and a token's sums are multiplied by one
-// over its scale.
+// bits), and a token's sums are multiplied by one over its scale. With PAIR there is a third row,
+// what those two left times 2^22, and an input keeps all its bits (the general kernel, which takes
+// pairs without ZHIP_OPTION_WIDE_DECODE, has them too): the matrix instruction has the rows anyway.
 // PAIR: a SILU_PAIR step, an output tile's gate rows and then its up rows (the general kernel's
 // time grows with the tokens: 2 x 8192 x 2048 f16 at eight 39 us, here 17).
 // LONG: k = 512 NP q.parts; workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
 // walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums.
 template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
 __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(StreamArgs q) {
-    static_assert(SPLIT || pieces_fit<NP, F16>(), "the tokens' pieces must fit LDS");
     static_assert(SPLIT || !LONG, "the stretches of a long row read the tokens from the planes");
     static_assert(!PAIR || !LONG, "gate / up steps take whole rows");
     constexpr uint32_t PER = PAIR ? 2u : 1u;  // weight tiles an output tile
-    constexpr uint32_t PIECES = F16 ? 2u : 3u;
+    constexpr uint32_t PIECES = pieces_of(F16, PAIR);
+    static_assert(SPLIT || pieces_fit<NP, PIECES>(), "the tokens' pieces must fit LDS");
     const MvArgs &a = q.a;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *lds_part = reinterpret_cast<float *>(lds);
@@ -262,7 +269,7 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     } else {
         // Wave w takes token w, lane l its vectors l, l + 64, ... (a wave without a token reads an
         // empty buffer). A token's values depend on nothing but its inputs.
-        constexpr uint32_t ROW = piece_row<NP, F16>(), PIECES_AT = (LDS_BYTES - 64u - pieces_bytes<NP, F16>()) & ~15u;
+        constexpr uint32_t ROW = piece_row<NP>(), PIECES_AT = (LDS_BYTES - 64u - pieces_bytes<NP, PIECES>()) & ~15u;
         constexpr uint32_t FREE = PIECES_AT < PART_BYTES ? 0u : (PIECES_AT - PART_BYTES) / (WAVES * SLOT);
         constexpr int EARLY = FREE < DEPTH - 1 ? FREE : DEPTH - 1;  // pieces of weights asked for meanwhile
         const __amdgpu_buffer_rsrc_t xbuf = make_buffer(a.x + (wave < a.m ? (size_t)wave * a.xr : 0u), wave < a.m ? 4u * a.k : 0u);
@@ -303,10 +310,10 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
             if (lane == 0) lds_inverse[wave] = inverse;
 #pragma unroll
             for (int j = 0; j < 2 * NP; j++) {
-                uint2 hi, lo;
-                f16_pieces(v[j], scale, hi, lo);
-                *reinterpret_cast<uint2 *>(mine + 8u * (lane + 64u * j)) = hi;
-                *reinterpret_cast<uint2 *>(mine + 8u * ROW + 8u * (lane + 64u * j)) = lo;
+                uint2 w[PIECES];
+                f16_pieces<PIECES>(v[j], scale, w);
+#pragma unroll
+                for (uint32_t p = 0; p < PIECES; p++) *reinterpret_cast<uint2 *>(mine + 8u * p * ROW + 8u * (lane + 64u * j)) = w[p];
             }
         } else {
 #pragma unroll
@@ -336,7 +343,7 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     auto finish = [&](uint32_t p, const hf32x16 &sum) __attribute__((always_inline)) {
         float *part = lds_part + (p & 1u) * (WAVES * 256u);
 #pragma unroll
-        for (int i = 0; i < 4; i++) part[wave * 256u + 64u * i + lane] = F16 ? fmaf(sum[4 + i], 1.0f / 2048.0f, sum[i]) : (sum[i] + sum[4 + i]) + sum[8 + i];
+        for (int i = 0; i < 4; i++) part[wave * 256u + 64u * i + lane] = !F16 ? (sum[i] + sum[4 + i]) + sum[8 + i] : fmaf(PIECES == 3 ? fmaf(sum[8 + i], 1.0f / 2048.0f, sum[4 + i]) : sum[4 + i], 1.0f / 2048.0f, sum[i]);
         lds_barrier();
         // Buffer p % 2 is written again in step p + 2, after the barrier of step p + 1, which a
         // wave passes only when it has read what it needs here. The 256 outputs of a tile are
@@ -424,8 +431,9 @@ __global__ __launch_bounds__(256) void matvec_bf16_split_kernel(MvArgs a, uint2 
 }
 
 // The same for matvec_f16: the token scaled by the power of two that puts its largest
-// magnitude in [2^14, 2^15) and split into its f16 rounding and what that left times 2^11
-// (planes [2][tokens][k]), and one over the scale.
+// magnitude in [2^14, 2^15) and split into PIECES f16 values a weight (planes
+// [piece][tokens][k]), and one over the scale.
+template <uint32_t PIECES>
 __global__ __launch_bounds__(256) void matvec_f16_split_kernel(MvArgs a, uint2 *planes, float *inverse) {
     __shared__ float red[4];
     extern __shared__ float4 staged[];  // the token: k / 4 vectors
@@ -445,7 +453,12 @@ __global__ __launch_bounds__(256) void matvec_f16_split_kernel(MvArgs a, uint2 *
     float scale, inv;
     f16_scale(big, scale, inv);
     if (tid == 0) inverse[blockIdx.x] = inv;
-    for (uint32_t i = tid; i < k4; i += 256u) f16_pieces(staged[i], scale, planes[(size_t)blockIdx.x * k4 + i], planes[(size_t)(gridDim.x + blockIdx.x) * k4 + i]);
+    for (uint32_t i = tid; i < k4; i += 256u) {
+        uint2 w[PIECES];
+        f16_pieces<PIECES>(staged[i], scale, w);
+#pragma unroll
+        for (uint32_t p = 0; p < PIECES; p++) planes[(size_t)(p * gridDim.x + blockIdx.x) * k4 + i] = w[p];
+    }
 }
 
 template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
@@ -483,8 +496,8 @@ static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 gri
     case 4: return launch_blocks<4, SPLIT, F16, LONG, PAIR>(d, q, grid);
     case 5: return launch_blocks<5, SPLIT, F16, LONG, PAIR>(d, q, grid);
     case 6: return launch_blocks<6, SPLIT, F16, LONG, PAIR>(d, q, grid);
-    case 7: return launch_blocks<7, SPLIT || !pieces_fit<7, F16>(), F16, LONG, PAIR>(d, q, grid);
-    default: return launch_blocks<8, SPLIT || !pieces_fit<8, F16>(), F16, LONG, PAIR>(d, q, grid);
+    case 7: return launch_blocks<7, SPLIT || !pieces_fit<7, pieces_of(F16, PAIR)>(), F16, LONG, PAIR>(d, q, grid);
+    default: return launch_blocks<8, SPLIT || !pieces_fit<8, pieces_of(F16, PAIR)>(), F16, LONG, PAIR>(d, q, grid);
     }
 }
 
@@ -502,8 +515,10 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
     const uint32_t tail = (a.rows - 32u * rounds * groups + 7u) / 8u;
     StreamArgs q{a, (uint32_t)(used < w_bytes ? used : w_bytes), rounds, tail / groups, tail % groups, groups % 8u == 0 ? 1u : 0u, nullptr, 0u, 0u, 0u, 0u, nullptr, 1u, nullptr};
     // The tokens are split (and normalised) by a launch of their own for rows taken in stretches
-    // (no workgroup sees a whole token), and for bf16 rows whose pieces do not fit LDS.
-    const bool split = a.k > (f16 ? 4096u : 3072u);
+    // (no workgroup sees a whole token), and for rows whose pieces do not fit LDS (three of them a token above
+    // 3072 weights).
+    const uint32_t token_pieces = pieces_of(f16, pair);
+    const bool split = a.k > (token_pieces == 2u ? 4096u : 3072u);
     // Rows of more than 4096 weights (the FFN-down shapes; the general kernel takes them token by
     // token) go in stretches of up to 4096 columns. Stretches of equal length (14336 = 4 x 3584,
     // 8192 = 2 x 4096 ...) go out as one launch: `launches` workgroups share a walker's tiles, a
@@ -511,14 +526,15 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
     // epilogue (their sums wait in the workspace, behind the tokens' planes).
     const uint32_t pieces = a.k / 512u, launches = (a.k + 4095u) / 4096u;
     const bool together = launches > 1u && pieces % launches == 0u && split && launches <= kMatvecMaxParts && cus >= launches;
-    const uint64_t planes_bytes = (((f16 ? 4ull : 6ull) * a.m * a.k + 4ull * a.m + 64u) + 255u) & ~255ull;
+    const uint64_t planes_bytes = ((2ull * token_pieces * a.m * a.k + 4ull * a.m + 64u) + 255u) & ~255ull;
     if (split) {
-        const uint64_t bytes = (f16 ? 4ull : 6ull) * a.m * a.k;
+        const uint64_t bytes = 2ull * token_pieces * a.m * a.k;
         if (!d.work) return fail(d, ZHIP_E_GPU, "%s: no workspace", name);
         if (bytes >= 0xfffffff0ull) return fail(d, ZHIP_E_BAD_COMMAND, "%s: a step of %u tokens", name, a.m);
         if (zhip_result r = d.work->reserve(d, planes_bytes + (together ? (uint64_t)launches * 8u * a.rows * sizeof(float) : 0ull))) return r;
         float *inverse = reinterpret_cast<float *>(d.work->data + bytes);
-        if (f16) hipLaunchKernelGGL(matvec_f16_split_kernel, dim3(a.m), dim3(256), a.k * 4u, d.stream, a, reinterpret_cast<uint2 *>(d.work->data), inverse);
+        if (f16 && pair) hipLaunchKernelGGL(matvec_f16_split_kernel<3>, dim3(a.m), dim3(256), a.k * 4u, d.stream, a, reinterpret_cast<uint2 *>(d.work->data), inverse);
+        else if (f16) hipLaunchKernelGGL(matvec_f16_split_kernel<2>, dim3(a.m), dim3(256), a.k * 4u, d.stream, a, reinterpret_cast<uint2 *>(d.work->data), inverse);
         else hipLaunchKernelGGL(matvec_bf16_split_kernel, dim3(a.m), dim3(256), a.k * 4u, d.stream, a, reinterpret_cast<uint2 *>(d.work->data));
         if (zhip_result r = check_launch(d, name)) return r;
         q.planes = d.work->data;
@@ -570,7 +586,7 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
             q.plane_first = first;
             zhip_result r;
             if (pair) {
-                if (f16) r = launch_for_k<false, true, false, true>(d, q, grid);  // (a pair's rows are at most 4096 weights)
+                if (f16) r = launch_for_k<false, true, false, true>(d, q, grid);
                 else r = split ? launch_for_k<true, false, false, true>(d, q, grid) : launch_for_k<false, false, false, true>(d, q, grid);
             } else if (f16) r = split ? launch_for_k<true, true>(d, q, grid) : launch_for_k<false, true>(d, q, grid);
             else r = split ? launch_for_k<true, false>(d, q, grid) : launch_for_k<false, false>(d, q, grid);
