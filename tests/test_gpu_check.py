@@ -340,6 +340,34 @@ def test_matvec_bf16_several_tokens_special_values(ctx_wide):
     assert np.all(np.isnan(got[3]))
 
 
+@pytest.mark.parametrize("pair,k", [(False, 1024), (False, 4608), (False, 8192), (True, 1024), (True, 4096)])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_infinities(ctx_wide, half, pair, k):
+    """An infinite input gives infinite outputs on the matrix cores too, whatever else its token holds,
+    a NaN gives NaNs, and neither reaches another token."""
+    c = ctx_wide
+    m, n = 5, (16 << 20) // (2 * k) + 1
+    x = np.abs(c.random(m * k, 1)).reshape(m, k) + np.float32(0.5)
+    x[0, 3], x[0, 7] = np.inf, 1e30
+    x[1, 5] = -np.inf
+    x[2, 9] = np.nan
+    x[4] *= np.float32(2.0 ** -140)                # below the normal numbers
+    w = np.full((2 * n if pair else n, k), 0.5, np.float32)
+    if pair:
+        w[:n, 5] = -0.5
+    bits = w.astype(np.float16).view(np.uint16) if half == "f16" else synth.to_bf16_bits(w.reshape(-1))
+    out = c.output(m * n)
+    c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=1e-6, silu_pair=pair, half=n if pair else 0),
+                        [c.upload(x), c.upload(bits), out, c.upload(x)], (K.div_ceil(n, K.matvec_rows), m, 1))
+    got = c.read(out).reshape(m, n)
+    assert np.all(np.isposinf(got[0])) and np.all(np.isneginf(got[1])) and np.all(np.isnan(got[2]))
+    g, u = x.astype(np.float64) @ w[0].astype(np.float64), x.astype(np.float64) @ w[-1].astype(np.float64)
+    want = g * sigmoid64(g) * u if pair else u
+    assert rel_err(got[3], np.full(n, want[3])) <= 1e-5
+    if not pair and half == "f16":
+        assert rel_err(got[4], np.full(n, want[4])) <= 1e-5
+
+
 @pytest.mark.parametrize("half", HALVES)
 def test_matvec_bf16_silu_pair(ctx, half):
     c = ctx

@@ -146,18 +146,28 @@ __device__ __forceinline__ uint2 bf16_piece(const float4 &v, uint32_t p) {
     return w;
 }
 
-// The power of two that puts a token's largest magnitude `big` in [2^14, 2^15), and one over it.
+// The larger of `big` and the magnitudes in v, infinities left out with FINITE (and NaNs always).
+template <bool FINITE>
+__device__ __forceinline__ float largest(float big, const float4 &v) {
+    const float x[4] = {fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w)};
+#pragma unroll
+    for (int j = 0; j < 4; j++) big = fmaxf(big, FINITE && x[j] == __builtin_inff() ? 0.f : x[j]);
+    return big;
+}
+
+// The power of two that puts a token's largest finite magnitude `big` in [2^14, 2^15) (2^126 for one
+// below the normal numbers), and one over it.
 __device__ __forceinline__ void f16_scale(float big, float &scale, float &inverse) {
     const int e = (int)((__float_as_uint(big) >> 23) & 0xffu);  // biased exponent; 0 for zero and subnormals
     int se = 127 + 14 - (e - 127);                               // scale = 2^(14 - (e - 127)), kept normal both ways
     se = se < 1 ? 1 : se > 253 ? 253 : se;
-    const bool unit = e == 0 || e == 255;
-    scale = unit ? 1.0f : __uint_as_float((uint32_t)se << 23);
-    inverse = unit ? 1.0f : __uint_as_float((uint32_t)(254 - se) << 23);
+    scale = __uint_as_float((uint32_t)se << 23);
+    inverse = __uint_as_float((uint32_t)(254 - se) << 23);
 }
 
 // Four scaled values as their f16 roundings, what those left times 2^11 and, with PIECES 3, what that left
-// times 2^22: eleven significant bits each, an f32 input's 24 in three.
+// times 2^22: eleven significant bits each, an f32 input's 24 in three. Infinities and NaNs are what they are
+// in the first; what an infinity leaves, a NaN, becomes a finite number, any being as good beside it.
 template <uint32_t PIECES>
 __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (&w)[PIECES]) {
     const float x[4] = {v.x, v.y, v.z, v.w};
@@ -166,7 +176,7 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (
     for (int j = 0; j < 4; j++) {
         // The scale is a power of two, so x * scale - q in one fused operation is exact, and so is what the next leaves.
         q[0][j] = (_Float16)(x[j] * scale);
-        const float rest = fmaf(x[j], scale, -(float)q[0][j]) * 2048.0f;
+        const float rest = fmaxf(fmaf(x[j], scale, -(float)q[0][j]) * 2048.0f, -32768.0f);
         q[1][j] = (_Float16)rest;
         if constexpr (PIECES == 3) q[2][j] = (_Float16)((rest - (float)q[1][j]) * 2048.0f);
     }
@@ -302,9 +312,16 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
         if constexpr (F16) {
             float big = 0.f;
 #pragma unroll
-            for (int j = 0; j < 2 * NP; j++) big = fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fmaxf(fabsf(v[j].z), fabsf(v[j].w)), big));
+            for (int j = 0; j < 2 * NP; j++) big = largest<false>(big, v[j]);
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off, 64));
+            if (big == __builtin_inff()) {
+                big = 0.f;
+#pragma unroll
+                for (int j = 0; j < 2 * NP; j++) big = largest<true>(big, v[j]);
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off, 64));
+            }
             float scale, inverse;
             f16_scale(big, scale, inverse);
             if (lane == 0) lds_inverse[wave] = inverse;
@@ -441,10 +458,7 @@ __global__ __launch_bounds__(256) void matvec_f16_split_kernel(MvArgs a, uint2 *
     __syncthreads();
     const uint32_t tid = threadIdx.x, k4 = a.k / 4u;
     float big = 0.f;
-    for (uint32_t i = tid; i < k4; i += 256u) {
-        const float4 v = staged[i];
-        big = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fmaxf(fabsf(v.z), fabsf(v.w)), big));
-    }
+    for (uint32_t i = tid; i < k4; i += 256u) big = largest<true>(big, staged[i]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off, 64));
     if ((tid & 63u) == 0) red[tid >> 6] = big;
