@@ -601,7 +601,7 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
             zhip_result r;
             if (pair) {
                 if (f16) r = launch_for_k<false, true, false, true>(d, q, grid);
-                else r = split ? launch_for_k<true, false, false, true>(d, q, grid) : launch_for_k<false, false, false, true>(d, q, grid);
+                else r = launch_for_k<false, false, false, true>(d, q, grid);  // (above 3072 weights that is the split tokens' kernel)
             } else if (f16) r = split ? launch_for_k<true, true>(d, q, grid) : launch_for_k<false, true>(d, q, grid);
             else r = split ? launch_for_k<true, false>(d, q, grid) : launch_for_k<false, false>(d, q, grid);
             if (r != ZHIP_OK) return r;

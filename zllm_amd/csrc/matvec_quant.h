@@ -894,6 +894,7 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
 constexpr int kRowDepth = 1;
 template <class P, int MT, bool PAIR, bool TURNS, int SEG_LOG2>
 __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
+    static_assert(PAIR || !TURNS, "rows in turn are a pair's");
     const MvArgs &a = q.a;
     extern __shared__ float4 lds4[];
     __shared__ float red[4 * MT];
@@ -1546,20 +1547,18 @@ static zhip_result run_slices(const Dispatch &d, const KArgs &q, uint32_t lds, u
     return check_launch(d, P::name());
 }
 
-template <class P, int MT, bool PAIR, bool TURNS = false>
-static zhip_result run_row(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
-    if (lds > 65536u) {
-        const bool ok = q.seg_log2 == 4u ? lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, TURNS, 4>, 160 * 1024 - 64>()
-                      : q.seg_log2 == 5u ? lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, TURNS, 5>, 160 * 1024 - 64>()
-                                         : lds_opt_in<matvec_quant_row_kernel<P, MT, PAIR, TURNS, 6>, 160 * 1024 - 64>();
-        if (!ok) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
-    }
-    switch (q.seg_log2) {
-    case 4: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, TURNS, 4>), dim3(blocks), dim3(256), lds, d.stream, q); break;
-    case 5: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, TURNS, 5>), dim3(blocks), dim3(256), lds, d.stream, q); break;
-    default: hipLaunchKernelGGL((matvec_quant_row_kernel<P, MT, PAIR, TURNS, 6>), dim3(blocks), dim3(256), lds, d.stream, q); break;
-    }
+// Which gate / up steps take their two rows in turn (see launch_quant).
+template <class P, int MT, bool PAIR, int SEG_LOG2> constexpr bool row_turns() { return PAIR && MT == 2 && !(P::PAIR2 && SEG_LOG2 == 6); }
+template <class P, int MT, bool PAIR, int SEG_LOG2>
+static zhip_result run_row_seg(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
+    constexpr auto kernel = matvec_quant_row_kernel<P, MT, PAIR, row_turns<P, MT, PAIR, SEG_LOG2>(), SEG_LOG2>;
+    if (lds > 65536u && !lds_opt_in<kernel, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, d.stream, q);
     return check_launch(d, P::name());
+}
+template <class P, int MT, bool PAIR>
+static zhip_result run_row(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
+    return q.seg_log2 == 4u ? run_row_seg<P, MT, PAIR, 4>(d, q, lds, blocks) : q.seg_log2 == 5u ? run_row_seg<P, MT, PAIR, 5>(d, q, lds, blocks) : run_row_seg<P, MT, PAIR, 6>(d, q, lds, blocks);
 }
 
 template <class P, int MT, bool PAIR, int STG>
@@ -1723,8 +1722,7 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             const uint32_t cap = cus * (three ? 3u : 2u), row_blocks = row_want < cap ? row_want : cap;
             const uint32_t row_lds = mt * q.tasks * kTaskStride * 4u;
             if (mt == 1u) r = pair ? run_row<P, 1, true>(d, q, row_lds, row_blocks) : run_row<P, 1, false>(d, q, row_lds, row_blocks);
-            else if (pair) r = P::PAIR2 && q.seg_log2 == 6u ? run_row<P, 2, P::PAIR2, !P::PAIR2>(d, q, row_lds, row_blocks) : run_row<P, 2, true, true>(d, q, row_lds, row_blocks);
-            else r = run_row<P, 2, false>(d, q, row_lds, row_blocks);
+            else r = pair ? run_row<P, 2, true>(d, q, row_lds, row_blocks) : run_row<P, 2, false>(d, q, row_lds, row_blocks);
         } else if (mt == 1u) r = pair ? run_quant<P, 1, true, 1>(d, q, lds, blocks) : run_quant<P, 1, false, 1>(d, q, lds, blocks);
         else if (mt == 2u) {
             if (small && P::STAGE2 != 2) r = pair ? run_quant<P, 2, true, 2>(d, q, lds, blocks) : run_quant<P, 2, false, 2>(d, q, lds, blocks);
