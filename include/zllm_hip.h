@@ -52,15 +52,21 @@ enum {
  * hosts record command lists per submit (src/agility/host.zig:520-548). */
 #define ZHIP_OPTION_NO_REPLAY 1u
 /* matvec_bf16 / matvec_f16 over 16 MB or more of weights (k = 1024 ... 16384 in
- * steps of 512) read the weights once for all of a step's tokens on the matrix
+ * steps of 512; gate / up steps over 16 MB or more of gate rows, k = 1024 ...
+ * 4096) read the weights once for all of a step's tokens on the matrix
  * cores, at every width from one token on, so that a token's bits do not depend
  * on the width of the step it ran in (src/sched/sched.zig:55-58,
- * src/plan/qwen35.zig:380-381). For deployments that verify speculated tokens
- * on these matrices: a step of 2..8 tokens then costs what one token does
- * (151936 x 1024 bf16: 55 us at any width; without the flag 52 / 75 / 122 us at
- * 1 / 4 / 8 tokens). Without the flag every width runs the kernel that takes the
- * tokens one pass each, whose one-token step is ~6 % faster; either way the
- * route depends on the matrix alone, never on the step. */
+ * src/plan/qwen35.zig:380-381). For deployments that decode or verify around
+ * eight tokens a step on these matrices: a step of 2..8 tokens then costs what
+ * one token does, which is more than one token costs without the flag. us at
+ * 1 / 2 / 4 / 8 tokens with the flag, and without (f16, RMSNorm prologue):
+ *   151936 x 1024     53 / 54 / 54 / 54       54 / 57 / 65 / 105
+ *   2 x 8192 x 2048   18 / 18 / 18 / 18       14 / 15 / 17 / 38
+ *   4096 x 4096       13 / 13 / 13 / 14       8 / 12 / 15 / 24
+ * Inputs are taken with all their 24 bits, except that matvec_f16 steps other
+ * than gate / up ones keep 22 (relative to the token's largest input). Weights
+ * are taken to be finite: an infinite or NaN weight makes its outputs NaN.
+ * Either way the route depends on the matrix alone, never on the step. */
 #define ZHIP_OPTION_WIDE_DECODE 2u
 
 typedef struct zhip_options {
@@ -131,7 +137,9 @@ zhip_result zhip_set_file(zhip_context *context, const void *bytes, size_t len);
  * one for the submit token. `*out_count` receives the completions written; a
  * batch producing more than `capacity` fails with ZHIP_E_INVALID_ARGUMENT
  * before anything runs. On ZHIP_E_UNSUPPORTED_KERNEL the submission in
- * progress is dropped. */
+ * progress is dropped. The destinations of a submit's reads are its own until
+ * it returns: where it fails, what they hold is undefined (a long read is handed
+ * over while its last bytes still arrive). */
 zhip_result zhip_execute(zhip_context *context, const uint32_t *words, size_t n_words,
     zhip_completion *out_completions, size_t capacity, size_t *out_count);
 

@@ -7,7 +7,8 @@
 //
 // Arithmetic. v_mfma_f32_32x32x16_bf16 multiplies 32 rows of inputs by 32 weight rows over
 // sixteen positions. The weights are bf16 already and reach the instruction as loaded. An f32
-// input is the exact sum of three bf16 values (its upper sixteen bits, the upper sixteen bits of
+// input is the exact sum of three bf16 values (f16 weights have their own split, see F16 below;
+// of bf16: its upper sixteen bits, the upper sixteen bits of
 // what that left, and the rest: eight significant bits each), so a token enters as three operand
 // rows, every product is exact in the f32 accumulator, and the three rows' sums are added at the
 // end. Eight tokens fill 24 of the 32 operand rows; the other eight are zeros. A token's rows
@@ -197,7 +198,7 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (
 // what those two left times 2^22, and an input keeps all its bits (the general kernel, which takes
 // pairs without ZHIP_OPTION_WIDE_DECODE, has them too): the matrix instruction has the rows anyway.
 // PAIR: a SILU_PAIR step, an output tile's gate rows and then its up rows (the general kernel's
-// time grows with the tokens: 2 x 8192 x 2048 f16 at eight 39 us, here 17).
+// time grows with the tokens: 2 x 8192 x 2048 f16 at eight 38 us, here 18).
 // LONG: k = 512 NP q.parts; workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
 // walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums.
 template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>

@@ -23,6 +23,8 @@
 //   1024 x 3072, accumulating, at 1 / 2             4.9 / 6.1 -> 3.6 / 4.0
 //   2560 x 4096 / 4096 x 4096, one token            8.8 / 9.6 -> 6.3 / 8.1
 //   2 x 8192 x 2048 / 2 x 9728 x 2560, one token    15.4 / 23.4 -> 13.0 / 18.5
+//   2 x 5120 x 5120 / 2 x 13824 x 5120, one token   22.6 / 53.5 -> 19.9 / 50.5 (f16, three registers of whose
+//                                                   pair do not fit: 22.9 / 53.3 -> 20.9 / 52.9)
 //   151936 x 1024 (311 MB), one token               52.8 -> 52.2 (6.0 TB/s)
 // Short launches are bound by the launch itself (about 2.3 us with nothing in it) and one trip to
 // memory, long ones by HBM.
