@@ -64,8 +64,7 @@ enum {
  *   2 x 8192 x 2048   18 / 18 / 18 / 18       14 / 15 / 17 / 38
  *   4096 x 4096       13 / 13 / 13 / 14       8 / 12 / 15 / 24
  * Inputs are taken with all their 24 bits, except that matvec_f16 steps other
- * than gate / up ones keep 22 (relative to the token's largest input). Weights
- * are taken to be finite: an infinite or NaN weight makes its outputs NaN.
+ * than gate / up ones keep 22 (relative to the token's largest input).
  * Either way the route depends on the matrix alone, never on the step. */
 #define ZHIP_OPTION_WIDE_DECODE 2u
 

@@ -366,6 +366,32 @@ def test_matvec_bf16_several_tokens_infinities(ctx_wide, half, pair, k):
         assert rel_err(got[4], np.full(n, want[4])) <= 1e-5
 
 
+@pytest.mark.parametrize("pair,k", [(False, 1024), (False, 4608), (False, 8192), (True, 1024), (True, 4096)])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_infinite_weights(ctx_wide, half, pair, k):
+    """An infinite weight gives infinite outputs on the matrix cores too, of inputs that are one piece and of
+    inputs that are three, and touches no other row's."""
+    c = ctx_wide
+    m, n = 3, (16 << 20) // (2 * k) + 1
+    x = np.abs(c.random(m * k, 1)).reshape(m, k) + np.float32(0.5)
+    x[0, 11], x[1, 11] = 1.0, np.float32(1.2345678)
+    w = np.full((2 * n if pair else n, k), 0.5, np.float32)
+    w[-n:][5, 11], w[-n:][n - 1, 11] = np.inf, -np.inf
+    if pair:
+        w[7, 11] = np.inf
+    bits = w.astype(np.float16).view(np.uint16) if half == "f16" else (w.view(np.uint32) >> 16).astype(np.uint16).reshape(-1)
+    out = c.output(m * n)
+    c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=1e-6, silu_pair=pair, half=n if pair else 0),
+                        [c.upload(x), c.upload(bits), out, c.upload(x)], (K.div_ceil(n, K.matvec_rows), m, 1))
+    got = c.read(out).reshape(m, n)
+    assert np.all(np.isposinf(got[:, 5])) and np.all(np.isneginf(got[:, n - 1]))
+    if pair:
+        assert np.all(np.isposinf(got[:, 7]))
+    others = [j for j in range(n) if j not in (5, n - 1) and not (pair and j == 7)]
+    g = x.astype(np.float64).sum(axis=1) * 0.5
+    assert rel_err(got[:, others], np.repeat((g * sigmoid64(g) * g if pair else g)[:, None], len(others), axis=1)) <= 1e-5
+
+
 @pytest.mark.parametrize("half", HALVES)
 def test_matvec_bf16_silu_pair(ctx, half):
     c = ctx

@@ -361,7 +361,11 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     auto finish = [&](uint32_t p, const hf32x16 &sum) __attribute__((always_inline)) {
         float *part = lds_part + (p & 1u) * (WAVES * 256u);
 #pragma unroll
-        for (int i = 0; i < 4; i++) part[wave * 256u + 64u * i + lane] = !F16 ? (sum[i] + sum[4 + i]) + sum[8 + i] : fmaf(PIECES == 3 ? fmaf(sum[8 + i], 1.0f / 2048.0f, sum[4 + i]) : sum[4 + i], 1.0f / 2048.0f, sum[i]);
+        for (int i = 0; i < 4; i++) {
+            const float all = !F16 ? (sum[i] + sum[4 + i]) + sum[8 + i] : fmaf(PIECES == 3 ? fmaf(sum[8 + i], 1.0f / 2048.0f, sum[4 + i]) : sum[4 + i], 1.0f / 2048.0f, sum[i]);
+            // (an infinite weight makes an infinity of an input's first piece, but NaNs of pieces that are zero)
+            part[wave * 256u + 64u * i + lane] = fabsf(sum[i]) == __builtin_inff() ? sum[i] : all;
+        }
         lds_barrier();
         // Buffer p % 2 is written again in step p + 2, after the barrier of step p + 1, which a
         // wave passes only when it has read what it needs here. The 256 outputs of a tile are
