@@ -338,6 +338,27 @@ def test_matvec_bf16_several_tokens_special_values(ctx_wide):
     assert np.all(np.isnan(got[3]))
 
 
+@pytest.mark.parametrize("k", [1536, 2048, 3072, 4096])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_pair_error(ctx, ctx_wide, half, k):
+    """A gate / up step on the matrix cores is no further from float64 than the default context's kernel, in the
+    2-norm over thousands of outputs a token (both are sums of f32 in another order, whose errors over that many
+    outputs are steady to a few in a hundred)."""
+    m, n, eps = 8, (16 << 20) // (2 * k) + 1, 1e-6
+    x, nw = ctx.rand.standard_normal((m, k), dtype=np.float32), ctx.random(k, 1)
+    bits, values = random_half(ctx, 2 * n * k, (3 / k) ** 0.5, half)
+    p = np.stack([norm_row(t, nw, eps) for t in x]) @ values.reshape(2 * n, k).astype(np.float64).T
+    want = p[:, :n] * sigmoid64(p[:, :n]) * p[:, n:]
+
+    def error(c):
+        out = c.output(m * n)
+        c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=eps, norm=True, silu_pair=True, half=n),
+                            [c.upload(x), c.upload(bits), out, c.upload(nw)], (K.div_ceil(n, K.matvec_rows), m, 1))
+        return np.linalg.norm(c.read(out).reshape(m, n) - want) / np.linalg.norm(want)
+
+    assert error(ctx_wide) <= 1.05 * error(ctx)
+
+
 @pytest.mark.parametrize("pair,k", [(False, 1024), (False, 4608), (False, 8192), (True, 1024), (True, 4096)])
 @pytest.mark.parametrize("half", HALVES)
 def test_matvec_bf16_several_tokens_infinities(ctx_wide, half, pair, k):
