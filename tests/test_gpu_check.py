@@ -1815,6 +1815,29 @@ def test_matmul_q8_0_int8_whole_steps_keep_token_bits(ctx):
         assert got[first : first + count].tobytes() == run(first, count).tobytes(), "token chunking changed bits"
 
 
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 1024, 1152])
+def test_matmul_q8_0_int8_scales_in_chunks(ctx, k):
+    """matmul_q8_0's kernel for 128-deep steps brings the scales sixteen units at a time: fewer
+    steps than its ring has slots, chunks that end with k and chunks that do not, both tile
+    heights, ragged rows; against float64 over the rounded activations, 1e-5
+    (src/kernels/check.zig:839-871), and a token alone against the whole step bit for bit."""
+    c, t, n, rows = ctx, TensorType.q8_0, 8230, 97
+    x = c.random(rows * k, 1).reshape(rows, k)
+    xs = oracle.round_like_llama(ORACLE_TYPE[t], x)
+    raw, values = quant_rows(c, t, n, k)
+    wa = c.gpu_weights(t, raw, k)
+
+    def run(first, count, wide):
+        out = c.output(count * wide)
+        launch_int8(c, t, quantize_x(c, t, c.upload(x[first : first + count]), count, k), wa, out, count, wide, k, 0, None)
+        return c.read(out).reshape(count, wide)
+
+    got = run(0, rows, n)  # 64-token tiles
+    assert rel_err(got, xs.astype(np.float64) @ values.astype(np.float64).T) <= 1e-5
+    for first, count in ((0, 1), (31, 33), (96, 1)):  # 32-token tiles, over the first rows of the matrix
+        assert run(first, count, 100).tobytes() == np.ascontiguousarray(got[first : first + count, :100]).tobytes()
+
+
 def test_silu_mul(ctx):
     c = ctx
     rows, width = 7, 10_001

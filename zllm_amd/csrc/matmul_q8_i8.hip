@@ -6,12 +6,9 @@
 //
 // The work per output and unit is one 32-deep integer dot product (the int8 matrix cores do
 // 1024 of them per instruction) and its scaling by dx * dw, which does not factor out of the
-// sum over units. On MI355X matrix and vector instructions of a SIMD's waves do not overlap
-// (measured: an instruction stream of both takes the sum of their times), a wave-wide f32
-// multiply-add takes ~1.4 ns of a SIMD with two waves resident, an int -> float conversion
-// 1.9 ns, v_mfma_i32_32x32x32_i8 16.5 ns and v_mfma_f32_32x32x1_2b_f32 29.7 ns. Scaled with
-// three vector operations per output and unit (scale product, conversion, multiply-add) the
-// scaling takes five times the dot products' time and bounds the kernel. So:
+// sum over units. A stream of matrix and vector instructions takes the sum of their times here;
+// with four waves a SIMD an f32 add or multiply-add takes 1.1 - 1.3 ns of it, an int -> float conversion
+// 2.0 ns, v_mfma_i32_32x32x32_i8 14 - 16 ns and v_mfma_f32_32x32x1_2b_f32 28 ns. So:
 //  * the scale products are a matrix instruction: v_mfma_f32_32x32x1_2b_f32 (two independent
 //    32 x 32 outer products: lanes 0-31 and 32-63 each give a column of row scales and a row of
 //    token scales) yields dx * dw for two token tiles, rounded once to f32 like the vector
@@ -19,13 +16,20 @@
 //  * the integer sums start from the bits of 1.5 * 2^23 (the matrix instruction's addend): the
 //    result's bits are then those of the float 1.5 * 2^23 + sum, and one exact f32 subtraction
 //    replaces the conversion.
-// Two full-rate vector operations per output and unit remain.
+// Two full-rate vector operations per output and unit remain: 60 ns a unit and 32 x 32 tile in
+// registers alone, of the 100 ns that large steps take with their loads, reads and barriers.
+// Short steps are bound by the launch, the trips to memory and the exchange at the end.
 //
-// Tiling as in matmul_q8_bf16.hip: a workgroup computes 128 (or 64, or 32) tokens x 64 matrix rows;
-// wave w multiplies rows 32 (w % 2) .. + 31 by all the tile's tokens over unit w / 2 of every
-// step, lane l holding row (token) l % 32 and bytes 16 (l / 32) .. + 15 of the unit. Operands
-// arrive straight in LDS (range-checked buffers: what lies past a binding reads as zero) three
-// steps ahead, every wave issuing its share; fragments are read one step ahead. The four units'
+// A workgroup computes 64 (or 32) tokens x 64 matrix rows; wave w multiplies rows 32 (w % 2) .. + 31
+// by all the tile's tokens over unit w / 2 of every 128-deep step, lane l holding row (token) l % 32 and bytes
+// 16 (l / 32) .. + 15 of the unit. Operands arrive straight in LDS (range-checked buffers: what lies
+// past a binding reads as zero) three steps ahead, every wave issuing its share. The scales arrive
+// four steps at a time: a step's alone are 8 and 16 bytes of a line a row and token, and a step that
+// asked for them moved as many lines for its scales as for its operands, which made it 0.57 us long whatever
+// the tile (64 x 4096 x 4096 18.8 -> 13.8 us, 512 x 3072 x 1024 11.8 -> 10.9). At most 128 registers
+// a wave and 80 KB a workgroup, so that two workgroups share a CU and one multiplies while the
+// other starts or exchanges (512 x 1024 x 6144 22.3 -> 17.1 us, 512 x 4096 x 4096 35.0 -> 31.6; a
+// workgroup of 128 tokens and sixteen waves a CU: 20.9, 31.6). The four units'
 // sums meet through LDS at the end, always as (u0 + u2) + (u1 + u3): a token's bits depend
 // neither on the tokens beside it nor on the tile height.
 #include <hip/hip_runtime.h>
@@ -45,16 +49,16 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int BN = 64, BK = 128, WAVES = 8, THREADS = 64 * WAVES;
-// One step in LDS: token lines [token][128 B], weight lines [row][128 B], then per wave 256 bytes
-// of row scales ([8 rows][4 f16], the rest filler) and 256 bytes of token scales ([16 tokens][4 f32]).
-template <int TT> constexpr int abuf_bytes() { return 32 * TT * 128; }
-constexpr int WBUF = BN * 128, SBUF = WAVES * 256, DBUF = WAVES * 256;
-// (and, with 32-token tiles, a spare KB where the loads of the four waves that have no token
-// lines to bring land their nothing)
-template <int TT> constexpr int buf_bytes() { return abuf_bytes<TT>() + WBUF + SBUF + DBUF + (TT == 1 ? 1024 : 0); }
-// Three buffers, or the exchange of the four units' sums that reuses them (8 waves x 3 inboxes x TT KB).
-template <int TT> constexpr int lds_bytes() { return 3 * buf_bytes<TT>() > 8 * 3 * TT * 1024 ? 3 * buf_bytes<TT>() : 8 * 3 * TT * 1024; }
-static_assert(lds_bytes<4>() <= 160 * 1024, "the buffers must fit the CU's LDS");
+// A step in LDS: token lines [token][128 B], then weight lines [row][128 B]; four steps in the ring.
+// The scales come four steps (sixteen units) at a time: [token][16 f32], then [row][16 f16], twice.
+constexpr int RING = 4, WBUF = BN * 128, SBUF = BN * 32;
+template <int TW>
+struct Tile {
+    static constexpr int BM = 32 * TW, ABUF = BM * 128, BUF = ABUF + WBUF, DBUF = BM * 64, CHUNK = DBUF + SBUF;
+    // The rings, or the exchange of the four units' sums that reuses them (8 waves x 3 inboxes x TW KB).
+    static constexpr int RINGS = RING * BUF + 2 * CHUNK, EXCHANGE = WAVES * 3 * TW * 1024, LDS = RINGS > EXCHANGE ? RINGS : EXCHANGE;
+    static_assert(2 * LDS <= 160 * 1024, "two workgroups' buffers must fit the CU's LDS");
+};
 
 struct Q8I8Args {
     const uint8_t *qx;  // rows x k int8
@@ -92,80 +96,75 @@ __device__ __forceinline__ void sync_keeping_loads() {
 // at the LDS's full rate.
 __device__ __forceinline__ uint32_t line_key(uint32_t row) { return (row & 7u) ^ ((row >> 3) & 1u); }
 
-template <int TT>
-struct Frags {
-    i32x4 w, tok[TT];  // the row's and each tile's token's sixteen bytes of the unit
-    float dw, dx[(TT + 1) / 2];  // the row's scale; the scale of the lane's token in tile 2 pair + lane / 32
-};
-
-template <int TT>
-__global__ __launch_bounds__(THREADS) void matmul_q8_i8_kernel(Q8I8Args a) {
+template <int TW>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void matmul_q8_i8_kernel(Q8I8Args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    constexpr int BM = 32 * TT, ABUF = abuf_bytes<TT>(), BUF = buf_bytes<TT>();
-    constexpr int XL = (TT + 1) / 2;      // token-line loads a wave issues per step (32-token tiles: four of the waves bring nothing)
-    constexpr int PER_STEP = XL + 3;
+    typedef Tile<TW> T;
+    constexpr uint32_t BUF = T::BUF, CHUNKS_AT = RING * BUF, CHUNK = T::CHUNK;
+    constexpr int PAIRS = (TW + 1) / 2;
+    // Lines a wave loads a step, of tokens and of rows; token lines of a scale load; loads a step and a chunk.
+    constexpr uint32_t XROWS = T::BM / WAVES, WROWS = BN / WAVES;
+    constexpr int PER_STEP = 2, DL = XROWS / 4, PER_CHUNK = DL + 1;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t j0 = blockIdx.x * BN, t0 = blockIdx.y * BM;
+    const uint32_t j0 = blockIdx.x * BN, t0 = blockIdx.y * T::BM;
     const uint32_t steps = a.k / BK;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
 
-    // ---- this wave's loads: token blocks wave and wave + 8 (8 tokens x 128 B each), weight
-    // rows 8 wave .. + 7, their scales and the scales of tokens 16 wave .. + 15.
+    // ---- this wave's loads: token lines XROWS wave .. (with 32-token tiles half a wave's load), weight
+    // lines WROWS wave ..; a chunk's scales of the same lines, a word a lane.
     const __amdgpu_buffer_rsrc_t xbuf = make_buffer(a.qx, a.qx_bytes), wbuf = make_buffer(a.w, a.w_bytes), dbuf = make_buffer(a.dx, a.dx_bytes);
-    uint32_t xoff[XL];
-#pragma unroll
-    for (int i = 0; i < XL; i++) {
-        const uint32_t row = 8u * (wave + 8u * i) + (lane >> 3);
-        xoff[i] = row < (uint32_t)BM ? (t0 + row) * a.k + 16u * ((lane & 7u) ^ line_key(row)) : 0xF0000000u;
-    }
-    const uint32_t wrow = 8u * wave + (lane >> 3);
+    const uint32_t xrow = XROWS * wave + (lane >> 3);
+    const uint32_t xoff = (t0 + xrow) * a.k + 16u * ((lane & 7u) ^ line_key(xrow));
+    const uint32_t wrow = WROWS * wave + (lane >> 3);
     const uint32_t woff = (j0 + wrow) * a.row_bytes + 16u * ((lane & 7u) ^ line_key(wrow));
-    const uint32_t soff = lane < 16u ? (j0 + 8u * wave + (lane >> 1)) * a.row_bytes + a.k + 4u * (lane & 1u) : 0xF0000000u;
-    const uint32_t dtok = 16u * wave + (lane >> 2);
-    const uint32_t doff = dtok < (uint32_t)BM ? ((t0 + dtok) * (a.k / 32u) + (lane & 3u)) * 4u : 0xF0000000u;
+    // (A step past the end of k is asked for like the rest, so that every wait counts the same loads,
+    // but as the last one: nothing reads it.)
     auto fetch = [&](uint32_t buf, uint32_t step) __attribute__((always_inline)) {
-        const uint32_t base = lds0 + buf * BUF;
+        const uint32_t base = lds0 + buf * BUF, at = 128u * min(step, steps - 1u);
+        if (XROWS == 8u || lane < 8u * XROWS) load_lds_b128(xbuf, base + 128u * XROWS * wave, xoff, at);
+        load_lds_b128(wbuf, base + T::ABUF + 128u * WROWS * wave, woff, at);
+    };
+    // Units 4 p .. + 3 of token t lie at position p ^ (t / 4 % 4) of its 64 bytes: a step's reads of
+    // sixteen tokens fall in sixteen bank groups. (What a ragged last chunk asks for past the end of
+    // k is the next row's, or past the buffer's end and zero; nothing reads it. The lanes' offsets
+    // are worked out again every time: kept, they would not fit the registers.)
+    auto fetch_scales = [&](uint32_t parity, uint32_t chunk) __attribute__((always_inline)) {
+        const uint32_t base = lds0 + CHUNKS_AT + parity * CHUNK;
+        uint32_t l = lane;
+        asm volatile("" : "+v"(l));
+        const uint32_t first = (t0 + XROWS * wave + (l >> 4)) * (a.k / 8u) + 64u * chunk;
 #pragma unroll
-        for (int i = 0; i < XL; i++)
-            load_lds_b128(xbuf, base + (8u * (wave + 8u * i) < (uint32_t)BM ? 1024u * (wave + 8u * i) : (uint32_t)(ABUF + WBUF + SBUF + DBUF)), xoff[i], 128u * step);
-        load_lds_b128(wbuf, base + ABUF + 1024u * wave, woff, 128u * step);
-        load_lds_b32(wbuf, base + ABUF + WBUF + 256u * wave, soff, 8u * step);
-        load_lds_b32(dbuf, base + ABUF + WBUF + SBUF + 256u * wave, doff, 16u * step);
+        for (uint32_t i = 0; i < (uint32_t)DL; i++)
+            load_lds_b32(dbuf, base + 64u * (XROWS * wave + 4u * i), first + i * (a.k / 2u) + 4u * ((l & 15u) ^ (4u * ((XROWS / 4u * wave + i) & 3u))), 0);
+        load_lds_b32(wbuf, base + T::DBUF + 32u * WROWS * wave, (j0 + WROWS * wave + (l >> 3)) * a.row_bytes + a.k + 32u * chunk + 4u * (l & 7u), 0);
     };
 
-    // ---- this wave's fragments
+    // ---- this wave's fragments: rows 32 wn .. + 31, the TW token tiles, unit kq of a step
     const uint32_t lrow = lane & 31u, h = lane >> 5, wn = wave & 1u, kq = wave >> 1;
-    const uint32_t key = line_key(lrow);
-    const uint32_t wr = 32u * wn + lrow;
-    const uint32_t chunk = 16u * ((2u * kq + h) ^ key);
+    const uint32_t chunk = 16u * ((2u * kq + h) ^ line_key(lrow));
     const uint32_t a_at = lrow * 128u + chunk;
-    const uint32_t w_at = ABUF + wr * 128u + chunk;
-    const uint32_t s_at = ABUF + WBUF + 256u * (wr >> 3) + 8u * (wr & 7u) + 2u * kq;
-    const uint32_t d_at = ABUF + WBUF + SBUF + 16u * (32u * h + lrow) + 4u * kq;
+    const uint32_t w_at = T::ABUF + (32u * wn + lrow) * 128u + chunk;
+    const uint32_t s_at = CHUNKS_AT + T::DBUF + 32u * (32u * wn + lrow) + 2u * kq;
+    const uint32_t d_at = CHUNKS_AT + 64u * ((TW == 1 ? 0u : 32u * h) + lrow) + 4u * kq, d_key = 16u * (lrow >> 2 & 3u);
 
-    f32x16 acc[TT];
+    float acc[TW][16];
 #pragma unroll
-    for (int i = 0; i < TT; i++)
+    for (int i = 0; i < TW; i++)
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[i][e] = 0.f;
 
-    Frags<TT> f;
-    auto read_tile = [&](uint32_t buf, int tt) __attribute__((always_inline)) {
-        f.tok[tt] = *reinterpret_cast<const i32x4 *>(lds + buf * BUF + a_at + 4096 * tt);
+    i32x4 w, tok[TW];    // the row's and each tile's token's sixteen bytes of the unit
+    float dw, dx[PAIRS];  // the row's scale; the scale of the lane's token in tile 2 pair + lane / 32
+    // The operands of the step in buffer `buf` of the ring, its scales those of the chunk at `at`.
+    auto read_step = [&](uint32_t buf, uint32_t at) __attribute__((always_inline)) {
+        w = *reinterpret_cast<const i32x4 *>(lds + buf * BUF + w_at);
+        dw = (float)*reinterpret_cast<const _Float16 *>(lds + at + s_at + 8u * buf);
+#pragma unroll
+        for (int tt = 0; tt < TW; tt++) tok[tt] = *reinterpret_cast<const i32x4 *>(lds + buf * BUF + a_at + 4096 * tt);
+#pragma unroll
+        for (int pair = 0; pair < PAIRS; pair++) dx[pair] = *reinterpret_cast<const float *>(lds + at + (d_at + ((16u * buf) ^ d_key)) + 4096 * pair);
     };
-    auto read_scales = [&](uint32_t buf, int pair) __attribute__((always_inline)) {
-        f.dx[pair] = *reinterpret_cast<const float *>(lds + buf * BUF + d_at + 1024 * pair);
-    };
-    auto read_rows = [&](uint32_t buf) __attribute__((always_inline)) {
-        f.w = *reinterpret_cast<const i32x4 *>(lds + buf * BUF + w_at);
-        f.dw = (float)*reinterpret_cast<const _Float16 *>(lds + buf * BUF + s_at);
-    };
-    // A tile's matrix instructions run for ~100 cycles before their results can be read, and only
-    // two waves share a SIMD: a tile's scaling (32 vector instructions) is issued after the next
-    // tiles' matrix instructions, the last tile's after the next step's first ones. A tile's
-    // fragments of the next step are read into its registers once its matrix instructions have
-    // been issued.
     // The integer sums start from the bits of 1.5 * 2^23: bits + sum are then the bits of the
     // float 1.5 * 2^23 + sum (|sum| <= 32 * 127 * 127 < 2^22, one unit in the last place is 1), and
     // the exact subtraction below replaces a conversion (half the rate of an addition here).
@@ -175,138 +174,85 @@ __global__ __launch_bounds__(THREADS) void matmul_q8_i8_kernel(Q8I8Args a) {
 #pragma unroll
     for (int e = 0; e < 16; e++) magic[e] = MAGIC_BITS;
     asm volatile("" : "+v"(magic));  // sixteen registers, set once
-    i32x16 sums_left = magic;
-    f32x16 scale_left = {};
-    auto scale_into = [&](f32x16 &to, const i32x16 &sums, const f32x16 &scale) __attribute__((always_inline)) {
-        const f32x16 exact = __builtin_bit_cast(f32x16, sums) - MAGIC;
+    auto multiply = [&]() __attribute__((always_inline)) {
+        const f32x32 none = {};
 #pragma unroll
-        for (int e = 0; e < 16; e++) to[e] = fmaf(exact[e], scale[e], to[e]);
-    };
-    auto low = [](const f32x32 &v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15); };
-    auto high = [](const f32x32 &v) { return __builtin_shufflevector(v, v, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31); };
-    auto multiply = [&](uint32_t nxt_buf) __attribute__((always_inline)) {
-        const i32x16 zero_i = magic;
-        const f32x32 zero_f = {};
-        i32x16 sums[TT];
-        f32x32 scale[(TT + 1) / 2];
-        sums[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.w, f.tok[0], zero_i, 0, 0, 0);
-        scale[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(f.dw, f.dx[0], zero_f, 0, 0, 0);
-        if constexpr (TT == 1) {
-            // One tile: its scaling follows the next step's matrix instructions.
-            read_tile(nxt_buf, 0);
-            read_scales(nxt_buf, 0);
-            read_rows(nxt_buf);
-            scale_into(acc[0], sums_left, scale_left);
-            sums_left = sums[0];
-            scale_left = low(scale[0]);
-            return;
-        }
-        sums[TT - 1 < 1 ? 0 : 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.w, f.tok[TT - 1 < 1 ? 0 : 1], zero_i, 0, 0, 0);
-        read_tile(nxt_buf, 0);
-        read_tile(nxt_buf, 1);
-        read_scales(nxt_buf, 0);
-        scale_into(acc[TT - 1], sums_left, scale_left);
-        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
-        if constexpr (TT == 4) {
-            sums[2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.w, f.tok[2], zero_i, 0, 0, 0);
-            scale[1] = __builtin_amdgcn_mfma_f32_32x32x1f32(f.dw, f.dx[1], zero_f, 0, 0, 0);
-            scale_into(acc[0], sums[0], low(scale[0]));
-            sums[3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.w, f.tok[3], zero_i, 0, 0, 0);
-            read_tile(nxt_buf, 2);
-            read_tile(nxt_buf, 3);
-            read_scales(nxt_buf, 1);
-            read_rows(nxt_buf);
-            scale_into(acc[1], sums[1], high(scale[0]));
-            scale_into(acc[2], sums[2], low(scale[1]));
-            sums_left = sums[3];
-            scale_left = high(scale[1]);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 5, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 64, 0);
-        } else {
-            read_rows(nxt_buf);
-            scale_into(acc[0], sums[0], low(scale[0]));
-            sums_left = sums[TT - 1 < 1 ? 0 : 1];
-            scale_left = high(scale[0]);
-            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
+        for (int pair = 0; pair < PAIRS; pair++) {
+            i32x16 sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, tok[2 * pair], magic, 0, 0, 0);
+            const f32x32 scale = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dx[pair], none, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[2 * pair][e] = fmaf(__int_as_float(sums[e]) - MAGIC, scale[e], acc[2 * pair][e]);
+            if (2 * pair + 1 < TW) {
+                sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, tok[2 * pair + 1 < TW ? 2 * pair + 1 : 0], magic, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[2 * pair + 1 < TW ? 2 * pair + 1 : 0][e] = fmaf(__int_as_float(sums[e]) - MAGIC, scale[16 + e], acc[2 * pair + 1 < TW ? 2 * pair + 1 : 0][e]);
+            }
         }
     };
 
-    // Steps past the end of k are loaded like the others (zeros or whatever follows in the
-    // operands; nothing reads them), so that every wait counts the same loads.
+    fetch_scales(0, 0);
     fetch(0, 0);
     fetch(1, 1);
     fetch(2, 2);
-    sync_keeping_loads<2 * PER_STEP>();  // step 0 has landed
-#pragma unroll
-    for (int tt = 0; tt < TT; tt++) read_tile(0, tt);
-#pragma unroll
-    for (int pair = 0; pair < (TT + 1) / 2; pair++) read_scales(0, pair);
-    read_rows(0);
-    sync_keeping_loads<PER_STEP>();      // step 1 has landed; buffer 0 has been read
+    sync_keeping_loads<2 * PER_STEP>();  // the first scales and step 0 have landed
 
-    // Step s multiplies the fragments of step s and reads those of step s + 1 from buffer
-    // (s + 1) % 3, while buffer s % 3 is refilled with step s + 3.
-    auto step = [&](uint32_t s, uint32_t cur_buf, uint32_t nxt_buf) __attribute__((always_inline)) {
-        fetch(cur_buf, s + 3u);
-        multiply(nxt_buf);
-        sync_keeping_loads<PER_STEP>();  // step s + 2 has landed; buffer (s + 1) % 3 has been read
+    // Step s multiplies buffer s % 4 while buffer (s + 3) % 4 is refilled. A chunk's first step asks for
+    // the next chunk's scales.
+    uint32_t at = 0;  // the chunk of step s's scales
+    auto step = [&](uint32_t s, auto phase) __attribute__((always_inline)) {
+        constexpr uint32_t p = decltype(phase)::value;
+        read_step(p, at);
+        if (p == 0) fetch_scales(at == 0u ? 1u : 0u, s / 4u + 1u);
+        fetch((p + 3u) & 3u, s + 3u);
+        if (p == 3) at = at == 0u ? CHUNK : 0u;
+        multiply();
+        // (Nothing of a step's scaling may be left for later: its operands would pile up in registers.)
+#pragma unroll
+        for (int i = 0; i < TW; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) asm volatile("" : "+v"(acc[i][e]));
+        sync_keeping_loads<2 * PER_STEP + (p < 2 ? PER_CHUNK : 0)>();  // step s + 1 has landed; buffer s % 4 has been read
     };
     uint32_t s = 0;
-    for (; s + 3u <= steps; s += 3u) {
-        step(s, 0, 1);
-        step(s + 1u, 1, 2);
-        step(s + 2u, 2, 0);
+    for (; s + 4u <= steps; s += 4u) {
+        step(s, std::integral_constant<uint32_t, 0>{});
+        step(s + 1u, std::integral_constant<uint32_t, 1>{});
+        step(s + 2u, std::integral_constant<uint32_t, 2>{});
+        step(s + 3u, std::integral_constant<uint32_t, 3>{});
     }
-    if (s < steps) { step(s, 0, 1); s++; }
-    if (s < steps) { step(s, 1, 2); s++; }
-    scale_into(acc[TT - 1], sums_left, scale_left);
+    if (s < steps) step(s, std::integral_constant<uint32_t, 0>{});
+    if (s + 1u < steps) step(s + 1u, std::integral_constant<uint32_t, 1>{});
+    if (s + 2u < steps) step(s + 2u, std::integral_constant<uint32_t, 2>{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still land in LDS during the exchange
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 
-    // The four units of a tile meet in LDS: the wave of unit q keeps token tile q % TT (with
-    // 64-token tiles, units q and q + 2 each keep half of tile q % 2: parts 2 (q / 2) and + 1 of the
-    // lane's four groups of sums; with 32-token tiles unit q keeps part q) and hands the rest to
-    // their owners.
+    // The four units of a tile meet in LDS: a row half's 4 TW quarters of tiles (quarter p of tile tt: the
+    // lane's sums 4 p .. + 3) are shared out, quarter i to the wave of unit i / TW, and each wave hands the
+    // others' to their owners.
     f32x4 *inbox = reinterpret_cast<f32x4 *>(lds);
-    constexpr int PARTS = TT;
-    auto owner_of = [](int tt, int part) { return TT == 4 ? tt : TT == 2 ? tt + 2 * (part / 2) : part; };
-    auto slot = [&](uint32_t owner, uint32_t from, int part) {
-        return (((owner * 2u + wn) * 3u + ((from + 3u - owner) & 3u)) * PARTS + part) * 64u + lane;
+    auto slot = [&](uint32_t owner, uint32_t from, int i) {
+        return (((owner * 2u + wn) * 3u + ((from + 3u - owner) & 3u)) * TW + i) * 64u + lane;
     };
+    auto mine = [&](int i) { return f32x4{acc[i / 4][4 * (i % 4)], acc[i / 4][4 * (i % 4) + 1], acc[i / 4][4 * (i % 4) + 2], acc[i / 4][4 * (i % 4) + 3]}; };
     auto send = [&](auto quarter) __attribute__((always_inline)) {
         constexpr int Q = decltype(quarter)::value;
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                if (owner_of(tt, p) == Q) continue;
-                inbox[slot(owner_of(tt, p), Q, TT == 4 ? p : TT == 2 ? p % 2 : 0)] = f32x4{acc[tt][4 * p], acc[tt][4 * p + 1], acc[tt][4 * p + 2], acc[tt][4 * p + 3]};
-            }
+        for (int i = 0; i < 4 * TW; i++)
+            if (i / TW != Q) inbox[slot(i / TW, Q, i % TW)] = mine(i);
     };
     const bool aligned = ((a.out_stride | a.col0) & 3u) == 0u && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0u;
     // In each 32 x 32 tile the lane holds rows 8 p + 4 (lane / 32) .. + 3, p < 4, of token
-    // lane % 32: sixteen contiguous bytes of the token's output row per group.
+    // lane % 32: sixteen contiguous bytes of the token's output row per quarter.
     auto collect = [&](auto quarter) __attribute__((always_inline)) {
         constexpr int Q = decltype(quarter)::value;
-        constexpr int tile = Q % TT;
-        const uint32_t t = t0 + 32u * tile + lrow;
 #pragma unroll
-        for (int i = 0; i < PARTS; i++) {
-            constexpr int first = TT == 4 ? 0 : TT == 2 ? 2 * (Q / 2) : Q;
-            const int p = first + i;
+        for (int i = Q * TW; i < (Q + 1) * TW; i++) {
+            const uint32_t t = t0 + 32u * (i / 4) + lrow, col = j0 + 32u * wn + 8u * (i % 4) + 4u * h;
             f32x4 part[4];
 #pragma unroll
-            for (int from = 0; from < 4; from++)
-                part[from] = from == Q ? f32x4{acc[tile][4 * p], acc[tile][4 * p + 1], acc[tile][4 * p + 2], acc[tile][4 * p + 3]} : inbox[slot(Q, from, i)];
+            for (int from = 0; from < 4; from++) part[from] = from == Q ? mine(i) : inbox[slot(Q, from, i % TW)];
             f32x4 v = (part[0] + part[2]) + (part[1] + part[3]);
-            const uint32_t col = j0 + 32u * wn + 8u * p + 4u * h;
             if (t >= a.rows || col >= a.n) continue;
             float *o = a.out + (size_t)t * a.out_stride + a.col0 + col;
             if (aligned && col + 3u < a.n) {
@@ -337,20 +283,12 @@ __global__ __launch_bounds__(THREADS) void matmul_q8_i8_kernel(Q8I8Args a) {
     }
 }
 
-template <int TT>
+template <int TW>
 zhip_result launch_tile(const Dispatch &d, const char *name, const Q8I8Args &a) {
-    auto kernel = matmul_q8_i8_kernel<TT>;
-    constexpr int bytes = lds_bytes<TT>();
-    static bool configured = false;
-    if (!configured) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", name, bytes);
-        }
-        configured = true;
-    }
-    const dim3 grid((a.n + BN - 1) / BN, (a.rows + 32 * TT - 1) / (32 * TT));
-    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), bytes, d.stream, a);
+    typedef Tile<TW> T;
+    if (!lds_opt_in<matmul_q8_i8_kernel<TW>, T::LDS>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", name, T::LDS);
+    const dim3 grid((a.n + BN - 1) / BN, (a.rows + T::BM - 1) / T::BM);
+    hipLaunchKernelGGL((matmul_q8_i8_kernel<TW>), grid, dim3(THREADS), T::LDS, d.stream, a);
     return check_launch(d, name);
 }
 
@@ -367,10 +305,11 @@ zhip_result launch_matmul_q8_i8(const Dispatch &d, const char *name, const uint8
     a.qx = qx; a.w = w; a.dx = dx; a.out = out;
     a.rows = rows; a.n = n; a.k = k; a.col0 = col0; a.out_stride = out_stride; a.accumulate = accumulate;
     a.row_bytes = row_bytes; a.qx_bytes = qx_bytes; a.w_bytes = w_bytes; a.dx_bytes = dx_bytes;
-    // 128-token tiles unless those leave half of the CUs idle: then 64-token tiles on twice the
-    // CUs, then 32-token tiles.
+    // 64-token tiles, two workgroups a CU, unless they leave half of the CUs idle: then 32-token
+    // tiles. us, 64 / 32: 512 x 1024 x 2048 (256 workgroups of 64 tokens) 7.9 / 8.3, 201 x 2560 x
+    // 4096 (256) 13.8 / 15.1, 512 x 1024 x 6144 17.1 / 21.2; 512 x 2048 x 1024 (128) 10.7 / 8.6,
+    // 64 x 4096 x 4096 (64) 18.0 / 13.8.
     const uint64_t columns = (n + BN - 1) / BN, cus = (uint64_t)d.dev->compute_units;
-    if (rows > 64u && 2u * ((rows + 127u) / 128u) * columns > cus) return launch_tile<4>(d, name, a);
     if (rows > 32u && 2u * ((rows + 63u) / 64u) * columns > cus) return launch_tile<2>(d, name, a);
     return launch_tile<1>(d, name, a);
 }
