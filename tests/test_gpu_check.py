@@ -700,6 +700,34 @@ def test_quant_matvec_mfma_variant(ctx, t, pair, rows, n, k, prologue):
         assert got[tk].tobytes() == c.read(single)[:stride].tobytes(), "a token's sums differ between a lone launch and a multi-token launch"
 
 
+@pytest.mark.parametrize("pair,rows,n,k,prologue", [
+    (False, 8, 40, 256, "norm"),       # one block a row
+    (True, 5, 33, 768, "norm_act"),    # three blocks, gate and up tiles of different teams, a ragged last tile
+    (False, 3, 8240, 1024, "plain"),   # four teams, more than one round
+    (False, 6, 4130, 1280, "norm"),    # two teams, a second tile for some workgroups, in halves
+    (True, 1, 4112, 1792, "norm"),
+    (False, 8, 100, 2304, "norm_act"),  # nine blocks over sixteen waves
+    (True, 4, 4128, 4096, "norm"),     # a block a wave
+    (False, 7, 272, 4352, "plain"),    # seventeen blocks: two for one wave
+    (True, 8, 48, 7936, "norm"),
+    (False, 2, 40, 8448, "norm_act"),  # three parts
+    (True, 5, 272, 9728, "norm"),
+    (False, 8, 2576, 14592, "plain"),  # four parts, several tiles a workgroup
+    (False, 1, 19, 32512, "norm"),     # eight parts
+])
+@pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_quant_matvec_mfma_any_row_length(ctx, t, pair, rows, n, k, prologue):
+    """The matrix-core id over rows of any number of blocks, under the bounds of the case above."""
+    test_quant_matvec_mfma_variant(ctx, t, pair, rows, n, k, prologue)
+
+
+@pytest.mark.parametrize("k", [32, 96, 288, 1056, 2080, 4128, 8224])
+def test_matvec_q8_0_mfma_ragged_rows(ctx, k):
+    """Q8_0 rows whose last 256-weight block is short, one unit of it to all but one."""
+    test_quant_matvec_mfma_variant(ctx, TensorType.q8_0, False, 5, 70, k, "norm")
+    test_quant_matvec_mfma_variant(ctx, TensorType.q8_0, True, 8, 35, k, "plain")
+
+
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate", [
     (8, 200, 1024, 3, 7, True),      # partial last tile, unaligned rows
     (5, 96, 4096, 4, 8, False),      # aligned rows: 16-byte stores

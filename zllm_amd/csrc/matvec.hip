@@ -313,24 +313,51 @@ __global__ __launch_bounds__(256) void matvec_kernel(MvArgs a) {
     }
 }
 
+// The matrix-core variant of the quantized formats, any row length (matvec_mfma_rows.hip) ...
+bool matvec_mfma_rows_accepts(const MvArgs &a);
+zhip_result launch_matvec_mfma_rows(const Dispatch &d, const MvArgs &a, int type);
+// ... and the kernels that are the faster ones on some shapes: Q4_K and Q5_K over rows of 2048 weights, or 6144 ..
+// 32768 in parts of 2048 (matvec_mfma_resident.hip), Q8_0 over the same (matvec_q8_mfma_stream.hip), Q6_K, Q3_K and
+// Q8_0 over long walks of tiles (matvec_q6k_mfma_stream.hip).
 bool matvec_q4k_mfma_resident_accepts(const MvArgs &a);
 zhip_result launch_matvec_q4k_mfma_resident(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
-// The matrix-core variant of matvec_q8_0 for k of 2048, 4096 or 6144 .. 32768 in parts (matvec_q8_mfma_stream.hip).
-bool matvec_q8_mfma_stream_accepts(const MvArgs &a);
-zhip_result launch_matvec_q8_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
-// matvec_bf16 on the matrix cores, the weights read once for all tokens (matvec_bf16_mfma_stream.hip).
-bool matvec_bf16_mfma_stream_accepts(const MvArgs &a);
-zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16);
 bool matvec_q5k_mfma_resident_accepts(const MvArgs &a);
 zhip_result launch_matvec_q5k_mfma_resident(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
-// matvec_q6_k on the matrix cores for k of 1024, 2048, 3072, 4096 or 6144 .. 32768 in parts (matvec_q6k_mfma_stream.hip).
+bool matvec_q8_mfma_stream_accepts(const MvArgs &a);
+zhip_result launch_matvec_q8_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
 bool matvec_q6k_mfma_stream_accepts(const MvArgs &a);
 zhip_result launch_matvec_q6k_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
 bool matvec_q3k_mfma_stream_accepts(const MvArgs &a);
 zhip_result launch_matvec_q3k_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
-// matvec_q8_0 over rows of 1024 weights in the same kernel: a tile's rows as one flat stretch.
 bool matvec_q8_0_mfma_flat_accepts(const MvArgs &a);
 zhip_result launch_matvec_q8_0_mfma_flat(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
+// Which of them takes a matrix under the matrix-core id: a property of the matrix alone, since they add in
+// different orders and a token's bits must not depend on the width of its step. us at one / four / eight
+// tokens, weights from HBM, these kernels / matvec_mfma_rows.hip:
+//  * Q4_K, Q5_K, Q8_0, rows of 2048 weights: Q4_K 4096 outputs 6.8 6.8 6.9 / 6.7 7.2 8.0, 2 x 8192 10.1 10.0 10.2 / 9.8
+//    10.4 11.1, Q8_0 4096 6.9 7.0 7.1 / 7.1 7.5 8.1. Rows of 4096: Q4_K 4096 outputs 10.3 10.3 10.8 / 6.9 7.7 10.0,
+//    2 x 14336 21.8 21.1 21.7 / 20.1 19.5 21.2, Q5_K 27.7 27.7 28.4 / 22.3 22.5 24.5, Q8_0 4096 10.9 10.9 11.3 / 7.8 8.1 9.9.
+//  * the same in parts of 2048, no gate / up pair (and of Q8_0 fewer than 8192 outputs): Q4_K 4096 x 8192 11.1
+//    11.3 11.6 / 9.5 11.5 15.5, 4096 x 14336 15.1 14.9 15.5 / 13.8 14.4 16.6, Q3_K 4096 x 8192 12.7 12.6 13.3 / 9.9 11.2 14.3,
+//    Q8_0 2048 x 6144 9.2 9.5 9.5 / 8.4 9.8 13.0. Pairs: Q4_K 2 x 8192 x 8192 26.8 27.4 27.7 / 21.4 21.9 24.1, Q8_0 37.2
+//    38.0 39.0 / 27.7 28.9 31.9; 57344 x 8192 Q8_0 (four and eight tokens) 113.9 118.9 / 85.9 91.6.
+//  * Q6_K, Q3_K and Q8_0 rows of 1024 weights: from twelve tiles of sixteen outputs a CU on (Q3_K: eight). Q6_K (rows of 1024
+//    weights always: 4096 outputs 7.3 7.2 7.3 / 6.6 7.1 7.7) 64000 x 4096 (four and eight tokens) 46.4 49.7 / 51.2 52.9, 32000 x 4096 28.6 29.6 / 28.7 30.6, 4096 x 4096 14.7 15.5 /
+//    8.6 10.3; Q3_K 64000 x 4096 38.9 40.9 / 42.9 44.1, 2 x 14336 x 4096 23.5 25.3 / 23.6 25.6, 4096 x 4096 12.7 13.3 / 7.4 9.4;
+//    Q8_0 151936 x 1024 33.1 33.2 / 36.1 36.0, 50257 x 1024 16.9 16.8 / 16.7 16.8, 2 x 3072 x 1024 9.0 9.1 / 7.3 7.9.
+static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
+    const bool pair = a.flags & FLAG_SILU_PAIR, parts = a.k > 4096u;
+    const uint64_t tiles = ((uint64_t)a.rows * (pair ? 2u : 1u) + 15u) / 16u, cus = (uint64_t)d.dev->compute_units;
+    switch (type) {
+    case 4: case 5: return a.k == 2048u || (parts && !pair);
+    case 8: return a.k == 1024u ? tiles >= 12u * cus : a.k == 2048u || (parts && !pair && a.rows < 8192u);
+    case 6: return a.k == 1024u || tiles >= 12u * cus;
+    default: return parts ? !pair || tiles >= 8u * cus : tiles >= 8u * cus;
+    }
+}
+// matvec_bf16 on the matrix cores, the weights read once for all tokens (matvec_bf16_mfma_stream.hip).
+bool matvec_bf16_mfma_stream_accepts(const MvArgs &a);
+zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16);
 // Which matrices take it: 16 MB of weights or more, and gate / up pairs of 32 MB or more, in
 // contexts opened with ZHIP_OPTION_WIDE_DECODE, and then at every width from one token on: the
 // kernel sums in another order than the general one, and a token's bits must not depend on the
@@ -446,28 +473,18 @@ static zhip_result launch_matvec(const Dispatch &d, bool quant) {
     // inputs in LDS, adds in the same order and lost on every shape measured (figures there).
     if (kSplitInputs<D> && matvec_half_row_accepts(a)) return launch_matvec_half_row(d, a, std::is_same<D, DecF16>::value);
 
-    // MatvecVariant (wg 512, lanes 64, rows 16) names the matrix-core variants: a wave per sixteen rows.
+    // MatvecVariant (wg 512, lanes 64, rows 16) names the matrix-core variants: sixteen rows a tile.
     const bool matrix_cores = quant && v.lanes == 64u && v.rows == 16u && (D::CHUNK == 4 || D::CHUNK == 8 || D::CHUNK == 6 || D::CHUNK == 5 || D::CHUNK == 3);
-    if (D::CHUNK == 3 && matrix_cores && matvec_q3k_mfma_stream_accepts(a)) return launch_matvec_q3k_mfma_stream(d, a, d.bind[2].size);
-    // (matvec_q5_k: the Q4_K kernel for k of 2048, 4096 or 6144 .. 32768 in parts, with the fifth bits; other shapes run the default variant)
-    if (D::CHUNK == 5 && matrix_cores && matvec_q5k_mfma_resident_accepts(a)) return launch_matvec_q5k_mfma_resident(d, a, d.bind[2].size);
-    // (matvec_q6_k and matvec_q3_k: k of 1024, 2048, 3072, 4096 or 6144 .. 32768 in parts; every workgroup builds the tokens' operands, prologue included)
-    if (D::CHUNK == 6 && matrix_cores && matvec_q6k_mfma_stream_accepts(a)) return launch_matvec_q6k_mfma_stream(d, a, d.bind[2].size);
-    // The kernels that keep the tokens' operands in registers (k of 2048 or 4096, longer rows in parts of 2048, and whole tiles) compute a step's prologue (RMSNorm, silu(x / act_div):
-    // src/kernels/matvec_quant.wgsl.hbs:73-89) themselves: their operands are built from one
-    // round of loads, which the norm weights join (C3 at four tokens with the FFN launch's
-    // RMSNorm: 22.6 us, 26.1 us with a pass of its own in front, 20.7 us without a prologue).
-    if (D::CHUNK == 8 && matrix_cores && matvec_q8_0_mfma_flat_accepts(a)) return launch_matvec_q8_0_mfma_flat(d, a, d.bind[2].size);
-    const bool resident = D::CHUNK == 4 && matrix_cores && matvec_q4k_mfma_resident_accepts(a);
-    const bool q8_stream = D::CHUNK == 8 && matrix_cores && matvec_q8_mfma_stream_accepts(a);
-    if (resident) return launch_matvec_q4k_mfma_resident(d, a, d.bind[2].size);
-    // The same id on matvec_q8_0 (a one-token step too, so that a token's bits do not depend on
-    // the step it ran in).
-    if (q8_stream) return launch_matvec_q8_mfma_stream(d, a, d.bind[2].size);
-    // Shapes these kernels do not take run the default variant under the id as well: the
-    // matrix-core kernels that once stood in for them (a k-sliced Q4_K kernel, the compensated
-    // prefill tiling for Q8_0) lost to it at two to four tokens on every shape measured
-    // (Q4_K 4096 x 14336 at four tokens: 71.7 against 21.9 us; 5120 x 5120: 28.0 against 21.2).
+    if (matrix_cores) {
+        const bool older = older_mfma_pays(d, a, D::CHUNK);
+        if (D::CHUNK == 4 && older && matvec_q4k_mfma_resident_accepts(a)) return launch_matvec_q4k_mfma_resident(d, a, d.bind[2].size);
+        if (D::CHUNK == 5 && older && matvec_q5k_mfma_resident_accepts(a)) return launch_matvec_q5k_mfma_resident(d, a, d.bind[2].size);
+        if (D::CHUNK == 6 && older && matvec_q6k_mfma_stream_accepts(a)) return launch_matvec_q6k_mfma_stream(d, a, d.bind[2].size);
+        if (D::CHUNK == 3 && older && matvec_q3k_mfma_stream_accepts(a)) return launch_matvec_q3k_mfma_stream(d, a, d.bind[2].size);
+        if (D::CHUNK == 8 && older && matvec_q8_0_mfma_flat_accepts(a)) return launch_matvec_q8_0_mfma_flat(d, a, d.bind[2].size);
+        if (D::CHUNK == 8 && older && matvec_q8_mfma_stream_accepts(a)) return launch_matvec_q8_mfma_stream(d, a, d.bind[2].size);
+        if (matvec_mfma_rows_accepts(a)) return launch_matvec_mfma_rows(d, a, D::CHUNK);
+    }
     // The tuned kernel takes rows of whole 64-weight tasks.
     if (D::CHUNK != 0 && p.k % 64u == 0) return launch_matvec_quant(d, a, D::CHUNK);
 

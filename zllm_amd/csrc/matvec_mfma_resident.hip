@@ -1,5 +1,6 @@
 // matvec_q4_k and matvec_q5_k, matrix-core variant (MatvecVariant wg 512, lanes 64, rows 16) for
-// k = 2048 or 4096 (longer rows in parts, below) and steps of up to eight tokens. The per-weight work is done once for all
+// k = 2048 (longer rows in parts, below) and steps of up to eight tokens; the other row lengths are
+// matvec_mfma_rows.hip's. The per-weight work is done once for all
 // tokens: the weights enter v_mfma_f32_16x16x32_f16 as the exact f16 values 16 + q (the nibble
 // dropped into the mantissa of 16.0; Q5_K: 32 + q with the fifth bit), every token as two f16
 // rows, the rounding of its inputs and what that left times 2^11, under a per-token power of
@@ -8,11 +9,10 @@
 // column of ones (src/ref/tensor.zig:94-117). Nothing is recomputed and nothing but partial
 // results crosses LDS.
 //
-// A 512-thread workgroup is eight waves that split k eight ways (one or two
-// 256-weight blocks a wave). A wave builds its k range of all tokens' f16 rows
+// A 512-thread workgroup is eight waves that split k eight ways (a
+// 256-weight block a wave). A wave builds its k range of all tokens' f16 rows
 // once, straight into matrix-core operands that stay in registers for the
-// whole kernel (64 VGPRs at k = 4096), together with the rows' sub-block sums
-// (32 VGPRs). It then walks over sixteen-row weight tiles, persistent
+// whole kernel, together with the rows' sub-block sums. It then walks over sixteen-row weight tiles, persistent
 // workgroups taking tiles b, b + G, ...: a tile's sixteen rows are one contiguous
 // stretch of the matrix and travel as a flat copy through a ring of three LDS
 // slots that the workgroup shares, every wave loading a share of it by wave-wide
@@ -39,7 +39,7 @@
 // 14.8 us (12.1 + the sums' launch) against 10.3 / 14.3 / 19.2 / 21.6 / 40.9 us at one / two /
 // three / four / eight tokens on the default variant; 8192 x 28672 34.3 - 36.4 us against
 // 46.4 / 69.7 / 133.8 us at one / four / eight; 28672 x 8192 with the RMSNorm prologue 37.7 -
-// 38.6 us against 26.7 / 83.7 / 169.0.
+// 38.6 us against 26.7 / 83.7 / 169.0. (Gate / up pairs over such rows are matvec_mfma_rows.hip's.)
 //
 // Contract as the other variants (src/kernels/matvec_quant.wgsl.hbs); a token's
 // result does not depend on how many tokens share the launch.
@@ -78,12 +78,11 @@ struct ResQ5 {
     static constexpr float BIAS = 32.0f;
     static const char *name() { return "matvec_q5_k"; }
 };
-// A tile in LDS: the flat copy of its sixteen rows (NB = 256-weight blocks of a wave's k range:
-// a row is 8 NB blocks, nine or eleven lines a block column of the eight waves).
-template <class F, int NB> constexpr uint32_t tile_bytes() { return 16u * 8u * F::BLOCK * NB; }
+// A tile in LDS: the flat copy of its sixteen rows of eight blocks (a wave's k range is one).
+template <class F> constexpr uint32_t tile_bytes() { return 16u * 8u * F::BLOCK; }
 // Wave-wide loads of 1 KB a tile takes, and how many a wave issues (the slots past the tile's end ask for nothing).
-template <class F, int NB> constexpr uint32_t tile_kb() { return tile_bytes<F, NB>() / 1024u; }
-template <class F, int NB> constexpr int tile_loads() { return (int)((tile_kb<F, NB>() + 7u) / 8u); }
+template <class F> constexpr uint32_t tile_kb() { return tile_bytes<F>() / 1024u; }
+template <class F> constexpr int tile_loads() { return (int)((tile_kb<F>() + 7u) / 8u); }
 
 struct ResArgs {
     MvArgs a;
@@ -163,12 +162,12 @@ __device__ __forceinline__ rf16x8 nibbles(ru32x2 w, ru32x2 fifth, uint32_t mask,
     return __builtin_bit_cast(rf16x8, r);
 }
 
-// NB: 256-weight blocks of a wave's k range (k = 2048 NB). LONG (NB = 1): k = 2048 q.parts;
+// k = 2048; LONG: k = 2048 q.parts,
 // workgroup b multiplies columns 2048 (b % parts) .. (part `kpart`) of the tiles that walker b / parts takes, and
 // matvec_kquant_mfma_parts_sum_kernel adds the parts in their order and applies the epilogue.
-template <class F, bool PAIR, int NB, bool LONG>
+template <class F, bool PAIR, bool LONG>
 __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(ResArgs q) {
-    static_assert(!LONG || NB == 1, "parts of a long row are 2048 columns");
+    static_assert(!LONG || !PAIR, "pairs over long rows are matvec_mfma_rows.hip's");
     constexpr int DEPTH = LONG ? kLongDepth : kDepth;
     const MvArgs &a = q.a;
     __shared__ float lds_scale[16];               // [8 ..]: one over each token's scale
@@ -195,7 +194,7 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
     auto rows_of = [&](uint32_t p) { return (q.split && p / per >= q.rounds) ? 8u : 16u; };
     auto row0 = [&](uint32_t p) { return out0(p) + ((PAIR && (p & 1u)) ? a.half : 0u); };
 
-    // A tile's loads. The tile's sixteen rows are one contiguous stretch of the matrix, 18 NB
+    // A tile's loads. The tile's sixteen rows are one contiguous stretch of the matrix, 18
     // KB of whole lines, and travel as a flat copy into one of the ring's slots, which the whole
     // workgroup shares: load g = LOADS wave + j brings lines 8 g .. 8 g + 7 (the slots past the
     // tile's last line go against an empty buffer and land their zeros in a spare KB, so that
@@ -203,8 +202,8 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
     // belongs at position l % 8 of it: chunk c of a line of row r sits at position c ^ (r % 8).
     // The whole address is the lane's offset. Past the run's last tile the loads still run, but
     // against the empty buffer: zeros land and nothing is fetched.
-    constexpr int LOADS = tile_loads<F, NB>();
-    constexpr uint32_t TILE = tile_bytes<F, NB>(), ROW_LINES = 8u * F::BLOCK * NB / 128u, TILE_LOADS = tile_kb<F, NB>();
+    constexpr int LOADS = tile_loads<F>();
+    constexpr uint32_t TILE = tile_bytes<F>(), ROW_LINES = 8u * F::BLOCK / 128u, TILE_LOADS = tile_kb<F>();
     __shared__ __align__(16) uint8_t lds_ring[DEPTH * TILE + 1024u];
     const uint32_t ring0 = (uint32_t)(uintptr_t)lds_ring;
     const uint32_t uwave = __builtin_amdgcn_readfirstlane(wave);
@@ -236,23 +235,23 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
     // one 4 .. 7, and they swap what the other needs. An absent token's rows read the last
     // token's inputs under a scale of zero: no branches, so all of the lane's loads go out together.
     const uint32_t tok = l16 >> 1, sub = l16 & 1u, tsrc = tok < a.m ? tok : a.m - 1u;
-    float4 raw[NB * 8];
+    float4 raw[8];
     {
-        const float *xt = a.x + (size_t)tsrc * a.xr + 2048u * kpart + NB * 256u * wave + 8u * g + 4u * sub;
+        const float *xt = a.x + (size_t)tsrc * a.xr + 2048u * kpart + 256u * wave + 8u * g + 4u * sub;
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) raw[s] = *reinterpret_cast<const float4 *>(xt + 32 * s);
+        for (int s = 0; s < 8; s++) raw[s] = *reinterpret_cast<const float4 *>(xt + 32 * s);
     }
     // A step's prologue (src/kernels/matvec_quant.wgsl.hbs:73-89) on the same registers, in the
     // default variant's arithmetic: RMSNorm times the norm weights (the wave ranges' sums of
     // squares meet in LDS, added in the order of the ranges) and / or silu(x / act_div).
     // (the sum of squares of a long row is not any one workgroup's: it comes ready in q.scales)
     const bool norm = (a.flags & FLAG_NORM) != 0, act = a.act_div > 0.f;
-    float4 gw[NB * 8];
+    float4 gw[8];
     float ready = 0.f;  // (asked for before the first weights, like the inputs)
     if (norm) {
-        const float *gt = a.norm_w + 2048u * kpart + NB * 256u * wave + 8u * g + 4u * sub;
+        const float *gt = a.norm_w + 2048u * kpart + 256u * wave + 8u * g + 4u * sub;
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) gw[s] = *reinterpret_cast<const float4 *>(gt + 32 * s);
+        for (int s = 0; s < 8; s++) gw[s] = *reinterpret_cast<const float4 *>(gt + 32 * s);
         if (LONG) ready = q.scales[tsrc];
     }
     load_tile(0, 0);
@@ -263,7 +262,7 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
         } else {
             float ss = 0.f;
 #pragma unroll
-            for (int s = 0; s < NB * 8; s++) ss += raw[s].x * raw[s].x + raw[s].y * raw[s].y + raw[s].z * raw[s].z + raw[s].w * raw[s].w;
+            for (int s = 0; s < 8; s++) ss += raw[s].x * raw[s].x + raw[s].y * raw[s].y + raw[s].z * raw[s].z + raw[s].w * raw[s].w;
             ss += __shfl_xor(ss, 1, 64);
             ss += __shfl_xor(ss, 16, 64);
             ss += __shfl_xor(ss, 32, 64);
@@ -275,14 +274,14 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
             rs = 1.0f / sqrtf(total / (float)a.k + a.eps);
         }
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) {
+        for (int s = 0; s < 8; s++) {
             raw[s].x = raw[s].x * rs * gw[s].x; raw[s].y = raw[s].y * rs * gw[s].y;
             raw[s].z = raw[s].z * rs * gw[s].z; raw[s].w = raw[s].w * rs * gw[s].w;
         }
     }
     if (act) {
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) {
+        for (int s = 0; s < 8; s++) {
             raw[s].x = silu_f(raw[s].x / a.act_div); raw[s].y = silu_f(raw[s].y / a.act_div);
             raw[s].z = silu_f(raw[s].z / a.act_div); raw[s].w = silu_f(raw[s].w / a.act_div);
         }
@@ -294,7 +293,7 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
     {
         float big = 0.f;
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) big = fmaxf(fmaxf(fabsf(raw[s].x), fabsf(raw[s].y)), fmaxf(fmaxf(fabsf(raw[s].z), fabsf(raw[s].w)), big));
+        for (int s = 0; s < 8; s++) big = fmaxf(fmaxf(fabsf(raw[s].x), fabsf(raw[s].y)), fmaxf(fmaxf(fabsf(raw[s].z), fabsf(raw[s].w)), big));
         big = fmaxf(big, __shfl_xor(big, 1, 64));
         big = fmaxf(big, __shfl_xor(big, 16, 64));
         big = fmaxf(big, __shfl_xor(big, 32, 64));
@@ -312,11 +311,11 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
         return __uint_as_float((uint32_t)(inverse ? 254 - se : se) << 23);
     };
     if (tid < 8u) lds_scale[8 + tid] = tid < a.m ? scale_of(tid, true) : 1.0f;  // read after a later barrier
-    rf16x8 xf[NB * 8];
+    rf16x8 xf[8];
     {
         const float scale = tok < a.m ? scale_of(tok, false) : 0.f;
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) {
+        for (int s = 0; s < 8; s++) {
             const float x[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
             // The scale is a power of two, so x * scale - hi in one fused operation is exact.
             _Float16 hi[4], lo[4];
@@ -338,63 +337,54 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
     }
     // The rows' sub-block sums, by the matrix cores (the rows times a column of ones): every
     // lane gets the sums of its own two tokens (operand rows 4 g .. 4 g + 3), whatever its column.
-    float2 xsum[NB * 8];
+    float2 xsum[8];
     {
         const ru32x4 ones = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
 #pragma unroll
-        for (int s = 0; s < NB * 8; s++) {
+        for (int s = 0; s < 8; s++) {
             const rf32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[s], __builtin_bit_cast(rf16x8, ones), rf32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             xsum[s] = float2{fmaf(d[1], 1.0f / 2048.0f, d[0]), fmaf(d[3], 1.0f / 2048.0f, d[2])};
         }
     }
 
-    // The lane's reads of its wave's blocks of a tile: row l16 of the flat copy, blocks
-    // NB wave + i. Byte f of the copy sits at 128 (f / 128) + 16 ((f / 16 % 8) ^ (l16 % 8)) + f % 16.
+    // The lane's reads of its wave's block of a tile, of row l16 of the flat copy. Byte f of the copy sits at 128 (f / 128) + 16 ((f / 16 % 8) ^ (l16 % 8)) + f % 16.
     auto at_byte = [&](uint32_t f) { return (f & ~127u) + 16u * (((f >> 4) & 7u) ^ (l16 & 7u)) + (f & 15u); };
-    uint32_t at_header[NB], at_fifth[NB], at_nibbles[NB][4];
+    const uint32_t block = 8u * F::BLOCK * l16 + F::BLOCK * wave, at_header = at_byte(block), at_fifth = at_byte(block + 16u + 8u * g);
+    uint32_t at_nibbles[4];
 #pragma unroll
-    for (uint32_t i = 0; i < NB; i++) {
-        const uint32_t block = 8u * F::BLOCK * NB * l16 + F::BLOCK * (NB * wave + i);
-        at_header[i] = at_byte(block);
-        at_fifth[i] = at_byte(block + 16u + 8u * g);
-#pragma unroll
-        for (uint32_t c = 0; c < 4; c++) at_nibbles[i][c] = at_byte(block + F::NIBBLES_AT + 32u * c + 8u * g);
-    }
+    for (uint32_t c = 0; c < 4; c++) at_nibbles[c] = at_byte(block + F::NIBBLES_AT + 32u * c + 8u * g);
 
     float held = 0.f;  // the gate tile's result, until the up tile's arrives
     // Multiplies tile p from its slot and leaves the wave's partial sums in LDS.
     auto multiply = [&](uint32_t p, uint32_t slot) __attribute__((always_inline)) {
         float acc[2] = {0.f, 0.f};  // tokens 2 g and 2 g + 1, matrix row row0 + l16, this wave's k range
         const uint8_t *tile = lds_ring + slot * TILE;
+        const ru32x4 h = *reinterpret_cast<const ru32x4 *>(tile + at_header);
+        const float d = half_bits_to_float(h.x & 0xffffu), dmin = half_bits_to_float(h.x >> 16);
+        // The eight 6-bit scales and minimums as bytes of four words (src/ref/tensor.zig:94-98).
+        const uint32_t sc_lo_ = h.y & 0x3f3f3f3fu, mn_lo_ = h.z & 0x3f3f3f3fu;
+        const uint32_t sc_hi_ = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+        uint32_t mn_hi = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
+        // (kept apart from the masks above: a clean byte converts to f32 in one instruction,
+        // a 6-bit field of the raw word needs two)
+        uint32_t sc_lo = sc_lo_, mn_lo = mn_lo_, sc_hi = sc_hi_;
+        asm volatile("" : "+v"(sc_lo), "+v"(mn_lo), "+v"(sc_hi), "+v"(mn_hi));
+        ru32x2 bits = {0u, 0u};  // Q5_K: bit sb of a byte is the fifth bit of the position's weight in sub-block sb
+        if (F::FIFTH) bits = *reinterpret_cast<const ru32x2 *>(tile + at_fifth);
 #pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const ru32x4 h = *reinterpret_cast<const ru32x4 *>(tile + at_header[i]);
-            const float d = half_bits_to_float(h.x & 0xffffu), dmin = half_bits_to_float(h.x >> 16);
-            // The eight 6-bit scales and minimums as bytes of four words (src/ref/tensor.zig:94-98).
-            const uint32_t sc_lo_ = h.y & 0x3f3f3f3fu, mn_lo_ = h.z & 0x3f3f3f3fu;
-            const uint32_t sc_hi_ = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
-            uint32_t mn_hi = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
-            // (kept apart from the masks above: a clean byte converts to f32 in one instruction,
-            // a 6-bit field of the raw word needs two)
-            uint32_t sc_lo = sc_lo_, mn_lo = mn_lo_, sc_hi = sc_hi_;
-            asm volatile("" : "+v"(sc_lo), "+v"(mn_lo), "+v"(sc_hi), "+v"(mn_hi));
-            ru32x2 bits = {0u, 0u};  // Q5_K: bit sb of a byte is the fifth bit of the position's weight in sub-block sb
-            if (F::FIFTH) bits = *reinterpret_cast<const ru32x2 *>(tile + at_fifth[i]);
+        for (uint32_t c = 0; c < 4; c++) {
+            const ru32x2 wq = *reinterpret_cast<const ru32x2 *>(tile + at_nibbles[c]);
 #pragma unroll
-            for (uint32_t c = 0; c < 4; c++) {
-                const ru32x2 wq = *reinterpret_cast<const ru32x2 *>(tile + at_nibbles[i][c]);
-#pragma unroll
-                for (uint32_t half = 0; half < 2; half++) {
-                    const uint32_t sb = 2u * c + half, shift = 8u * (sb & 3u);
-                    const float dsc = d * (float)(((sb < 4u ? sc_lo : sc_hi) >> shift) & 0xffu);
-                    const float off = fmaf(F::BIAS, dsc, dmin * (float)(((sb < 4u ? mn_lo : mn_hi) >> shift) & 0xffu));
-                    const ru32x2 fifth = {sb ? bits.x >> sb : bits.x, sb ? bits.y >> sb : bits.y};
-                    const rf16x8 wf = half ? nibbles<F, true>(wq, fifth, q.nibble_mask, sixteen) : nibbles<F, false>(wq, fifth, q.nibble_mask, sixteen);
-                    const rf32x4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[8 * i + sb], wf, rf32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    const float2 xs = xsum[8 * i + sb];
-                    acc[0] = fmaf(-off, xs.x, fmaf(dsc, fmaf(r[1], 1.0f / 2048.0f, r[0]), acc[0]));
-                    acc[1] = fmaf(-off, xs.y, fmaf(dsc, fmaf(r[3], 1.0f / 2048.0f, r[2]), acc[1]));
-                }
+            for (uint32_t half = 0; half < 2; half++) {
+                const uint32_t sb = 2u * c + half, shift = 8u * (sb & 3u);
+                const float dsc = d * (float)(((sb < 4u ? sc_lo : sc_hi) >> shift) & 0xffu);
+                const float off = fmaf(F::BIAS, dsc, dmin * (float)(((sb < 4u ? mn_lo : mn_hi) >> shift) & 0xffu));
+                const ru32x2 fifth = {sb ? bits.x >> sb : bits.x, sb ? bits.y >> sb : bits.y};
+                const rf16x8 wf = half ? nibbles<F, true>(wq, fifth, q.nibble_mask, sixteen) : nibbles<F, false>(wq, fifth, q.nibble_mask, sixteen);
+                const rf32x4 r = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[sb], wf, rf32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                const float2 xs = xsum[sb];
+                acc[0] = fmaf(-off, xs.x, fmaf(dsc, fmaf(r[1], 1.0f / 2048.0f, r[0]), acc[0]));
+                acc[1] = fmaf(-off, xs.y, fmaf(dsc, fmaf(r[3], 1.0f / 2048.0f, r[2]), acc[1]));
             }
         }
         float *part = &lds_part[p & 1u][0][0];
@@ -517,8 +507,8 @@ zhip_result launch_matvec_parts_sum(const Dispatch &d, const char *name, const M
 // one or two blocks a wave, or rows of 6144 .. 32768 weights in parts of 2048.
 bool matvec_q4k_mfma_resident_accepts(const MvArgs &a) {
     const bool pair = a.flags & FLAG_SILU_PAIR;
-    const bool parts = a.k > 4096u && a.k % 2048u == 0 && a.k / 2048u <= kMatvecMaxParts;
-    return a.m >= 1 && a.m <= 8 && (a.k == 2048u || a.k == 4096u || parts) && a.rows % 16u == 0 && (!pair || a.half % 16u == 0);
+    const bool parts = !pair && a.k > 4096u && a.k % 2048u == 0 && a.k / 2048u <= kMatvecMaxParts;
+    return a.m >= 1 && a.m <= 8 && (a.k == 2048u || parts) && a.rows % 16u == 0 && (!pair || a.half % 16u == 0);
 }
 
 template <class F>
@@ -539,7 +529,7 @@ static zhip_result launch_resident(const Dispatch &d, const MvArgs &a, uint64_t 
     ResArgs q{a, (uint32_t)w_bytes, mask, bias_bits, halves ? 0u : tiles / groups, left, (halves || 2u * left <= groups) ? 1u : 0u, parts, nullptr, nullptr};
     const dim3 grid(groups * parts);
     if (parts > 1u) {
-        const uint64_t bytes = (uint64_t)parts * (pair ? 2u : 1u) * 8u * a.rows * sizeof(float);
+        const uint64_t bytes = (uint64_t)parts * 8u * a.rows * sizeof(float);
         if (!d.work) return fail(d, ZHIP_E_GPU, "%s: no workspace", F::name());
         if (zhip_result r = d.work->reserve(d, kPartsScalesBytes + bytes)) return r;
         q.partial = reinterpret_cast<float *>(d.work->data + kPartsScalesBytes);
@@ -547,17 +537,12 @@ static zhip_result launch_resident(const Dispatch &d, const MvArgs &a, uint64_t 
             q.scales = reinterpret_cast<const float *>(d.work->data);
             if (zhip_result r = launch_matvec_parts_scales(d, F::name(), a, reinterpret_cast<float *>(d.work->data))) return r;
         }
-        if (pair) hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, true, 1, true>), grid, dim3(THREADS), 0, d.stream, q);
-        else hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, 1, true>), grid, dim3(THREADS), 0, d.stream, q);
+        hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, true>), grid, dim3(THREADS), 0, d.stream, q);
         if (zhip_result r = check_launch(d, F::name())) return r;
         return launch_matvec_parts_sum(d, F::name(), a, q.partial, parts);
-    } else if (a.k == 2048u) {
-        if (pair) hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, true, 1, false>), grid, dim3(THREADS), 0, d.stream, q);
-        else hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, 1, false>), grid, dim3(THREADS), 0, d.stream, q);
-    } else {
-        if (pair) hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, true, 2, false>), grid, dim3(THREADS), 0, d.stream, q);
-        else hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, 2, false>), grid, dim3(THREADS), 0, d.stream, q);
     }
+    if (pair) hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, true, false>), grid, dim3(THREADS), 0, d.stream, q);
+    else hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, false>), grid, dim3(THREADS), 0, d.stream, q);
     return check_launch(d, F::name());
 }
 

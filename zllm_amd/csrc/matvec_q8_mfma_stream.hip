@@ -1,5 +1,6 @@
-// matvec_q8_0, matrix-core variant for steps of up to eight tokens and k = 2048 or 4096 (longer
-// rows in parts, below): the
+// matvec_q8_0, matrix-core variant for steps of up to eight tokens and k = 2048 (longer
+// rows in parts, below; the other row lengths, and gate / up pairs over long rows, are
+// matvec_mfma_rows.hip's): the
 // weight stream is read once for all tokens of the step and nothing but partial sums crosses
 // LDS. Contract as the other variants (src/kernels/matvec_quant.wgsl.hbs with the decoder of
 // src/kernels/quant/q8_0_dot.wgsl:5-14): out[t][col0 + j] (+)= sum over 32-weight blocks of
@@ -14,10 +15,10 @@
 // scale multiplies the block's sum afterwards. A token's rows meet no other token's anywhere:
 // its results do not depend on how many tokens share the launch.
 //
-// Layout of the work. A 512-thread workgroup is eight waves that split k eight ways (8 or 16
+// Layout of the work. A 512-thread workgroup is eight waves that split k eight ways (8
 // blocks a wave); a wave builds its k range of all tokens' rows once, straight into operands
-// that stay in registers (64 VGPRs at k = 4096). Persistent workgroups take sixteen-row weight
-// tiles b, b + G, ...; a wave's part of a tile (its 256 or 512 bytes of each of the sixteen
+// that stay in registers. Persistent workgroups take sixteen-row weight
+// tiles b, b + G, ...; a wave's part of a tile (its 256 bytes of each of the sixteen
 // rows, and their scales) arrives in a private ring of LDS slots by wave-wide direct loads of
 // whole lines, a tile or more ahead, and each lane reads its row's eight bytes of a block back
 // for one matrix instruction. (The matrix instruction wants lane l to hold row l % 16, so a
@@ -400,12 +401,12 @@ __global__ __launch_bounds__(THREADS) void matvec_q8_mfma_stream_kernel(StreamAr
 
 }  // namespace
 
-// Whether this kernel can run the (already validated) arguments: whole tiles, k split into 4, 8
-// or 16 blocks a wave.
+// Whether this kernel can run the (already validated) arguments: whole tiles, k split into eight
+// blocks a wave.
 bool matvec_q8_mfma_stream_accepts(const MvArgs &a) {
     // (rows of 6144 .. 32768 weights in parts of 2048)
-    const bool parts = a.k > 4096u && a.k % 2048u == 0 && a.k / 2048u <= kMatvecMaxParts;
-    return a.m >= 1 && a.m <= 8 && (a.k == 2048u || a.k == 4096u || parts) && (!(a.flags & FLAG_SILU_PAIR) || a.half % 16u == 0) && a.rows % 16u == 0 &&
+    const bool parts = !(a.flags & FLAG_SILU_PAIR) && a.k > 4096u && a.k % 2048u == 0 && a.k / 2048u <= kMatvecMaxParts;
+    return a.m >= 1 && a.m <= 8 && (a.k == 2048u || parts) && (!(a.flags & FLAG_SILU_PAIR) || a.half % 16u == 0) && a.rows % 16u == 0 &&
            a.xr % 4u == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0;
 }
 
@@ -440,7 +441,7 @@ zhip_result launch_matvec_q8_mfma_stream(const Dispatch &d, const MvArgs &a, uin
     if (tiles < groups) { q.rounds = 0; q.left = tiles; }
     const dim3 grid(groups * parts);
     if (parts > 1u) {
-        const uint64_t bytes = (uint64_t)parts * ((a.flags & FLAG_SILU_PAIR) ? 2u : 1u) * 8u * a.rows * sizeof(float);
+        const uint64_t bytes = (uint64_t)parts * 8u * a.rows * sizeof(float);
         if (!d.work) return fail(d, ZHIP_E_GPU, "matvec_q8_0: no workspace");
         if (zhip_result r = d.work->reserve(d, kPartsScalesBytes + bytes)) return r;
         q.partial = reinterpret_cast<float *>(d.work->data + kPartsScalesBytes);
@@ -451,7 +452,7 @@ zhip_result launch_matvec_q8_mfma_stream(const Dispatch &d, const MvArgs &a, uin
         if (zhip_result r = launch_blocks<8, true>(d, q, grid)) return r;
         return launch_matvec_parts_sum(d, "matvec_q8_0", a, q.partial, parts);
     }
-    return a.k == 2048u ? launch_blocks<8>(d, q, grid) : launch_blocks<16>(d, q, grid);
+    return launch_blocks<8>(d, q, grid);
 }
 
 }  // namespace zhip
