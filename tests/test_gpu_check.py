@@ -223,6 +223,16 @@ def test_matvec_half_rows_in_registers(ctx, half, pair, k, n):
         assert rel_err(whole, want) <= 1e-5
 
 
+@pytest.mark.parametrize("k,n", [
+    (1024, 12300), (1024, 20500),    # 25 and 42 MB: four and eight tokens a workgroup
+    (2048, 6200),                    # four, two groups
+    (2568, 5000), (4096, 7400),      # two; past 60 MB rows of more than 3072 weights run the general kernel
+])
+def test_matvec_half_rows_in_registers_groups_of_tokens(ctx, k, n):
+    """The sizes from which a workgroup takes more of a step's tokens, under the bounds of the case above."""
+    test_matvec_half_rows_in_registers(ctx, "bf16", False, k, n)
+
+
 @pytest.mark.parametrize("m,n,k,half_row,accumulate,norm", [
     # 16 MB of gate rows and more: the matrix cores, a tile of gate rows and then one of up rows,
     # for every count of pieces in a row.

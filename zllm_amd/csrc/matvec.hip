@@ -366,18 +366,17 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
 // depends on the width, so such a context has steps of eight tokens at the price of its one-token
 // steps, and pays for them at one token and, up to 40 MB or so, at four. With the RMSNorm prologue, this
 // kernel / a default context's (matvec_half_row.hip, and matvec_kernel past its registers) at 1, 2, 4, 8 tokens, f16:
-//   4096 x 2048 (16 MB)          8.4 8.4 8.5 8.6 / 5.1 5.7 7.1 15.5 us
-//   8192 x 2048                  11.3 11.3 11.2 11.5 / 7.7 8.4 10.4 22.2
-//   4096 x 4096                  13.0 13.2 13.2 13.5 / 8.4 12.0 14.6 24.1
-//   151936 x 1024                52.9 53.6 54.2 54.3 / 53.6 56.8 64.9 105
-//   2 x 8192 x 1024 (32 MB)      10.1 10.0 10.0 10.0 / 8.8 9.4 11.7 19.1
-//   2 x 4096 x 2048 (32 MB)      12.3 12.4 12.6 12.9 / 8.2 8.7 10.7 24.2
+//   4096 x 2048 (16 MB)          8.4 8.4 8.5 8.6 / 5.1 5.6 6.6 8.9 us
+//   8192 x 2048                  11.0 11.0 10.9 11.1 / 7.3 8.0 9.9 13.3
+//   4096 x 4096                  13.0 13.2 13.2 13.5 / 8.4 9.2 11.7 17.2
+//   151936 x 1024                52.9 53.6 54.2 54.3 / 53.6 56.8 61.5 85.7
+//   2 x 8192 x 1024 (32 MB)      9.5 9.5 9.5 9.5 / 8.5 9.1 11.3 16.2
+//   2 x 4096 x 2048 (32 MB)      12.2 12.1 12.2 12.2 / 7.9 8.3 9.9 13.9
 //   2 x 8192 x 2048              17.8 17.9 17.9 18.0 / 13.6 14.6 17.2 38.1
 //   2 x 14336 x 4096             46.8 47.9 47.9 50.5 / 40.9 51.3 61.1 107
 // and below the line, where only the default kernels run:
-//   4096 x 1024 (8 MB)           3.7 3.9 5.5 8.2
-//   3072 x 2048                  4.4 4.9 6.3 14.8
-//   2 x 4096 x 1024 (16 MB)      5.3 5.6 7.7 12.9
+//   4096 x 1024 (8 MB)           3.9 4.0 4.5 5.9
+//   2048 x 2048 (8 MB)           4.2 4.9 4.9 6.0
 constexpr uint64_t kBf16StreamBytes = 16ull << 20;
 static bool bf16_stream_pays(const Dispatch &d, const MvArgs &a) {
     const uint64_t bytes = (uint64_t)a.rows * a.row_bytes;  // (of a pair: of its gate rows)

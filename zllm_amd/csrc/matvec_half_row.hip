@@ -1,5 +1,6 @@
 // matvec_bf16 and matvec_f16 with the inputs in registers: steps of one to eight tokens over
-// rows of up to 5120 weights, as long as a lane's inputs of all the tokens fit.
+// rows of up to 5120 weights. A workgroup takes as many of the tokens as a lane's registers hold
+// the inputs of, or fewer (see launch), others the rest.
 //
 // Such a launch reads a few MB and lasts a few microseconds, most of them trips to memory one
 // behind the other. Here there is one: the tokens' inputs and the norm weights are asked for
@@ -17,9 +18,9 @@
 // bits are the same in both and at every width.
 //
 // Measured from a graph over different weights (bf16; before: matvec.hip's kernel):
-//   2048 x 1024, RMSNorm, at 1 / 2 / 4 / 8 tokens   4.0 / 4.4 / 5.9 / 9.1 -> 2.7 / 3.3 / 4.1 / 5.8 us
-//   1024 x 2048, accumulating, at 1 / 2 / 4         4.4 / 5.4 / 7.5 -> 3.2 / 3.6 / 4.3
-//   2 x 3072 x 1024, RMSNorm, at 1 / 2 / 4          6.0 / 6.4 / 11.4 -> 4.4 / 4.8 / 7.1
+//   2048 x 1024, RMSNorm, at 1 / 2 / 4 / 8 tokens   4.0 / 4.4 / 5.9 / 9.1 -> 2.7 / 3.1 / 3.7 / 4.1 us
+//   1024 x 2048, accumulating, at 1 / 2 / 4 / 8     4.4 / 5.4 / 7.5 / 11.5 -> 3.2 / 3.6 / 3.9 / 4.6
+//   2 x 3072 x 1024, RMSNorm, at 1 / 2 / 4 / 8      6.0 / 6.4 / 11.4 / 10.4 -> 4.4 / 4.8 / 6.0 / 8.5
 //   1024 x 3072, accumulating, at 1 / 2             4.9 / 6.1 -> 3.6 / 4.0
 //   2560 x 4096 / 4096 x 4096, one token            8.8 / 9.6 -> 6.3 / 8.1
 //   2 x 8192 x 2048 / 2 x 9728 x 2560, one token    15.4 / 23.4 -> 13.0 / 18.5
@@ -46,6 +47,10 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
     extern __shared__ float4 xs4[];
     __shared__ float red[4 * MT];
     constexpr int OUTS = PAIR ? ROWS / 2 : ROWS, XV = (ITERS + 1) / 2;
+    // A step of more tokens than the registers hold: workgroups of their own for every MT of them.
+    a.x += (size_t)(MT * blockIdx.y) * a.xr;
+    a.out += (size_t)(MT * blockIdx.y) * a.out_stride;
+    a.m -= MT * blockIdx.y;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t k4 = a.k / 4u, tasks = a.k / 8u;
     const uint32_t passes = (a.rows + OUTS - 1u) / OUTS;
@@ -204,14 +209,18 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
 
 template <class D, int MT, int ITERS>
 zhip_result launch_iters(const Dispatch &d, const MvArgs &a) {
+    // (Groups of tokens: blocks a multiple of the eight dies, so that the groups' workgroups of the same rows
+    // share an L2; at three groups of 170 blocks 2 x 4096 x 2048 took 17.6 us instead of 12.4.)
     // Two workgroups a CU (three and more measured slower everywhere but on gate / up pairs of 200 MB:
     // 4096 x 4096 8.1, 8.7, 9.4 us at two, three, four a CU), a row a pass (a gate / up pair: its two rows),
     // two where a row is no more than two loads a lane: 2048 x 1024 2.9 -> 2.7 us, but 1024 x 2048 3.2 -> 3.4.
     const bool pair = (a.flags & FLAG_SILU_PAIR) != 0;
     constexpr int ROWS = ITERS <= 2 ? 2 : 1;
     const uint32_t outs = pair ? 1u : (uint32_t)ROWS;
-    const uint32_t want = ((a.rows + outs - 1u) / outs + 3u) / 4u, cap = 2u * (uint32_t)d.dev->compute_units;
-    const dim3 grid(want < cap ? want : cap);
+    const uint32_t want = ((a.rows + outs - 1u) / outs + 3u) / 4u, groups = (a.m + MT - 1u) / MT, all = 2u * (uint32_t)d.dev->compute_units;
+    uint32_t cap = all / groups, blocks = want < cap ? want : cap;
+    if (groups > 1u) blocks = want < cap ? (want + 7u) & ~7u : cap & ~7u;
+    const dim3 grid(blocks ? blocks : 1u, groups);
     const uint32_t lds = MT * a.k * 4u;
     if (pair) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2>), grid, dim3(256), lds, d.stream, a);
     else hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS>), grid, dim3(256), lds, d.stream, a);
@@ -228,21 +237,40 @@ zhip_result launch_tokens(const Dispatch &d, const MvArgs &a) {
 // The longest rows, in 512 weights, for a lane's inputs of one, two, up to four and up to eight tokens.
 constexpr uint32_t kIters1 = 10, kIters2 = 6, kIters4 = 4, kIters8 = 2;
 
+// How many tokens a workgroup takes: the fewer the sooner it has them in its registers and the more
+// workgroups share the multiply, but each group of tokens reads the weights over again, from L2 where
+// the groups keep step (their workgroups of the same rows lie on one die). us, tokens a workgroup in brackets:
+//   five and eight tokens  2048 x 2048 (8 MB) 5.5 6.0 [2], 6.2 6.6 [4], 5.9 7.1 [1]; 2048 x 1024 3.9 4.1 [2], 4.6 5.0 [4], 6.0 6.2 [8]; 14336 x 1024 (29 MB) 12.1 12.7 [4], 13.0 13.2 [8],
+//     40000 x 1024 (82 MB) 27.4 28.8 [4], 27.2 27.5 [8];
+//     2 x 3072 x 1024 (13 MB) 7.6 8.5 [2], 7.6 8.7 [4], 9.2 10.4 [8]; 2 x 4096 x 2048 (34 MB) 12.4 14.5 [2], 12.9 13.9 [4];
+//     14336 x 2048 (59 MB) 20.1 23.6 [2], 19.4 20.4 [4]; 151936 x 1024 at eight 128 [2], 101 [4], 86 [8]
+//   three and four tokens  2048 x 2048 4.8 4.9 [2], 6.1 6.1 [4]; 2 x 3072 x 1024 5.8 6.0 [2], 6.1 6.8 [4]; 2 x 4096 x 2048 10.3 10.7
+//     [2], 9.6 10.0 [4]; 32003 x 2048 (131 MB) 32.6 34.0 [2], 26.1 26.4 [4]
+// and what ran matvec.hip's kernel before, for want of registers, now / then, at two, three, four and eight tokens:
+//   2560 x 2560 at three, four, five and eight 6.2 6.4 6.8 7.8 [2] / 10.7 10.8 16.8 17.1; 32003 x 2560 (164 MB) at three, four and
+//     eight 35.8 37.6 56.8 [2] / 42.6 43.7 75.0; 2048 x 2048 at five and eight 5.5 6.0 / 11.3 11.9
+//   2560 x 3584 (18 MB) 7.0 7.5 8.2 11.6 [1] / 9.5 12.1 12.3 19.9; 4096 x 4096 (34 MB) 9.2 10.4 11.7 17.2 [1] / 11.5 13.5 13.6 22.7;
+//     8192 x 4096 (67 MB) 15.5 17.5 20.3 31.0 [1] / 19.0 19.2 19.5 34.3, and past 60 MB it is that kernel's: 2 x 7168 x 3584
+//     (103 MB) 30.9 30.8 33.0 46.7 / 24.2 24.2 24.6 43.9.
+constexpr uint64_t kSplitBytes = 24ull << 20, kWideBytes = 40ull << 20, kLoneBytes = 60ull << 20;
+uint64_t bytes_of(const MvArgs &a) { return (uint64_t)a.rows * a.row_bytes * ((a.flags & FLAG_SILU_PAIR) ? 2u : 1u); }
+
 template <class D>
 zhip_result launch(const Dispatch &d, const MvArgs &a) {
-    if (a.m == 1u) return launch_tokens<D, 1, kIters1>(d, a);
-    if (a.m == 2u) return launch_tokens<D, 2, kIters2>(d, a);
-    if (a.m <= 4u) return launch_tokens<D, 4, kIters4>(d, a);
+    const uint32_t iters = (a.k + 511u) / 512u;
+    if (a.m == 1u || iters > kIters2) return launch_tokens<D, 1, kIters1>(d, a);
+    if (a.m == 2u || iters > kIters4 || bytes_of(a) <= kSplitBytes) return launch_tokens<D, 2, kIters2>(d, a);
+    if (a.m <= 4u || iters > kIters8 || bytes_of(a) <= kWideBytes) return launch_tokens<D, 4, kIters4>(d, a);
     return launch_tokens<D, 8, kIters8>(d, a);
 }
 
 }  // namespace
 
-// The validated call of a 16-bit format: as many tokens as the registers hold for its rows, and a
+// The validated call of a 16-bit format: rows whose inputs of one token fit the registers, and a
 // matrix (each half of a pair) that 32-bit offsets reach.
 bool matvec_half_row_accepts(const MvArgs &a) {
-    const uint32_t iters = (a.k + 511u) / 512u, most = a.m == 1u ? kIters1 : a.m == 2u ? kIters2 : a.m <= 4u ? kIters4 : a.m <= 8u ? kIters8 : 0u;
-    return iters <= most && (uint64_t)a.rows * a.row_bytes <= 0x7fffffffu;
+    const uint32_t iters = (a.k + 511u) / 512u;
+    return a.m <= 8u && iters <= kIters1 && (a.m == 1u || iters <= kIters2 || bytes_of(a) <= kLoneBytes) && (uint64_t)a.rows * a.row_bytes <= 0x7fffffffu;
 }
 zhip_result launch_matvec_half_row(const Dispatch &d, const MvArgs &a, bool f16) { return f16 ? launch<DecF16>(d, a) : launch<DecBF16>(d, a); }
 
