@@ -724,6 +724,7 @@ def test_quant_matvec_mfma_variant(ctx, t, pair, rows, n, k, prologue):
     (True, 5, 272, 9728, "norm"),
     (False, 8, 2576, 14592, "plain"),  # four parts, several tiles a workgroup
     (False, 1, 19, 32512, "norm"),     # eight parts
+    (False, 8, 32776, 256, "norm"),    # four teams, many rounds: what is accumulated onto is in flight for two of them
 ])
 @pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
 def test_quant_matvec_mfma_any_row_length(ctx, t, pair, rows, n, k, prologue):

@@ -567,13 +567,15 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
         return norm && !early && !LONG ? sum * norm_scale(my_token) : sum;
     };
     // Adds up a round's tiles, behind the barrier that follows their multiply: an output tile is two
-    // waves' to add, others from one output tile to the next.
+    // waves' to add, others from one output tile to the next. (Four teams' four output tiles a round use
+    // every place of lds_before: they stay with the same waves, or those of the next round would fill a place that is still read.)
+    constexpr uint32_t adders = teams == 4u ? 3u : 7u;
     auto sum_up = [&](uint32_t round) __attribute__((always_inline)) {
         const float *part = &lds_part[round & 1u][0][0];
         const bool whole = pair && teams > 1u;  // the round has both tiles of an output
         for (uint32_t of = 0; of < teams; of += whole ? 2u : 1u) {
             const uint32_t p = round * teams + of, o = output(p);
-            if (p >= count || (wave >> 1) != (o & 7u)) continue;
+            if (p >= count || (wave >> 1) != (o & adders)) continue;
             const float sum = team_sum(part, of);
             if (LONG) {
                 if (my_token < a.m && my_row < rows_of(p)) store_apart(q.partial + kSums + ((size_t)((pair ? 2u : 1u) * kpart + (pair ? p & 1u : 0u)) * 8u + my_token) * a.rows + out0(p) + my_row, sum);
@@ -604,7 +606,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
         if (accumulate) {
             for (uint32_t of = 0; of < teams; of++) {
                 const uint32_t p = round * teams + of, o = output(p);
-                if (p >= count || (wave >> 1) != (o & 7u) || (pair && (p & 1u))) continue;
+                if (p >= count || (wave >> 1) != (o & adders) || (pair && (p & 1u))) continue;
                 const bool there = my_token < a.m && my_row < rows_of(p);
                 const uint32_t at = there ? (my_token * a.out_stride + a.col0 + out0(p) + my_row) * 4u : kNowhere;
                 load_lds_b32(make_buffer(a.out, 0x7fffffffu), (uint32_t)(uintptr_t)(lds_ptr)&lds_before[o & 3u][64u * (wave & 1u)], at);
