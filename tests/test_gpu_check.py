@@ -711,20 +711,20 @@ def test_quant_matvec_mfma_variant(ctx, t, pair, rows, n, k, prologue):
 
 
 @pytest.mark.parametrize("pair,rows,n,k,prologue", [
-    (False, 8, 40, 256, "norm"),       # one block a row
-    (True, 5, 33, 768, "norm_act"),    # three blocks, gate and up tiles of different teams, a ragged last tile
+    # (rows of other lengths than 1024 and whole 2048s in matrices of more than 8 << 20 weights, or the default kernels run)
+    (False, 8, 32776, 256, "norm"),    # one block a row
+    (True, 5, 5473, 768, "norm_act"),  # three blocks, gate and up tiles of different teams, a ragged last tile
     (False, 3, 8240, 1024, "plain"),   # four teams, more than one round
-    (False, 6, 4130, 1280, "norm"),    # two teams, a second tile for some workgroups, in halves
+    (False, 6, 6562, 1280, "norm"),    # two teams, a second tile for some workgroups, in halves
     (True, 1, 4112, 1792, "norm"),
-    (False, 8, 100, 2304, "norm_act"),  # nine blocks over sixteen waves
+    (False, 8, 3652, 2304, "norm_act"),  # nine blocks over sixteen waves
     (True, 4, 4128, 4096, "norm"),     # a block a wave
-    (False, 7, 272, 4352, "plain"),    # seventeen blocks: two for one wave
-    (True, 8, 48, 7936, "norm"),
-    (False, 2, 40, 8448, "norm_act"),  # three parts
-    (True, 5, 272, 9728, "norm"),
+    (False, 7, 1936, 4352, "plain"),   # seventeen blocks: two for one wave
+    (True, 8, 536, 7936, "norm"),
+    (False, 2, 1000, 8448, "norm_act"),  # three parts
+    (True, 5, 440, 9728, "norm"),
     (False, 8, 2576, 14592, "plain"),  # four parts, several tiles a workgroup
-    (False, 1, 19, 32512, "norm"),     # eight parts
-    (False, 8, 32776, 256, "norm"),    # four teams, many rounds: what is accumulated onto is in flight for two of them
+    (False, 1, 267, 32512, "norm"),    # eight parts
 ])
 @pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
 def test_quant_matvec_mfma_any_row_length(ctx, t, pair, rows, n, k, prologue):
@@ -735,8 +735,35 @@ def test_quant_matvec_mfma_any_row_length(ctx, t, pair, rows, n, k, prologue):
 @pytest.mark.parametrize("k", [32, 96, 288, 1056, 2080, 4128, 8224])
 def test_matvec_q8_0_mfma_ragged_rows(ctx, k):
     """Q8_0 rows whose last 256-weight block is short, one unit of it to all but one."""
-    test_quant_matvec_mfma_variant(ctx, TensorType.q8_0, False, 5, 70, k, "norm")
-    test_quant_matvec_mfma_variant(ctx, TensorType.q8_0, True, 8, 35, k, "plain")
+    n = (8 << 20) // k // 8 * 8
+    test_quant_matvec_mfma_variant(ctx, TensorType.q8_0, False, 5, n + 14, k, "norm")
+    test_quant_matvec_mfma_variant(ctx, TensorType.q8_0, True, 8, n // 2 + 11, k, "plain")
+
+
+@pytest.mark.parametrize("k,n,pair", [
+    (768, 50, False), (1024, 4104, False), (1792, 300, False),  # 12, 16 and 28 tasks: four, four and two rows a wave
+    (2560, 3280, False), (4096, 2060, False),  # past 8 << 20 weights, three and four tokens: two a workgroup
+    (4096, 11000, False), (2048, 12400, True),  # past 24 MB and, pairs, 16 MB (three tokens), inputs in LDS
+    (2304, 70, True),
+    (5120, 100, False), (4352, 4000, False),  # two slices: one token a workgroup, two
+    (12288, 50, False), (16384, 60, False),   # three, four
+])
+@pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_quant_matvec_groups_of_tokens(ctx, t, k, n, pair):
+    """Every width of a step gives each token the bits that it gets alone, through whichever kernel the width takes."""
+    c = ctx
+    x, raw = c.random(8 * k, 3).reshape(8, k), synth.random_blocks(c.rand, t.name, (2 if pair else 1) * n, k)
+    wa, init, nw = c.gpu_weights(t, raw, k), c.random(8 * (n + 3), 2), c.upload(np.ones(k, np.float32))
+    p = P.MatvecBf16(n=n, k=k, col0=1, out_stride=n + 3, eps=1e-6, norm=not pair and k <= 4096, accumulate=not pair, silu_pair=pair, half=n if pair else 0)
+
+    def run(m, at=0):
+        out = c.upload(init[at * (n + 3):][:m * (n + 3)])
+        c.launcher().launch(K.weight_kernel("matvec", t), p, [c.upload(x[at:at + m]), wa, out, nw], (K.div_ceil(n, K.matvec_rows), m, 1))
+        return c.read(out).reshape(m, n + 3)
+
+    alone = np.concatenate([run(1, at) for at in range(8)])
+    for m in (2, 3, 4, 5, 7, 8):
+        assert run(m).tobytes() == alone[:m].tobytes(), m
 
 
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate", [

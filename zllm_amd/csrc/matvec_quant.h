@@ -30,13 +30,14 @@
 // Kernels. matvec_quant_kernel (steps of one to four tokens, any row length): inputs are read
 // from a bank-conflict-free padded LDS copy kept in task order, once per task for both rows of
 // a pass (two outputs, or the gate and up rows of one output with SILU_PAIR), the next task's
-// vectors loaded before the current one is multiplied. matvec_quant_row_kernel (one or two tokens, at
-// most one task per lane, i.e. k <= 4096): the lane's 64 inputs never change from row to row,
+// vectors loaded before the current one is multiplied. matvec_quant_row_kernel (one or two tokens a
+// workgroup, at most one task per lane, i.e. k <= 4096): the lane's 64 inputs never change from row to row,
 // so they live in registers and the loop touches nothing but the weight stream; it asks for the
 // token's inputs (and norm weights) before its first weights: loads complete in order within a
 // wave, so inputs requested behind a weight row would wait for that row's trip to memory before
-// the staging could start. matvec_quant_slices_kernel: the same for one token over longer rows,
-// a 64-task slice of the row a wave. matvec_quant_long_kernel: steps of several tokens over
+// the staging could start. matvec_quant_slices_kernel: the same over longer rows,
+// a 64-task slice of the row a wave. Both take steps of more tokens as further workgroups for the same rows
+// where that is the faster way (tokens_in_registers). matvec_quant_long_kernel: steps of several tokens over
 // rows too long for the tokens to share LDS, tile by tile.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -162,7 +163,8 @@ struct KQ8 {
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = false;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
-    static constexpr bool PASS2 = false;
+    static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
+    static constexpr uint32_t REG_SLICES = 4;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
     static const char *name() { return "matvec_q8_0"; }
     struct Raw {
         uint4 q[4];
@@ -236,7 +238,8 @@ struct KQ3 {
     static constexpr bool ALL4 = false;           // (four at once measured slower on every shape: 1024 x 4096 7.7 against 7.1 us)
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
-    static constexpr bool PASS2 = false;
+    static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
+    static constexpr uint32_t REG_SLICES = 3;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
     static const char *name() { return "matvec_q3_k"; }
     struct Raw {
         uint4 u[2];
@@ -325,7 +328,8 @@ struct KQ4 {
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
-    static constexpr bool PASS2 = false;
+    static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
+    static constexpr uint32_t REG_SLICES = 2;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
     static const char *name() { return "matvec_q4_k"; }
     struct Raw {
         uint4 h, q0, q1;
@@ -409,14 +413,11 @@ struct KQ5 {
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
-    // A step of more than two tokens over 10 MB of rows or more runs as passes of two tokens in
-    // registers: the fifth bits leave the general kernel too few registers for more tokens' sums.
-    // Four tokens, general / passes of two: 9728 x 2560 21.7 / 17.6 us, 14336 x 4096 30.0 / 23.8,
-    // 50257 x 2560 82 / 57, 8192 x 2048 (11 MB) 11.8 / 10.7; below, the second launch costs more
-    // than it gains (3072 x 1024 6.0 / 6.9, 2 x 3072 x 1024 8.1 / 10.4). The other formats'
-    // general kernels are the faster ones at three and four tokens (14336 x 4096 at four tokens
-    // against twice the two-token launch: Q4_K 18.5 / 22, Q6_K 21.7 / 29, Q8_0 21.6 / 27).
-    static constexpr bool PASS2 = true;
+    // The fifth bits leave the general kernel too few registers for three or more tokens' sums: rows
+    // of up to 64 tasks always run two tokens a workgroup (four tokens, general / that: 9728 x 2560 21.7 /
+    // 17.6 us, 14336 x 4096 30.0 / 23.8, 50257 x 2560 55.9 / 51.5).
+    static constexpr bool TWO = true;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
+    static constexpr uint32_t REG_SLICES = 3;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
     static const char *name() { return "matvec_q5_k"; }
     struct Raw {
         uint4 h, b0, b1, q0, q1;
@@ -508,7 +509,8 @@ struct KQ6 {
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = false;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
-    static constexpr bool PASS2 = false;
+    static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
+    static constexpr uint32_t REG_SLICES = 4;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
     static const char *name() { return "matvec_q6_k"; }
     struct Raw {
         uint4 l0, l1, hv;
@@ -894,6 +896,8 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
 constexpr int kRowDepth = 1;
 template <class P, int MT, bool PAIR, bool TURNS, int SEG_LOG2>
 __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
+    q.t0 += MT * blockIdx.y;  // (a step of more tokens: workgroups of their own for every MT of them)
+    const bool full = MT == 1 || q.t0 + MT <= q.a.m;  // (of two tokens the second may be absent: it runs as the first again and is not stored)
     static_assert(PAIR || !TURNS, "rows in turn are a pair's");
     const MvArgs &a = q.a;
     extern __shared__ float4 lds4[];
@@ -916,7 +920,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
         const uint32_t i = tid + 256u * j;
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            const float4 *xrow = reinterpret_cast<const float4 *>(a.x + (size_t)(q.t0 + t) * a.xr);
+            const float4 *xrow = reinterpret_cast<const float4 *>(a.x + (size_t)(q.t0 + (full ? t : 0)) * a.xr);
             xv[t][j] = i < k4 ? xrow[i] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
@@ -1032,6 +1036,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
         if (lane < nkept && j < a.rows) {
 #pragma unroll
             for (int t = 0; t < MT; t++) {
+                if (t > 0 && !full) break;
                 float r = PAIR ? silu_f(kept0[t]) * kept1[t] : kept0[t];
                 if (accumulate) r += a.out[out_at(t, j)];
                 a.out[out_at(t, j)] = r;
@@ -1074,6 +1079,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
             if (tsub == SEG - 1u && j < a.rows) {
 #pragma unroll
                 for (int t = 0; t < MT; t++) {
+                    if (t > 0 && !full) break;
                     float r = PAIR ? silu_f(s0[t]) * s1[t] : s0[t];
                     if (accumulate) r += a.out[out_at(t, j)];
                     a.out[out_at(t, j)] = r;
@@ -1356,6 +1362,8 @@ static zhip_result run_long(const Dispatch &d, const KArgs &q, uint32_t blocks) 
 // K4: the most vectors of four inputs a token has (4096: k <= 16384; 8192: k <= 32768).
 template <class P, int MT, bool PAIR, int R, int NW, int K4 = 4096>
 __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
+    q.t0 += MT * blockIdx.y;
+    const bool full = MT == 1 || q.t0 + MT <= q.a.m;
     const MvArgs &a = q.a;
     extern __shared__ float4 lds4[];  // the tokens in task order, padded per task; then the partial sums [parity][group][unit of the round][slice][row][token][lane]
     __shared__ float red[4 * MT];
@@ -1375,7 +1383,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
     const bool active = task < tasks;
     const bool norm = (a.flags & FLAG_NORM) != 0, accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
     const float4 *nw = reinterpret_cast<const float4 *>(a.norm_w);
-    auto token_row = [&](int t) { return reinterpret_cast<const float4 *>(a.x + (size_t)(q.t0 + t) * a.xr); };
+    auto token_row = [&](int t) { return reinterpret_cast<const float4 *>(a.x + (size_t)(q.t0 + (full ? t : 0)) * a.xr); };
 
     // Unit n of the group's walk: R consecutive units a round, the groups' rounds interleaved.
     auto unit_of = [&](uint32_t n) { return ((n / R) * groups + group) * R + n % R; };
@@ -1493,7 +1501,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
             for (uint32_t i = 0; i < kMine; i++) {
                 const uint32_t r = slice + i * slices, u = unit_of(round * R + r);
 #pragma unroll
-                for (int t = 0; t < MT; t++) held[i][t] = (lane == 63u && r < (uint32_t)R && u < units) ? a.out[out_at(t, u)] : 0.f;
+                for (int t = 0; t < MT; t++) held[i][t] = (lane == 63u && r < (uint32_t)R && u < units && (t == 0 || full)) ? a.out[out_at(t, u)] : 0.f;
             }
         }
 #pragma unroll
@@ -1529,7 +1537,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
                     for (int j = 0; j < kRows; j++) acc[j] += theirs[sl * kCell + (j * MT + t) * 64u + lane];
                 }
                 const float s0 = segment_sum(acc[0], 6u), s1 = PAIR ? segment_sum(acc[kRows - 1], 6u) : 0.f;
-                if (lane == 63u && u < units) {
+                if (lane == 63u && u < units && (t == 0 || full)) {
                     float res = PAIR ? silu_f(s0) * s1 : s0;
                     if (accumulate) res += held[i][t];
                     a.out[out_at(t, u)] = res;
@@ -1543,17 +1551,24 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
 template <class P, int MT, bool PAIR, int R, int NW, int K4 = 4096>
 static zhip_result run_slices(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     if (!lds_opt_in<matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
-    hipLaunchKernelGGL((matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>), dim3(blocks), dim3(64 * NW), lds, d.stream, q);
+    hipLaunchKernelGGL((matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>), dim3(blocks, (q.a.m - q.t0 + MT - 1u) / MT), dim3(64 * NW), lds, d.stream, q);
     return check_launch(d, P::name());
 }
 
-// Which gate / up steps take their two rows in turn (see launch_quant).
+// A gate / up step of two tokens takes its
+// gate and up rows in turn (TURNS), except whole-wave rows of the formats whose two rows
+// fit beside two tokens' inputs (PAIR2). Two tokens with the RMSNorm prologue, through the
+// general kernel / rows in turn, 2 x 9728 x 2560: Q5_K 31.0 / 16.0 us, Q8_0 20.3 / 16.5,
+// Q6_K 18.6 / 16.8; 2 x 14336 x 4096: 44.3 / 23.6, 30.7 / 25.5, 28.3 / 25.3; both rows
+// in a pass / in turn, 2 x 8192 x 2048 (two rows to a wave's pass): Q4_K 12.5 / 8.8,
+// Q3_K 13.1 / 9.3, and 2 x 14336 x 4096: Q4_K 20.2 / 20.4, Q3_K 21.7 / 21.7. One token
+// gains nothing from it (2 x 14336 x 4096 Q4_K 15.6 / 16.3, Q5_K 19.6 / 19.8).
 template <class P, int MT, bool PAIR, int SEG_LOG2> constexpr bool row_turns() { return PAIR && MT == 2 && !(P::PAIR2 && SEG_LOG2 == 6); }
 template <class P, int MT, bool PAIR, int SEG_LOG2>
 static zhip_result run_row_seg(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     constexpr auto kernel = matvec_quant_row_kernel<P, MT, PAIR, row_turns<P, MT, PAIR, SEG_LOG2>(), SEG_LOG2>;
     if (lds > 65536u && !lds_opt_in<kernel, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, d.stream, q);
+    hipLaunchKernelGGL(kernel, dim3(blocks, (q.mt + MT - 1u) / MT), dim3(256), lds, d.stream, q);
     return check_launch(d, P::name());
 }
 template <class P, int MT, bool PAIR>
@@ -1575,6 +1590,49 @@ static zhip_result run_quant(const Dispatch &d, const KArgs &q, uint32_t lds, ui
     return check_launch(d, P::name());
 }
 
+// How many tokens a workgroup takes with their inputs in registers (0: the step goes to the kernels with
+// inputs in LDS, up to four tokens a pass over the weights). One token a workgroup costs a launch little beyond its first
+// trip to memory, so small matrices, whose weights the L2 holds for the other tokens, take that; two share a
+// weight's unpacking, which counts more the longer the launch; four tokens' sums beside their inputs do not
+// fit, and reading the weights from memory for the four costs the least once the matrix has outgrown the L2s.
+// All of them add in the same order. us at 2 / 3 / 4 / 8 tokens, inputs in LDS (two tokens: registers) / one
+// token a workgroup / two:
+//   Q8_0 2048 x 1024       3.7 6.0 6.8 13.4 / 3.1 3.3 3.3 3.9 / 3.7 3.8 3.8 4.1
+//   Q4_K 2048 x 2048       4.3 6.4 7.3 14.4 / 3.6 4.1 4.1 5.4 / 4.3 4.6 4.6 5.5
+//   Q6_K 2560 x 2560       5.9 8.5 10.0 19.1 / 5.7 6.3 7.1 10.8 / 5.9 7.6 7.6 9.8
+//   Q8_0 2 x 3072 x 1024   4.8 6.3 7.1 14.0 / 5.3 5.8 6.3 7.6 / 4.7 5.2 5.2 6.9
+//   Q4_K 4096 x 4096       7.0 9.1 10.6 20.1 / 6.6 7.7 8.6 13.4 / 6.9 8.0 8.0 11.2
+//   Q8_0 4096 x 4096       7.3 - 12.4 22.6 / - / 7.3 - 9.0 12.3
+//   Q4_K 2 x 6912 x 2304   - 14.5 17.4 34.4 / - / - 16.1 15.9 26.0
+//   Q8_0 14336 x 4096      - 19.1 22.5 43.5 / - / - 19.5 20.5 31.2
+//   Q6_K 32000 x 4096      - - 40.7 78.8 / - / - - 43.5 73.9
+//   Q8_0 40000 x 1024      - - 15.9 30.1 / - / - - 14.5 22.8
+//   Q8_0 151936 x 1024     - - 41.9 78.5 / - / - - 47.0 76.7
+// and over rows of two and more slices of 64 tasks:
+//   Q4_K 2560 x 5120       9.5 11.2 13.0 24.1 / 8.8 10.4 12.0 20.5 / 9.5 11.4 11.5 16.2
+//   Q8_0 4096 x 8192       11.2 15.4 17.2 31.7 / 10.7 14.8 16.2 28.0 / 11.3 14.2 14.9 24.3
+//   Q5_K 2560 x 9728       13.3 19.7 19.9 37.2 / 12.5 14.9 17.6 31.0 / -
+//   Q6_K 5120 x 10240      18.4 34.7 39.4 75 / 17.6 24.1 28.9 53.1 / -
+//   Q4_K 4096 x 11008      15.1 16.3 18.9 34.9 / 13.0 18.6 20.7 37.0 / -
+//   Q8_0 4096 x 14336      - - 27.7 52.9 / - / - - 26.6 47.0
+//   Q4_K 4096 x 14336      - - - 43.8 / - / - - - 46.4
+template <class P>
+static uint32_t tokens_in_registers(const MvArgs &a, uint32_t tasks) {
+    const bool pair = a.flags & FLAG_SILU_PAIR;
+    const uint64_t weights = (uint64_t)a.rows * a.k, bytes = (uint64_t)a.rows * a.row_bytes * (pair ? 2u : 1u);
+    if (a.m < 2u) return 0u;
+    if (tasks <= 64u) {
+        if (!pair && weights <= (a.m <= 4u ? 8u << 20 : 9u << 19)) return 1u;
+        if (a.m == 2u || a.m > 4u || P::TWO) return 2u;
+        return bytes <= (a.m == 4u ? (tasks <= 32u ? 48u << 20 : 96u << 20) : pair ? 16u << 20 : 24u << 20) ? 2u : 0u;
+    }
+    if (pair || tasks > 256u) return 0u;
+    const uint32_t slices = (tasks + 63u) / 64u;
+    if (slices == 2u) return a.m <= 3u && weights <= 16u << 20 ? 1u : a.m != 3u || P::REG_SLICES > 3u ? 2u : 0u;
+    if (slices == 3u) return a.m == 2u || P::REG_SLICES >= 3u ? 1u : 0u;
+    return a.m == 2u || (a.m >= 4u && P::REG_SLICES >= 4u) ? 2u : 0u;
+}
+
 // Launches the multiply for validated arguments: one pass per group of up to
 // four tokens (a pass of three has kernels of its own: in the four-token ones a quarter of the
 // multiply-adds would go to a token that is not there).
@@ -1583,34 +1641,41 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
     KArgs q{};
     q.a = a;
     q.tasks = a.k / 64u;
-    q.seg_log2 = q.tasks == 16u ? 4u : q.tasks == 32u ? 5u : 6u;
+    q.seg_log2 = q.tasks <= 16u ? 4u : q.tasks <= 32u ? 5u : 6u;
     q.nm = Masks{0x0f0f0f0fu, 0xf0f0f0f0u, 0x03030303u, 0x01010101u};
     const bool pair = a.flags & FLAG_SILU_PAIR;
     const uint32_t rpi = 64u >> q.seg_log2;
     const uint64_t tok_lds = (uint64_t)q.tasks * kTaskStride * 4u + (uint64_t)q.tasks * P::NSUM * 4u;
     const uint64_t max_lds = 160u * 1024u - 64u;
     if (tok_lds > max_lds) return fail(d, ZHIP_E_BAD_COMMAND, "%s: k = %u does not fit workgroup memory", P::name(), a.k);
+    // Rows of up to 16384 weights whose inputs stay in registers: a token or two a workgroup, the rest of
+    // the step's tokens in workgroups of their own (the blocks a multiple of the eight dies, so that those of
+    // the same rows share an L2).
+    if (const uint32_t mt = tokens_in_registers<P>(a, q.tasks)) {
+        const uint32_t groups = (a.m + mt - 1u) / mt, cus = (uint32_t)d.dev->compute_units;
+        auto shared_out = [&](uint32_t want, uint32_t all) {
+            const uint32_t cap = all / groups;
+            if (groups == 1u) return want < cap ? want : cap;
+            const uint32_t blocks = want < cap ? (want + 7u) & ~7u : cap & ~7u;
+            return blocks ? blocks : 1u;
+        };
+        q.t0 = 0;
+        q.mt = a.m;
+        if (q.tasks <= 64u) {
+            const uint32_t want = ((a.rows + rpi - 1u) / rpi + 3u) / 4u, blocks = shared_out(want, 2u * cus), lds = mt * q.tasks * kTaskStride * 4u;
+            if (mt == 1u) return pair ? run_row<P, 1, true>(d, q, lds, blocks) : run_row<P, 1, false>(d, q, lds, blocks);
+            return pair ? run_row<P, 2, true>(d, q, lds, blocks) : run_row<P, 2, false>(d, q, lds, blocks);
+        }
+        // (of two tokens eight waves for two or four slices, six for three: twelve would spill)
+        const uint32_t slices = (q.tasks + 63u) / 64u, nw = slices != 3u ? 8u : mt == 1u ? 12u : 6u, groups_here = nw / slices;
+        const uint32_t blocks = shared_out((a.rows + groups_here * 2u - 1u) / (groups_here * 2u), cus);
+        const uint32_t lds = mt * q.tasks * kTaskStride * 4u + 2u * nw * 2u * mt * 256u;
+        if (mt == 1u) return nw == 12u ? run_slices<P, 1, false, 2, 12>(d, q, lds, blocks) : run_slices<P, 1, false, 2, 8>(d, q, lds, blocks);
+        return nw == 6u ? run_slices<P, 2, false, 2, 6>(d, q, lds, blocks) : run_slices<P, 2, false, 2, 8>(d, q, lds, blocks);
+    }
     for (uint32_t t0 = 0; t0 < a.m;) {
         uint32_t left = a.m - t0;
-        // (PASS2: see KQ5)
-        const bool pass2 = P::PASS2 && q.tasks <= 64u && (uint64_t)a.rows * a.row_bytes * (pair ? 2u : 1u) >= 10u << 20;
-        const uint32_t most = pass2 ? 2u : 4u;
-        uint32_t mt = left >= most ? most : left;
-        // A step of exactly two tokens over rows of 65 .. 256 tasks keeps both tokens' slices in
-        // registers like the one-token step (Q4_K 4096 x 14336: 16.5 us tile by tile).
-        if (a.m == 2u && !pair && q.tasks > 64u && q.tasks <= 256u) {
-            q.t0 = 0;
-            q.mt = 2;
-            // (eight waves for two or four slices, six for three: twelve would spill)
-            const uint32_t slices = (q.tasks + 63u) / 64u, nw = slices == 3u ? 6u : 8u, groups_here = nw / slices;
-            const uint32_t cus = (uint32_t)d.dev->compute_units;
-            const uint32_t want = (a.rows + groups_here * 2u - 1u) / (groups_here * 2u);
-            const uint32_t blocks = want < cus ? want : cus;
-            const uint32_t lds2 = 2u * q.tasks * kTaskStride * 4u + 2u * nw * 2u * 2u * 256u;
-            const zhip_result r = nw == 6u ? run_slices<P, 2, false, 2, 6>(d, q, lds2, blocks) : run_slices<P, 2, false, 2, 8>(d, q, lds2, blocks);
-            if (r != ZHIP_OK) return r;
-            break;
-        }
+        uint32_t mt = left >= 4u ? 4u : left;
         // Two workgroups a CU must fit their staged tokens in the 160 KB of LDS. Where the
         // pass's tokens do not, the rows are long (64 tasks or more) and the step is taken tile
         // by tile with all of them (matvec_quant_long_kernel).
@@ -1684,16 +1749,8 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             t0 += q.mt;
             continue;
         }
-        // Steps of one or two tokens over rows of up to 64 tasks keep the lanes' inputs in registers,
-        // and so do Q5_K's longer steps, two tokens a pass. A two-token gate / up step takes its
-        // gate and up rows in turn (TURNS), except whole-wave rows of the formats whose two rows
-        // fit beside two tokens' inputs (PAIR2). Two tokens with the RMSNorm prologue, through the
-        // general kernel / rows in turn, 2 x 9728 x 2560: Q5_K 31.0 / 16.0 us, Q8_0 20.3 / 16.5,
-        // Q6_K 18.6 / 16.8; 2 x 14336 x 4096: 44.3 / 23.6, 30.7 / 25.5, 28.3 / 25.3; both rows
-        // in a pass / in turn, 2 x 8192 x 2048 (two rows to a wave's pass): Q4_K 12.5 / 8.8,
-        // Q3_K 13.1 / 9.3, and 2 x 14336 x 4096: Q4_K 20.2 / 20.4, Q3_K 21.7 / 21.7. One token
-        // gains nothing from it (2 x 14336 x 4096 Q4_K 15.6 / 16.3, Q5_K 19.6 / 19.8).
-        const bool xreg = (a.m <= 2u || pass2) && q.tasks <= 64u;
+        // One token over rows of up to 64 tasks keeps the lanes' inputs in registers.
+        const bool xreg = a.m == 1u && q.tasks <= 64u;
         const uint32_t per_unit = pair ? rpi : rpi * (xreg ? 1u : 2u);
         const uint32_t units = (a.rows + per_unit - 1u) / per_unit;
         const uint32_t want = (units + 3u) / 4u;
@@ -1717,12 +1774,10 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             // 9.8, Q6_K 10.9 / 10.8, Q8_0 12.05 / 11.7, gate / up pairs of Q4_K 14.4 / 13.9, of
             // Q5_K 18.3 / 17.2; 4096 x 4096 Q4_K 4.9 / 4.2; 28672 x 2048 Q4_K 8.0 / 9.05.
             const uint32_t cus = (uint32_t)d.dev->compute_units;
-            // (two tokens' inputs leave the registers for two waves a SIMD: two workgroups)
-            const bool three = mt == 1u && !pair && (uint64_t)rpi * a.row_bytes <= 3072u && passes >= cus * 48u;
+            const bool three = !pair && (uint64_t)rpi * a.row_bytes <= 3072u && passes >= cus * 48u;
             const uint32_t cap = cus * (three ? 3u : 2u), row_blocks = row_want < cap ? row_want : cap;
-            const uint32_t row_lds = mt * q.tasks * kTaskStride * 4u;
-            if (mt == 1u) r = pair ? run_row<P, 1, true>(d, q, row_lds, row_blocks) : run_row<P, 1, false>(d, q, row_lds, row_blocks);
-            else r = pair ? run_row<P, 2, true>(d, q, row_lds, row_blocks) : run_row<P, 2, false>(d, q, row_lds, row_blocks);
+            const uint32_t row_lds = q.tasks * kTaskStride * 4u;
+            r = pair ? run_row<P, 1, true>(d, q, row_lds, row_blocks) : run_row<P, 1, false>(d, q, row_lds, row_blocks);
         } else if (mt == 1u) r = pair ? run_quant<P, 1, true, 1>(d, q, lds, blocks) : run_quant<P, 1, false, 1>(d, q, lds, blocks);
         else if (mt == 2u) {
             if (small && P::STAGE2 != 2) r = pair ? run_quant<P, 2, true, 2>(d, q, lds, blocks) : run_quant<P, 2, false, 2>(d, q, lds, blocks);
