@@ -1552,6 +1552,21 @@ def test_quantize_q8_long_rows(ctx, t, k):
         assert np.max(np.abs(q.astype(np.float64) * np.repeat(d, 256, axis=1) - want) / (step / 2)) <= 1.0001
 
 
+@pytest.mark.parametrize("t,k", [(TensorType.q8_0, k) for k in (32, 1024, 1056, 3040, 4096, 5152, 8192, 8224)] +
+                                 [(TensorType.q4_k, k) for k in (256, 1280, 2048, 3328, 6144, 7424, 8448, 12544)])
+def test_quantize_q8_norm_row_lengths(ctx, t, k):
+    """The RMSNorm prologue at the ends of the lengths a thread keeps one to eight loads of, and past them: the
+    oracle's integers and scales."""
+    c = ctx
+    block, rows = K.act_block(t), 3
+    x, nw = c.random(rows * k, 3).reshape(rows, k), c.random(k, 1)
+    x[1, k - 1], x[2, 1:] = -300.0, 0
+    qx, dx = quantize_x(c, t, c.upload(x), rows, k, mode=1, eps=1e-6, nw=c.upload(nw))
+    q, d = read_q8(c, qx, dx, rows, k)
+    wq, wd = oracle.quantize_q8(x, block, mode=1, eps=1e-6, nw=nw)
+    assert np.array_equal(q, wq) and np.array_equal(d[:, : k // block].view(np.uint32), wd.view(np.uint32))
+
+
 def _llama_kats():
     import json
     import os

@@ -1,14 +1,13 @@
 // quantize_q8: rows of activations rounded to 8-bit blocks for the int8 prefill
 // multiply, value for value as llama.cpp's x86 CPU backend rounds them
-// (src/kernels/quantize_q8.wgsl, src/ref/matmul.zig:197-247). A wave takes U
-// consecutive chunks of 256 values of one row, four values a lane and chunk
+// (src/kernels/quantize_q8.wgsl, src/ref/matmul.zig:197-247). A wave takes a
+// chunk of 256 values of a row, four values a lane
 // (a chunk is one Q8_K block, or eight Q8_0 blocks of eight lanes each), and a
 // workgroup is four such waves on neighbouring chunks. A chunk's rounding is a
 // chain of dependent operations behind one 16-byte load, so what hides it is
-// other waves: without the RMSNorm prologue U is one. With it a workgroup
-// first adds the row's squares together and then takes all of the row's
-// chunks, up to four a wave, all their loads issued before the first is
-// rounded. The largest magnitude of a
+// other waves. With the RMSNorm prologue a workgroup
+// takes a whole row, every fourth chunk a wave, first adds the row's squares together and then
+// rounds. The largest magnitude of a
 // block is found with row-local DPP steps (and, for Q8_K, four lane reads),
 // the first position that holds it with a ballot. Every operation whose rounding
 // decides a value is an operation of its own (the library is compiled with
@@ -52,123 +51,180 @@ __device__ __forceinline__ float max_of_wave(float v) {
     return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
-template <int U>
-__global__ __launch_bounds__(256) void quantize_q8_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx, const float *nw) {
+// The 8-bit values of one 256-value chunk of a row, four a lane from `first` on (lanes past the row hold zeros and
+// store nothing), and its scale or scales.
+__device__ __forceinline__ void round_chunk(const QuantizeQ8Params &p, const qf32x4 &v, bool live, size_t base, uint32_t lane, uint32_t *qx, float *dx) {
+    // The lane's first largest magnitude: a strict > scan from the left.
+    float mag = fabsf(v[0]), value = v[0];
+#pragma unroll
+    for (int e = 1; e < 4; e++) {
+        const float a = fabsf(v[e]);
+        if (a > mag) {
+            mag = a;
+            value = v[e];
+        }
+    }
+    int q[4] = {0, 0, 0, 0};
+    float d = 0.f;
+    if (p.block == 256u) {
+        // Q8_K: the value itself (with its sign) at the first position of the largest
+        // magnitude: the lowest lane that holds it.
+        const float amax = max_of_wave(mag);
+        const uint64_t holders = __ballot(mag == amax);
+        const float lead = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(value), (int)__ffsll((unsigned long long)holders) - 1));
+        if (amax != 0.f) {
+            const float iscale = __fdiv_rn(-127.0f, lead);
+            d = __fdiv_rn(1.0f, iscale);
+#pragma unroll
+            for (int e = 0; e < 4; e++) q[e] = min(127, nearest_int(__fmul_rn(iscale, v[e])));
+        }
+    } else {
+        const float amax = max_of_eight(mag);
+        if (amax != 0.f) {
+            const float d32 = __fdiv_rn(amax, 127.0f);
+            const float id = __fdiv_rn(127.0f, amax);
+            d = (float)(_Float16)d32;
+#pragma unroll
+            for (int e = 0; e < 4; e++) q[e] = nearest_int(__fmul_rn(v[e], id));
+        }
+    }
+    if (!live) return;
+    qx[base / 4u] = ((uint32_t)q[0] & 0xffu) | (((uint32_t)q[1] & 0xffu) << 8) | (((uint32_t)q[2] & 0xffu) << 16) | (((uint32_t)q[3] & 0xffu) << 24);
+    if (((4u * lane) & (p.block - 1u)) == 0u) dx[base >> (p.block == 256u ? 8 : 5)] = d;  // (a division by the block would be one of 64 bits)
+}
+
+// A double of each lane plus that of the lane 32, 16, 8, 4, 2 and 1 away (by turns: after the step of 8 the rows
+// of sixteen repeat every eight lanes, so a rotation by 4 is the exchange): every lane ends with the wave's sum.
+template <int CTRL>
+__device__ __forceinline__ double add_with(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xf, 0xf, true), hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+    return v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double sum_of_wave(double v) {
+    uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const auto lo32 = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false), hi32 = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    v = __builtin_bit_cast(double, (uint64_t)hi32[0] << 32 | lo32[0]) + __builtin_bit_cast(double, (uint64_t)hi32[1] << 32 | lo32[1]);
+    b = __builtin_bit_cast(uint64_t, v);
+    const auto lo16 = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false), hi16 = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    v = __builtin_bit_cast(double, (uint64_t)hi16[0] << 32 | lo16[0]) + __builtin_bit_cast(double, (uint64_t)hi16[1] << 32 | lo16[1]);
+    v = add_with<0x128>(v);     // row_ror:8
+    v = add_with<0x124>(v);     // row_ror:4
+    v = add_with<0x4E>(v);      // quad_perm [2, 3, 0, 1]
+    return add_with<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+}
+// The RMSNorm factor as ggml computes it (src/ref/ops.zig:25-41): f32 squares
+// summed and divided in f64, an f32 mean, add, sqrt and reciprocal (then x * scale, then * w).
+__device__ __forceinline__ float norm_factor(const QuantizeQ8Params &p, double ss, double (&squares)[4]) {
+    ss = sum_of_wave(ss);
+    if ((threadIdx.x & 63u) == 0u) squares[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = (squares[0] + squares[1]) + (squares[2] + squares[3]);
+    const float mean = (float)(ss / (double)p.k);
+    // (sqrtf is the correctly rounded square root under hipcc's default options; the
+    // __fsqrt_rn intrinsic is the hardware's approximate one here and gave some rows a
+    // scale one unit in the last place away from ggml's)
+    return __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, p.eps)));
+}
+
+// The RMSNorm prologue over a row of up to 1024 J values: the row and its weights are read once and
+// kept in registers. gridDim.x workgroups a row: each adds up the whole row's squares and rounds its share of the
+// chunks. What bounds it is the chain of the two trips (the row, the stores) and a wave's rounding, 0.2 us a chunk
+// where it has the SIMD to itself. us, a row read twice by one workgroup (once for the sum) / this: 64 x 4096 4.6 / 2.5, 64 x 5120
+// 6.2 / 2.9, 128 x 4096 4.6 / 2.8, 201 x 2560 4.4 / 3.1, 512 x 1024 3.1 / 2.4, 512 x 4096 6.0 / 4.8.
+template <int J>
+__global__ __launch_bounds__(256) void quantize_q8_norm_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx, const float *nw) {
     __shared__ double squares[4];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, row = blockIdx.y;
-    const float *xr = x + (size_t)row * p.k;
-    float scale = 1.0f;
-    if (p.mode == 1u) {
-        // RMSNorm as ggml computes it (src/ref/ops.zig:25-41): f32 squares
-        // summed and divided in f64, an f32 mean, add, sqrt and reciprocal,
-        // then x * scale, then * w. (Four loads at a time: one after the other, a long
-        // row's pass over itself is a chain of trips to L2.)
-        double ss = 0.0;
-        for (uint32_t i0 = 4u * threadIdx.x; i0 < p.k; i0 += 4096u) {
-            qf32x4 r[4];
+    const uint32_t at = 4u * threadIdx.x;
+    const size_t row = (size_t)blockIdx.y * p.k;
+    qf32x4 v[J], w[J];
 #pragma unroll
-            for (uint32_t j = 0; j < 4; j++) r[j] = i0 + 1024u * j < p.k ? *reinterpret_cast<const qf32x4 *>(xr + i0 + 1024u * j) : qf32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < J; j++) v[j] = at + 1024u * j < p.k ? *reinterpret_cast<const qf32x4 *>(x + row + at + 1024u * j) : qf32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (uint32_t j = 0; j < 4; j++) {
-                if (i0 + 1024u * j >= p.k) break;
+    for (int j = 0; j < J; j++) w[j] = *reinterpret_cast<const qf32x4 *>(nw + (at + 1024u * j < p.k ? at + 1024u * j : 0u));
+    double ss = 0.0;
 #pragma unroll
-                for (int e = 0; e < 4; e++) ss += (double)__fmul_rn(r[j][e], r[j][e]);
-            }
-        }
+    for (int j = 0; j < J; j++)
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        if (lane == 0) squares[wave] = ss;
-        __syncthreads();
-        ss = (squares[0] + squares[1]) + (squares[2] + squares[3]);
-        const float mean = (float)(ss / (double)p.k);
-        // (sqrtf is the correctly rounded square root under hipcc's default options; the
-        // __fsqrt_rn intrinsic is the hardware's approximate one here and gave some rows a
-        // scale one unit in the last place away from ggml's)
-        scale = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, p.eps)));
+        for (int e = 0; e < 4; e++) ss += (double)__fmul_rn(v[j][e], v[j][e]);
+    const float scale = norm_factor(p, ss, squares);
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        if (J > 1 && j % gridDim.x != blockIdx.x) continue;
+        const bool live = at + 1024u * j < p.k;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[j][e] = live ? __fmul_rn(__fmul_rn(v[j][e], scale), w[j][e]) : 0.f;
+        round_chunk(p, v[j], live, row + at + 1024u * j, threadIdx.x & 63u, qx, dx);
     }
-
-    // The workgroup's spans of 4 U chunks: one (blockIdx.x) without the prologue; with it, all
-    // of the row's, so that the row's squares are added once.
-    for (uint32_t span = blockIdx.x; span * (1024u * U) < p.k; span += gridDim.x) {
-        const uint32_t first = ((span * 4u + wave) * U) * 256u + 4u * lane;  // the lane's first position of the wave's first chunk
-        qf32x4 v[U];
-        bool live[U];
+}
+// The same over rows of any length, read twice.
+__global__ __launch_bounds__(256) void quantize_q8_norm_long_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx, const float *nw) {
+    __shared__ double squares[4];
+    const uint32_t at = 4u * threadIdx.x;
+    const size_t row = (size_t)blockIdx.y * p.k;
+    auto four = [&](const float *from, uint32_t i0, qf32x4 (&r)[4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            live[u] = first + 256u * u < p.k;
-            v[u] = qf32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        if (p.mode == 2u) {
-            // silu(gate) * up over a row of gate | up (src/kernels/silu_mul.wgsl).
-            qf32x4 gate[U], up[U];
+        for (uint32_t j = 0; j < 4; j++) r[j] = i0 + 1024u * j < p.k ? *reinterpret_cast<const qf32x4 *>(from + i0 + 1024u * j) : qf32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    double ss = 0.0;
+    for (uint32_t i0 = at; i0 < p.k; i0 += 4096u) {
+        qf32x4 r[4];
+        four(x + row, i0, r);
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const float *g = x + (size_t)row * 2u * p.k + (live[u] ? first + 256u * u : 0u);
-                gate[u] = *reinterpret_cast<const qf32x4 *>(g);
-                up[u] = *reinterpret_cast<const qf32x4 *>(g + p.k);
-            }
+        for (uint32_t j = 0; j < 4; j++)
 #pragma unroll
-            for (int u = 0; u < U; u++)
+            for (int e = 0; e < 4; e++) ss += (double)__fmul_rn(r[j][e], r[j][e]);
+    }
+    const float scale = norm_factor(p, ss, squares);
+    for (uint32_t i0 = at; i0 - at < p.k; i0 += 4096u) {  // (whole waves: a chunk's lanes look at each other)
+        qf32x4 r[4], w[4];
+        four(x + row, i0, r);
+        four(nw, i0, w);
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[u][i] = live[u] ? gate[u][i] / (1.0f + expf(-gate[u][i])) * up[u][i] : 0.f;
-        } else {
-            qf32x4 w[U];
+        for (uint32_t j = 0; j < 4; j++) {
+            const bool live = i0 + 1024u * j < p.k;
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const qf32x4 got = *reinterpret_cast<const qf32x4 *>(xr + (live[u] ? first + 256u * u : 0u));
-                if (live[u]) v[u] = got;
-                if (p.mode == 1u) w[u] = *reinterpret_cast<const qf32x4 *>(nw + (live[u] ? first + 256u * u : 0u));
-            }
-            if (p.mode == 1u) {
-#pragma unroll
-                for (int u = 0; u < U; u++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[u][e] = live[u] ? __fmul_rn(__fmul_rn(v[u][e], scale), w[u][e]) : 0.f;
-            }
-        }
-
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            // The lane's first largest magnitude: a strict > scan from the left.
-            float mag = fabsf(v[u][0]), value = v[u][0];
-#pragma unroll
-            for (int e = 1; e < 4; e++) {
-                const float a = fabsf(v[u][e]);
-                if (a > mag) {
-                    mag = a;
-                    value = v[u][e];
-                }
-            }
-            int q[4] = {0, 0, 0, 0};
-            float d = 0.f;
-            if (p.block == 256u) {
-                // Q8_K: the value itself (with its sign) at the first position of the largest
-                // magnitude: the lowest lane that holds it.
-                const float amax = max_of_wave(mag);
-                const uint64_t holders = __ballot(mag == amax);
-                const float lead = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(value), (int)__ffsll((unsigned long long)holders) - 1));
-                if (amax != 0.f) {
-                    const float iscale = __fdiv_rn(-127.0f, lead);
-                    d = __fdiv_rn(1.0f, iscale);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) q[e] = min(127, nearest_int(__fmul_rn(iscale, v[u][e])));
-                }
-            } else {
-                const float amax = max_of_eight(mag);
-                if (amax != 0.f) {
-                    const float d32 = __fdiv_rn(amax, 127.0f);
-                    const float id = __fdiv_rn(127.0f, amax);
-                    d = (float)(_Float16)d32;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) q[e] = nearest_int(__fmul_rn(v[u][e], id));
-                }
-            }
-            if (!live[u]) continue;
-            const size_t base = (size_t)row * p.k + first + 256u * u;
-            qx[base / 4u] = ((uint32_t)q[0] & 0xffu) | (((uint32_t)q[1] & 0xffu) << 8) | (((uint32_t)q[2] & 0xffu) << 16) | (((uint32_t)q[3] & 0xffu) << 24);
-            if ((4u * lane) % p.block == 0u) dx[base / p.block] = d;
+            for (int e = 0; e < 4; e++) r[j][e] = live ? __fmul_rn(__fmul_rn(r[j][e], scale), w[j][e]) : 0.f;
+            round_chunk(p, r[j], live, row + i0 + 1024u * j, threadIdx.x & 63u, qx, dx);
         }
     }
+}
+
+// Without the prologue: a chunk a wave.
+__global__ __launch_bounds__(256) void quantize_q8_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx) {
+    const uint32_t at = 1024u * blockIdx.x + 4u * threadIdx.x;
+    const bool live = at < p.k;
+    const size_t row = blockIdx.y;
+    qf32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (p.mode == 2u) {
+        // silu(gate) * up over a row of gate | up (src/kernels/silu_mul.wgsl).
+        const float *g = x + row * 2u * p.k + (live ? at : 0u);
+        qf32x4 gate = *reinterpret_cast<const qf32x4 *>(g), up = *reinterpret_cast<const qf32x4 *>(g + p.k);
+        // (zeros give zeros: no branch around each of the four, whose chains overlap)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            gate[i] = live ? gate[i] : 0.f;
+            up[i] = live ? up[i] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = gate[i] / (1.0f + expf(-gate[i])) * up[i];
+    } else if (live) {
+        v = *reinterpret_cast<const qf32x4 *>(x + row * p.k + at);
+    }
+    round_chunk(p, v, live, row * p.k + at, threadIdx.x & 63u, qx, dx);
+}
+
+// Workgroups a row: as many as leave each a CU of its own, two up to a row a CU. One / two / four (0.25 us ahead
+// of the kernel as it is): 64 x 4096 4.1 / 3.2 / 2.7 us, 128 x 4096 4.2 / 3.3 / 3.5, 201 x 2560 3.5 / 3.4 / 3.4, 256 x 1792 3.0 / 2.6,
+// 256 x 4096 4.2 / 4.3 / 6.2; past it 300 x 5120 5.8 / 6.8 / 7.7, 512 x 2048 3.2 / 4.0, 512 x 4096 5.6 / 6.9 / 9.3.
+template <int J>
+static void launch_norm(const Dispatch &d, const QuantizeQ8Params &p, uint32_t spans, const float *x, uint32_t *qx, float *dx, const float *nw) {
+    if constexpr (J < 8) {
+        if (spans > (uint32_t)J) return launch_norm<J + 1>(d, p, spans, x, qx, dx, nw);
+    }
+    const uint32_t rows = d.grid[1], cus = (uint32_t)d.dev->compute_units;
+    const uint32_t each = cus / rows > 2u ? cus / rows : 2u, parts = rows > cus ? 1u : each < (uint32_t)J ? each : (uint32_t)J;
+    hipLaunchKernelGGL(quantize_q8_norm_kernel<J>, dim3(parts, rows), dim3(256), 0, d.stream, p, x, qx, dx, nw);
 }
 
 zhip_result launch_quantize_q8(const Dispatch &d) {
@@ -194,17 +250,14 @@ zhip_result launch_quantize_q8(const Dispatch &d) {
     const float *x = reinterpret_cast<const float *>(d.bind[1].ptr), *nw = reinterpret_cast<const float *>(d.bind[4].ptr);
     uint32_t *qx = reinterpret_cast<uint32_t *>(d.bind[2].ptr);
     float *dx = reinterpret_cast<float *>(d.bind[3].ptr);
-    // One chunk a wave, whatever the size: against two and four (the choice before, where that
-    // left two workgroups a CU), inputs in the Infinity Cache, 512 x 3072 with the SiLU-pair prologue
-    // 4.7 / 5.5 / 6.3 us, 512 x 4096 without one 3.8 / 3.9 / 4.2, 512 x 14336 with the prologue 13.9 / 13.8 /
-    // 15.9, 201 x 9728 with it 5.3 / 5.9 / 7.5; only 512 x 14336 without one is faster with two, 8.9 / 8.6.
-    // With the RMSNorm prologue a workgroup takes its whole row.
-    const uint32_t n_chunks = d.grid[0];
-    const bool whole = p.mode == 1u;
-    const dim3 grid(whole ? 1u : (n_chunks + 3u) / 4u, d.grid[1]);
-    if (whole && n_chunks > 8u) hipLaunchKernelGGL(quantize_q8_kernel<4>, grid, dim3(256), 0, d.stream, p, x, qx, dx, nw);
-    else if (whole && n_chunks > 4u) hipLaunchKernelGGL(quantize_q8_kernel<2>, grid, dim3(256), 0, d.stream, p, x, qx, dx, nw);
-    else hipLaunchKernelGGL(quantize_q8_kernel<1>, grid, dim3(256), 0, d.stream, p, x, qx, dx, nw);
+    // One chunk a wave, whatever the size: against two and four, inputs in the Infinity Cache, 512 x 3072 with the
+    // SiLU-pair prologue 4.7 / 5.5 / 6.3 us, 512 x 4096 without one 3.8 / 3.9 / 4.2, 512 x 14336 with the prologue
+    // 13.9 / 13.8 / 15.9, 201 x 9728 with it 5.3 / 5.9 / 7.5; only 512 x 14336 without one is faster with
+    // two, 8.9 / 8.6. (With the block's index shifted, not divided: 4.5, -, 13.1 and 5.5 us.)
+    const uint32_t spans = (d.grid[0] + 3u) / 4u;
+    if (p.mode != 1u) hipLaunchKernelGGL(quantize_q8_kernel, dim3(spans, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx);
+    else if (spans <= 8u) launch_norm<1>(d, p, spans, x, qx, dx, nw);
+    else hipLaunchKernelGGL(quantize_q8_norm_long_kernel, dim3(1, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx, nw);
     return check_launch(d, "quantize_q8");
 }
 
