@@ -144,6 +144,35 @@ def test_matvec_bf16_several_tokens(ctx, ctx_wide, wide, half, m, n, k, col0, pa
     assert np.array_equal(got[:, keep].astype(np.float32), want[:, keep].astype(np.float32))
 
 
+@pytest.mark.parametrize("m,n,k,accumulate", [
+    (8, 1900, 4608, True),    # three equal stretches
+    (3, 1644, 5120, False),   # two
+    (8, 1290, 6656, True),    # three, the last past the row by two lines a wave
+    (8, 1030, 8192, True),    # four
+    (1, 1000, 8704, True),    # three, the last past the row
+    (11, 587, 14336, False),  # seven; two launches of tokens
+    (5, 519, 16384, True),    # eight
+])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_stretches(ctx, ctx_wide, half, m, n, k, accumulate):
+    """Rows taken in stretches whose workgroups split the tokens, under the bounds of the case above."""
+    test_matvec_bf16_several_tokens(ctx, ctx_wide, True, half, m, n, k, 3, 2, accumulate, False)
+
+
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_stretch_past_the_row(ctx_wide, half):
+    """The last stretch's columns past a row are the next row's first: an infinity there stays in its own row."""
+    c, n, k = ctx_wide, 1000, 8704
+    bits, values = random_half(c, n * k, k ** -0.5, half)
+    bits.reshape(n, k)[1::2, :300] = 0x7c00 if half == "f16" else 0x7f80
+    out, wa = c.output(2 * n), c.upload(bits)
+    c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=1e-6), [c.upload(np.ones(2 * k, np.float32)), wa, out, wa],
+                        (K.div_ceil(n, K.matvec_rows), 2, 1))
+    got = c.read(out)[: 2 * n].reshape(2, n)
+    assert np.isposinf(got[:, 1::2]).all()
+    assert rel_err(got[0, ::2], values.reshape(n, k)[::2].astype(np.float64).sum(axis=1)) <= 1e-5
+
+
 def test_matvec_bf16_several_tokens_many_rows(ctx_wide):
     """More than forty 32-row tiles on every workgroup: the outputs kept back in workgroup
     memory are stored in the middle of the run, not only at its end."""

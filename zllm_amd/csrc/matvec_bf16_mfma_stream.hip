@@ -204,10 +204,10 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (
 // PAIR: a SILU_PAIR step, an output tile's gate rows and then its up rows (the general kernel's
 // time grows with the tokens: 2 x 8192 x 2048 f16 at eight 38 us, here 18).
 // LONG: k = 512 NP q.parts; workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
-// walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums.
+// walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums. Without the RMSNorm prologue no
+// workgroup needs more of a token than its stretch (an F16 token's scale is then the stretch's own).
 template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
 __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(StreamArgs q) {
-    static_assert(SPLIT || !LONG, "the stretches of a long row read the tokens from the planes");
     static_assert(!PAIR || !LONG, "gate / up steps take whole rows");
     constexpr uint32_t PER = PAIR ? 2u : 1u;  // weight tiles an output tile
     constexpr uint32_t PIECES = pieces_of(F16, PAIR);
@@ -250,7 +250,9 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
         // every step, but against an empty buffer: zeros land and nothing is fetched; the same
         // for the rows a share of the last rows does not have)
         const uint32_t o = load_tile / PER;
-        const __amdgpu_buffer_rsrc_t buf = o < count ? wbuf : nobuf;
+        // (and for the pieces past the row that the last stretch of one that does not divide has)
+        const bool beyond = LONG && !SPLIT && 1024u * NP * kpart + 128u * (NP * wave + load_piece) >= a.row_bytes;
+        const __amdgpu_buffer_rsrc_t buf = o < count && !beyond ? wbuf : nobuf;
         const uint32_t base = (first_row(o) + (PAIR && (load_tile & 1u) ? a.half : 0u)) * a.row_bytes + 128u * load_piece, rows = rows_of(o);
         const uint32_t dst = ring0 + load_slot * (WAVES * SLOT);
 #pragma unroll
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
         constexpr uint32_t ROW = piece_row<NP>(), PIECES_AT = (LDS_BYTES - 64u - pieces_bytes<NP, PIECES>()) & ~15u;
         constexpr uint32_t FREE = PIECES_AT < PART_BYTES ? 0u : (PIECES_AT - PART_BYTES) / (WAVES * SLOT);
         constexpr int EARLY = FREE < DEPTH - 1 ? FREE : DEPTH - 1;  // pieces of weights asked for meanwhile
-        const __amdgpu_buffer_rsrc_t xbuf = make_buffer(a.x + (wave < a.m ? (size_t)wave * a.xr : 0u), wave < a.m ? 4u * a.k : 0u);
+        const __amdgpu_buffer_rsrc_t xbuf = make_buffer(a.x + (wave < a.m ? (size_t)wave * a.xr : 0u) + 512u * NP * kpart, wave < a.m ? 4u * min(a.k, a.row_bytes / 2u - 512u * NP * kpart) : 0u);
         const __amdgpu_buffer_rsrc_t gbuf = make_buffer(a.norm_w, (a.flags & FLAG_NORM) && wave < a.m ? 4u * a.k : 0u);
         float4 v[2 * NP], g[2 * NP];
 #pragma unroll
@@ -508,7 +510,7 @@ zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
 // Whether this kernel can run the (already validated) arguments: k split into whole lines a
 // wave; a gate / up pair only over rows that one workgroup takes whole.
 // (rows of more than 4096 weights are taken in stretches of columns: equal ones in one launch, workgroups sharing a
-// tile, with a launch for their sums; unequal ones a launch each; up to 16384: the split launch stages a token in 64 KB of LDS)
+// tile, with a launch for their sums; unequal ones behind the RMSNorm prologue a launch each; up to 16384: the split launch stages a token in 64 KB of LDS)
 bool matvec_bf16_mfma_stream_accepts(const MvArgs &a) {
     if ((a.flags & FLAG_SILU_PAIR) && (a.k > 4096u || ((uint64_t)a.half + a.rows + 64u) * a.row_bytes >= 0xfffffff0ull)) return false;
     return a.m >= 1 && a.k >= 1024u && a.k <= 16384u && a.k % 512u == 0 && a.act_div == 0.f && a.rows >= 1 &&
@@ -541,19 +543,37 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
     const uint32_t rounds = (a.rows / 32u) / groups;
     const uint32_t tail = (a.rows - 32u * rounds * groups + 7u) / 8u;
     StreamArgs q{a, (uint32_t)(used < w_bytes ? used : w_bytes), rounds, tail / groups, tail % groups, groups % 8u == 0 ? 1u : 0u, nullptr, 0u, 0u, 0u, 0u, nullptr, 1u, nullptr};
-    // The tokens are split (and normalised) by a launch of their own for rows taken in stretches
-    // (no workgroup sees a whole token), and for rows whose pieces do not fit LDS (three of them a token above
-    // 3072 weights).
-    const uint32_t token_pieces = pieces_of(f16, pair);
-    const bool split = a.k > (token_pieces == 2u ? 4096u : 3072u);
     // Rows of more than 4096 weights (the FFN-down shapes; the general kernel takes them token by
     // token) go in stretches of up to 4096 columns. Stretches of equal length (14336 = 4 x 3584,
-    // 8192 = 2 x 4096 ...) go out as one launch: `launches` workgroups share a walker's tiles, a
+    // 8192 = 4 x 2048 ...) go out as one launch: `launches` workgroups share a walker's tiles, a
     // stretch each, and a second launch adds the stretches' sums in their order and applies the
     // epilogue (their sums wait in the workspace, behind the tokens' planes).
-    const uint32_t pieces = a.k / 512u, launches = (a.k + 4095u) / 4096u;
-    const bool together = launches > 1u && pieces % launches == 0u && split && launches <= kMatvecMaxParts && cus >= launches;
-    const uint64_t planes_bytes = ((2ull * token_pieces * a.m * a.k + 4ull * a.m + 64u) + 255u) & ~255ull;
+    const uint32_t token_pieces = pieces_of(f16, pair), pieces = a.k / 512u, fits = token_pieces == 2u ? 8u : 6u;
+    uint32_t launches = (a.k + 4095u) / 4096u;
+    // Without the RMSNorm prologue the workgroups split their stretches' tokens themselves: in stretches of up to 3072 columns
+    // (what fits LDS in bf16, and in f16 the sums are the shorter ones), equal ones where two more than the fewest at most are, or with a last one that ends past the
+    // row. Behind the prologue the tokens are split (and normalised) by a launch of their own, and so are those of
+    // shorter rows whose pieces do not fit (three of them a token above 3072 weights). us at one / four / eight tokens, ACCUMULATE,
+    // split in front / by the workgroups:
+    //   2048 x 8192 f16    18.4 19.2 20.2 / 13.1 13.3 13.2    bf16 17.6 19.1 21.2 / 13.0 13.2 13.0
+    //   2560 x 9728        31.8 33.1 35.6 / 16.3 16.4 16.5         30.5 32.6 38.7 / 17.2 17.7 18.0   (unequal: a launch a stretch)
+    //   4096 x 14336       32.7 33.4 34.2 / 27.7 27.7 27.5         31.9 32.9 34.5 / 27.6 27.5 27.5
+    //   2048 x 5120        14.0 14.7 15.6 / 11.2 11.3 11.3         13.4 14.6 16.6 / 11.5 11.6 11.7
+    // (f16 in two stretches of 4096, 2048 x 8192: 14.6 15.0 15.1; in three of 3584, 2560 x 9728: 16.6 16.8 17.0; relative
+    // errors as before, 1.02e-7 .. 1.11e-7, bf16 8.7e-8 .. 9.7e-8)
+    const uint32_t fewest = (pieces + 5u) / 6u;
+    const bool own = launches > 1u && !(a.flags & FLAG_NORM) && fewest + 2u <= kMatvecMaxParts && fewest + 2u <= cus;
+    if (own) {
+        launches = fewest;
+        for (uint32_t n = fewest + 2u; n >= fewest; n--) launches = pieces % n == 0u ? n : launches;
+    }
+    const bool split = !own && pieces > fits;
+    const bool together = own || (launches > 1u && pieces % launches == 0u && split && launches <= kMatvecMaxParts && cus >= launches);
+    const uint64_t planes_bytes = own ? 0ull : ((2ull * token_pieces * a.m * a.k + 4ull * a.m + 64u) + 255u) & ~255ull;
+    if (own) {
+        if (!d.work) return fail(d, ZHIP_E_GPU, "%s: no workspace", name);
+        if (zhip_result r = d.work->reserve(d, (uint64_t)launches * 8u * a.rows * sizeof(float))) return r;
+    }
     if (split) {
         const uint64_t bytes = 2ull * token_pieces * a.m * a.k;
         if (!d.work) return fail(d, ZHIP_E_GPU, "%s: no workspace", name);
@@ -580,7 +600,7 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
         q.rounds = lrounds; q.tail_base = ltail / walkers; q.tail_rem = ltail % walkers; q.by_die = walkers % 8u == 0 ? 1u : 0u;
         q.parts = launches;
         q.partial = reinterpret_cast<float *>(d.work->data + planes_bytes);
-        q.a.k = 512u * (pieces / launches);
+        q.a.k = 512u * ((pieces + launches - 1u) / launches);
         q.plane_first = 0;
         for (uint32_t t0 = 0; t0 < a.m; t0 += 8u) {
             q.a.x = a.x + (size_t)t0 * a.xr;
@@ -588,10 +608,14 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
             q.a.m = a.m - t0 < 8u ? a.m - t0 : 8u;
             q.a.flags = a.flags & ~FLAG_NORM;
             q.t0 = t0;
-            if (zhip_result r = f16 ? launch_for_k<true, true, true>(d, q, dim3(walkers * launches)) : launch_for_k<true, false, true>(d, q, dim3(walkers * launches))) return r;
+            const dim3 all(walkers * launches);
+            zhip_result r;
+            if (own) r = f16 ? launch_for_k<false, true, true>(d, q, all) : launch_for_k<false, false, true>(d, q, all);
+            else r = f16 ? launch_for_k<true, true, true>(d, q, all) : launch_for_k<true, false, true>(d, q, all);
+            if (r != ZHIP_OK) return r;
             MvArgs sum = q.a;
             sum.k = a.k;
-            if (zhip_result r = launch_matvec_parts_sum(d, name, sum, q.partial, launches)) return r;
+            if ((r = launch_matvec_parts_sum(d, name, sum, q.partial, launches)) != ZHIP_OK) return r;
         }
         return ZHIP_OK;
     }
