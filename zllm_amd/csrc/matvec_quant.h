@@ -13,8 +13,9 @@
 // lane that owns a task loads its vectors and the block's scales, so every byte
 // of the weight stream is loaded by exactly one lane per use and a wave's load
 // instruction falls in one contiguous span of the matrix. A row has k / 64
-// tasks: lane l takes tasks l, l + 64, ...; rows of 1024 or 2048 weights pack
-// four or two to a wave pass so that no lane idles.
+// tasks: lane l takes tasks l, l + 64, ...; rows of up to 1024 or 2048 weights pack
+// four or two to a wave pass so that fewer lanes idle (Q3_K 50257 x 1792 21.1 -> 13.8 us; the
+// lanes' sums reduce over fewer lanes, what they leave out being zeros: the same bits).
 //
 // Arithmetic. Per task and token the lane computes, for each sub-block s of
 // the task, scale_s * sum(q * x) - min_s * sum(x): the block formula with
