@@ -795,6 +795,21 @@ def test_quant_matvec_groups_of_tokens(ctx, t, k, n, pair):
         assert run(m).tobytes() == alone[:m].tobytes(), m
 
 
+@pytest.mark.parametrize("t,k,n", [(t, k, n) for t in (TensorType.q3_k, TensorType.q6_k) for k, n in ((1024, 509), (2048, 509), (3072, 512), (3072, 2800))])
+def test_quant_matvec_mfma_error(ctx, t, k, n):
+    """Q3_K and Q6_K rows of the lengths that the id has always had matrix-core sums for, whatever the number of rows: the
+    relative error against float64 (2-norm) within 1.5e-7. Measured: 0.9e-7 .. 1.2e-7 (the order of the additions moves it
+    by 0.1e-7); a lane's chain of the default variant gives 1.9e-7 .. 2.2e-7."""
+    c, rows = ctx, 4
+    x = np.random.default_rng(k).standard_normal((rows, k), dtype=np.float32)
+    raw, values = quant_rows(c, t, n, k)
+    wa, out = c.gpu_weights(t, raw, k), c.output(rows * n)
+    c.launcher().launch_pipeline(c.set.matvec(c.rec, K.weight_kernel("matvec", t), MFMA_VARIANT), P.MatvecBf16(n=n, k=k, col0=0, out_stride=n),
+                                 [c.upload(x), wa, out, wa], (K.div_ceil(n, MFMA_VARIANT.group_rows()), rows, 1))
+    want = x.astype(np.float64) @ values.astype(np.float64).T
+    assert np.linalg.norm(c.read(out).reshape(rows, n) - want) <= 1.5e-7 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate", [
     (8, 200, 1024, 3, 7, True),      # partial last tile, unaligned rows
     (5, 96, 4096, 4, 8, False),      # aligned rows: 16-byte stores
