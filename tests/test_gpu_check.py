@@ -810,6 +810,33 @@ def test_quant_matvec_mfma_error(ctx, t, k, n):
     assert np.linalg.norm(c.read(out).reshape(rows, n) - want) <= 1.5e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("k,n", [(768, 11000), (1280, 6600), (2560, 3400), (4096, 2060), (4352, 2000), (9728, 900)])
+@pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_quant_matvec_mfma_infinities(ctx, t, k, n):
+    """An output that the default variant makes infinite is that infinity under the matrix-core id too: infinite inputs, finite
+    ones beside them, inputs below the normal numbers; and no other token notices."""
+    c, rows = ctx, 7
+    x = c.random(rows * k, 1).reshape(rows, k)
+    x[0, 77], x[0, 78] = np.inf, 1e6
+    x[2, k - 1] = -np.inf
+    x[4] *= np.float32(2.0 ** -132)
+    x[6, 5] = x[6, 300 % k] = np.inf
+    raw, values = quant_rows(c, t, n, k)
+    xa, wa = c.upload(x), c.gpu_weights(t, raw, k)
+    p = lambda: P.MatvecBf16(n=n, k=k, col0=0, out_stride=n)
+    out, want = c.output(rows * n), c.output(rows * n)
+    c.launcher().launch_pipeline(c.set.matvec(c.rec, K.weight_kernel("matvec", t), MFMA_VARIANT), p(), [xa, wa, out, wa], (K.div_ceil(n, MFMA_VARIANT.group_rows()), rows, 1))
+    c.launcher().launch(K.weight_kernel("matvec", t), p(), [xa, wa, want, wa], (K.div_ceil(n, K.matvec_rows), rows, 1))
+    got, want = c.read(out).reshape(rows, n), c.read(want).reshape(rows, n)
+    infinite = np.isinf(want)
+    assert infinite[0].any() or t in (TensorType.q3_k, TensorType.q6_k)  # (whose default variant gives NaNs)
+    assert np.array_equal(got[infinite], want[infinite])
+    exact = x[[1, 3, 4, 5]].astype(np.float64) @ values.astype(np.float64).T
+    for i, tk in enumerate((1, 3, 5)):
+        assert rel_err(got[tk], exact[(0, 1, 3)[i]]) <= 1e-5
+    assert np.max(np.abs(got[4] - exact[2])) <= (k // 256 + 1) * 2.0 ** -149 + 1e-5 * np.max(np.abs(exact[2]))  # (a rounding to 2^-149 a block)
+
+
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate", [
     (8, 200, 1024, 3, 7, True),      # partial last tile, unaligned rows
     (5, 96, 4096, 4, 8, False),      # aligned rows: 16-byte stores

@@ -469,39 +469,45 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
             if (norm) v[t] *= gv[b];
             big[t] = fmaxf(fmaxf(fabsf(v[t][0]), fabsf(v[t][1])), fmaxf(fabsf(v[t][2]), fabsf(v[t][3])));
         }
-        // The power of two that puts the block's largest magnitude of a token in [2^14, 2^15).
+        // The power of two that puts the block's largest magnitude of a token in [2^14, 2^15) (2^126 at most).
         const uint32_t exponent = __float_as_uint(over_tokens<G>(big, lane, [](float x, float y) { return fmaxf(x, y); })) >> 23;
         uint32_t up = 268u - exponent;
-        up = up > 253u ? 253u : up;
-        if (exponent == 0u || exponent == 255u) up = 127u;
-        up <<= 23;
+        up = (up > 253u ? 253u : up) << 23;
         if (lane < (uint32_t)G) *reinterpret_cast<float *>(lds + operands_at + INVERSE_AT + 4u * lane) = __uint_as_float((254u << 23) - up);
+        // (An infinity's rounding leaves inf - inf: INFINITE makes that a zero. The finite inputs of its block, under the scale
+        // that the infinity's exponent gives, vanish beside it. One branch a group of tokens, so that their chains still overlap.)
+        auto put = [&](auto infinite) __attribute__((always_inline)) {
+            constexpr bool INFINITE = decltype(infinite)::value;
+            auto rest = [](float v, float scale, _Float16 rounded) { return INFINITE && !(fabsf((float)rounded) <= 65504.f) ? (_Float16)0.f : (_Float16)fmaf(v, scale, -(float)rounded); };
 #pragma unroll
-        for (int t = 0; t < G; t++) {
-            const uint32_t bits = __builtin_amdgcn_readlane(up, t);
-            const float scale = __uint_as_float(bits);
-            _Float16 hi[4], lo[4];
+            for (int t = 0; t < G; t++) {
+                const uint32_t bits = __builtin_amdgcn_readlane(up, t);
+                const float scale = __uint_as_float(bits);
+                _Float16 hi[4], lo[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                hi[e] = (_Float16)(v[t][e] * scale);
-                lo[e] = (_Float16)fmaf(v[t][e], scale, -(float)hi[e]);
-            }
-            *reinterpret_cast<f16x4 *>(place + 32u * t) = f16x4{hi[0], hi[2], hi[1], hi[3]};
-            *reinterpret_cast<f16x4 *>(place + 32u * t + 16u) = f16x4{lo[0], lo[2], lo[1], lo[3]};
-            if (F::MINS) {
-                // The unit's sum, over 32, the same way: half lane / 8 of the sums' rows.
-                float sum = (v[t][0] + v[t][1]) + (v[t][2] + v[t][3]);
-                sum = add_dpp<0xB1>(sum);
-                sum = add_dpp<0x4E>(sum);
-                sum = add_dpp<0x141>(sum);
-                const float part = scale * 0.03125f;
-                const _Float16 sum_hi = (_Float16)(sum * part), sum_lo = (_Float16)fmaf(sum, part, -(float)sum_hi);
-                if ((lane & 7u) == 0u) {
-                    *reinterpret_cast<_Float16 *>(lds + operands_at + SUMS_AT + 32u * t + 2u * (lane >> 3)) = sum_hi;
-                    *reinterpret_cast<_Float16 *>(lds + operands_at + SUMS_AT + 32u * t + 16u + 2u * (lane >> 3)) = sum_lo;
+                for (int e = 0; e < 4; e++) {
+                    hi[e] = (_Float16)(v[t][e] * scale);
+                    lo[e] = rest(v[t][e], scale, hi[e]);
+                }
+                *reinterpret_cast<f16x4 *>(place + 32u * t) = f16x4{hi[0], hi[2], hi[1], hi[3]};
+                *reinterpret_cast<f16x4 *>(place + 32u * t + 16u) = f16x4{lo[0], lo[2], lo[1], lo[3]};
+                if (F::MINS) {
+                    // The unit's sum, over 32, the same way: half lane / 8 of the sums' rows.
+                    float sum = (v[t][0] + v[t][1]) + (v[t][2] + v[t][3]);
+                    sum = add_dpp<0xB1>(sum);
+                    sum = add_dpp<0x4E>(sum);
+                    sum = add_dpp<0x141>(sum);
+                    const float part = scale * 0.03125f;
+                    const _Float16 sum_hi = (_Float16)(sum * part), sum_lo = rest(sum, part, sum_hi);
+                    if ((lane & 7u) == 0u) {
+                        *reinterpret_cast<_Float16 *>(lds + operands_at + SUMS_AT + 32u * t + 2u * (lane >> 3)) = sum_hi;
+                        *reinterpret_cast<_Float16 *>(lds + operands_at + SUMS_AT + 32u * t + 16u + 2u * (lane >> 3)) = sum_lo;
+                    }
                 }
             }
-        }
+        };
+        put(std::false_type{});
+        if (__ballot(exponent == 255u)) put(std::true_type{});
     };
     // Operand row l16 is token l16 / 2's, from where the token lies (an absent token's rows are whatever lies
     // there: they meet no other token's); positions of the sums' rows past the eight units are zeros. The lane's
