@@ -9,6 +9,7 @@ import pytest
 
 import oracle
 from gpucheck import bound_err, rel_err
+from zllm_amd import cmd
 from zllm_amd import kernels as K
 from zllm_amd import synth
 from zllm_amd.kernels import Kernel, TensorType, params as P
@@ -835,6 +836,43 @@ def test_quant_matvec_mfma_infinities(ctx, t, k, n):
     for i, tk in enumerate((1, 3, 5)):
         assert rel_err(got[tk], exact[(0, 1, 3)[i]]) <= 1e-5
     assert np.max(np.abs(got[4] - exact[2])) <= (k // 256 + 1) * 2.0 ** -149 + 1e-5 * np.max(np.abs(exact[2]))  # (a rounding to 2^-149 a block)
+
+
+@pytest.mark.parametrize("t,k,n", [(TensorType.q8_0, 2560, 3300), (TensorType.q6_k, 4096, 64)])
+def test_quant_matvec_mfma_wide_output_stride(ctx, t, k, n):
+    """Tokens' outputs further apart than 32-bit byte offsets behind the first reach: each adds to what it holds."""
+    c, rows, stride = ctx, 8, 0x1260_0000 // 4
+    assert 7 * stride * 4 > 1 << 31
+    x, init = c.random(rows * k, 3).reshape(rows, k), c.random(rows * n, 2).reshape(rows, n)
+    raw, values = quant_rows(c, t, n, k)
+    wa, out = c.gpu_weights(t, raw, k), c.output(7 * stride + n)
+    for tk in range(rows):
+        c.rec.write_buffer(out.buffer, 4 * tk * stride, init[tk])
+    c.launcher().launch_pipeline(c.set.matvec(c.rec, K.weight_kernel("matvec", t), MFMA_VARIANT), P.MatvecBf16(n=n, k=k, col0=0, out_stride=stride, accumulate=True),
+                                 [c.upload(x), wa, out, wa], (K.div_ceil(n, MFMA_VARIANT.group_rows()), rows, 1))
+    got = np.zeros((rows, n), np.float32)
+    for tk in range(rows):
+        c.rec.read_buffer(1 << 30 | tk, out.buffer, 4 * tk * stride, got[tk].view(np.uint8))
+    c.rec.destroy(cmd.Kind.buffer, out.buffer)
+    c.flush()
+    assert rel_err(got, init + x.astype(np.float64) @ values.astype(np.float64).T) <= 1e-5
+
+
+def test_quant_matvec_mfma_wide_input_stride(ctx):
+    """Tokens' inputs further apart than 32-bit byte offsets behind the first reach."""
+    c, t, rows, n, k, stride = ctx, TensorType.q8_0, 8, 3300, 2560, 0x2600_0000 // 4
+    assert 7 * stride * 4 > 1 << 32
+    x = c.random(rows * k, 3).reshape(rows, k)
+    raw, values = quant_rows(c, t, n, k)
+    xa, wa, out = c.output(7 * stride + k), c.gpu_weights(t, raw, k), c.output(rows * n)
+    for tk in range(rows):
+        c.rec.write_buffer(xa.buffer, 4 * tk * stride, x[tk])
+    c.launcher().launch_pipeline(c.set.matvec(c.rec, K.weight_kernel("matvec", t), MFMA_VARIANT), P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, x_stride=stride // 4),
+                                 [xa, wa, out, wa], (K.div_ceil(n, MFMA_VARIANT.group_rows()), rows, 1))
+    got = c.read(out).reshape(rows, n)
+    c.rec.destroy(cmd.Kind.buffer, xa.buffer)
+    c.flush()
+    assert rel_err(got, x.astype(np.float64) @ values.astype(np.float64).T) <= 1e-5
 
 
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate", [

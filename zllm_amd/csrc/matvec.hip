@@ -485,14 +485,14 @@ static zhip_result launch_matvec(const Dispatch &d, bool quant) {
     const bool small = weights <= 8u << 20 && !always;
     const bool matrix_cores = quant && v.lanes == 64u && v.rows == 16u && !small && (D::CHUNK == 4 || D::CHUNK == 8 || D::CHUNK == 6 || D::CHUNK == 5 || D::CHUNK == 3);
     if (matrix_cores) {
-        const bool older = older_mfma_pays(d, a, D::CHUNK);
+        const bool rows = matvec_mfma_rows_accepts(a), older = !rows || older_mfma_pays(d, a, D::CHUNK);
         if (D::CHUNK == 4 && older && matvec_q4k_mfma_resident_accepts(a)) return launch_matvec_q4k_mfma_resident(d, a, d.bind[2].size);
         if (D::CHUNK == 5 && older && matvec_q5k_mfma_resident_accepts(a)) return launch_matvec_q5k_mfma_resident(d, a, d.bind[2].size);
         if (D::CHUNK == 6 && older && matvec_q6k_mfma_stream_accepts(a)) return launch_matvec_q6k_mfma_stream(d, a, d.bind[2].size);
         if (D::CHUNK == 3 && older && matvec_q3k_mfma_stream_accepts(a)) return launch_matvec_q3k_mfma_stream(d, a, d.bind[2].size);
         if (D::CHUNK == 8 && older && matvec_q8_0_mfma_flat_accepts(a)) return launch_matvec_q8_0_mfma_flat(d, a, d.bind[2].size);
         if (D::CHUNK == 8 && older && matvec_q8_mfma_stream_accepts(a)) return launch_matvec_q8_mfma_stream(d, a, d.bind[2].size);
-        if (matvec_mfma_rows_accepts(a)) return launch_matvec_mfma_rows(d, a, D::CHUNK);
+        if (rows) return launch_matvec_mfma_rows(d, a, D::CHUNK);
     }
     // The tuned kernel takes rows of whole 64-weight tasks.
     if (D::CHUNK != 0 && p.k % 64u == 0) return launch_matvec_quant(d, a, D::CHUNK);

@@ -59,6 +59,7 @@ constexpr uint32_t WAVES = 16, THREADS = 64 * WAVES;
 constexpr uint32_t GROUP = 8u * 16u + 16u, INVERSE_AT = 32u * GROUP, SUMS_AT = INVERSE_AT + 16u, OPERANDS = SUMS_AT + 128u;
 
 constexpr uint32_t kMaxParts = 8;  // rows of up to 32768 weights
+constexpr uint32_t kOutBytes = 0x7fffffff;  // how far behind a.out a step that accumulates reads
 constexpr uint32_t kScales = kMaxParts * 8u, kSums = kScales + 8u;
 
 struct RowsArgs {
@@ -615,7 +616,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
                 if (p >= count || (wave >> 1) != (o & adders) || (pair && (p & 1u))) continue;
                 const bool there = my_token < a.m && my_row < rows_of(p);
                 const uint32_t at = there ? (my_token * a.out_stride + a.col0 + out0(p) + my_row) * 4u : kNowhere;
-                load_lds_b32(make_buffer(a.out, 0x7fffffffu), (uint32_t)(uintptr_t)(lds_ptr)&lds_before[o & 3u][64u * (wave & 1u)], at);
+                load_lds_b32(make_buffer(a.out, kOutBytes), (uint32_t)(uintptr_t)(lds_ptr)&lds_before[o & 3u][64u * (wave & 1u)], at);
             }
         }
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -718,8 +719,12 @@ zhip_result launch_format(const Dispatch &d, const MvArgs &a) {
 
 }  // namespace
 
-// Whether the kernel can run the (already validated) arguments.
-bool matvec_mfma_rows_accepts(const MvArgs &a) { return a.m >= 1u && a.m <= 8u && a.k <= kMaxParts * WAVES * 256u; }
+// Whether the kernel can run the (already validated) arguments: rows of up to eight parts, and inputs and (where it adds
+// to them) outputs that its 32-bit offsets reach, of eight tokens so that the route is the same at every width.
+bool matvec_mfma_rows_accepts(const MvArgs &a) {
+    const uint64_t x_end = (7ull * a.xr + a.k) * 4u, out_end = (7ull * a.out_stride + a.col0 + a.rows) * 4u;
+    return a.m >= 1u && a.m <= 8u && a.k <= kMaxParts * WAVES * 256u && x_end < kNowhere && (!(a.flags & FLAG_ACCUMULATE) || out_end <= kOutBytes);
+}
 zhip_result launch_matvec_mfma_rows(const Dispatch &d, const MvArgs &a, int type) {
     switch (type) {
     case 3: return launch_format<RowsQ3>(d, a);
