@@ -838,6 +838,20 @@ def test_quant_matvec_mfma_infinities(ctx, t, k, n):
     assert np.max(np.abs(got[4] - exact[2])) <= (k // 256 + 1) * 2.0 ** -149 + 1e-5 * np.max(np.abs(exact[2]))  # (a rounding to 2^-149 a block)
 
 
+@pytest.mark.parametrize("n,pair", [(1024, False), (9000, False), (3072, True)])
+@pytest.mark.parametrize("t", [TensorType.q4_k, TensorType.q5_k])
+def test_quant_matvec_mfma_short_rows_are_the_default_variants(ctx, t, n, pair):
+    """Q4_K and Q5_K rows of 1024 weights in matrices of up to 12 << 20 weights: the default variant's launch under the
+    matrix-core id too, bit for bit."""
+    c, rows, k = ctx, 4, 1024
+    raw = synth.random_blocks(c.rand, t.name, (2 if pair else 1) * n, k)
+    xa, wa, out, want = c.upload(c.random(rows * k, 3)), c.gpu_weights(t, raw, k), c.output(rows * n), c.output(rows * n)
+    p = lambda: P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, silu_pair=pair, half=n if pair else 0)
+    c.launcher().launch_pipeline(c.set.matvec(c.rec, K.weight_kernel("matvec", t), MFMA_VARIANT), p(), [xa, wa, out, wa], (K.div_ceil(n, MFMA_VARIANT.group_rows()), rows, 1))
+    c.launcher().launch(K.weight_kernel("matvec", t), p(), [xa, wa, want, wa], (K.div_ceil(n, K.matvec_rows), rows, 1))
+    assert c.read_bytes(out).tobytes() == c.read_bytes(want).tobytes()
+
+
 @pytest.mark.parametrize("t,k,n", [(TensorType.q8_0, 2560, 3300), (TensorType.q6_k, 4096, 64)])
 def test_quant_matvec_mfma_wide_output_stride(ctx, t, k, n):
     """Tokens' outputs further apart than 32-bit byte offsets behind the first reach: each adds to what it holds."""

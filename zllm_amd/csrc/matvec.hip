@@ -477,12 +477,15 @@ static zhip_result launch_matvec(const Dispatch &d, bool quant) {
     // launch is over before the matrix cores' sixteen-row tiles have their operands built. us at 1 / 4 / 8 tokens,
     // matrix cores / default: Q8_0 1024 x 3072 5.8 6.4 8.1 / 3.2 4.3 5.8, Q4_K 4096 x 1792 6.5 7.0 8.0 / 3.9 5.6 7.8,
     // Q3_K 2560 x 2560 6.5 7.2 9.0 / 4.3 7.0 9.1, Q6_K 6.8 7.5 9.5 / 4.4 7.1 9.8; above, Q4_K 4096 x 4096 6.9 7.4 7.7 /
-    // 5.7 8.1 11.2. Not so rows of 1024 weights, of whole 2048s and, in Q6_K and Q3_K, of 3072: the matrix cores' sums are the ones nearer to the
+    // 5.7 8.1 11.2. Not so rows of whole 2048s, in Q8_0, Q6_K and Q3_K of 1024 and in Q6_K and Q3_K of 3072: the matrix cores' sums are the ones nearer to the
     // exact (relative error, matrix cores / default: at 1024 weights Q8_0 1.15e-7 / 1.36e-7, Q3_K 1.13e-7 / 2.13e-7, Q6_K 1.05e-7 /
     // 2.22e-7, at 3072 Q3_K 0.90e-7 / 1.96e-7, Q6_K 1.06e-7 / 2.05e-7), and callers of the id have always had them there.
+    // Q4_K and Q5_K rows of 1024 weights want sixteen million weights (four tiles a CU: a round of the kernel's four teams). Q4_K
+    // 4096 outputs 6.3 6.8 7.6 / 3.2 4.1 5.4, 9000 8.1 8.7 9.5 / 3.8 6.1 8.0, 11718 8.0 8.8 9.6 / 3.9 6.3 9.2, 16384 6.9 6.9 7.6 / 4.4 7.4 11.0.
     const uint64_t weights = (uint64_t)a.rows * a.k * (pair ? 2u : 1u);
-    const bool always = a.k == 1024u || a.k % 2048u == 0 || (a.k == 3072u && (D::CHUNK == 3 || D::CHUNK == 6));
-    const bool small = weights <= 8u << 20 && !always;
+    constexpr bool Q36 = D::CHUNK == 3 || D::CHUNK == 6, Q45 = D::CHUNK == 4 || D::CHUNK == 5;
+    const bool always = a.k % 2048u == 0 || (a.k == 1024u && !Q45) || (a.k == 3072u && Q36);
+    const bool small = !always && weights <= (Q45 && a.k == 1024u ? 12u << 20 : 8u << 20);
     const bool matrix_cores = quant && v.lanes == 64u && v.rows == 16u && !small && (D::CHUNK == 4 || D::CHUNK == 8 || D::CHUNK == 6 || D::CHUNK == 5 || D::CHUNK == 3);
     if (matrix_cores) {
         const bool rows = matvec_mfma_rows_accepts(a), older = !rows || older_mfma_pays(d, a, D::CHUNK);
