@@ -345,14 +345,18 @@ zhip_result launch_matvec_q8_0_mfma_flat(const Dispatch &d, const MvArgs &a, uin
 //    weights always: 4096 outputs 7.3 7.2 7.3 / 6.6 7.1 7.7) 64000 x 4096 (four and eight tokens) 46.4 49.7 / 51.2 52.9, 32000 x 4096 28.6 29.6 / 28.7 30.6, 4096 x 4096 14.7 15.5 /
 //    8.6 10.3; Q3_K 64000 x 4096 38.9 40.9 / 42.9 44.1, 2 x 14336 x 4096 23.5 25.3 / 23.6 25.6, 4096 x 4096 12.7 13.3 / 7.4 9.4;
 //    Q8_0 151936 x 1024 33.1 33.2 / 36.1 36.0, 50257 x 1024 16.9 16.8 / 16.7 16.8, 2 x 3072 x 1024 9.0 9.1 / 7.3 7.9.
+//  * Q3_K rows of 1024 weights, no pair: but where the tiles of a CU fill matvec_mfma_rows.hip's rounds of four. 4096 outputs 6.4 6.4 6.5 /
+//    6.6 7.1 7.7, 9000 7.9 8.0 8.2 / 9.1 9.7 10.2, 16384 (four a CU) 8.3 8.3 8.6 / 7.3 7.2 7.5, 20480 9.4 9.4 9.7 / 9.7 9.6 9.9, 24576 9.4 9.3 9.6 / 9.9 9.6 10.0,
+//    32000 (eight) 10.9 11.0 11.5 / 10.3 10.0 10.4.
 static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
     const bool pair = a.flags & FLAG_SILU_PAIR, parts = a.k > 4096u;
     const uint64_t tiles = ((uint64_t)a.rows * (pair ? 2u : 1u) + 15u) / 16u, cus = (uint64_t)d.dev->compute_units;
+    const uint64_t each = (tiles + cus - 1u) / cus;
     switch (type) {
     case 4: case 5: return a.k == 2048u || (parts && !pair);
     case 8: return a.k == 1024u ? tiles >= 12u * cus : a.k == 2048u || (parts && !pair && a.rows < 8192u);
     case 6: return a.k == 1024u || tiles >= 12u * cus;
-    default: return parts ? !pair || tiles >= 8u * cus : tiles >= 8u * cus;
+    default: return (parts && !pair) || (a.k == 1024u && !pair && !(each == 4u || each == 7u || each == 8u)) || tiles >= 8u * cus;
     }
 }
 // matvec_bf16 on the matrix cores, the weights read once for all tokens (matvec_bf16_mfma_stream.hip).
