@@ -348,6 +348,10 @@ zhip_result launch_matvec_q8_0_mfma_flat(const Dispatch &d, const MvArgs &a, uin
 //  * Q3_K rows of 1024 weights, no pair: but where the tiles of a CU fill matvec_mfma_rows.hip's rounds of four. 4096 outputs 6.4 6.4 6.5 /
 //    6.6 7.1 7.7, 9000 7.9 8.0 8.2 / 9.1 9.7 10.2, 16384 (four a CU) 8.3 8.3 8.6 / 7.3 7.2 7.5, 20480 9.4 9.4 9.7 / 9.7 9.6 9.9, 24576 9.4 9.3 9.6 / 9.9 9.6 10.0,
 //    32000 (eight) 10.9 11.0 11.5 / 10.3 10.0 10.4.
+//  * Q6_K in parts, no pair: from four tiles a CU on. 4096 x 6144 14.7 14.7 15.4 / 11.9 12.5 14.1, 8192 x 8192 19.6 19.4 20.5 / 18.5 18.8 20.5,
+//    8192 x 14336 28.2 28.2 30.3 / 28.0 27.8 30.0, 16384 x 6144 26.0 25.9 27.7 / 26.8 26.9 28.8, 16384 x 14336 43.8 44.1 47.4 / 46.9 47.3 50.5,
+//    28672 x 14336 72.9 73.7 76.5 / 78.9 79.5 83.1; pairs 2 x 14336 x 6144 41.3 41.8 44.4 / 41.0 41.9 44.2, 2 x 14336 x 8192 46.2 46.6 49.6 / 44.2
+//    45.3 48.3, 2 x 14336 x 14336 75.4 77.5 82.4 / 76.3 78.0 82.7.
 static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
     const bool pair = a.flags & FLAG_SILU_PAIR, parts = a.k > 4096u;
     const uint64_t tiles = ((uint64_t)a.rows * (pair ? 2u : 1u) + 15u) / 16u, cus = (uint64_t)d.dev->compute_units;
@@ -355,7 +359,7 @@ static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
     switch (type) {
     case 4: case 5: return a.k == 2048u || (parts && !pair);
     case 8: return a.k == 1024u ? tiles >= 12u * cus : a.k == 2048u || (parts && !pair && a.rows < 8192u);
-    case 6: return a.k == 1024u || tiles >= 12u * cus;
+    case 6: return a.k == 1024u || (parts ? !pair && tiles >= 4u * cus : tiles >= 12u * cus);
     default: return (parts && !pair) || (a.k == 1024u && !pair && !(each == 4u || each == 7u || each == 8u)) || tiles >= 8u * cus;
     }
 }

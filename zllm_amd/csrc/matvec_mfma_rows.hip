@@ -12,13 +12,13 @@
 // is applied to a unit's sum.
 //
 // Layout. A workgroup of sixteen waves takes tiles of sixteen rows (eight where whole tiles do not
-// share out), all of k: a wave has one or two blocks of every row of its tiles, and of rows of up to half
+// share out), all of k: a wave has one or two (Q6_K: one) blocks of every row of its tiles, and of rows of up to half
 // (a quarter) as many blocks as waves two (four) teams take a tile each. The wave brings its blocks' inputs
 // in, turns them into operands through its own LDS and keeps them in registers; its weights arrive by direct loads of
 // 16 bytes a lane, sixteen rows' pieces in a row, two or one blocks ahead in slots of its own: it waits
 // for no one. One barrier a round, behind which two waves add the partial sums of a tile and
 // store. The RMSNorm factor is left to the outputs, so nothing waits for the row's squares either. Rows of more than
-// 8192 weights are shared by k / 4096 workgroups, which leave their sums to a launch of their own.
+// 8192 weights (Q6_K: 4096) are shared by k / 4096 workgroups, which leave their sums to a launch of their own.
 //
 // What bounds it: short launches the chain launch - inputs - operands - multiply - sum, of which the
 // operands' VALU and LDS work grows with the tokens (0.3 us a token at k = 4096, every workgroup the
@@ -137,6 +137,7 @@ template <bool FIFTH>
 struct RowsQ45 {
     static constexpr uint32_t BLOCK = FIFTH ? 176 : 144, CHUNKS = BLOCK / 16;
     static constexpr uint32_t SLOTS = 3;
+    static constexpr uint32_t MOST = 2;   // blocks a wave keeps of a row
     static constexpr bool MINS = true;    // has minimums
     static constexpr bool RAGGED = false;  // rows are whole blocks
     static constexpr bool SPLIT = false;   // a row's scales lie behind its weights
@@ -192,7 +193,10 @@ struct RowsQ45 {
 // Q6_K (blocks padded to 224 bytes): a weight is d * s * (q - 32) with s a signed byte for sixteen weights. The
 // product s * (q - 32) has up to 13 bits: its rounding to f16 and what that leaves are an instruction each.
 struct RowsQ6 {
-    static constexpr uint32_t BLOCK = 224, CHUNKS = 14, SLOTS = 2;
+    // (a wave keeps one block of a row: with two the kernel spilled, at 128 registers. Rows of 17 .. 32 blocks in two parts against
+    // that, at one / four / eight tokens: 16384 x 8192 34.0 34.2 37.0 -> 29.1 28.9 31.1 us, 2 x 8192 x 6144 31.3 32.9 35.9 -> 26.9 27.5 29.8, 4096 x
+    // 5120 12.6 13.1 16.5 -> 11.8 12.2 13.8, 2560 x 6912 11.2 12.2 15.5 -> 12.2 12.5 14.1)
+    static constexpr uint32_t BLOCK = 224, CHUNKS = 14, SLOTS = 2, MOST = 1;
     static constexpr bool MINS = false, RAGGED = false, SPLIT = false;
     static const char *name() { return "matvec_q6_k"; }
     static __device__ __forceinline__ uint32_t chunk_at(uint32_t, uint32_t b, uint32_t c, uint32_t) { return BLOCK * b + 16u * c; }
@@ -238,7 +242,7 @@ struct RowsQ6 {
 // scales - 32 and d): a weight is d * s * (q - 4), the product exact in f16. Blocks are 128 bytes, so their
 // units are permuted by the row: unpermuted, sixteen rows' reads would meet in two banks.
 struct RowsQ3 {
-    static constexpr uint32_t BLOCK = 128, CHUNKS = 8, SLOTS = 3;
+    static constexpr uint32_t BLOCK = 128, CHUNKS = 8, SLOTS = 3, MOST = 2;
     static constexpr bool MINS = false, RAGGED = false, SPLIT = false;
     static const char *name() { return "matvec_q3_k"; }
     static __device__ __forceinline__ uint32_t chunk_at(uint32_t, uint32_t b, uint32_t c, uint32_t row) { return BLOCK * b + 16u * (c ^ (row & 7u)); }
@@ -267,7 +271,7 @@ struct RowsQ3 {
 // Q8_0 split rows (k signed bytes, then k / 32 f16 scales): in a slot a row's 256 bytes and its eight
 // scales. The scale, eleven bits of its own, meets a unit's sums.
 struct RowsQ8 {
-    static constexpr uint32_t BLOCK = 272, CHUNKS = 17, SLOTS = 2;
+    static constexpr uint32_t BLOCK = 272, CHUNKS = 17, SLOTS = 2, MOST = 2;
     static constexpr bool MINS = false, RAGGED = true, SPLIT = true;
     static const char *name() { return "matvec_q8_0"; }
     static __device__ __forceinline__ uint32_t chunk_at(uint32_t k, uint32_t b, uint32_t c, uint32_t) { return c < 16u ? 256u * b + 16u * c : k + 16u * b; }
@@ -690,7 +694,7 @@ template <class F>
 zhip_result launch_format(const Dispatch &d, const MvArgs &a) {
     const bool pair = (a.flags & FLAG_SILU_PAIR) != 0, norm = (a.flags & FLAG_NORM) != 0;
     const uint32_t blocks = (a.k + 255u) / 256u, tiles = (a.rows + 15u) / 16u;
-    const uint32_t parts = blocks > 2u * WAVES ? (blocks + WAVES - 1u) / WAVES : 1u;
+    const uint32_t parts = blocks > F::MOST * WAVES ? (blocks + WAVES - 1u) / WAVES : 1u;
     const uint32_t most = (uint32_t)d.dev->compute_units / parts;
     if (most == 0u) return fail(d, ZHIP_E_GPU, "%s: %d compute units for %u parts of a row", F::name(), d.dev->compute_units, parts);
     const uint32_t groups = tiles < most ? (2u * tiles <= most ? 2u * tiles : tiles) : most;
@@ -711,7 +715,9 @@ zhip_result launch_format(const Dispatch &d, const MvArgs &a) {
         else hipLaunchKernelGGL(matvec_mfma_rows_sum_kernel<false>, sums, dim3(256), 0, d.stream, a, q.partial, parts, norm && a.act_div <= 0.f);
         return check_launch(d, F::name());
     }
-    if (blocks > WAVES) return launch_act<F, 2, 1, false>(d, q);
+    if constexpr (F::MOST > 1u) {
+        if (blocks > WAVES) return launch_act<F, 2, 1, false>(d, q);
+    }
     if (blocks > WAVES / 2u) return launch_act<F, 1, 1, false>(d, q);
     if (blocks > WAVES / 4u || count < 4u) return launch_act<F, 1, 2, false>(d, q);
     return launch_act<F, 1, 4, false>(d, q);
