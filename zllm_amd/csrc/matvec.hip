@@ -352,6 +352,12 @@ zhip_result launch_matvec_q8_0_mfma_flat(const Dispatch &d, const MvArgs &a, uin
 //    8192 x 14336 28.2 28.2 30.3 / 28.0 27.8 30.0, 16384 x 6144 26.0 25.9 27.7 / 26.8 26.9 28.8, 16384 x 14336 43.8 44.1 47.4 / 46.9 47.3 50.5,
 //    28672 x 14336 72.9 73.7 76.5 / 78.9 79.5 83.1; pairs 2 x 14336 x 6144 41.3 41.8 44.4 / 41.0 41.9 44.2, 2 x 14336 x 8192 46.2 46.6 49.6 / 44.2
 //    45.3 48.3, 2 x 14336 x 14336 75.4 77.5 82.4 / 76.3 78.0 82.7.
+//  * gate / up pairs from seven tiles a CU on (Q6_K: rows of 3072 and 4096 weights), other rows of 3072 weights earlier still (twelve blocks for sixteen waves). Q3_K 2 x 14336 x 4096 with
+//    RMSNorm 23.7 23.4 25.2 / 24.6 24.6 26.9, without 22.1 21.8 23.7 / 24.3 24.0 25.8, 2 x 12288 x 4096 23.5 23.4 25.2 / 20.5 19.8 22.0,
+//    2 x 14336 x 2048 15.0 15.0 16.1 / 15.4 15.8 16.3, 2 x 14336 x 6144 36.9 37.3 39.8 / 39.3 40.8 44.6; Q6_K 2 x 14336 x 4096 28.0 26.8 28.6 / 27.5 27.0 28.5,
+//    without RMSNorm 26.0 25.1 26.8 / 27.2 26.8 28.1, 2 x 12288 x 4096 26.8 26.7 28.3 / 22.6 22.6 24.3. Rows of 3072: Q3_K 12288 outputs 14.7 14.5 15.3 /
+//    12.1 12.3 14.6, 16384 14.5 14.3 15.1 / 14.4 14.7 16.9, 32000 20.2 20.2 21.5 / 23.9 24.5 26.8, 2 x 4096 14.2 13.9 14.7 / 9.5 9.9 12.0, 2 x 6144 14.4
+//    14.1 14.9 / 14.6 14.9 17.1; Q6_K 20480 20.7 20.2 21.5 / 18.1 17.9 20.3, 24576 20.6 20.5 21.5 / 21.0 20.3 22.8, 32000 24.0 23.7 25.1 / 25.7 25.4 27.9, 2 x 12288 23.9 23.6 24.9 / 21.0 20.4 22.7.
 static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
     const bool pair = a.flags & FLAG_SILU_PAIR, parts = a.k > 4096u;
     const uint64_t tiles = ((uint64_t)a.rows * (pair ? 2u : 1u) + 15u) / 16u, cus = (uint64_t)d.dev->compute_units;
@@ -359,8 +365,11 @@ static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
     switch (type) {
     case 4: case 5: return a.k == 2048u || (parts && !pair);
     case 8: return a.k == 1024u ? tiles >= 12u * cus : a.k == 2048u || (parts && !pair && a.rows < 8192u);
-    case 6: return a.k == 1024u || (parts ? !pair && tiles >= 4u * cus : tiles >= 12u * cus);
-    default: return (parts && !pair) || (a.k == 1024u && !pair && !(each == 4u || each == 7u || each == 8u)) || tiles >= 8u * cus;
+    case 6: return a.k == 1024u || (parts ? !pair && tiles >= 4u * cus : tiles >= (pair && a.k >= 3072u ? 7u : a.k == 3072u ? 6u : 12u) * cus);
+    default:
+        if (a.k == 1024u) return pair ? tiles >= 8u * cus : tiles >= 8u * cus || !(each == 4u || each == 7u || each == 8u);
+        if (a.k == 3072u) return tiles >= (pair ? 3u : 4u) * cus;
+        return pair ? tiles >= 7u * cus : parts || tiles >= 8u * cus;
     }
 }
 // matvec_bf16 on the matrix cores, the weights read once for all tokens (matvec_bf16_mfma_stream.hip).
