@@ -777,6 +777,7 @@ def test_matvec_q8_0_mfma_ragged_rows(ctx, k):
     (2304, 70, True),
     (5120, 100, False), (4352, 4000, False),  # two slices: one token a workgroup, two
     (12288, 50, False), (16384, 60, False),   # three, four
+    (2048, 26500, False), (2560, 27000, False),  # past 13 and 43 thousand wave passes: seven (Q6_K: five and eight) tokens with inputs in LDS
 ])
 @pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
 def test_quant_matvec_groups_of_tokens(ctx, t, k, n, pair):

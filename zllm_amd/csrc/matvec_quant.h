@@ -155,6 +155,8 @@ __device__ __forceinline__ float dot_bytes(uint32_t word, const float4 &x, float
 // the start of a stretch of rows (base: the row's offset in the stretch) and fetch() loads them
 // through a range-checked buffer that begins at the stretch.
 
+constexpr uint32_t kAny = 0xffffffffu / 1000u;
+
 // Q8_0 split rows (src/kernels/repack_q8_0.wgsl): k signed bytes, then k / 32
 // f16 scales. Task = 64 consecutive weights, two blocks of 32 with a scale each;
 // no minimum, so the input sums go unused.
@@ -166,6 +168,7 @@ struct KQ8 {
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 4;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_PASSES[2][4] = {{kAny, kAny, 28, kAny}, {kAny, kAny, 70, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q8_0"; }
     struct Raw {
         uint4 q[4];
@@ -241,6 +244,7 @@ struct KQ3 {
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 3;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_PASSES[2][4] = {{26, kAny, 13, 30}, {65, kAny, 33, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q3_k"; }
     struct Raw {
         uint4 u[2];
@@ -331,6 +335,7 @@ struct KQ4 {
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 2;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_PASSES[2][4] = {{30, kAny, 18, 30}, {kAny, kAny, 90, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q4_k"; }
     struct Raw {
         uint4 h, q0, q1;
@@ -419,6 +424,7 @@ struct KQ5 {
     // 17.6 us, 14336 x 4096 30.0 / 23.8, 50257 x 2560 55.9 / 51.5).
     static constexpr bool TWO = true;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 3;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_PASSES[2][4] = {{kAny, kAny, kAny, kAny}, {kAny, kAny, kAny, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q5_k"; }
     struct Raw {
         uint4 h, b0, b1, q0, q1;
@@ -512,6 +518,7 @@ struct KQ6 {
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 4;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_PASSES[2][4] = {{kAny, kAny, 24, kAny}, {43, 64, 22, 38}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q6_k"; }
     struct Raw {
         uint4 l0, l1, hv;
@@ -1617,6 +1624,22 @@ static zhip_result run_quant(const Dispatch &d, const KArgs &q, uint32_t lds, ui
 //   Q4_K 4096 x 11008      15.1 16.3 18.9 34.9 / 13.0 18.6 20.7 37.0 / -
 //   Q8_0 4096 x 14336      - - 27.7 52.9 / - / - - 26.6 47.0
 //   Q4_K 4096 x 14336      - - - 43.8 / - / - - - 46.4
+// Five to eight tokens over a large matrix: twos read it three or four times, from further away the larger it is, the kernels with
+// inputs in LDS twice; seven tokens are four twos but a pass of four and one of three. us at 5 / 6 / 7 / 8 tokens, inputs in
+// LDS / two a workgroup (wave passes: rows of up to 16 tasks four a pass, up to 32 two, longer ones weighed by their idle lanes):
+//   Q6_K 14336 x 2560 (23 thousand passes)  28.4 31.1 33.4 36.4 / 28.3 28.3 34.8 35.0
+//   Q6_K 28672 x 2560 (46)                  48.3 53.2 58.3 63.1 / 50.9 51.9 64.9 65.2
+//   Q6_K 65536 x 2560 (105)                 95.1 105 115 125 / 110 112 143 142
+//   Q6_K 20480 x 4096 (20)                  44.0 46.9 51.5 54.9 / 39.0 39.6 48.7 49.0
+//   Q6_K 65536 x 4096 (66)                  110 114 124 134 / 114 116 147 146
+//   Q3_K 28672 x 4096 (29)                  49.3 54.6 60.7 65.9 / 47.0 47.1 60.2 60.3
+//   Q3_K 65536 x 4096 (66)                  99.2 109 120 134 / 101 101 132 132
+//   Q3_K 28672 x 2048 (14), two a pass      27.9 29.6 33.6 36.9 / 27.3 27.3 33.9 34.2
+//   Q3_K 65536 x 2048 (33), two a pass      53.6 58.4 65.4 71.7 / 56.6 57.8 73.8 73.8
+//   Q4_K 65536 x 2048 (33), two a pass      49.3 53.6 59.1 64.5 / 50.6 52.1 65.9 66.0
+//   Q4_K 65536 x 2560 (105)                 85.0 94.3 104 114 / 82.6 82.8 109 109
+//   Q8_0 65536 x 2048 (33), two a pass      60.1 64.2 66.1 71.6 / 54.0 55.3 68.8 67.5
+//   Q8_0 65536 x 2560 (105)                 90.0 101 111 120 / 92.4 94.4 120 119
 template <class P>
 static uint32_t tokens_in_registers(const MvArgs &a, uint32_t tasks) {
     const bool pair = a.flags & FLAG_SILU_PAIR;
@@ -1624,6 +1647,8 @@ static uint32_t tokens_in_registers(const MvArgs &a, uint32_t tasks) {
     if (a.m < 2u) return 0u;
     if (tasks <= 64u) {
         if (!pair && weights <= (a.m <= 4u ? 8u << 20 : 9u << 19)) return 1u;
+        const uint64_t passes = tasks <= 16u ? a.rows / 4u : tasks <= 32u ? a.rows / 2u : (uint64_t)a.rows * 64u / tasks;
+        if (!pair && a.m > 4u && passes >= 1000ull * P::REG_PASSES[tasks > 32u][a.m - 5u]) return 0u;
         if (a.m == 2u || a.m > 4u || P::TWO) return 2u;
         return bytes <= (a.m == 4u ? (tasks <= 32u ? 48u << 20 : 96u << 20) : pair ? 16u << 20 : 24u << 20) ? 2u : 0u;
     }
