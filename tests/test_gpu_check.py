@@ -160,6 +160,13 @@ def test_matvec_bf16_several_tokens_stretches(ctx, ctx_wide, half, m, n, k, accu
     test_matvec_bf16_several_tokens(ctx, ctx_wide, True, half, m, n, k, 3, 2, accumulate, False)
 
 
+@pytest.mark.parametrize("k", [4608, 5120, 6144, 9728, 11776, 14336])  # 5 + 4, 2 x 5, 2 x 6, 7 + 6 + 6, 8 + 8 + 7 and 4 x 7 512s
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_stretches_behind_the_norm(ctx, ctx_wide, half, k):
+    """With the RMSNorm prologue the tokens are split ahead of the stretches, equal ones (one launch) and unequal ones."""
+    test_matvec_bf16_several_tokens(ctx, ctx_wide, True, half, 5, (8 << 20) // k + 3, k, 3, 2, True, True)
+
+
 @pytest.mark.parametrize("half", HALVES)
 def test_matvec_bf16_several_tokens_stretch_past_the_row(ctx_wide, half):
     """The last stretch's columns past a row are the next row's first: an infinity there stays in its own row."""
@@ -646,7 +653,7 @@ def test_quant_matvec_pair_rows_in_turn(ctx, t, k, rows, n):
     (2304, True, 5, 3315),
 ])
 def test_matvec_q5_k_passes_of_two(ctx, k, pair, rows, n):
-    """Q5_K steps of more than two tokens over 10 MB of rows and more."""
+    """Q5_K steps of more than two tokens: two a workgroup with their inputs in registers, whatever the matrix (here 10 MB)."""
     assert n * K.row_bytes(TensorType.q5_k, k) * (2 if pair else 1) >= 10 << 20
     test_quant_matvec_long_rows(ctx, TensorType.q5_k, k, pair, rows, n)
 
@@ -680,13 +687,13 @@ MFMA_VARIANT = K.MatvecVariant(wg=512, lanes=64, rows=16)
     (True, 5, 96, 4096),      # four slabs
     (False, 3, 100, 2048),    # accumulate epilogue, an odd token count
     (False, 1, 530, 1024),    # one token, more than one workgroup
-    # k of 2048 or 4096 and whole tiles: the kernel with the tokens' operands in registers
+    # k of 2048 and whole tiles: the kernel with the tokens' operands in registers; 4096: matvec_mfma_rows.hip's
     (False, 8, 4112, 4096),   # 257 tiles: a second tile for the first workgroup
     (True, 8, 4128, 4096),    # gate and up tiles of 258 output tiles
     (True, 3, 64, 2048),      # one block a wave
     (False, 2, 48, 2048),
     # rows of more than 4096 weights: workgroups that share a tile, 2048 columns each (with the
-    # RMSNorm prologue the tokens' scales come from a launch of their own)
+    # RMSNorm prologue the tokens' scales come from a launch of their own); gate / up pairs matvec_mfma_rows.hip's
     (False, 8, 1296, 14336),  # seven parts, 81 tiles over 36 walkers: two rounds and nine tiles in halves
     (True, 4, 528, 8192),     # four parts, gate and up, fewer tiles than walkers
     (False, 5, 4096, 6144),   # three parts, 256 tiles over 85 walkers: one whole tile left over
@@ -695,8 +702,8 @@ MFMA_VARIANT = K.MatvecVariant(wg=512, lanes=64, rows=16)
 @pytest.mark.parametrize("prologue", ["plain", "norm", "norm_act"])
 @pytest.mark.parametrize("t", [TensorType.q4_k, TensorType.q5_k])
 def test_quant_matvec_mfma_variant(ctx, t, pair, rows, n, k, prologue):
-    """The matrix-core variant of matvec_q4_k and matvec_q5_k (a wave per sixteen rows; Q5_K has
-    it for k of 2048 or 4096 and whole tiles, its other cases run the default variant): every
+    """The matrix-core variant of matvec_q4_k and matvec_q5_k (sixteen rows a tile; small matrices of rows
+    of 1024 weights run the default variant): every
     row within 1e-5 of float64 over the decoded weights, each token bitwise
     equal to its lone launch, and nothing outside the outputs touched; also
     with the prologues the planner's launches carry (RMSNorm times its weights
@@ -741,15 +748,18 @@ def test_quant_matvec_mfma_variant(ctx, t, pair, rows, n, k, prologue):
 
 
 @pytest.mark.parametrize("pair,rows,n,k,prologue", [
-    # (rows of other lengths than 1024 and whole 2048s in matrices of more than 8 << 20 weights, or the default kernels run)
-    (False, 8, 32776, 256, "norm"),    # one block a row
+    # (matrices of more than 8 << 20 weights, or at most lengths the default kernels run)
+    (False, 8, 32776, 256, "norm"),    # one block a row: four teams, three rounds
     (True, 5, 5473, 768, "norm_act"),  # three blocks, gate and up tiles of different teams, a ragged last tile
-    (False, 3, 8240, 1024, "plain"),   # four teams, more than one round
+    (False, 3, 8240, 1024, "plain"),   # two teams (Q4_K and Q5_K: the default kernels)
+    (False, 5, 12300, 1024, "norm"),   # four teams of four blocks (but Q6_K)
     (False, 6, 6562, 1280, "norm"),    # two teams, a second tile for some workgroups, in halves
     (True, 1, 4112, 1792, "norm"),
+    (False, 2, 6700, 1280, "norm_act"),
     (False, 8, 3652, 2304, "norm_act"),  # nine blocks over sixteen waves
     (True, 4, 4128, 4096, "norm"),     # a block a wave
     (False, 7, 1936, 4352, "plain"),   # seventeen blocks: two for one wave
+    (False, 3, 1700, 5120, "norm_act"),
     (True, 8, 536, 7936, "norm"),
     (False, 2, 1000, 8448, "norm_act"),  # three parts
     (True, 5, 440, 9728, "norm"),
@@ -795,6 +805,72 @@ def test_quant_matvec_groups_of_tokens(ctx, t, k, n, pair):
     alone = np.concatenate([run(1, at) for at in range(8)])
     for m in (2, 3, 4, 5, 7, 8):
         assert run(m).tobytes() == alone[:m].tobytes(), m
+
+
+@pytest.mark.parametrize("t,k,n,pair", [
+    # (256 compute units: twelve tiles of sixteen outputs each are 49152 outputs)
+    (TensorType.q8_0, 1024, 49171, False),    # rows as one flat stretch
+    (TensorType.q8_0, 1024, 24600, True),
+    (TensorType.q6_k, 2048, 49171, False),    # two, three and four units of a row
+    (TensorType.q6_k, 2048, 24600, True),
+    (TensorType.q6_k, 3072, 24587, False),
+    (TensorType.q6_k, 3072, 14341, True),
+    (TensorType.q6_k, 4096, 49171, False),
+    (TensorType.q6_k, 4096, 14341, True),
+    (TensorType.q6_k, 6144, 16397, False),    # parts
+    (TensorType.q3_k, 1024, 32771, False),
+    (TensorType.q3_k, 1024, 16400, True),
+    (TensorType.q3_k, 2048, 32771, False),
+    (TensorType.q3_k, 2048, 14341, True),
+    (TensorType.q3_k, 3072, 16389, False),
+    (TensorType.q3_k, 3072, 6149, True),
+    (TensorType.q3_k, 4096, 32771, False),
+    (TensorType.q3_k, 4096, 14341, True),
+    (TensorType.q3_k, 6144, 14341, True),     # parts of a pair
+])
+@pytest.mark.parametrize("rows,prologue", [(1, "plain"), (3, "norm"), (8, "norm_act")])
+def test_quant_matvec_mfma_large_matrices(ctx, t, k, n, pair, rows, prologue):
+    """The sizes from which the matrix-core id's streaming kernel takes a matrix, for every instance of it, at both of its
+    token counts, with a ragged last tile, under the bounds of test_quant_matvec_mfma_variant. (The matrix is 509 rows over and
+    over, and its up rows 503: no multiple of anything that the kernels step by.)"""
+    c, eps, col0 = ctx, 1e-6, 3
+    norm, div = prologue != "plain", 4 if prologue == "norm_act" else 0
+    x, nw = c.random(rows * k, 3).reshape(rows, k), c.random(k, 1.5)
+    x[0] *= np.float32(1e-3)
+    sets = [quant_rows(c, t, r, k) for r in ((509, 503) if pair else (509,))]
+    # (indexing is row by row: tile what a row is)
+    raw = np.concatenate([np.resize(np.ascontiguousarray(r).view(np.uint8).reshape(len(v), -1), (n, r.nbytes // len(v))) for r, v in sets])
+    stride = col0 + n + 2
+    init = c.random(rows * stride, 2).reshape(rows, stride)
+    xa, wa, na = c.upload(x), c.gpu_weights(t, raw, k), c.upload(nw)
+    x64 = np.stack([norm_row(r, nw if norm else None, eps) for r in x])
+    if div:
+        x64 = (x64 / div) * sigmoid64(x64 / div)
+    sums = [np.tile(x64 @ v.reshape(-1, k).astype(np.float64).T, -(-n // (v.size // k)))[:, :n] for _, v in sets]
+    want = sums[0] * sigmoid64(sums[0]) * sums[1] if pair else sums[0]
+    accumulate = not pair
+    variant = K.MatvecVariant(MFMA_VARIANT.wg, MFMA_VARIANT.lanes, MFMA_VARIANT.rows, div)
+    pipeline = c.set.matvec(c.rec, K.weight_kernel("matvec", t), variant)
+
+    def run(first, count):
+        out = c.upload(init[first : first + count])
+        p = P.MatvecBf16(n=n, k=k, col0=col0, out_stride=stride, eps=eps, norm=norm, accumulate=accumulate, silu_pair=pair, half=n if pair else 0)
+        c.launcher().launch_pipeline(pipeline, p, [xa if count == rows else c.upload(x[first : first + count]), wa, out, na], (K.div_ceil(n, variant.group_rows()), count, 1))
+        return c.read(out).reshape(count, stride)
+
+    got = run(0, rows)
+    for tk in range(rows):
+        base = init[tk, col0 : col0 + n] if accumulate else 0
+        assert np.max(np.abs(got[tk, col0 : col0 + n] - (want[tk] + base))) <= 1e-5 * np.max(np.abs(want[tk])) + 1e-6 * np.max(np.abs(base)), tk
+    mask = np.ones(stride, dtype=bool)
+    mask[col0 : col0 + n] = False
+    assert np.array_equal(got[:, mask].view(np.uint32), init[:, mask].view(np.uint32))
+    if rows > 1:
+        for tk in (0, rows - 1):
+            assert got[tk].tobytes() == run(tk, 1).tobytes(), "a token's sums differ between a lone launch and a multi-token launch"
+    for arg in (wa, xa):
+        c.rec.destroy(cmd.Kind.buffer, arg.buffer)
+    c.flush()
 
 
 @pytest.mark.parametrize("t,k,n", [(t, k, n) for t in (TensorType.q3_k, TensorType.q6_k) for k, n in ((1024, 509), (2048, 509), (3072, 512), (3072, 2800))])
@@ -893,22 +969,23 @@ def test_quant_matvec_mfma_wide_input_stride(ctx):
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate", [
     (8, 200, 1024, 3, 7, True),      # partial last tile, unaligned rows
     (5, 96, 4096, 4, 8, False),      # aligned rows: 16-byte stores
-    (3, 100, 2080, 0, 0, True),      # k = 65 blocks: a ragged last step
+    (3, 100, 2080, 0, 0, True),      # k = 65 blocks in a small matrix: the default variant
     (1, 530, 1024, 0, 2, False),     # one token
-    (8, 4112, 4096, 0, 0, False),    # 257 sixteen-row tiles: the kernel that streams whole tiles, two tiles on one workgroup
-    (7, 4112, 2048, 5, 7, True),     # the same with eight blocks a wave, unaligned outputs, accumulating
+    (8, 4112, 4096, 0, 0, False),    # 257 sixteen-row tiles: two tiles on one workgroup
+    (7, 4112, 2048, 5, 7, True),     # the kernel that streams whole tiles, unaligned outputs, accumulating
     (2, 1536, 4096, 0, 0, True),
-    (8, 4112, 1024, 0, 0, False),    # rows of 1024 weights: the kernel that moves a tile's 32 rows as one flat stretch
+    (8, 4112, 1024, 0, 0, False),    # rows of 1024 weights
     (3, 4128, 1024, 5, 7, True),
     (4, 5, 1024, 1, 2, True),        # fewer rows than a unit of eight
     # rows of more than 4096 weights: workgroups that share a tile, 2048 columns each
     (8, 1296, 14336, 3, 7, True),    # seven parts, 81 tiles over 36 walkers
     (3, 4096, 6144, 0, 0, False),    # three parts, 256 tiles over 85 walkers
     (5, 48, 8192, 0, 0, False),      # four parts, fewer tiles than walkers
+    (6, 8192, 8192, 0, 0, True),     # from 8192 outputs on matvec_mfma_rows.hip's
     (2, 272, 20480, 0, 0, False),    # ten parts
 ])
 def test_matvec_q8_0_mfma_variant(ctx, rows, n, k, col0, pad, accumulate):
-    """The matrix-core variant of matvec_q8_0 (the id of a wave per sixteen rows): every
+    """The matrix-core variant of matvec_q8_0 (sixteen rows a tile): every
     token within 1e-5 of float64 over the decoded weights whatever its magnitude (each token
     is scaled by its own power of two), each token bitwise equal to its lone launch, nothing
     outside the outputs touched."""
@@ -942,7 +1019,7 @@ def test_matvec_q8_0_mfma_variant(ctx, rows, n, k, col0, pad, accumulate):
 
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("rows,n,k", [(8, 4128, 4096), (3, 64, 2048), (5, 3072, 1024), (2, 4104, 1024),
-                                      (6, 528, 8192), (3, 1304, 6144)])  # rows in four and in three parts (1304 outputs: whole rounds and a ragged tail)
+                                      (6, 528, 8192), (3, 1304, 6144)])  # rows of up to 32 blocks: two a wave (Q6_K: in two parts)
 @pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q6_k, TensorType.q3_k])
 def test_matvec_q8_0_mfma_variant_silu_pair(ctx, t, rows, n, k, norm):
     """The matrix-core variant of matvec_q8_0, matvec_q6_k and matvec_q3_k on the fused gate / up step (SILU_PAIR: gate rows,
@@ -978,9 +1055,8 @@ def test_matvec_q8_0_mfma_variant_silu_pair(ctx, t, rows, n, k, norm):
 @pytest.mark.parametrize("rows,n,k", [(6, 4112, 4096), (3, 96, 2048), (2, 200, 1024), (4, 4128, 1024), (5, 1040, 14336)])
 def test_matvec_q8_0_mfma_variant_prologues(ctx, rows, n, k, prologue):
     """The matrix-core variant of matvec_q8_0 on steps with the RMSNorm and silu(x / act_div)
-    prologues (src/kernels/matvec_quant.wgsl.hbs:73-89), which the streaming kernel computes
-    as it builds the tokens' operands (200 rows of 1024 weights: the kernel that takes a
-    tile's rows as one flat stretch, a workgroup's share of the last rows); 1e-5 against float64, each token bitwise equal to its lone launch."""
+    prologues (src/kernels/matvec_quant.wgsl.hbs:73-89), which the kernels compute
+    as they build the tokens' operands; 1e-5 against float64, each token bitwise equal to its lone launch."""
     c = ctx
     div, eps = 4 if prologue == "norm_act" else 0, 1e-6
     x = c.random(rows * k, 3).reshape(rows, k)
@@ -1009,18 +1085,18 @@ def test_matvec_q8_0_mfma_variant_prologues(ctx, rows, n, k, prologue):
 
 
 @pytest.mark.parametrize("rows,n,k,col0,pad,accumulate,prologue", [
-    (8, 8224, 4096, 0, 0, False, None),        # whole rounds of 32-row tiles and a tail on every workgroup
-    (5, 9000, 4096, 0, 0, True, None),         # a ragged last unit of rows
+    (8, 8224, 4096, 0, 0, False, None),        # whole rounds of tiles and two more
+    (5, 9000, 4096, 0, 0, True, None),         # a ragged last tile
     (3, 100, 2048, 3, 7, True, None),          # fewer rows than workgroups, unaligned columns
     (1, 530, 2048, 0, 2, False, None),         # one token
     (6, 4100, 2048, 0, 0, False, "norm"),
     (4, 300, 4096, 5, 0, True, "norm_act"),
-    (2, 64, 1024, 0, 0, False, None),          # one unit a tile
+    (2, 64, 1024, 0, 0, False, None),          # the streaming kernel: one unit a tile
     (7, 8232, 1024, 0, 0, True, "norm"),
-    (3, 96, 3072, 0, 0, False, None),          # three units a tile
+    (3, 96, 3072, 0, 0, False, None),          # twelve blocks for sixteen waves
     (6, 1000, 3072, 3, 2, True, "norm"),
-    (2, 64, 5120, 0, 0, False, None),          # k the kernel does not take: the default variant's
-    # rows of more than 4096 weights: workgroups that share a tile, 2048 columns each
+    (2, 64, 5120, 0, 0, False, None),          # a small matrix of another length: the default variant's
+    # rows of more than 4096 weights: workgroups that share a tile, 2048 columns each (Q6_K: up to sixteen blocks each; the comments are Q3_K's)
     (8, 1300, 14336, 3, 2, True, None),        # seven parts, 36 walkers: whole rounds, a tail, a ragged last unit
     (4, 4096, 6144, 0, 0, False, None),        # three parts, at most four tokens
     (5, 200, 8192, 0, 0, True, "act"),         # four parts, fewer rows than walkers
@@ -1029,8 +1105,8 @@ def test_matvec_q8_0_mfma_variant_prologues(ctx, rows, n, k, prologue):
 ])
 @pytest.mark.parametrize("t", [TensorType.q6_k, TensorType.q3_k])
 def test_matvec_q6_k_mfma_variant(ctx, t, rows, n, k, col0, pad, accumulate, prologue):
-    """matvec_q6_k and matvec_q3_k on the matrix-core variant id (a wave per sixteen rows): the weights are read
-    once for all tokens of the step, the tokens split into two f16 rows by every workgroup (with
+    """matvec_q6_k and matvec_q3_k on the matrix-core variant id (sixteen rows a tile; the streaming kernel's larger
+    matrices are test_quant_matvec_mfma_large_matrices'): the weights are read once for all tokens of the step, the tokens split into two f16 rows by every workgroup (with
     the RMSNorm and silu(x / act_div) prologues of src/kernels/matvec_quant.wgsl.hbs:73-89 where
     the step has them). 1e-5 against float64; columns outside the launch untouched; each token bitwise equal
     to its lone launch."""
