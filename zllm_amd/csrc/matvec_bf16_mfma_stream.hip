@@ -203,7 +203,7 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (
 // pairs without ZHIP_OPTION_WIDE_DECODE, has them too): the matrix instruction has the rows anyway.
 // PAIR: a SILU_PAIR step, an output tile's gate rows and then its up rows (the general kernel's
 // time grows with the tokens: 2 x 8192 x 2048 f16 at eight 38 us, here 18).
-// LONG: k = 512 NP q.parts; workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
+// LONG: rows of q.parts stretches of 512 NP columns (the last one may end past the row); workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
 // walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums. Without the RMSNorm prologue no
 // workgroup needs more of a token than its stretch (an F16 token's scale is then the stretch's own).
 template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
@@ -517,18 +517,18 @@ bool matvec_bf16_mfma_stream_accepts(const MvArgs &a) {
            a.xr % 4u == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0 && a.row_bytes == 2u * a.k;
 }
 
-template <bool SPLIT, bool F16, bool LONG = false, bool PAIR = false>
-static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 grid) {
-    switch (q.a.k / 512u) {
-    case 2: return launch_blocks<2, SPLIT, F16, LONG, PAIR>(d, q, grid);
-    case 3: return launch_blocks<3, SPLIT, F16, LONG, PAIR>(d, q, grid);
-    case 4: return launch_blocks<4, SPLIT, F16, LONG, PAIR>(d, q, grid);
-    case 5: return launch_blocks<5, SPLIT, F16, LONG, PAIR>(d, q, grid);
-    case 6: return launch_blocks<6, SPLIT, F16, LONG, PAIR>(d, q, grid);
-    case 7: return launch_blocks<7, SPLIT || !pieces_fit<7, pieces_of(F16, PAIR)>(), F16, LONG, PAIR>(d, q, grid);
-    default: return launch_blocks<8, SPLIT || !pieces_fit<8, pieces_of(F16, PAIR)>(), F16, LONG, PAIR>(d, q, grid);
+// The stretches' lengths, in 512 columns: rows of up to 4096 weights 2 .. 8, longer rows 4 .. 8 behind the RMSNorm prologue (equal ones 5 .. 8), 3 .. 6 without.
+template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
+static zhip_result launch_np(const Dispatch &d, const StreamArgs &q, dim3 grid) {
+    constexpr int LOW = LONG ? (SPLIT ? 5 : 3) : SPLIT ? 4 : 2, HIGH = LONG && !SPLIT ? 6 : 8;
+    if constexpr (NP >= LOW && NP <= HIGH) {
+        if (q.a.k == 512u * NP) return launch_blocks<NP, SPLIT || !pieces_fit<NP, pieces_of(F16, PAIR)>(), F16, LONG, PAIR>(d, q, grid);
     }
+    if constexpr (NP < 8) return launch_np<NP + 1, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    else return fail(d, ZHIP_E_GPU, "%s: a stretch of %u columns", F16 ? "matvec_f16" : "matvec_bf16", q.a.k);
 }
+template <bool SPLIT, bool F16, bool LONG = false, bool PAIR = false>
+static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 grid) { return launch_np<2, SPLIT, F16, LONG, PAIR>(d, q, grid); }
 
 // f16: the weights are f16 (matvec_f16), bf16 otherwise.
 zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16) {
@@ -544,10 +544,11 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
     const uint32_t tail = (a.rows - 32u * rounds * groups + 7u) / 8u;
     StreamArgs q{a, (uint32_t)(used < w_bytes ? used : w_bytes), rounds, tail / groups, tail % groups, groups % 8u == 0 ? 1u : 0u, nullptr, 0u, 0u, 0u, 0u, nullptr, 1u, nullptr};
     // Rows of more than 4096 weights (the FFN-down shapes; the general kernel takes them token by
-    // token) go in stretches of up to 4096 columns. Stretches of equal length (14336 = 4 x 3584,
-    // 8192 = 4 x 2048 ...) go out as one launch: `launches` workgroups share a walker's tiles, a
+    // token) go in stretches of columns, by two rules: behind the RMSNorm prologue as few of up to 4096 as there can be (14336 = 4 x 3584, 8192 =
+    // 2 x 4096, 9728 = 3584 + 2 x 3072), without it see below (7 x 2048, 4 x 2048, 4 x 2560 less 512). Together in
+    // one launch, `launches` workgroups share a walker's tiles, a
     // stretch each, and a second launch adds the stretches' sums in their order and applies the
-    // epilogue (their sums wait in the workspace, behind the tokens' planes).
+    // epilogue (their sums wait in the workspace, behind the tokens' planes where there are any).
     const uint32_t token_pieces = pieces_of(f16, pair), pieces = a.k / 512u, fits = token_pieces == 2u ? 8u : 6u;
     uint32_t launches = (a.k + 4095u) / 4096u;
     // Without the RMSNorm prologue the workgroups split their stretches' tokens themselves: in stretches of up to 3072 columns

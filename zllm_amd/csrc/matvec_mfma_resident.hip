@@ -405,7 +405,7 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
         for (uint32_t wv = 1; wv < WAVES; wv++) sum += src[wv * 128u];
         sum *= lds_scale[8 + t];
         if (LONG) {
-            if (t < a.m && row < rows_of(p)) store_apart(q.partial + ((size_t)(per * kpart + (PAIR ? p & 1u : 0u)) * 8u + t) * a.rows + out0(p) + row, sum);
+            if (t < a.m && row < rows_of(p)) store_apart(q.partial + ((size_t)kpart * 8u + t) * a.rows + out0(p) + row, sum);
         } else if (PAIR && !(p & 1u)) {
             held = sum;
         } else {
@@ -504,7 +504,7 @@ zhip_result launch_matvec_parts_sum(const Dispatch &d, const char *name, const M
 }
 
 // Whether this kernel can run the (already validated) arguments: whole tiles, k split into
-// one or two blocks a wave, or rows of 6144 .. 32768 weights in parts of 2048.
+// a block a wave, or rows of 6144 .. 32768 weights in parts of 2048.
 bool matvec_q4k_mfma_resident_accepts(const MvArgs &a) {
     const bool pair = a.flags & FLAG_SILU_PAIR;
     const bool parts = !pair && a.k > 4096u && a.k % 2048u == 0 && a.k / 2048u <= kMatvecMaxParts;

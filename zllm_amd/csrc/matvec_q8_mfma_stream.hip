@@ -127,29 +127,29 @@ __device__ __forceinline__ void load_lds_b32(__amdgpu_buffer_rsrc_t buf, uint32_
     __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (lds_ptr)(uintptr_t)dst, 4, voffset, soffset, 0, 0);
 }
 
-// NS: 32-weight blocks of a wave's k range (k = 256 NS). The ring moves half tiles: the first or
+// NS: 32-weight blocks of a wave's k range. The ring moves half tiles: the first or
 // second NS / 2 blocks of the wave's range of a tile's sixteen rows. A slot: sixteen lines, then 256 bytes for the scales' load
 // (two bytes a block and row; zeros from idle lanes behind).
+constexpr int NS = 8;
 constexpr int DEPTH = 4;  // ring slots a wave: three half tiles in flight behind the one multiplied
-template <int NS> constexpr uint32_t slot_bytes() { return 16u * 32u * (NS / 2) + 256u; }
+constexpr uint32_t SLOT = 16u * 32u * (NS / 2) + 256u;
 constexpr uint32_t PART_BYTES = 2u * WAVES * 128u * 4u, SCALE_BYTES = 576u;  // [8 waves][8 tokens] maxima, [8] inverse scales, [8 waves][8 tokens] sums of squares
-template <int NS> constexpr uint32_t lds_bytes() { return PART_BYTES + SCALE_BYTES + WAVES * DEPTH * slot_bytes<NS>(); }
-static_assert(lds_bytes<16>() <= 160u * 1024u, "the rings must fit the CU's LDS");
+constexpr uint32_t LDS_BYTES = PART_BYTES + SCALE_BYTES + WAVES * DEPTH * SLOT;
+static_assert(LDS_BYTES <= 160u * 1024u, "the rings must fit the CU's LDS");
 
-// LONG (NS = 8): k = 2048 q.parts; workgroup i multiplies columns 2048 (i % parts) .. (part
+// k = 2048; LONG: k = 2048 q.parts, workgroup i multiplies columns 2048 (i % parts) .. (part
 // `kpart`) of the tiles that walker i / parts takes, and launch_matvec_parts_sum adds the parts.
-template <int NS, bool LONG>
+template <bool LONG>
 __global__ __launch_bounds__(THREADS) void matvec_q8_mfma_stream_kernel(StreamArgs q) {
-    static_assert(!LONG || NS == 8, "parts of a long row are 2048 columns");
     const MvArgs &a = q.a;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *lds_part = reinterpret_cast<float *>(lds);                  // [tile parity][wave][2 lane + token of the lane's two]
     float *lds_max = reinterpret_cast<float *>(lds + PART_BYTES);      // [wave][token]: the largest magnitude in the wave's range
     float *lds_inverse = lds_max + 64;                                 // [token]: one over the token's scale
-    static_assert(NS >= 8, "a half tile is whole 128-byte lines of every row");
     constexpr int PARTS = 2;  // ring slots a wave's range of a tile takes
     constexpr int HB = NS / PARTS;           // blocks of a half tile
-    constexpr uint32_t SLOT = slot_bytes<NS>(), LINE = 32u * HB, CHUNKS = 2u * HB;
+    constexpr uint32_t LINE = 32u * HB, CHUNKS = 2u * HB;
+    static_assert(LINE == 128u, "a half tile is whole lines of every row");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint8_t *ring = lds + PART_BYTES + SCALE_BYTES + wave * (DEPTH * SLOT);
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(THREADS) void matvec_q8_mfma_stream_kernel(StreamAr
     // With SILU_PAIR (src/kernels/matvec_quant.wgsl.hbs:110-125) an output tile is two weight
     // tiles, the gate rows and then the up rows `half` further down: tile p of the run is weight
     // tile p % per of output tile p / per.
-    const uint32_t per = (a.flags & FLAG_SILU_PAIR) ? 2u : 1u;
+    const uint32_t per = !LONG && (a.flags & FLAG_SILU_PAIR) ? 2u : 1u;
     const uint32_t kpart = LONG ? blockIdx.x % q.parts : 0u, walker = LONG ? blockIdx.x / q.parts : blockIdx.x, walkers = LONG ? gridDim.x / q.parts : gridDim.x;
     const bool extra = walker < (q.split ? 2u * q.left : q.left);
     const uint32_t count = per * (q.rounds + (extra ? 1u : 0u));
@@ -323,15 +323,9 @@ __global__ __launch_bounds__(THREADS) void matvec_q8_mfma_stream_kernel(StreamAr
     auto multiply = [&](auto half, uint32_t slot) __attribute__((always_inline)) {
         constexpr int H = decltype(half)::value;
         const uint8_t *t = ring + slot * SLOT;
-        uint32_t d[SWORDS];
-        if constexpr (SWORDS == 4) {
-            const su32x4 v = *reinterpret_cast<const su32x4 *>(t + 16u * LINE + l16 * 16u);
-            d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
-        } else {
-            static_assert(SWORDS == 2, "two or four words of scales a row");
-            const su32x2 v = *reinterpret_cast<const su32x2 *>(t + 16u * LINE + l16 * 8u);
-            d[0] = v.x; d[1] = v.y;
-        }
+        static_assert(SWORDS == 2, "two words of scales a row");
+        const su32x2 v = *reinterpret_cast<const su32x2 *>(t + 16u * LINE + l16 * 8u);
+        const uint32_t d[SWORDS] = {v.x, v.y};
 #pragma unroll
         for (int s = 0; s < HB; s++) {
             const su32x2 w = *reinterpret_cast<const su32x2 *>(t + r_at + 16u * ((2u * s + r_half) ^ r_key));
@@ -358,7 +352,7 @@ __global__ __launch_bounds__(THREADS) void matvec_q8_mfma_stream_kernel(StreamAr
             for (uint32_t wv = 1; wv < WAVES; wv++) sum += src[wv * 128u];
             sum *= lds_inverse[tk];
             if (LONG) {
-                if (tk < a.m && row < rows_of(p)) store_apart(q.partial + ((size_t)(per * kpart + (p % per)) * 8u + tk) * a.rows + out0(p) + row, sum);
+                if (tk < a.m && row < rows_of(p)) store_apart(q.partial + ((size_t)kpart * 8u + tk) * a.rows + out0(p) + row, sum);
             } else if (per == 2u && !(p & 1u)) {
                 held = sum;  // the gate tile's result, until the up tile's arrives
             } else {
@@ -410,18 +404,18 @@ bool matvec_q8_mfma_stream_accepts(const MvArgs &a) {
            a.xr % 4u == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0;
 }
 
-template <int NS, bool LONG = false>
+template <bool LONG>
 static zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
-    auto kernel = matvec_q8_mfma_stream_kernel<NS, LONG>;
+    auto kernel = matvec_q8_mfma_stream_kernel<LONG>;
     static bool configured = false;
     if (!configured) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<NS>()) != hipSuccess) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) != hipSuccess) {
             (void)hipGetLastError();
-            return fail(d, ZHIP_E_GPU, "matvec_q8_0: cannot reserve %u bytes of LDS", lds_bytes<NS>());
+            return fail(d, ZHIP_E_GPU, "matvec_q8_0: cannot reserve %u bytes of LDS", LDS_BYTES);
         }
         configured = true;
     }
-    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), lds_bytes<NS>(), d.stream, q);
+    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), LDS_BYTES, d.stream, q);
     return check_launch(d, "matvec_q8_0");
 }
 
@@ -449,10 +443,10 @@ zhip_result launch_matvec_q8_mfma_stream(const Dispatch &d, const MvArgs &a, uin
             q.scales = reinterpret_cast<const float *>(d.work->data);
             if (zhip_result r = launch_matvec_parts_scales(d, "matvec_q8_0", a, reinterpret_cast<float *>(d.work->data))) return r;
         }
-        if (zhip_result r = launch_blocks<8, true>(d, q, grid)) return r;
+        if (zhip_result r = launch_blocks<true>(d, q, grid)) return r;
         return launch_matvec_parts_sum(d, "matvec_q8_0", a, q.partial, parts);
     }
-    return launch_blocks<8>(d, q, grid);
+    return launch_blocks<false>(d, q, grid);
 }
 
 }  // namespace zhip

@@ -167,7 +167,7 @@ struct KQ8 {
     static constexpr bool DEFER = false;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
-    static constexpr uint32_t REG_SLICES = 4;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_SLICES = 4;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
     static constexpr uint32_t REG_PASSES[2][4] = {{kAny, kAny, 28, kAny}, {kAny, kAny, 70, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q8_0"; }
     struct Raw {
@@ -238,12 +238,12 @@ struct KQ8 {
 struct KQ3 {
     static constexpr uint32_t BLOCK_BYTES = 128;
     static constexpr int NSUM = 4;
-    static constexpr int STAGE2 = 2, STAGE4 = 2;  // tokens whose inputs are loaded at once
+    static constexpr int STAGE2 = 0, STAGE4 = 2;  // tokens whose inputs are loaded at once, of two and of three or four
     static constexpr bool ALL4 = false;           // (four at once measured slower on every shape: 1024 x 4096 7.7 against 7.1 us)
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
-    static constexpr uint32_t REG_SLICES = 3;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_SLICES = 3;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
     static constexpr uint32_t REG_PASSES[2][4] = {{26, kAny, 13, 30}, {65, kAny, 33, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q3_k"; }
     struct Raw {
@@ -329,12 +329,12 @@ struct KQ3 {
 struct KQ4 {
     static constexpr uint32_t BLOCK_BYTES = 144;
     static constexpr int NSUM = 2;
-    static constexpr int STAGE2 = 2, STAGE4 = 1;  // tokens whose inputs are loaded at once
+    static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
-    static constexpr uint32_t REG_SLICES = 2;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_SLICES = 2;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
     static constexpr uint32_t REG_PASSES[2][4] = {{30, kAny, 18, 30}, {kAny, kAny, 90, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q4_k"; }
     struct Raw {
@@ -415,15 +415,15 @@ struct KQ4 {
 struct KQ5 {
     static constexpr uint32_t BLOCK_BYTES = 176;
     static constexpr int NSUM = 2;
-    static constexpr int STAGE2 = 0, STAGE4 = 4;  // tokens whose inputs are loaded at once
-    static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
+    static constexpr int STAGE2 = 0, STAGE4 = 0;  // (rows of up to 4096 weights always have two tokens' inputs in registers)
+    static constexpr bool ALL4 = false;
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     // The fifth bits leave the general kernel too few registers for three or more tokens' sums: rows
     // of up to 64 tasks always run two tokens a workgroup (four tokens, general / that: 9728 x 2560 21.7 /
     // 17.6 us, 14336 x 4096 30.0 / 23.8, 50257 x 2560 55.9 / 51.5).
     static constexpr bool TWO = true;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
-    static constexpr uint32_t REG_SLICES = 3;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_SLICES = 3;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
     static constexpr uint32_t REG_PASSES[2][4] = {{kAny, kAny, kAny, kAny}, {kAny, kAny, kAny, kAny}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q5_k"; }
     struct Raw {
@@ -517,7 +517,7 @@ struct KQ6 {
     static constexpr bool DEFER = false;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
-    static constexpr uint32_t REG_SLICES = 4;  // three or more tokens keep their inputs in registers over rows of up to so many slices of 64 tasks
+    static constexpr uint32_t REG_SLICES = 4;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
     static constexpr uint32_t REG_PASSES[2][4] = {{kAny, kAny, 24, kAny}, {43, 64, 22, 38}};  // five .. eight tokens keep theirs up to so many thousand wave passes: see tokens_in_registers
     static const char *name() { return "matvec_q6_k"; }
     struct Raw {
@@ -1653,6 +1653,8 @@ static uint32_t tokens_in_registers(const MvArgs &a, uint32_t tasks) {
         return bytes <= (a.m == 4u ? (tasks <= 32u ? 48u << 20 : 96u << 20) : pair ? 16u << 20 : 24u << 20) ? 2u : 0u;
     }
     if (pair || tasks > 256u) return 0u;
+    // (REG_SLICES: what a format's unpacking costs beside the loads. Two slices: two tokens a workgroup whatever the format, but three tokens over more than
+    // 16 << 20 weights only from 4 on; three slices: one, from 3 on; four: two, of four tokens and more from 4 on.)
     const uint32_t slices = (tasks + 63u) / 64u;
     if (slices == 2u) return a.m <= 3u && weights <= 16u << 20 ? 1u : a.m != 3u || P::REG_SLICES > 3u ? 2u : 0u;
     if (slices == 3u) return a.m == 2u || P::REG_SLICES >= 3u ? 1u : 0u;
@@ -1692,12 +1694,12 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             if (mt == 1u) return pair ? run_row<P, 1, true>(d, q, lds, blocks) : run_row<P, 1, false>(d, q, lds, blocks);
             return pair ? run_row<P, 2, true>(d, q, lds, blocks) : run_row<P, 2, false>(d, q, lds, blocks);
         }
-        // (of two tokens eight waves for two or four slices, six for three: twelve would spill)
-        const uint32_t slices = (q.tasks + 63u) / 64u, nw = slices != 3u ? 8u : mt == 1u ? 12u : 6u, groups_here = nw / slices;
+        // (two tokens never over three slices: twelve waves would spill)
+        const uint32_t slices = (q.tasks + 63u) / 64u, nw = slices != 3u ? 8u : 12u, groups_here = nw / slices;
         const uint32_t blocks = shared_out((a.rows + groups_here * 2u - 1u) / (groups_here * 2u), cus);
         const uint32_t lds = mt * q.tasks * kTaskStride * 4u + 2u * nw * 2u * mt * 256u;
         if (mt == 1u) return nw == 12u ? run_slices<P, 1, false, 2, 12>(d, q, lds, blocks) : run_slices<P, 1, false, 2, 8>(d, q, lds, blocks);
-        return nw == 6u ? run_slices<P, 2, false, 2, 6>(d, q, lds, blocks) : run_slices<P, 2, false, 2, 8>(d, q, lds, blocks);
+        return run_slices<P, 2, false, 2, 8>(d, q, lds, blocks);
     }
     for (uint32_t t0 = 0; t0 < a.m;) {
         uint32_t left = a.m - t0;
@@ -1806,8 +1808,7 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
             r = pair ? run_row<P, 1, true>(d, q, row_lds, row_blocks) : run_row<P, 1, false>(d, q, row_lds, row_blocks);
         } else if (mt == 1u) r = pair ? run_quant<P, 1, true, 1>(d, q, lds, blocks) : run_quant<P, 1, false, 1>(d, q, lds, blocks);
         else if (mt == 2u) {
-            if (small && P::STAGE2 != 2) r = pair ? run_quant<P, 2, true, 2>(d, q, lds, blocks) : run_quant<P, 2, false, 2>(d, q, lds, blocks);
-            else r = pair ? run_quant<P, 2, true, P::STAGE2>(d, q, lds, blocks) : run_quant<P, 2, false, P::STAGE2>(d, q, lds, blocks);
+            r = pair ? run_quant<P, 2, true, P::STAGE2>(d, q, lds, blocks) : run_quant<P, 2, false, P::STAGE2>(d, q, lds, blocks);
         } else if (mt == 3u) {
             // (three tokens: the four-token pass's choices, at most three loaded at once)
             constexpr int STAGE3 = P::STAGE4 > 3 ? 3 : P::STAGE4;

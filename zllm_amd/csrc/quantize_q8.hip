@@ -5,9 +5,8 @@
 // (a chunk is one Q8_K block, or eight Q8_0 blocks of eight lanes each), and a
 // workgroup is four such waves on neighbouring chunks. A chunk's rounding is a
 // chain of dependent operations behind one 16-byte load, so what hides it is
-// other waves. With the RMSNorm prologue a workgroup
-// takes a whole row, every fourth chunk a wave, first adds the row's squares together and then
-// rounds. The largest magnitude of a
+// other waves. With the RMSNorm prologue every workgroup of a row (one to eight: see
+// launch_norm) first adds the whole row's squares together and then rounds its share of the chunks. The largest magnitude of a
 // block is found with row-local DPP steps (and, for Q8_K, four lane reads),
 // the first position that holds it with a ballot. Every operation whose rounding
 // decides a value is an operation of its own (the library is compiled with
