@@ -270,6 +270,17 @@ def test_matvec_half_rows_in_registers_groups_of_tokens(ctx, k, n):
     test_matvec_half_rows_in_registers(ctx, "bf16", False, k, n)
 
 
+@pytest.mark.parametrize("pair,k,n", [
+    (False, 512, 25000), (False, 512, 41500), (True, 512, 12600), (True, 512, 20800),  # rows of one load a lane: four, eight
+    (True, 1024, 6300), (True, 1024, 10400), (False, 1024, 12300), (False, 1024, 20500),
+    (False, 4400, 900), (True, 4400, 500),
+])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_half_rows_in_registers_groups_of_short_rows(ctx, half, pair, k, n):
+    """The same of both formats and of gate / up pairs, four and eight tokens a workgroup."""
+    test_matvec_half_rows_in_registers(ctx, half, pair, k, n)
+
+
 @pytest.mark.parametrize("m,n,k,half_row,accumulate,norm", [
     # 16 MB of gate rows and more: the matrix cores, a tile of gate rows and then one of up rows,
     # for every count of pieces in a row.
@@ -787,6 +798,9 @@ def test_matvec_q8_0_mfma_ragged_rows(ctx, k):
     (2304, 70, True),
     (5120, 100, False), (4352, 4000, False),  # two slices: one token a workgroup, two
     (12288, 50, False), (16384, 60, False),   # three, four
+    (5120, 300, True), (9728, 200, True), (17408, 40, False),  # inputs in LDS, whole and tile by tile
+    (2560, 41000, False),                        # Q6_K: past 64 thousand wave passes, six tokens
+    (2048, 25000, True), (2048, 56200, False),   # past 48 MB of a pair, four tokens, and past every format's packed passes, seven
     (2048, 26500, False), (2560, 27000, False),  # past 13 and 43 thousand wave passes: seven (Q6_K: five and eight) tokens with inputs in LDS
 ])
 @pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
@@ -803,7 +817,7 @@ def test_quant_matvec_groups_of_tokens(ctx, t, k, n, pair):
         return c.read(out).reshape(m, n + 3)
 
     alone = np.concatenate([run(1, at) for at in range(8)])
-    for m in (2, 3, 4, 5, 7, 8):
+    for m in range(2, 9):
         assert run(m).tobytes() == alone[:m].tobytes(), m
 
 

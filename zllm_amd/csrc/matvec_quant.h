@@ -163,7 +163,6 @@ constexpr uint32_t kAny = 0xffffffffu / 1000u;
 struct KQ8 {
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
-    static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = false;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
@@ -239,7 +238,6 @@ struct KQ3 {
     static constexpr uint32_t BLOCK_BYTES = 128;
     static constexpr int NSUM = 4;
     static constexpr int STAGE2 = 0, STAGE4 = 2;  // tokens whose inputs are loaded at once, of two and of three or four
-    static constexpr bool ALL4 = false;           // (four at once measured slower on every shape: 1024 x 4096 7.7 against 7.1 us)
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
@@ -330,7 +328,6 @@ struct KQ4 {
     static constexpr uint32_t BLOCK_BYTES = 144;
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
-    static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
@@ -416,7 +413,6 @@ struct KQ5 {
     static constexpr uint32_t BLOCK_BYTES = 176;
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 0;  // (rows of up to 4096 weights always have two tokens' inputs in registers)
-    static constexpr bool ALL4 = false;
     static constexpr bool DEFER = true;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     // The fifth bits leave the general kernel too few registers for three or more tokens' sums: rows
@@ -513,7 +509,6 @@ struct KQ6 {
     static constexpr uint32_t BLOCK_BYTES = 224;
     static constexpr int NSUM = 4;
     static constexpr int STAGE2 = 2, STAGE4 = 1;  // tokens whose inputs are loaded at once
-    static constexpr bool ALL4 = true;            // a launch of at most a workgroup a CU stages a pass of four at once
     static constexpr bool DEFER = false;
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
@@ -1787,11 +1782,8 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
         const uint32_t cap = (uint32_t)d.dev->compute_units * (xreg ? 3u : 2u);
         const uint32_t blocks = want < cap ? want : cap;
         zhip_result r;
-        // A launch of at most one workgroup a CU is a chain of trips to memory and has the CU's
-        // registers to itself: all of the pass's tokens go in one. With more workgroups a CU the
-        // format keeps what leaves the multiply its second wave a SIMD (STAGE2, STAGE4; 4096 x
-        // 4096 at four tokens with all at once: Q4_K 12.3 against 9.1 us, Q6_K 13.4 against 10.9).
-        const bool small = want <= (uint32_t)d.dev->compute_units;
+        // (What is loaded at once leaves the multiply its second wave a SIMD: STAGE2, STAGE4; 4096 x
+        // 4096 at four tokens with all at once: Q4_K 12.3 against 9.1 us, Q6_K 13.4 against 10.9.)
         if (xreg) {
             // (a pass of the row kernel is a wave's 64 / seg rows, or that many gate / up pairs)
             const uint32_t passes = (a.rows + rpi - 1u) / rpi, row_want = (passes + 3u) / 4u;
@@ -1812,11 +1804,9 @@ static zhip_result launch_quant(const Dispatch &d, const MvArgs &a) {
         } else if (mt == 3u) {
             // (three tokens: the four-token pass's choices, at most three loaded at once)
             constexpr int STAGE3 = P::STAGE4 > 3 ? 3 : P::STAGE4;
-            if (small && P::ALL4 && STAGE3 != 3) r = pair ? run_quant<P, 3, true, 3>(d, q, lds, blocks) : run_quant<P, 3, false, 3>(d, q, lds, blocks);
-            else r = pair ? run_quant<P, 3, true, STAGE3>(d, q, lds, blocks) : run_quant<P, 3, false, STAGE3>(d, q, lds, blocks);
+            r = pair ? run_quant<P, 3, true, STAGE3>(d, q, lds, blocks) : run_quant<P, 3, false, STAGE3>(d, q, lds, blocks);
         } else {
-            if (small && P::ALL4 && P::STAGE4 != 4) r = pair ? run_quant<P, 4, true, 4>(d, q, lds, blocks) : run_quant<P, 4, false, 4>(d, q, lds, blocks);
-            else r = pair ? run_quant<P, 4, true, P::STAGE4>(d, q, lds, blocks) : run_quant<P, 4, false, P::STAGE4>(d, q, lds, blocks);
+            r = pair ? run_quant<P, 4, true, P::STAGE4>(d, q, lds, blocks) : run_quant<P, 4, false, P::STAGE4>(d, q, lds, blocks);
         }
         if (r != ZHIP_OK) return r;
         t0 += q.mt;
