@@ -929,6 +929,25 @@ def test_quant_matvec_mfma_infinities(ctx, t, k, n):
     assert np.max(np.abs(got[4] - exact[2])) <= (k // 256 + 1) * 2.0 ** -149 + 1e-5 * np.max(np.abs(exact[2]))  # (a rounding to 2^-149 a block)
 
 
+@pytest.mark.parametrize("k,n", [(768, 11000), (1280, 6600), (2560, 3400), (4096, 2060), (5120, 1700), (9728, 900)])
+@pytest.mark.parametrize("t", [TensorType.q8_0, TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_quant_matvec_mfma_split_inputs(ctx, t, k, n):
+    """The matrix cores take an input in two f16 pieces where the default variant has f32: its error against float64 (2-norm) is no
+    larger than the default variant's, over inputs of one size and over ones with a large one in every block."""
+    c, rows = ctx, 4
+    raw, values = quant_rows(c, t, n, k)
+    wa, v64 = c.gpu_weights(t, raw, k), values.astype(np.float64)
+    p = lambda: P.MatvecBf16(n=n, k=k, col0=0, out_stride=n)
+    for large in (1, 1000):
+        x = np.random.default_rng(k).standard_normal((rows, k), dtype=np.float32)
+        x[:, ::256] *= np.float32(large)
+        xa, out, ref, want = c.upload(x), c.output(rows * n), c.output(rows * n), x.astype(np.float64) @ v64.T
+        c.launcher().launch_pipeline(c.set.matvec(c.rec, K.weight_kernel("matvec", t), MFMA_VARIANT), p(), [xa, wa, out, wa], (K.div_ceil(n, MFMA_VARIANT.group_rows()), rows, 1))
+        c.launcher().launch(K.weight_kernel("matvec", t), p(), [xa, wa, ref, wa], (K.div_ceil(n, K.matvec_rows), rows, 1))
+        error = [np.linalg.norm(c.read(o).reshape(rows, n) - want) for o in (out, ref)]
+        assert error[0] <= error[1], large
+
+
 @pytest.mark.parametrize("n,pair", [(1024, False), (9000, False), (3072, True)])
 @pytest.mark.parametrize("t", [TensorType.q4_k, TensorType.q5_k])
 def test_quant_matvec_mfma_short_rows_are_the_default_variants(ctx, t, n, pair):

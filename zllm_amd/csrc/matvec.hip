@@ -331,20 +331,26 @@ bool matvec_q3k_mfma_stream_accepts(const MvArgs &a);
 zhip_result launch_matvec_q3k_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
 bool matvec_q8_0_mfma_flat_accepts(const MvArgs &a);
 zhip_result launch_matvec_q8_0_mfma_flat(const Dispatch &d, const MvArgs &a, uint64_t w_bytes);
-// Which of them takes a matrix under the matrix-core id: a property of the matrix alone, since they add in
+// Which of them takes a matrix under the matrix-core id: a property of the launch's matrix (type, row length, its rows, pair or not) and of
+// the device's compute units, never of the step, since they add in
 // different orders and a token's bits must not depend on the width of its step. us at one / four / eight
 // tokens, weights from HBM, these kernels / matvec_mfma_rows.hip:
 //  * Q4_K, Q5_K, Q8_0, rows of 2048 weights: Q4_K 4096 outputs 6.8 6.8 6.9 / 6.7 7.2 8.0, 2 x 8192 10.1 10.0 10.2 / 9.8
-//    10.4 11.1, Q8_0 4096 6.9 7.0 7.1 / 7.1 7.5 8.1. Rows of 4096: Q4_K 4096 outputs 10.3 10.3 10.8 / 6.9 7.7 10.0,
-//    2 x 14336 21.8 21.1 21.7 / 20.1 19.5 21.2, Q5_K 27.7 27.7 28.4 / 22.3 22.5 24.5, Q8_0 4096 10.9 10.9 11.3 / 7.8 8.1 9.9.
-//  * the same in parts of 2048, no gate / up pair (and of Q8_0 fewer than 8192 outputs): Q4_K 4096 x 8192 11.1
-//    11.3 11.6 / 9.5 11.5 15.5, 4096 x 14336 15.1 14.9 15.5 / 13.8 14.4 16.6, Q3_K 4096 x 8192 12.7 12.6 13.3 / 9.9 11.2 14.3,
-//    Q8_0 2048 x 6144 9.2 9.5 9.5 / 8.4 9.8 13.0. Pairs: Q4_K 2 x 8192 x 8192 26.8 27.4 27.7 / 21.4 21.9 24.1, Q8_0 37.2
-//    38.0 39.0 / 27.7 28.9 31.9; 57344 x 8192 Q8_0 (four and eight tokens) 113.9 118.9 / 85.9 91.6.
+//    10.4 11.1, Q8_0 4096 6.9 7.0 7.1 / 7.1 7.5 8.1. Not rows of 4096: Q4_K 4096 outputs 10.3 10.3 10.8 / 6.9 7.7 10.0,
+//    2 x 14336 21.7 21.2 21.8 / 19.7 19.5 21.4, Q5_K 27.5 27.7 28.3 / 22.4 22.0 24.5, Q8_0 4096 10.9 10.8 11.3 / 7.8 8.1 10.2. (Without RMSNorm
+//    eight tokens over many rows pay for one to four: Q4_K 2 x 14336 20.1 20.0 19.9 / 19.5 18.3 20.5, Q8_0 14336 15.6 15.5 16.0 / 15.7 15.5 16.5.)
+//  * the same in parts of 2048, no gate / up pair (and of Q8_0 fewer than 8192 outputs): at four tokens the two are within 5 % of each other on most, at eight
+//    matvec_mfma_rows.hip is up to 40 % behind over few rows. Q4_K 2560 x 8192 9.8 9.8 9.9 / 10.4 11.0 13.1, 4096 x 8192 11.1 10.9 11.5 / 10.8 11.3 13.4, 4096 x 14336
+//    15.0 14.8 15.4 / 13.8 14.2 16.4, 16384 x 8192 21.8 22.0 22.8 / 20.9 21.1 23.4, Q5_K 4096 x 6144 12.2 12.2 12.4 / 11.2 11.8 14.0, 16384 x 14336 41.9 41.9 43.0 / 38.5 38.7 41.2,
+//    Q3_K 4096 x 6144 12.8 12.7 13.3 / 11.2 11.4 13.1, 16384 x 6144 22.9 22.6 24.1 / 24.4 24.7 26.8, Q8_0 2560 x 8192 10.8 10.9 11.2 / 11.4 12.1 13.3,
+//    4096 x 14336 18.7 18.9 19.4 / 17.1 18.1 18.9; past the line Q8_0 8192 x 6144 17.2 17.6 18.0 / 14.6 15.3 17.7, 16384 x 8192 32.7 33.7 34.8 / 27.6 28.5 30.5.
+//    Pairs: Q4_K 2 x 8192 x 8192 26.7 27.3 27.6 / 21.4 22.2 26.6, 2 x 14336 x 14336 61.0 62.2 62.9 / 52.6 55.2 55.8 (2 x 14336 x 6144 pays at eight, 32.1 32.6 32.9 / 30.2 31.9 36.8),
+//    Q8_0 2 x 8192 x 8192 37.2 38.0 39.0 / 27.7 28.8 31.4.
 //  * Q6_K, Q3_K and Q8_0 rows of 1024 weights: from twelve tiles of sixteen outputs a CU on (Q3_K: eight). Q6_K (rows of 1024
 //    weights always: 4096 outputs 7.3 7.2 7.3 / 6.6 7.1 7.7) 64000 x 4096 (four and eight tokens) 46.4 49.7 / 51.2 52.9, 32000 x 4096 28.6 29.6 / 28.7 30.6, 4096 x 4096 14.7 15.5 /
-//    8.6 10.3; Q3_K 64000 x 4096 38.9 40.9 / 42.9 44.1, 2 x 14336 x 4096 23.5 25.3 / 23.6 25.6, 4096 x 4096 12.7 13.3 / 7.4 9.4;
-//    Q8_0 151936 x 1024 33.1 33.2 / 36.1 36.0, 50257 x 1024 16.9 16.8 / 16.7 16.8, 2 x 3072 x 1024 9.0 9.1 / 7.3 7.9.
+//    8.6 10.3; Q3_K 64000 x 4096 38.9 40.9 / 42.9 44.1, 28672 x 4096 23.4 25.4 / 22.1 24.2, 4096 x 4096 12.7 13.3 / 7.4 9.4;
+//    Q8_0 151936 x 1024 33.1 33.2 / 36.1 36.0, 50257 x 1024 16.9 16.8 / 16.7 16.8, 2 x 3072 x 1024 9.0 9.1 / 7.3 7.9, 4096 x 1024 (one, four, eight) 7.3 7.3 7.4 / 6.4 6.9
+//    7.5, 1024 x 1024 6.7 6.8 6.9 / 5.9 6.5 7.2.
 //  * Q3_K rows of 1024 weights, no pair: but where the tiles of a CU fill matvec_mfma_rows.hip's rounds of four. 4096 outputs 6.4 6.4 6.5 /
 //    6.6 7.1 7.7, 9000 7.9 8.0 8.2 / 9.1 9.7 10.2, 16384 (four a CU) 8.3 8.3 8.6 / 7.3 7.2 7.5, 20480 9.4 9.4 9.7 / 9.7 9.6 9.9, 24576 9.4 9.3 9.6 / 9.9 9.6 10.0,
 //    32000 (eight) 10.9 11.0 11.5 / 10.3 10.0 10.4.

@@ -26,12 +26,18 @@
 // Scalar instructions count, sixteen waves sharing one scalar unit: a token's buffer each instead of one for all of
 // them, runtime team counts and sums held over two rounds cost 0.5 us a launch. Eight waves a workgroup with twice
 // the blocks each were slower (Q4_K 4096 x 4096 at four tokens 8.8 against 7.6 us), and so were parts of eight blocks
-// (4096 x 14336 16.0 against 14.4). Measured against the kernels before (us at one / four / eight tokens, weights from HBM):
-// Q4_K 4096 x 4096 with RMSNorm 10.3 10.3 10.8 -> 6.9 7.7 10.0, Q6_K 14.8 14.7 15.5 -> 7.8 8.6 10.3, Q3_K 12.8 12.7 13.3 -> 6.7 7.4 9.4,
-// Q8_0 10.9 10.9 11.3 -> 7.8 8.1 9.9, Q5_K 2 x 14336 x 4096 27.7 27.7 28.4 -> 22.3 22.5 24.5, Q6_K 4096 x 14336
-// 19.9 19.9 20.7 -> 18.0 18.2 20.1; lengths that ran the default variant before: Q4_K 4096 x 2560 5.1 9.2 18.0 -> 6.3 7.1 9.6, Q5_K
+// (4096 x 14336 16.0 against 14.4). Measured against the kernels before (us at one / four / eight tokens, weights from HBM, with RMSNorm but for
+// 4096 x 14336): Q4_K 4096 x 4096 10.3 10.3 10.8 -> 6.9 7.6 10.0, Q6_K 14.8 14.7 15.5 -> 7.9 8.3 10.1, Q3_K 12.8 12.7 13.3 -> 6.7 7.4 9.4,
+// Q8_0 10.9 10.9 11.3 -> 7.8 8.1 9.9, Q4_K 2 x 14336 x 4096 21.7 21.2 21.8 -> 19.7 19.5 21.4, Q5_K 27.5 27.7 28.3 -> 22.4 22.0 24.5, Q6_K 4096 x 14336
+// 19.9 19.9 20.7 -> 17.9 18.1 20.0; lengths that ran the default variant before: Q4_K 4096 x 2560 5.1 9.2 18.0 -> 6.3 7.1 9.6, Q5_K
 // 2 x 9728 x 2560 12.3 28.7 57.0 -> 16.8 17.4 19.9, Q4_K 2560 x 9728 8.2 17.8 33.0 -> 10.2 10.8 12.9, Q8_0 2 x 9728 x 2560
-// 12.0 25.4 49.9 -> 16.2 16.7 19.0 (one token pays for it, as on every matrix under this id).
+// 12.0 25.4 49.9 -> 16.2 16.7 19.0 (one and two tokens pay for it, as on every matrix under this id). Where eight tokens pay too, matvec.hip says so.
+//
+// Precision. Those lengths had f32 inputs in the default variant; here an input has 22 bits and its sign, 23 in all, down to 2^-17 of its block's largest
+// and fewer below (what is lost there is under 2^-39 of that largest). The outputs are the nearer ones to the exact all the same, since the sums are
+// shorter (relative error against float64, 48 tokens over rows of 1280 .. 6912 weights, default / here): Q8_0 1.22 - 1.29e-7 / 0.86 - 0.96e-7, Q3_K 1.95 - 2.00e-7 / 0.87 -
+// 0.96e-7, Q4_K 1.27 - 1.30e-7 / 1.03 - 1.11e-7, Q5_K 1.29 - 1.31e-7 / 1.07 - 1.12e-7, Q6_K 2.11 - 2.13e-7 / 1.00 - 1.08e-7, with RMSNorm 1.37 - 2.22e-7 / 1.06 - 1.31e-7; with
+// every 256th input a thousand times the others 1.44 - 3.34e-7 / 1.04 - 1.59e-7.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
