@@ -54,6 +54,9 @@
 // 33.9 / 32.9 / 35.6 us (41.7 us with the rows read line by line, row by row, by the kernel that
 // takes k = 2048 and 4096; the default variant 33.6 / 44.1 / 79.7 us).
 //
+// Which matrices come here is matvec.hip's to say (older_mfma_pays: rows of 1024 weights, and long walks of tiles);
+// the others, 14336 x 4096 and 4096 x 14336 in Q6_K among them, are matvec_mfma_rows.hip's by now.
+//
 // Rows of 6144 .. 32768 weights (a multiple of 2048; the FFN-down shapes), Q6_K and Q3_K: the
 // operands of so many positions do not fit a workgroup's registers, so k / 2048 workgroups share
 // a walker's tiles, each over two units of every tile's rows and under its own per-token scales;
