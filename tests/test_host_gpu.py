@@ -237,6 +237,49 @@ def test_kernel_ranges_are_checked_before_launch(ctx):
     c.flush()
 
 
+# One word; a piece less, exactly and more than one; two threads' share; more pieces than flags would make them longer.
+@pytest.mark.parametrize("size", [4, 131072 - 4, 131072, 131072 + 4, 786432 + 4, 2097152 + 4096 + 12])
+@pytest.mark.parametrize("reads", [1, 3, 17])
+def test_reads_arrive_whole_at_every_size(ctx, size, reads):
+    """A submit's reads, of whole buffers and from odd words on, over and over: in pieces behind flags,
+    or (more than sixteen reads) behind the stream's end."""
+    c = ctx
+    rng = np.random.default_rng(size + reads)
+    data = rng.integers(0, 255, size + 16, dtype=np.uint8)
+    buf = c.upload(data)
+    c.flush()
+    out = [np.zeros(size, np.uint8) for _ in range(reads)]
+    for turn in range(4):
+        data[:16] = rng.integers(0, 255, 16, dtype=np.uint8)
+        if turn != 2:  # (with and without a staged write ahead of the submit)
+            c.rec.write_buffer(buf.buffer, 0, data[:16].copy())
+        else:
+            data[:16] = last
+        last = data[:16].copy()
+        for i, o in enumerate(out):
+            o[:] = 0
+            c.rec.read_buffer(700 + i, buf.buffer, 4 * (i % 5), o)
+        done = c.flush()
+        assert [d.token for d in done] == [700 + i for i in range(reads)] + [c.token]
+        for i, o in enumerate(out):
+            assert np.array_equal(o, data[4 * (i % 5) :][:size]), (turn, i)
+        assert 0 < c.host.last_submit()[0] < 1e9
+
+
+def test_reads_over_one_destination_leave_the_last_one(ctx):
+    c = ctx
+    rng = np.random.default_rng(7)
+    first, second = rng.integers(0, 255, 1 << 20, dtype=np.uint8), rng.integers(0, 255, 1 << 20, dtype=np.uint8)
+    a, b = c.upload(first), c.upload(second)
+    dst = np.zeros(1 << 20, np.uint8)
+    c.rec.read_buffer(1, a.buffer, 0, dst)
+    c.rec.clear_buffer(a.buffer, 0, 1 << 20)  # (behind its read)
+    c.rec.read_buffer(2, b.buffer, 0, dst[: 1 << 19])
+    c.flush()
+    assert np.array_equal(dst[: 1 << 19], second[: 1 << 19]) and np.array_equal(dst[1 << 19 :], first[1 << 19 :])
+    assert not c.read(a).any()
+
+
 def test_missing_kernels_fail_the_batch_and_drop_the_submission(ctx):
     """Dispatching a pipeline created with an empty artifact fails with
     UnsupportedKernel, names the kernel, and drops the submission in progress

@@ -5,6 +5,8 @@
 // parameter block, bindings and arithmetic.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "common.h"
 #include "decode.h"
 
@@ -335,20 +337,58 @@ zhip_result launch_fill(hipStream_t stream, void *dst, uint64_t words, uint32_t 
     return hipGetLastError() == hipSuccess ? ZHIP_OK : ZHIP_E_GPU;
 }
 
-// The host's short transfers: a trip over the bus for 64 bytes or for 64 KB, and the launch. A
-// blit of the runtime's takes 4 us of host time more for the same.
+// ---- the host's transfers --------------------------------------------------------
+// Short writes: a trip over the bus for 64 bytes or for 64 KB, and the launch. A blit of the
+// runtime's takes 4 us of host time more for the same. The GPU's clock is left in `stamp`.
 template <class T>
-__global__ __launch_bounds__(256) void copy_kernel(T *dst, const T *src, uint64_t n) {
+__global__ __launch_bounds__(256) void copy_kernel(T *dst, const T *src, uint64_t n, uint64_t *stamp) {
     for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) dst[i] = src[i];
+    if (threadIdx.x == 0) __hip_atomic_store(stamp, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t bytes) {
-    if (bytes == 0) return ZHIP_OK;
-    const bool wide = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | bytes) & 15u) == 0;
+// Reads: `n` units to pinned memory, piece after piece; the last workgroup to finish a piece
+// leaves `ticket` in the piece's flag, where the host waits for it, and behind the last piece the
+// GPU's clock in `stamp`. `arrived` (a counter a piece) is zero before and after. An event and a stream
+// synchronization behind a read cost 2 us more than the flag, a pair of timing events around a
+// submit 5 us (the first one keeps the next kernel from starting), pieces as copies of the runtime's
+// with an event each up to 2 us of idle bus a piece.
+template <class T>
+__global__ __launch_bounds__(256) void read_kernel(T *dst, const T *src, uint64_t n, uint64_t piece, uint32_t *arrived, uint32_t *flags, uint32_t ticket, uint64_t *stamp) {
+    for (uint64_t at = 0, p = 0; at < n; at += piece, p++) {
+        const uint64_t end = at + piece < n ? at + piece : n;
+        for (uint64_t i = at + (uint64_t)blockIdx.x * 256u + threadIdx.x; i < end; i += (uint64_t)gridDim.x * 256u) dst[i] = src[i];
+        // Every wave's stores have reached host memory before the workgroup is counted.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x != 0) continue;
+        if (__hip_atomic_fetch_add(arrived + p, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1u) continue;
+        __hip_atomic_store(arrived + p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (end == n) __hip_atomic_store(stamp, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(flags + p, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+namespace {
+bool wide_copy(const void *dst, const void *src, uint64_t bytes) { return ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | bytes) & 15u) == 0; }
+}  // namespace
+
+// (0 bytes: the stamp alone)
+zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t *stamp) {
+    const bool wide = wide_copy(dst, src, bytes);
     const uint64_t n = bytes / (wide ? 16u : 4u);
-    const dim3 grid(blocks_for(n, 256, 256));
-    if (wide) hipLaunchKernelGGL(copy_kernel<uint4>, grid, dim3(256), 0, stream, static_cast<uint4 *>(dst), static_cast<const uint4 *>(src), n);
-    else hipLaunchKernelGGL(copy_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), n);
+    const dim3 grid(n ? blocks_for(n, 256, 256) : 1u);
+    if (wide) hipLaunchKernelGGL(copy_kernel<uint4>, grid, dim3(256), 0, stream, static_cast<uint4 *>(dst), static_cast<const uint4 *>(src), n, stamp);
+    else hipLaunchKernelGGL(copy_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), n, stamp);
+    return hipGetLastError() == hipSuccess ? ZHIP_OK : ZHIP_E_GPU;
+}
+
+// `piece` is a multiple of 16 bytes; one flag and one counter a piece.
+zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint32_t *flags, uint32_t ticket, uint64_t *stamp) {
+    const bool wide = wide_copy(dst, src, bytes);
+    const uint64_t unit = wide ? 16u : 4u, n = bytes / unit;
+    const dim3 grid(blocks_for(std::min(n, piece / unit), 256, 128));
+    if (wide) hipLaunchKernelGGL(read_kernel<uint4>, grid, dim3(256), 0, stream, static_cast<uint4 *>(dst), static_cast<const uint4 *>(src), n, piece / unit, arrived, flags, ticket, stamp);
+    else hipLaunchKernelGGL(read_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), n, piece / unit, arrived, flags, ticket, stamp);
     return hipGetLastError() == hipSuccess ? ZHIP_OK : ZHIP_E_GPU;
 }
 

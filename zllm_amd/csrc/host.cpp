@@ -23,13 +23,18 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "common.h"
@@ -216,6 +221,100 @@ struct TimingKey {
 };
 struct TimingTotal { uint64_t ns = 0, count = 0; };
 
+// Reads of a submit that the host waits for by their pieces' flags, and pieces of one.
+constexpr uint32_t kFlaggedReads = 16, kMostPieces = 16, kFlags = kFlaggedReads * kMostPieces;
+// Pinned, written by the GPU: its clock behind a submit's last staged write and behind its last read, a flag a piece.
+struct Signals {
+    uint64_t begin, end;
+    uint32_t flags[kFlags];
+};
+
+// A read on its way from its staging, which the GPU fills piece by piece, to its destination.
+struct Handover {
+    uint8_t *dst;
+    const uint8_t *src;
+    uint64_t size, piece;
+    const uint32_t *flags;
+    uint32_t ticket;
+};
+
+inline void pause_cpu() {
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+    __builtin_ia32_pause();
+#endif
+}
+
+// A second thread for long reads: one copies 28 GB/s from pinned memory, the bus brings 54. Pieces
+// go to whichever of the two is free, in order; the thread sleeps but for the time between start()
+// and finish(), and looks at nothing of the context.
+class HandoverThread {
+  public:
+    // (no thread to be had: the caller copies alone)
+    void start(const Handover &job) {
+        std::lock_guard<std::mutex> hold(lock_);
+        job_ = job;
+        next_.store(0, std::memory_order_relaxed);
+        open_ = true;
+        if (!thread_.joinable()) {
+            try {
+                thread_ = std::thread([this] { run(); });
+            } catch (const std::system_error &) {
+            }
+        }
+        wake_.notify_one();
+    }
+    // The next piece that nobody has taken.
+    uint64_t take() { return next_.fetch_add(1, std::memory_order_relaxed); }
+    // When this returns the thread copies nothing any more. `failed`: what the GPU has not
+    // brought will not come.
+    void finish(bool failed) {
+        std::unique_lock<std::mutex> hold(lock_);
+        open_ = false;
+        give_up_.store(failed, std::memory_order_relaxed);
+        idle_.wait(hold, [this] { return !busy_; });
+        give_up_.store(false, std::memory_order_relaxed);
+    }
+    ~HandoverThread() {
+        {
+            std::lock_guard<std::mutex> hold(lock_);
+            stop_ = true;
+        }
+        wake_.notify_one();
+        if (thread_.joinable()) thread_.join();
+    }
+
+  private:
+    void run() {
+        std::unique_lock<std::mutex> hold(lock_);
+        for (;;) {
+            wake_.wait(hold, [this] { return stop_ || open_; });
+            if (stop_) return;
+            const Handover job = job_;
+            busy_ = true;
+            hold.unlock();
+            bool more = true;
+            while (more) {
+                const uint64_t p = take();
+                if (p * job.piece >= job.size) break;
+                while (__atomic_load_n(job.flags + p, __ATOMIC_ACQUIRE) != job.ticket && !give_up_.load(std::memory_order_relaxed)) pause_cpu();
+                more = !give_up_.load(std::memory_order_relaxed);
+                if (more) memcpy(job.dst + p * job.piece, job.src + p * job.piece, std::min(job.piece, job.size - p * job.piece));
+            }
+            hold.lock();
+            busy_ = false;
+            open_ = false;
+            idle_.notify_one();
+        }
+    }
+    std::mutex lock_;
+    std::condition_variable wake_, idle_;
+    std::thread thread_;
+    Handover job_{};
+    std::atomic<uint64_t> next_{0};
+    std::atomic<bool> give_up_{false};
+    bool open_ = false, busy_ = false, stop_ = false;
+};
+
 }  // namespace zhip
 
 using namespace zhip;
@@ -265,7 +364,11 @@ struct zhip_context {
     std::vector<uint32_t> released;
     uint8_t *download = nullptr;  // pinned
     uint64_t download_size = 0;
-    std::vector<hipEvent_t> read_events;  // one behind each piece of a long read
+    Signals *signals = nullptr;   // pinned
+    uint32_t *arrived = nullptr;  // on the device: kFlags counters of read_kernel's workgroups
+    uint32_t ticket = 0;          // of the last submit that waited for flags
+    double tick_ns = 10.0;        // of the GPU's clock
+    HandoverThread handover;
 
     // Small writes wait here, pinned, for the copy kernel queued for each on the stream;
     // upload_used bytes of it are taken, and nothing is in flight when that is 0.
@@ -346,11 +449,9 @@ void drop_pending(zhip_context *c) {
 // launched there later (2 us of host time). They never outlast the batch: zhip_execute and
 // everything that does not order against the stream waits for them first.
 constexpr uint64_t kStagedWrite = 64u << 10, kUploadBytes = 4 * kStagedWrite;
-// Reads of up to this many bytes are a kernel's stores to pinned memory too.
-constexpr uint64_t kSmallRead = 64u << 10;
-// Longer reads than this arrive in pieces, each handed to its destination while the next ones
-// cross the bus: 8 MB (512 tokens of 4096 values) take 150 us to arrive and 285 us to hand over.
-constexpr uint64_t kReadPiece = 512u << 10, kMostPieces = 16;
+// Reads are a kernel's stores to pinned memory too. They arrive in pieces of at least this many
+// bytes, each handed to its destination while the next ones cross the bus, and from kSharedRead on by two threads.
+constexpr uint64_t kReadPiece = 128u << 10, kSharedRead = 768u << 10;
 
 zhip_result finish_writes(zhip_context *c) {
     if (c->upload_used == 0) return ZHIP_OK;
@@ -384,7 +485,7 @@ zhip_result write_device(zhip_context *c, uint8_t *dst, const void *src, uint64_
     uint8_t *at = c->upload + c->upload_used;
     memcpy(at, src, len);
     c->upload_used += room;
-    if (launch_copy(c->stream, dst, at, len) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "%s: launch failed", what);
+    if (launch_copy(c->stream, dst, at, len, &c->signals->begin) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "%s: launch failed", what);
     return ZHIP_OK;
 }
 
@@ -612,6 +713,47 @@ zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **ou
     return ZHIP_OK;
 }
 
+// Whether the submit's end is its last read, so that the host can wait for the reads' flags.
+bool ends_in_flagged_reads(const zhip_context *c) {
+    if (c->profiling || c->ops.empty() || c->ops.back().kind != Op::read || c->ops.back().size == 0) return false;
+    size_t reads = 0;
+    for (const Read &rd : c->reads) reads += rd.size > 0;
+    return reads <= kFlaggedReads;
+}
+
+uint64_t piece_bytes(uint64_t size) { return std::max<uint64_t>(kReadPiece, (size / kMostPieces + 4096u) & ~4095ull); }
+
+// Waits for a piece. The stream is asked now and then, for what may keep a flag from being set.
+zhip_result wait_flag(zhip_context *c, const uint32_t *flag) {
+    for (uint32_t spins = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != c->ticket; spins++) {
+        pause_cpu();
+        if (spins % 8192u != 0) continue;
+        const hipError_t e = hipStreamQuery(c->stream);
+        if (e == hipSuccess) return ZHIP_OK;
+        (void)hipGetLastError();
+        if (e != hipErrorNotReady) return hip_check(c, e, "hipStreamQuery");
+    }
+    return ZHIP_OK;
+}
+
+// A read, from its staging to its destination, piece by piece as they arrive.
+zhip_result hand_over(zhip_context *c, const Read &rd, uint32_t first_flag) {
+    const uint32_t *flags = c->signals->flags + first_flag;
+    const Handover job{rd.dst, c->download + rd.staging_offset, rd.size, piece_bytes(rd.size), flags, c->ticket};
+    if (zhip_result r = wait_flag(c, flags)) return r;
+    const bool shared = rd.size >= kSharedRead;
+    if (shared) c->handover.start(job);
+    zhip_result result = ZHIP_OK;
+    for (uint64_t next = 0; result == ZHIP_OK;) {
+        const uint64_t p = shared ? c->handover.take() : next++, at = p * job.piece;
+        if (at >= job.size) break;
+        result = wait_flag(c, flags + p);
+        if (result == ZHIP_OK) memcpy(job.dst + at, job.src + at, std::min(job.piece, job.size - at));
+    }
+    if (shared) c->handover.finish(result != ZHIP_OK);
+    return result;
+}
+
 // Runs everything queued since the last submit, waits for it, completes reads.
 zhip_result run_queue(zhip_context *c) {
     if (c->read_bytes > c->download_size) {
@@ -619,7 +761,7 @@ zhip_result run_queue(zhip_context *c) {
         c->download = nullptr;
         c->download_size = 0;
         const uint64_t size = std::max<uint64_t>(c->read_bytes, 1u << 20);
-        if (zhip_result r = hip_check(c, hipHostMalloc(reinterpret_cast<void **>(&c->download), size, hipHostMallocDefault), "hipHostMalloc")) return r;
+        if (zhip_result r = hip_check(c, hipHostMalloc(reinterpret_cast<void **>(&c->download), size, hipHostMallocCoherent), "hipHostMalloc")) return r;
         c->download_size = size;
     }
     if (zhip_result r = finish_null_stream(c)) return r;
@@ -627,19 +769,21 @@ zhip_result run_queue(zhip_context *c) {
     std::vector<TimingKey> keys;
     uint64_t dispatches = 0;
     size_t next_read = 0;
-    struct Piece {
-        uint8_t *dst;
-        const uint8_t *src;
-        uint64_t size;
-    };
-    std::vector<Piece> pieces;  // of the long reads, in order; read_events[i] is behind piece i
+    const bool flagged = ends_in_flagged_reads(c);
+    uint32_t next_flags = 0;
     // Parameter blocks the GPU wrote are read back while resolving the launches: before the
     // timed region and before any capture.
     const size_t prefix = (c->use_graphs && !c->profiling) ? replayable_prefix(c) : 0;
     zhip_context::Replay *replay = nullptr;
     if (prefix > 0)
         if (zhip_result r = find_replay(c, prefix, &replay)) return r;
-    if (zhip_result r = hip_check(c, hipEventRecord(c->ev_begin, c->stream), "hipEventRecord")) return r;
+    if (flagged) {
+        c->ticket++;
+        // The submit's staged writes have left the clock, or nothing is there to wait for.
+        if (c->upload_used == 0 && launch_copy(c->stream, c->signals, c->signals, 0, &c->signals->begin) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "submit: launch failed");
+    } else if (zhip_result r = hip_check(c, hipEventRecord(c->ev_begin, c->stream), "hipEventRecord")) {
+        return r;
+    }
     bool replayed = false;
     if (replay) {
         if (hipGraphLaunch(replay->exec, c->stream) == hipSuccess) {
@@ -686,40 +830,36 @@ zhip_result run_queue(zhip_context *c) {
             if (rd.size == 0) break;
             const uint8_t *from = s->dev + op.src_offset;
             uint8_t *to = c->download + rd.staging_offset;
-            if (rd.size <= kSmallRead) {
-                if (launch_copy(c->stream, to, from, rd.size) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "read_buffer: launch failed");
+            if (flagged) {
+                const uint64_t piece = piece_bytes(rd.size);
+                if (launch_read(c->stream, to, from, rd.size, piece, c->arrived + next_flags, c->signals->flags + next_flags, c->ticket, &c->signals->end) != ZHIP_OK)
+                    return set_error(c, ZHIP_E_GPU, "read_buffer: launch failed");
+                next_flags += kMostPieces;
                 break;
             }
-            // (a read over an earlier one's destination is handed over behind it)
-            bool apart = true;
-            for (size_t i = 0; i + 1 < next_read; i++) apart &= c->reads[i].size == 0 || rd.dst + rd.size <= c->reads[i].dst || c->reads[i].dst + c->reads[i].size <= rd.dst;
-            const uint64_t piece = apart ? std::max<uint64_t>(kReadPiece, (rd.size / kMostPieces + 4096u) & ~4095ull) : rd.size;
-            for (uint64_t done = 0; done < rd.size; done += piece) {
-                const uint64_t size = std::min(piece, rd.size - done);
-                if (zhip_result r = hip_check(c, hipMemcpyAsync(to + done, from + done, size, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync")) return r;
-                if (rd.size <= piece) break;  // (in one piece: handed over at the end)
-                if (c->read_events.size() == pieces.size()) {
-                    hipEvent_t ev;
-                    if (zhip_result r = hip_check(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return r;
-                    c->read_events.push_back(ev);
-                }
-                if (zhip_result r = hip_check(c, hipEventRecord(c->read_events[pieces.size()], c->stream), "hipEventRecord")) return r;
-                pieces.push_back(Piece{rd.dst + done, to + done, size});
-            }
+            if (zhip_result r = hip_check(c, hipMemcpyAsync(to, from, rd.size, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync")) return r;
             break;
         }
         }
     }
-    if (zhip_result r = hip_check(c, hipEventRecord(c->ev_end, c->stream), "hipEventRecord")) return r;
-    for (size_t i = 0; i < pieces.size(); i++) {
-        if (zhip_result r = hip_check(c, hipEventSynchronize(c->read_events[i]), "hipEventSynchronize")) return r;
-        memcpy(pieces[i].dst, pieces[i].src, pieces[i].size);
+    c->last_dispatches = dispatches;
+    if (flagged) {
+        next_flags = 0;
+        for (const Read &rd : c->reads) {
+            if (rd.size == 0) continue;
+            if (zhip_result r = hand_over(c, rd, next_flags)) return r;
+            next_flags += kMostPieces;
+        }
+        c->upload_used = 0;
+        const uint64_t begin = __atomic_load_n(&c->signals->begin, __ATOMIC_RELAXED), end = __atomic_load_n(&c->signals->end, __ATOMIC_RELAXED);
+        c->last_ns = end > begin ? (uint64_t)((double)(end - begin) * c->tick_ns) : 0;
+        return ZHIP_OK;
     }
+    if (zhip_result r = hip_check(c, hipEventRecord(c->ev_end, c->stream), "hipEventRecord")) return r;
     if (zhip_result r = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
     c->upload_used = 0;
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, c->ev_begin, c->ev_end) == hipSuccess) c->last_ns = (uint64_t)((double)ms * 1e6);
-    c->last_dispatches = dispatches;
     for (size_t i = 0; i < timed; i++) {
         float dms = 0.f;
         if (hipEventElapsedTime(&dms, c->events[2 * i], c->events[2 * i + 1]) != hipSuccess) continue;
@@ -727,11 +867,8 @@ zhip_result run_queue(zhip_context *c) {
         t.ns += (uint64_t)((double)dms * 1e6);
         t.count++;
     }
-    for (const Read &rd : c->reads) {
-        bool in_pieces = false;
-        for (const Piece &p : pieces) in_pieces |= p.src == c->download + rd.staging_offset;
-        if (rd.size > 0 && !in_pieces) memcpy(rd.dst, c->download + rd.staging_offset, rd.size);
-    }
+    for (const Read &rd : c->reads)
+        if (rd.size > 0) memcpy(rd.dst, c->download + rd.staging_offset, rd.size);
     return ZHIP_OK;
 }
 
@@ -1037,20 +1174,18 @@ zhip_result zhip_create(const zhip_options *options, zhip_context **out_context)
     snprintf(c->caps.name, sizeof c->caps.name, "%s", prop.name[0] ? prop.name : "AMD Instinct (gfx950)");
     snprintf(c->caps.arch, sizeof c->caps.arch, "%s", prop.gcnArchName);
     if (char *colon = strchr(c->caps.arch, ':')) *colon = 0;
-    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&c->ev_begin) != hipSuccess || hipEventCreate(&c->ev_end) != hipSuccess) {
+    int clock_khz = 0;
+    if (hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, index) == hipSuccess && clock_khz > 0) c->tick_ns = 1e6 / (double)clock_khz;
+    // (The fixed scratch array's address is looked up here alone, while the device is current.)
+    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&c->ev_begin) != hipSuccess || hipEventCreate(&c->ev_end) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&c->signals), sizeof(Signals), hipHostMallocCoherent) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void **>(&c->arrived), kFlags * sizeof(uint32_t)) != hipSuccess || launch_fill(c->stream, c->arrived, kFlags, 0) != ZHIP_OK ||
+        hipStreamSynchronize(c->stream) != hipSuccess || no_alloc_setup(index, c->info) != ZHIP_OK) {
         (void)hipGetLastError();
-        delete c;
+        (void)zhip_destroy(c);
         return ZHIP_E_GPU;
     }
-    // The device is current: the one place the fixed scratch array's address is looked up.
-    if (no_alloc_setup(index, c->info) != ZHIP_OK) {
-        (void)hipEventDestroy(c->ev_begin);
-        (void)hipEventDestroy(c->ev_end);
-        (void)hipStreamDestroy(c->stream);
-        delete c;
-        return ZHIP_E_GPU;
-    }
+    memset(c->signals, 0, sizeof(Signals));
     *out_context = c;
     return ZHIP_OK;
 }
@@ -1080,7 +1215,8 @@ zhip_result zhip_destroy(zhip_context *c) {
         if (e.exec) (void)hipGraphExecDestroy(e.exec);
     c->work.release();
     for (hipEvent_t ev : c->events) (void)hipEventDestroy(ev);
-    for (hipEvent_t ev : c->read_events) (void)hipEventDestroy(ev);
+    if (c->arrived) (void)hipFree(c->arrived);
+    if (c->signals) (void)hipHostFree(c->signals);
     if (c->download) (void)hipHostFree(c->download);
     if (c->upload) (void)hipHostFree(c->upload);
     if (c->ev_begin) (void)hipEventDestroy(c->ev_begin);
