@@ -2161,3 +2161,33 @@ def test_silu_mul(ctx):
     c.launcher().launch(Kernel.silu_mul, P.SiluMul(n, width), [c.upload(gu), act], K.elementwise(n))
     g = gu[:, :width].astype(np.float64)
     assert rel_err(c.read(act), g * sigmoid64(g) * gu[:, width:]) <= 1e-6
+
+
+@pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+@pytest.mark.parametrize("n,k", [(24700, 2048), (28700, 256), (14370, 768)])
+def test_matmul_int8_k_formats_tall_matrices_repeat_their_rows(ctx, t, n, k):
+    """The launches whose waves walk all of k, over one, two and four token tiles, in column order
+    and die by die (matrices of 24 MB and more, 193 column tiles, no multiple of the eight dies), short rows
+    whose parts are empty, ragged rows and tokens: a matrix that repeats 1000 rows gives the bits that
+    the 1000 rows alone give, in launches of a part of k a wave."""
+    c, base, stride = ctx, 1000, n + 5
+    rows = 300
+    x = c.random(rows * k, 1).reshape(rows, k)
+    raw, _ = quant_rows(c, t, base, k)
+    row = np.ascontiguousarray(raw).reshape(-1).view(np.uint8).reshape(base, -1)
+    wide = np.ascontiguousarray(np.resize(row, (n, row.shape[1])))
+    small, tall = c.gpu_weights(t, raw, k), c.gpu_weights(t, wide, k)
+    init = c.random(rows * base, 0.5).reshape(rows, base)
+    columns = np.arange(n) % base
+    for count, accumulate in ((20, 0), (33, 1), (64, 0), (70, 0), (130, 1), (200, 0), (300, 0)):
+        act = quantize_x(c, t, c.upload(x[:count]), count, k)
+        out = c.upload(init[:count])
+        launch_int8(c, t, act, small, out, count, base, k, accumulate, None)
+        want = c.read(out).reshape(count, base)
+        start = np.zeros((count, stride), np.float32)
+        start[:, 2 : 2 + n] = init[:count, columns]
+        out = c.upload(start)
+        launch_int8(c, t, act, tall, out, count, n, k, accumulate, None, col0=2, stride=stride)
+        got = c.read(out).reshape(count, stride)
+        assert np.array_equal(got[:, 2 : 2 + n].view(np.uint32), want[:, columns].view(np.uint32)), (count, accumulate)
+        assert not got[:, :2].any() and not got[:, 2 + n :].any()

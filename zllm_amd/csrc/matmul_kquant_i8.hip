@@ -63,6 +63,7 @@ struct KqArgs {
     float *out;
     uint32_t rows, n, k, col0, out_stride, accumulate, row_bytes;
     uint32_t qx_bytes, w_bytes, dx_bytes;
+    uint32_t by_die;  // workgroups renumbered die by die
 };
 
 // A part's LDS: a ring of three token tiles, the tiles' scales, which are used a step later, and
@@ -294,7 +295,15 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
     constexpr bool UNIT_SCALES = NT == 1 && P::HAS_MIN;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, lrow = lane & 31u, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = wave % S, group = wave / S;
-    const uint32_t n0 = blockIdx.x * (32u * RW) + 32u * group, t0 = blockIdx.y * (32u * NT);
+    // The chip deals workgroups out to its eight dies in turn. Renumbered, those of a column of the matrix follow one
+    // another on one die, whose L2 then has the column's weights for all but the first of them.
+    uint32_t column = blockIdx.x, tokens = blockIdx.y;
+    if (S == 1 && a.by_die) {
+        const uint32_t id = tokens * gridDim.x + column, dealt = (gridDim.x & ~7u) * gridDim.y, turn = id >> 3;
+        column = id < dealt ? (turn / gridDim.y << 3) + (id & 7u) : id / gridDim.y;
+        tokens = (id < dealt ? turn : id) % gridDim.y;
+    }
+    const uint32_t n0 = column * (32u * RW) + 32u * group, t0 = tokens * (32u * NT);
     const uint32_t blocks = a.k / 256u, first = part * blocks / S, mine = (part + 1u) * blocks / S - first;
     const uint32_t most = (blocks + S - 1u) / S;  // of any part
     const __amdgpu_buffer_rsrc_t xbuf = make_buffer(a.qx, a.qx_bytes), wbuf = make_buffer(a.w, a.w_bytes), dbuf = make_buffer(a.dx, a.dx_bytes);
@@ -557,44 +566,55 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const KqArgs &a) {
     return check_launch(d, name);
 }
 
-// Which launch takes the step; the bits are the same. A wave a part each (S = 4) unless a wave that
-// walks all of k is the faster one. us, all of k / a part each:
-//   Q3_K, four token tiles, from four and a half waves a CU on: 28672 x 4096 at 512 tokens 111 / 130, 18432 x
-//     2560 at 201 34 / 41, at 4096 52 / 52, at 8192 96 / 91; below, 16384 at 256 30 / 32, 44 / 42, 81 / 71
-//   Q4_K, two (the closed sums of four do not fit the registers), from five on: 28672 x 4096 at 512 168 / 192, at
-//     128 50 / 60; 14336 at 512 91 / 104, 20480 at 128 48 / 55; below, 14336 at 128 (three and a half) 35 / 30
-//   Q4_K and Q5_K, one, steps of up to 64 tokens whose parts would take a third round of workgroups:
-//     28672 x 4096 at 32 tokens Q4_K 25 / 28, Q5_K 28 / 32, at 64 36 / 38, 40 / 46; with two rounds, 14336 at 32, 23 / 16
-// Q5_K and Q6_K at two tiles gain nothing (28672 x 4096 at 512: 215 / 214, 214 / 190).
+// Which launch takes the step; the bits are the same. Workgroups that walk a part of k each (S = 4) have a CU to
+// themselves: a launch of w a CU takes w times one's time. Those that walk all of it (S = 1) share a CU two at a
+// time, and a pair takes less than twice a lone one's time: an odd one out costs `lone`, a pair `pair`. In k the
+// first kind's time grows like blocks + 3 (the exchange), the second's like blocks + 2. In units of such a
+// time, fitted to steps of 16 ... 512 tokens over sixteen matrices of 1024 x 3072 ... 28672 x 4096 and 4096 x 14336, every
+// launch of the list on each of them: the rule's launch is within 0.1 % (Q5_K 0.3 %, Q6_K 0.6 %) of the fastest one in the mean. (A line
+// at a number of workgroups, as here before, lost 1.6 % / 6.2 % / 2.7 % / 1.8 % of Q4_K's / Q5_K's / Q6_K's / Q3_K's time, and where a
+// last round was nearly empty 30 - 80 %: 96 x 19456 x 2560 Q4_K 34.9 -> 20.5 us, Q5_K 40.6 -> 22.5, Q3_K 25.1 -> 19.0; Q5_K
+// 512 x 12288 x 2560 63.4 -> 55.9, 64 x 28672 x 4096 Q4_K 33.1 -> 31.6.)
+struct Lone { uint32_t lone, pair; };
+struct Costs {
+    uint32_t parts[5];  // token tiles x row groups: 1 x 1, 1 x 2, 2 x 1, 2 x 2, 4 x 2
+    Lone whole[3];      // of 1, 2 and 4 token tiles, four row groups (0: none; of two planes, four tiles' closed sums do not fit the registers)
+};
+template <class P> constexpr Costs costs();
+template <> constexpr Costs costs<KqQ3>() { return {{19, 24, 22, 31, 42}, {{51, 73}, {67, 90}, {98, 118}}}; }
+template <> constexpr Costs costs<KqQ4>() { return {{14, 19, 18, 29, 39}, {{39, 56}, {50, 71}, {0, 0}}}; }
+template <> constexpr Costs costs<KqQ5>() { return {{13, 17, 19, 26, 40}, {{32, 47}, {51, 79}, {0, 0}}}; }
+template <> constexpr Costs costs<KqQ6>() { return {{17, 26, 21, 31, 43}, {{53, 74}, {66, 91}, {0, 0}}}; }
+
 template <class P>
-zhip_result launch_format(const Dispatch &d, const char *name, const KqArgs &a) {
-    const uint64_t cus = (uint64_t)d.dev->compute_units, groups = (a.n + 31u) / 32u;
-    auto tokens = [&](uint32_t nt) { return (uint64_t)((a.rows + 32u * nt - 1u) / (32u * nt)); };
-    if constexpr (P::PLANES == 1) {
-        if (a.rows > 64u && 2u * groups * tokens(4) >= 9u * cus) return launch_tile<P, 4, 4, 1>(d, name, a);
-    }
-    if constexpr (P::HAS_MIN) {
-        if constexpr (P::SHIFT == 3) {
-            if (a.rows > 32u && groups * tokens(2) >= 5u * cus) return launch_tile<P, 2, 4, 1>(d, name, a);
-        }
-        if (a.rows <= 64u && groups > 2u * cus) return launch_tile<P, 1, 4, 1>(d, name, a);
-    }
-    // One workgroup a CU at a time: the tile whose rounds take least. A round's time in eighths of
-    // the smallest tile's, measured at k = 4096 (Q4_K 9.3 / 12.6 / 11.0 / 16.8 / 24 us, Q6_K 10.2 /
-    // 14.9 / 11.8 / 17.1 / 23).
-    auto rounds = [&](uint32_t nt, uint32_t rw) { return ((groups + rw - 1u) / rw * tokens(nt) + cus - 1u) / cus; };
-    const uint64_t cost[5] = {8u * rounds(1, 1), 11u * rounds(1, 2), (P::HAS_MIN ? 10u : 9u) * rounds(2, 1), (P::HAS_MIN ? 15u : 13u) * rounds(2, 2),
-        (P::HAS_MIN ? 21u : 17u) * rounds(4, 2)};
+zhip_result launch_format(const Dispatch &d, const char *name, KqArgs a) {
+    constexpr Costs c = costs<P>();
+    const uint64_t cus = (uint64_t)d.dev->compute_units, groups = (a.n + 31u) / 32u, blocks = a.k / 256u;
+    auto per_cu = [&](uint32_t nt, uint32_t rw) { return ((groups + rw - 1u) / rw * ((a.rows + 32u * nt - 1u) / (32u * nt)) + cus - 1u) / cus; };
+    constexpr uint32_t shapes[5][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {4, 2}};
+    uint64_t least = ~0ull;
     int best = 0;
-    for (int i = 1; i < 5; i++)
-        if (cost[i] < cost[best]) best = i;
+    for (int i = 0; i < 8; i++) {
+        if (i >= 5 && c.whole[i - 5].lone == 0u) continue;
+        const uint64_t w = i < 5 ? per_cu(shapes[i][0], shapes[i][1]) : per_cu(1u << (i - 5), 4u);
+        const uint64_t cost = i < 5 ? c.parts[i] * w * (blocks + 3u) : (c.whole[i - 5].lone * (w & 1u) + c.whole[i - 5].pair * (w >> 1)) * (blocks + 2u);
+        if (cost < least) least = cost, best = i;
+    }
+    // Matrices too large for the dies' L2s, several token tiles: 24576 x 3072 and 28672 x 4096 at 256 ... 512 tokens 1 - 8 % faster
+    // column by column (two token tiles and one; four the same), matrices of up to 20 MB up to 4 % slower.
+    a.by_die = (uint64_t)a.n * a.row_bytes >= (24u << 20);
     switch (best) {
     case 0: return launch_tile<P, 1, 1, 4>(d, name, a);
     case 1: return launch_tile<P, 1, 2, 4>(d, name, a);
     case 2: return launch_tile<P, 2, 1, 4>(d, name, a);
     case 3: return launch_tile<P, 2, 2, 4>(d, name, a);
-    default: return launch_tile<P, 4, 2, 4>(d, name, a);
+    case 4: return launch_tile<P, 4, 2, 4>(d, name, a);
+    case 5: return launch_tile<P, 1, 4, 1>(d, name, a);
+    case 6: return launch_tile<P, 2, 4, 1>(d, name, a);
+    default: break;
     }
+    if constexpr (c.whole[2].lone != 0u) return launch_tile<P, 4, 4, 1>(d, name, a);
+    return fail(d, ZHIP_E_GPU, "%s: no launch", name);
 }
 
 }  // namespace
@@ -605,7 +625,7 @@ zhip_result launch_format(const Dispatch &d, const char *name, const KqArgs &a) 
 zhip_result launch_matmul_kquant_i8(const Dispatch &d, const char *name, int type, const uint8_t *qx, const uint8_t *w, const uint8_t *dx, float *out,
     uint32_t rows, uint32_t n, uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t qx_bytes, uint32_t w_bytes,
     uint32_t dx_bytes) {
-    const KqArgs a{qx, w, dx, out, rows, n, k, col0, out_stride, accumulate, row_bytes, qx_bytes, w_bytes, dx_bytes};
+    const KqArgs a{qx, w, dx, out, rows, n, k, col0, out_stride, accumulate, row_bytes, qx_bytes, w_bytes, dx_bytes, 0};
     switch (type) {
     case 3: return launch_format<KqQ3>(d, name, a);
     case 4: return launch_format<KqQ4>(d, name, a);
