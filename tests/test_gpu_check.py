@@ -325,6 +325,41 @@ def test_matvec_bf16_several_tokens_silu_pair(ctx_wide, half, m, n, k, half_row,
         assert np.array_equal(run([t])[0], got[t])
 
 
+@pytest.mark.parametrize("k,mb", [
+    (6336, 17), (6400, 4), (6400, 17),            # the general kernel; the shortest rows, from 4 MB on
+    (6464, 5), (6656, 5), (9664, 4), (9664, 17),  # a wave's last piece past the row; rows of whole 512s under 16 MB
+    (11520, 5), (16320, 4),                       # a wave's every piece past it
+])
+@pytest.mark.parametrize("half", HALVES)
+def test_matvec_bf16_several_tokens_long_rows(ctx_wide, half, k, mb):
+    """Long rows of whole lines, any number of them: within 1e-5 of float64, a token's bits the same alone, and
+    nothing of the row behind (an infinity at its start) in a row's sums."""
+    c, eps, n = ctx_wide, 1e-6, (mb << 20) // (2 * k) + 37
+    x, nw = c.random(11 * k, 3).reshape(11, k), c.random(k, 1)
+    bits, values = random_half(c, n * k, k ** -0.5, half)
+    bits, values = bits.reshape(-1, k), values.reshape(-1, k)
+    bits[7, 0] = 0x7C00 if half == "f16" else 0x7F80  # infinity
+    init = c.random(11 * n, 0.5).reshape(11, n)
+    wa, na = c.upload(bits), c.upload(nw)
+    rows = np.arange(n) != 7
+
+    def run(tokens, norm, accumulate):
+        out = c.upload(init[tokens])
+        p = P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=eps, norm=norm, accumulate=accumulate)
+        c.launcher().launch(Kernel["matvec_" + half], p, [c.upload(x[tokens]), wa, out, na], (K.div_ceil(n, K.matvec_rows), len(tokens), 1))
+        return c.read(out).reshape(len(tokens), n)
+
+    v64 = values.astype(np.float64)
+    for m, norm, accumulate in ((2, False, False), (8, False, True), (11, False, True), (3, True, True)):
+        got = run(list(range(m)), norm, accumulate)
+        xs = np.stack([norm_row(x[t], nw if norm else None, eps) for t in range(m)])
+        want = xs @ v64.T + (init[:m] if accumulate else 0.0)
+        assert rel_err(got[:, rows], want[:, rows]) <= 1e-5
+        assert not np.isfinite(got[:, 7]).any()
+        for t in (0, m - 1):
+            assert np.array_equal(run([t], norm, accumulate)[0][rows], got[t][rows])
+
+
 @pytest.mark.parametrize("k", [1024, 1536, 2048, 2560, 3072, 3584, 4096])
 @pytest.mark.parametrize("half", HALVES)
 def test_matvec_bf16_several_tokens_norm_is_every_kernels(ctx, ctx_wide, half, k):

@@ -381,7 +381,8 @@ static bool older_mfma_pays(const Dispatch &d, const MvArgs &a, int type) {
 // matvec_bf16 on the matrix cores, the weights read once for all tokens (matvec_bf16_mfma_stream.hip).
 bool matvec_bf16_mfma_stream_accepts(const MvArgs &a);
 zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16);
-// Which matrices take it: 16 MB of weights or more, and gate / up pairs of 32 MB or more, in
+// Which matrices take it: rows of whole 512s in matrices of 16 MB of weights or more, gate / up pairs of 32 MB or more,
+// and without the RMSNorm prologue, from 4 MB on, every matrix of rows of 6400 weights or more (no pairs), in
 // contexts opened with ZHIP_OPTION_WIDE_DECODE, and then at every width from one token on: the
 // kernel sums in another order than the general one, and a token's bits must not depend on the
 // width of the step it runs in (src/sched/sched.zig:55-58; src/plan/qwen35.zig:380-381), so the
@@ -400,10 +401,22 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
 // and below the line, where only the default kernels run:
 //   4096 x 1024 (8 MB)           3.9 4.0 4.5 5.9
 //   2048 x 2048 (8 MB)           4.2 4.9 4.9 6.0
-constexpr uint64_t kBf16StreamBytes = 16ull << 20;
+// Long rows are past the registers of matvec_half_row.hip, and the general kernel takes them token by token:
+// without the prologue, this kernel / the general one at 1, 2, 4, 8 tokens, f16:
+//   768 x 6400 (9 MB)            9.1 9.2 9.3 9.4 / 7.4 10.3 18.2 32.8
+//   1024 x 7168                  10.6 10.8 10.9 11.4 / 9.7 12.1 20.3 36.4
+//   400 x 9600                   9.1 9.0 9.1 9.4 / 9.0 15.4 28.0 52.6
+//   2688 x 8064 (41 MB)          14.9 14.9 15.1 15.9 / 13.5 16.9 28.5 52.4
+//   3328 x 11520                 21.1 21.2 21.6 21.3 / 22.5 35.0 61 114
+// and below that line: 1024 x 6144 11.1 11.3 11.4 11.6 / 9.0 11.3 18.4 32.3, 3200 x 5248 (33 MB) 13.8 14.3 14.5 13.9 / 10.8 13.4 21.2 40.1.
+// Shorter rows of no multiple of 512 stay with matvec_half_row.hip, which is the faster one at one and two tokens, at two by up to
+// 35 % (5376 x 1792 pair 13.3 / 9.5, 8064 x 2688 22.0 / 17.1; at eight 13.3 / 17.7, 22.5 / 31.6).
+constexpr uint64_t kBf16StreamBytes = kMatvecBf16StreamBytes, kBf16StreamLongBytes = 4ull << 20;
+constexpr uint32_t kBf16StreamLong = 6400u;
 static bool bf16_stream_pays(const Dispatch &d, const MvArgs &a) {
     const uint64_t bytes = (uint64_t)a.rows * a.row_bytes;  // (of a pair: of its gate rows)
-    return d.dev->wide_decode && bytes >= kBf16StreamBytes;
+    if (a.k % 512u == 0 && bytes >= kBf16StreamBytes) return d.dev->wide_decode;
+    return d.dev->wide_decode && a.k >= kBf16StreamLong && bytes >= kBf16StreamLongBytes && !(a.flags & FLAG_NORM);
 }
 // The 16-bit formats with the inputs in registers, one to eight tokens (matvec_half_row.hip).
 bool matvec_half_row_accepts(const MvArgs &a);

@@ -1,6 +1,7 @@
 // matvec_bf16 (and matvec_f16) on the matrix cores for steps of several tokens and k = 1024 ... 4096 in steps of
 // 512: the weight stream is read once for all tokens of the step and nothing but partial sums
-// crosses LDS. Contract of src/kernels/matvec_half.wgsl:1-133 with the bf16 decoder of
+// crosses LDS. (Rows of more than 4096 weights and no multiple of 512 are taken as if they ended in zeros: their lines are
+// whole, the ones past a row's end are asked for from an empty buffer, and the tokens' positions there are zeros.) Contract of src/kernels/matvec_half.wgsl:1-133 with the bf16 decoder of
 // src/kernels/half/bf16.wgsl:3-9: out[t][col0 + j] (+)= sum_i x[t][i] * w[j][i], the inputs
 // taken as the f32 values they are. (The reference gives every token a row of workgroups of its
 // own, so a step of M tokens reads the weights M times.)
@@ -65,8 +66,8 @@ constexpr uint32_t LDS_BYTES = PART_BYTES + RING_BYTES + KEPT * 1024u + 64u;  //
 // Kernels whose workgroups split their tokens themselves keep the pieces in LDS ([piece][token of
 // 8][k], rows padded by 16 bytes so that one chunk of neighbouring rows falls in different banks)
 // until the operands are read, at its end: ring slots below them take their weights meanwhile.
-// An f16 token of a step without a pair enters as two pieces, every other as three.
-constexpr uint32_t pieces_of(bool f16, bool pair) { return f16 && !pair ? 2u : 3u; }
+// An f16 token enters as two pieces, `whole` (steps of a pair, and over some long rows) as three, and so does every other.
+constexpr uint32_t pieces_of(bool f16, bool whole) { return f16 && !whole ? 2u : 3u; }
 template <int NP> constexpr uint32_t piece_row() { return 1024u * NP + 16u; }
 template <int NP, uint32_t PIECES> constexpr uint32_t pieces_bytes() { return 8u * PIECES * piece_row<NP>(); }
 template <int NP, uint32_t PIECES> constexpr bool pieces_fit() { return pieces_bytes<NP, PIECES>() <= LDS_BYTES - 64u; }
@@ -200,17 +201,20 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (
 // times 2^11, after a power of two has put its largest magnitude at 2^14 (an input keeps 22
 // bits), and a token's sums are multiplied by one over its scale. With PAIR there is a third row,
 // what those two left times 2^22, and an input keeps all its bits (the general kernel, which takes
-// pairs without ZHIP_OPTION_WIDE_DECODE, has them too): the matrix instruction has the rows anyway.
+// pairs without ZHIP_OPTION_WIDE_DECODE, has them too): the matrix instruction has the rows anyway. So over the long
+// rows that would be the general kernel's otherwise (no multiple of 512, or under 16 MB): an activation's products there, of a log-normal magnitude,
+// 768 x 6400, relative error 1.17e-7 with two, 1.08e-7 with three, 1.12e-7 in the general kernel. (In time three cost up to 10 %: 2560 x 9728
+// 16.7 -> 18.5 us.)
 // PAIR: a SILU_PAIR step, an output tile's gate rows and then its up rows (the general kernel's
 // time grows with the tokens: 2 x 8192 x 2048 f16 at eight 38 us, here 18).
 // LONG: rows of q.parts stretches of 512 NP columns (the last one may end past the row); workgroup i multiplies stretch i % parts (`kpart`) of the tiles that
 // walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums. Without the RMSNorm prologue no
 // workgroup needs more of a token than its stretch (an F16 token's scale is then the stretch's own).
-template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
+template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR, bool WHOLE>
 __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(StreamArgs q) {
     static_assert(!PAIR || !LONG, "gate / up steps take whole rows");
     constexpr uint32_t PER = PAIR ? 2u : 1u;  // weight tiles an output tile
-    constexpr uint32_t PIECES = pieces_of(F16, PAIR);
+    constexpr uint32_t PIECES = pieces_of(F16, WHOLE);
     static_assert(SPLIT || pieces_fit<NP, PIECES>(), "the tokens' pieces must fit LDS");
     const MvArgs &a = q.a;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -490,9 +494,9 @@ __global__ __launch_bounds__(256) void matvec_f16_split_kernel(MvArgs a, uint2 *
     }
 }
 
-template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
+template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR, bool WHOLE>
 zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
-    auto kernel = matvec_bf16_mfma_stream_kernel<NP, SPLIT, F16, LONG, PAIR>;
+    auto kernel = matvec_bf16_mfma_stream_kernel<NP, SPLIT, F16, LONG, PAIR, WHOLE>;
     static bool configured = false;
     if (!configured) {
         if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) != hipSuccess) {
@@ -508,27 +512,27 @@ zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
 }  // namespace
 
 // Whether this kernel can run the (already validated) arguments: k split into whole lines a
-// wave; a gate / up pair only over rows that one workgroup takes whole.
+// wave, and rows of whole lines where the workgroups split the tokens of long ones themselves (`own` below); a gate / up pair only over rows that one workgroup takes whole.
 // (rows of more than 4096 weights are taken in stretches of columns: equal ones in one launch, workgroups sharing a
 // tile, with a launch for their sums; unequal ones behind the RMSNorm prologue a launch each; up to 16384: the split launch stages a token in 64 KB of LDS)
 bool matvec_bf16_mfma_stream_accepts(const MvArgs &a) {
     if ((a.flags & FLAG_SILU_PAIR) && (a.k > 4096u || ((uint64_t)a.half + a.rows + 64u) * a.row_bytes >= 0xfffffff0ull)) return false;
-    return a.m >= 1 && a.k >= 1024u && a.k <= 16384u && a.k % 512u == 0 && a.act_div == 0.f && a.rows >= 1 &&
+    return a.m >= 1 && a.k >= 1024u && a.k <= 16384u && (a.k % 512u == 0 || (a.k % 64u == 0 && a.k > 4096u && !(a.flags & FLAG_NORM))) && a.act_div == 0.f && a.rows >= 1 &&
            a.xr % 4u == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0 && a.row_bytes == 2u * a.k;
 }
 
 // The stretches' lengths, in 512 columns: rows of up to 4096 weights 2 .. 8, longer rows 4 .. 8 behind the RMSNorm prologue (equal ones 5 .. 8), 3 .. 6 without.
-template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR>
+template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR, bool WHOLE>
 static zhip_result launch_np(const Dispatch &d, const StreamArgs &q, dim3 grid) {
     constexpr int LOW = LONG ? (SPLIT ? 5 : 3) : SPLIT ? 4 : 2, HIGH = LONG && !SPLIT ? 6 : 8;
     if constexpr (NP >= LOW && NP <= HIGH) {
-        if (q.a.k == 512u * NP) return launch_blocks<NP, SPLIT || !pieces_fit<NP, pieces_of(F16, PAIR)>(), F16, LONG, PAIR>(d, q, grid);
+        if (q.a.k == 512u * NP) return launch_blocks<NP, SPLIT || !pieces_fit<NP, pieces_of(F16, WHOLE)>(), F16, LONG, PAIR, WHOLE>(d, q, grid);
     }
-    if constexpr (NP < 8) return launch_np<NP + 1, SPLIT, F16, LONG, PAIR>(d, q, grid);
+    if constexpr (NP < 8) return launch_np<NP + 1, SPLIT, F16, LONG, PAIR, WHOLE>(d, q, grid);
     else return fail(d, ZHIP_E_GPU, "%s: a stretch of %u columns", F16 ? "matvec_f16" : "matvec_bf16", q.a.k);
 }
-template <bool SPLIT, bool F16, bool LONG = false, bool PAIR = false>
-static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 grid) { return launch_np<2, SPLIT, F16, LONG, PAIR>(d, q, grid); }
+template <bool SPLIT, bool F16, bool LONG = false, bool PAIR = false, bool WHOLE = PAIR>
+static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 grid) { return launch_np<2, SPLIT, F16, LONG, PAIR, WHOLE>(d, q, grid); }
 
 // f16: the weights are f16 (matvec_f16), bf16 otherwise.
 zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16) {
@@ -549,7 +553,7 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
     // one launch, `launches` workgroups share a walker's tiles, a
     // stretch each, and a second launch adds the stretches' sums in their order and applies the
     // epilogue (their sums wait in the workspace, behind the tokens' planes where there are any).
-    const uint32_t token_pieces = pieces_of(f16, pair), pieces = a.k / 512u, fits = token_pieces == 2u ? 8u : 6u;
+    const uint32_t token_pieces = pieces_of(f16, pair), pieces = (a.k + 511u) / 512u, fits = token_pieces == 2u ? 8u : 6u;
     uint32_t launches = (a.k + 4095u) / 4096u;
     // Without the RMSNorm prologue the workgroups split their stretches' tokens themselves: in stretches of up to 3072 columns
     // (what fits LDS in bf16, and in f16 the sums are the shorter ones), equal ones where two more than the fewest at most are, or with a last one that ends past the
@@ -568,6 +572,8 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
         launches = fewest;
         for (uint32_t n = fewest + 2u; n >= fewest; n--) launches = pieces % n == 0u ? n : launches;
     }
+    // (an input keeps all its bits where the general kernel was the alternative)
+    const bool whole = a.k % 512u != 0 || (uint64_t)a.rows * a.row_bytes < kMatvecBf16StreamBytes;
     const bool split = !own && pieces > fits;
     const bool together = own || (launches > 1u && pieces % launches == 0u && split && launches <= kMatvecMaxParts && cus >= launches);
     const uint64_t planes_bytes = own ? 0ull : ((2ull * token_pieces * a.m * a.k + 4ull * a.m + 64u) + 255u) & ~255ull;
@@ -611,7 +617,8 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
             q.t0 = t0;
             const dim3 all(walkers * launches);
             zhip_result r;
-            if (own) r = f16 ? launch_for_k<false, true, true>(d, q, all) : launch_for_k<false, false, true>(d, q, all);
+            if (own && f16) r = whole ? launch_for_k<false, true, true, false, true>(d, q, all) : launch_for_k<false, true, true>(d, q, all);
+            else if (own) r = launch_for_k<false, false, true>(d, q, all);
             else r = f16 ? launch_for_k<true, true, true>(d, q, all) : launch_for_k<true, false, true>(d, q, all);
             if (r != ZHIP_OK) return r;
             MvArgs sum = q.a;

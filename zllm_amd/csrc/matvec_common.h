@@ -94,6 +94,8 @@ __device__ __forceinline__ void stage_token(const MvArgs &a, uint32_t token, flo
 // outputs a.rows apart); this launch adds a tile's parts in the order of their columns and applies
 // the SILU_PAIR / ACCUMULATE epilogue (matvec_mfma_resident.hip).
 constexpr uint32_t kMatvecMaxParts = 16;  // rows of up to 32768 weights
+// The 16-bit matrices of whole 512s a row that ZHIP_OPTION_WIDE_DECODE moves to the matrix cores (matvec.hip).
+constexpr uint64_t kMatvecBf16StreamBytes = 16ull << 20;
 zhip_result launch_matvec_parts_sum(const Dispatch &d, const char *name, const MvArgs &a, const float *partial, uint32_t parts);
 // A step over such rows with the RMSNorm prologue: no workgroup sees a whole row, so a launch of
 // its own leaves each token's 1 / sqrt(mean(x^2) + eps) in scales[token] beforehand (the sum of
