@@ -172,4 +172,14 @@ zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t
 // Reads `bytes` to pinned memory in pieces: read_kernel, elementwise.hip.
 zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint32_t *flags, uint32_t ticket, uint64_t *stamp);
 
+// A launch's time by its workgroups, where two share a CU: a lone one's time, and a pair's, which is less than twice
+// that. An odd one out costs its CU a lone one's.
+struct SharedCu {
+    uint32_t lone, pair;
+    constexpr uint64_t of(uint64_t workgroups, uint64_t cus) const {
+        const uint64_t w = (workgroups + cus - 1u) / cus;
+        return lone * (w & 1u) + pair * (w >> 1);
+    }
+};
+
 }  // namespace zhip

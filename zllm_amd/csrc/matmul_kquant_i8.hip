@@ -575,10 +575,9 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const KqArgs &a) {
 // at a number of workgroups, as here before, lost 1.6 % / 6.2 % / 2.7 % / 1.8 % of Q4_K's / Q5_K's / Q6_K's / Q3_K's time, and where a
 // last round was nearly empty 30 - 80 %: 96 x 19456 x 2560 Q4_K 34.9 -> 20.5 us, Q5_K 40.6 -> 22.5, Q3_K 25.1 -> 19.0; Q5_K
 // 512 x 12288 x 2560 63.4 -> 55.9, 64 x 28672 x 4096 Q4_K 33.1 -> 31.6.)
-struct Lone { uint32_t lone, pair; };
 struct Costs {
     uint32_t parts[5];  // token tiles x row groups: 1 x 1, 1 x 2, 2 x 1, 2 x 2, 4 x 2
-    Lone whole[3];      // of 1, 2 and 4 token tiles, four row groups (0: none; of two planes, four tiles' closed sums do not fit the registers)
+    SharedCu whole[3];      // of 1, 2 and 4 token tiles, four row groups (0: none; of two planes, four tiles' closed sums do not fit the registers)
 };
 template <class P> constexpr Costs costs();
 template <> constexpr Costs costs<KqQ3>() { return {{19, 24, 22, 31, 42}, {{51, 73}, {67, 90}, {98, 118}}}; }
@@ -590,14 +589,13 @@ template <class P>
 zhip_result launch_format(const Dispatch &d, const char *name, KqArgs a) {
     constexpr Costs c = costs<P>();
     const uint64_t cus = (uint64_t)d.dev->compute_units, groups = (a.n + 31u) / 32u, blocks = a.k / 256u;
-    auto per_cu = [&](uint32_t nt, uint32_t rw) { return ((groups + rw - 1u) / rw * ((a.rows + 32u * nt - 1u) / (32u * nt)) + cus - 1u) / cus; };
+    auto workgroups = [&](uint32_t nt, uint32_t rw) { return (groups + rw - 1u) / rw * ((a.rows + 32u * nt - 1u) / (32u * nt)); };
     constexpr uint32_t shapes[5][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {4, 2}};
     uint64_t least = ~0ull;
     int best = 0;
     for (int i = 0; i < 8; i++) {
         if (i >= 5 && c.whole[i - 5].lone == 0u) continue;
-        const uint64_t w = i < 5 ? per_cu(shapes[i][0], shapes[i][1]) : per_cu(1u << (i - 5), 4u);
-        const uint64_t cost = i < 5 ? c.parts[i] * w * (blocks + 3u) : (c.whole[i - 5].lone * (w & 1u) + c.whole[i - 5].pair * (w >> 1)) * (blocks + 2u);
+        const uint64_t cost = i < 5 ? c.parts[i] * ((workgroups(shapes[i][0], shapes[i][1]) + cus - 1u) / cus) * (blocks + 3u) : c.whole[i - 5].of(workgroups(1u << (i - 5), 4u), cus) * (blocks + 2u);
         if (cost < least) least = cost, best = i;
     }
     // Matrices too large for the dies' L2s, several token tiles: 24576 x 3072 and 28672 x 4096 at 256 ... 512 tokens 1 - 8 % faster

@@ -31,6 +31,7 @@
 // the tile height.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -293,14 +294,20 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const Q8Args &a) {
 
 template <class H>
 zhip_result launch_as(const Dispatch &d, const char *name, const Q8Args &a) {
-    // The largest tile that keeps more than half of the CUs busy: what a CU can have in flight
-    // from memory bounds its share of the loads, so a short step is faster in many small tiles
-    // than in few large ones. 128 tokens x 64 rows, 64 x 64 (every weight converted twice as
-    // often), 32 x 64, 32 x 32. A token's sums are the same bits in all of them.
-    const uint64_t cus = (uint64_t)d.dev->compute_units, columns = (a.n + 63u) / 64u;
-    if (a.rows > 64u && 2u * ((a.rows + 127u) / 128u) * columns > cus) return launch_tile<4, H, 2>(d, name, a);
-    if (a.rows > 32u && 2u * ((a.rows + 63u) / 64u) * columns > cus) return launch_tile<2, H, 2>(d, name, a);
-    if (2u * ((a.rows + 31u) / 32u) * columns > cus) return launch_tile<1, H, 2>(d, name, a);
+    // 128 tokens x 64 rows, 64 x 64 (every weight converted twice as often), 32 x 64, 32 x 32: the tile whose workgroups take
+    // least. What a CU can have in flight from memory bounds its share of the loads, so a short step is faster in many small
+    // tiles than in few large ones; the largest have a CU to themselves. Costs fitted to all four at 16 ... 512 tokens over ten matrices of
+    // up to 8064 rows, within 0.2 % of the fastest one's time in the mean (the largest tile that kept half of the CUs busy, as here
+    // before, lost 1.3 %, at the worst 160 x 5120 x 2560 18.8 -> 14.8 us, 320 x 6144 x 1024 18.7 -> 14.6, 80 x 5120 x 2560 14.3 -> 11.1).
+    // A token's sums are the same bits in all of them.
+    constexpr SharedCu costs[4] = {{50, 100}, {40, 62}, {29, 43}, {24, 34}};
+    const uint64_t cus = (uint64_t)d.dev->compute_units;
+    auto cost = [&](int i, uint32_t tokens, uint32_t rows) { return costs[i].of((uint64_t)((a.rows + tokens - 1u) / tokens) * ((a.n + rows - 1u) / rows), cus); };
+    const uint64_t c[4] = {cost(0, 128u, 64u), cost(1, 64u, 64u), cost(2, 32u, 64u), cost(3, 32u, 32u)};
+    const uint64_t least = std::min(std::min(c[0], c[1]), std::min(c[2], c[3]));
+    if (c[0] == least) return launch_tile<4, H, 2>(d, name, a);
+    if (c[1] == least) return launch_tile<2, H, 2>(d, name, a);
+    if (c[2] == least) return launch_tile<1, H, 2>(d, name, a);
     return launch_tile<1, H, 1>(d, name, a);
 }
 

@@ -268,12 +268,17 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const Q8Args &a) {
 
 template <class H>
 zhip_result launch_as(const Dispatch &d, const char *name, const Q8Args &a) {
-    // The largest tile that keeps more than half of the CUs busy: 128 tokens x 128 rows, 64
-    // tokens x 128 rows (every weight converted twice as often), 64 x 64. A token's sums are the
-    // same bits in all three.
-    const uint64_t cus = (uint64_t)d.dev->compute_units, columns = (a.n + 127u) / 128u;
-    if (a.rows > 64u && 2u * ((a.rows + 127u) / 128u) * columns > cus) return launch_tile<4, H, 4>(d, name, a);
-    if (a.rows > 64u && 2u * ((a.rows + 63u) / 64u) * columns > cus) return launch_tile<2, H, 4>(d, name, a);
+    // 128 tokens x 128 rows (a CU to themselves), 64 tokens x 128 rows (every weight converted twice as often), 64 x 64: the
+    // tile whose workgroups take least, costs fitted to all three at 16 ... 512 tokens over six matrices of 8192 x 2560 ... 28672 x 4096, within
+    // 0.02 % of the fastest one's time in the mean (the largest tile that kept half of the CUs busy, above 64 tokens, as here before, lost
+    // 1.5 %: 64 x 28672 x 4096 47.5 -> 38.5 us, 160 x 10240 x 5120 40.0 -> 33.6, 320 x 12288 x 2560 45.1 -> 39.2). A token's sums are
+    // the same bits in all three.
+    constexpr SharedCu costs[3] = {{50, 100}, {42, 82}, {33, 54}};
+    const uint64_t cus = (uint64_t)d.dev->compute_units;
+    auto cost = [&](int i, uint32_t tokens, uint32_t rows) { return costs[i].of((uint64_t)((a.rows + tokens - 1u) / tokens) * ((a.n + rows - 1u) / rows), cus); };
+    const uint64_t c[3] = {cost(0, 128u, 128u), cost(1, 64u, 128u), cost(2, 64u, 64u)};
+    if (c[0] <= c[1] && c[0] <= c[2]) return launch_tile<4, H, 4>(d, name, a);
+    if (c[1] <= c[2]) return launch_tile<2, H, 4>(d, name, a);
     return launch_tile<2, H, 2>(d, name, a);
 }
 

@@ -305,12 +305,14 @@ zhip_result launch_matmul_q8_i8(const Dispatch &d, const char *name, const uint8
     a.qx = qx; a.w = w; a.dx = dx; a.out = out;
     a.rows = rows; a.n = n; a.k = k; a.col0 = col0; a.out_stride = out_stride; a.accumulate = accumulate;
     a.row_bytes = row_bytes; a.qx_bytes = qx_bytes; a.w_bytes = w_bytes; a.dx_bytes = dx_bytes;
-    // 64-token tiles, two workgroups a CU, unless they leave half of the CUs idle: then 32-token
-    // tiles. us, 64 / 32: 512 x 1024 x 2048 (256 workgroups of 64 tokens) 7.9 / 8.3, 201 x 2560 x
-    // 4096 (256) 13.8 / 15.1, 512 x 1024 x 6144 17.1 / 21.2; 512 x 2048 x 1024 (128) 10.7 / 8.6,
-    // 64 x 4096 x 4096 (64) 18.0 / 13.8.
+    // The tile whose workgroups, two a CU, take least: costs fitted to both tiles' times at 16 ... 512 tokens over sixteen
+    // matrices of 1024 x 3072 ... 28672 x 4096, where the rule's tile is the faster one but for 0.01 % of the time in the mean (64-token tiles
+    // wherever they kept half of the CUs busy, as here before, 0.6 %). us, 64 / 32: 512 x 1024 x 2048 (256 workgroups of 64
+    // tokens) 7.9 / 8.3, 201 x 2560 x 4096 (256) 13.8 / 15.1, 512 x 28672 x 4096 203 / 287; 80 x 5120 x 2560 (160) 12.9 / 10.1, 160 x
+    // 3072 x 1024 (144) 7.2 / 5.6, 512 x 2048 x 1024 (128) 10.7 / 8.6, 64 x 4096 x 4096 (64) 18.0 / 13.8.
+    constexpr SharedCu tall{52, 85}, flat{40, 60};
     const uint64_t columns = (n + BN - 1) / BN, cus = (uint64_t)d.dev->compute_units;
-    if (rows > 32u && 2u * ((rows + 63u) / 64u) * columns > cus) return launch_tile<2>(d, name, a);
+    if (tall.of((rows + 63u) / 64u * columns, cus) < flat.of((rows + 31u) / 32u * columns, cus)) return launch_tile<2>(d, name, a);
     return launch_tile<1>(d, name, a);
 }
 
