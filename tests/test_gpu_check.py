@@ -1435,6 +1435,40 @@ def test_matmul_bf16_mfma_tilings(ctx, rows, n, k):
     c.set.select_prefill(c.rec, K.Prefill.scalar_f32)
 
 
+@pytest.mark.parametrize("n", [5130, 28700])
+@pytest.mark.parametrize("path", ["int8", "bf16_mfma", "fp16_single"])
+def test_matmul_q8_0_tiles_by_their_rounds_keep_token_bits(ctx, path, n):
+    """Q8_0 steps whose tile is chosen by the rounds its workgroups take: 33 ... 160 tokens of matrices
+    that fill the CUs once and several times over (up to 64 tokens of 28700 rows in tiles of 128 rows),
+    against 300 tokens in the largest tiles, the same bits a token; those against float64
+    over the rounded operands, 1e-5."""
+    c, rows, k, t = ctx, 300, 256, TensorType.q8_0
+    x = c.random(rows * k, 1).reshape(rows, k)
+    raw, values = quant_rows(c, t, n, k)
+    wa = c.gpu_weights(t, raw, k)
+    if path == "int8":
+        xs = oracle.round_like_llama(ORACLE_TYPE[t], x)
+    else:
+        c.set.select_prefill(c.rec, K.Prefill[path])
+        narrow = synth.bf16_round if path == "bf16_mfma" else (lambda v: v.astype(np.float16).astype(np.float32))
+        xs, values = narrow(x), narrow(values)
+
+    def run(first, count):
+        out = c.upload(np.full((count, n), np.nan, np.float32))
+        if path == "int8":
+            launch_int8(c, t, quantize_x(c, t, c.upload(x[first : first + count]), count, k), wa, out, count, n, k, 0, None)
+        else:
+            c.launcher().launch(Kernel.matmul_q8_0_float, P.MatmulQuant(rows=count, n=n, k=k, col0=0, out_stride=n, accumulate=0, k_slice=k),
+                                [c.upload(x[first : first + count]), wa, out], (K.div_ceil(n, 64), K.div_ceil(count, 16), 1))
+        return c.read(out).reshape(count, n)
+
+    got = run(0, rows)
+    assert rel_err(got, xs.astype(np.float64) @ values.astype(np.float64).T) <= 1e-5
+    for first, count in ((0, 33), (20, 64), (84, 80), (140, 160)):
+        assert got[first : first + count].tobytes() == run(first, count).tobytes(), (first, count)
+    c.set.select_prefill(c.rec, K.Prefill.scalar_f32)
+
+
 @pytest.mark.parametrize("n", [2830, 8230])
 @pytest.mark.parametrize("rung", ["bf16_mfma", "fp16_single"])
 def test_matmul_q8_0_float_bf16_whole_steps_keep_token_bits(ctx, rung, n):
