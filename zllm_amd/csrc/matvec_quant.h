@@ -163,7 +163,7 @@ constexpr uint32_t kAny = 0xffffffffu / 1000u;
 struct KQ8 {
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
-    static constexpr bool DEFER = false;
+    static constexpr bool KEEPS = false;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 4;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -238,7 +238,7 @@ struct KQ3 {
     static constexpr uint32_t BLOCK_BYTES = 128;
     static constexpr int NSUM = 4;
     static constexpr int STAGE2 = 0, STAGE4 = 2;  // tokens whose inputs are loaded at once, of two and of three or four
-    static constexpr bool DEFER = true;
+    static constexpr bool KEEPS = true;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 3;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -328,7 +328,7 @@ struct KQ4 {
     static constexpr uint32_t BLOCK_BYTES = 144;
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
-    static constexpr bool DEFER = true;
+    static constexpr bool KEEPS = true;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 2;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -413,7 +413,7 @@ struct KQ5 {
     static constexpr uint32_t BLOCK_BYTES = 176;
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 0;  // (rows of up to 4096 weights always have two tokens' inputs in registers)
-    static constexpr bool DEFER = true;
+    static constexpr bool KEEPS = true;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     // The fifth bits leave the general kernel too few registers for three or more tokens' sums: rows
     // of up to 64 tasks always run two tokens a workgroup (four tokens, general / that: 9728 x 2560 21.7 /
@@ -509,7 +509,7 @@ struct KQ6 {
     static constexpr uint32_t BLOCK_BYTES = 224;
     static constexpr int NSUM = 4;
     static constexpr int STAGE2 = 2, STAGE4 = 1;  // tokens whose inputs are loaded at once
-    static constexpr bool DEFER = false;
+    static constexpr bool KEEPS = false;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 4;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -892,12 +892,22 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
 // multiply turns into a sum of zero; no address arithmetic, clamp or branch per lane is left.
 // The staging of the inputs, a task's dot product and the lanes' reduction are the code of the
 // kernel above, so the results are its bits.
+// A segment's sum, which segment_sum leaves in its last lane (and in every lane of a segment of sixteen), in all of its lanes.
+template <int SEG_LOG2>
+__device__ __forceinline__ float segment_total(float v, uint32_t lane) {
+    if (SEG_LOG2 == 4) return v;
+    const float last = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
+    if (SEG_LOG2 == 6) return last;
+    const float first = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 31));
+    return lane < 32u ? first : last;
+}
+
 // Passes whose loads are in flight ahead of the one multiplied. Measured on 14336 x 4096 Q4_K
 // (7.9 us with one): two or three passes ahead 8.6 / 9.8 us, and no better with fewer workgroups;
 // two passes asked for before the inputs are staged (instead of one) 8.7 us; the first pass
 // asked for only once the inputs have arrived 8.0 us.
 constexpr int kRowDepth = 1;
-template <class P, int MT, bool PAIR, bool TURNS, int SEG_LOG2>
+template <class P, int MT, bool PAIR, bool TURNS, int SEG_LOG2, bool KEEP>
 __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
     q.t0 += MT * blockIdx.y;  // (a step of more tokens: workgroups of their own for every MT of them)
     const bool full = MT == 1 || q.t0 + MT <= q.a.m;  // (of two tokens the second may be absent: it runs as the first again and is not stored)
@@ -1025,18 +1035,17 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
     const bool accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
     auto out_at = [&](int t, uint32_t j) { return (size_t)(q.t0 + t) * a.out_stride + a.col0 + j; };
 
-    // Whole-wave rows (SEG = 64) of a format with DEFER keep their finished sums in the lane of
-    // their number (the gate's and the up row's apart) and are finished and stored together,
-    // 64 outputs at a time: stores between the loads of the stream cost more than their bytes,
-    // and the activation runs once for 64 outputs instead of once a row.
-    constexpr bool kKeep = P::DEFER && SEG == 64u;
+    // With KEEP a pass's finished sums are kept in the rows' lanes of its number
+    // (the gate's and the up row's apart), and SEG passes' are finished and stored together:
+    // stores between the loads of the stream cost more than their bytes,
+    // and the activation runs once for 64 outputs instead of once a row. See run_row_seg.
     float kept0[MT], kept1[MT];
 #pragma unroll
     for (int t = 0; t < MT; t++) kept0[t] = kept1[t] = 0.f;
     uint32_t nkept = 0, kept_first = gwave;
     auto flush_kept = [&]() __attribute__((always_inline)) {
-        const uint32_t j = kept_first + lane * nwaves;
-        if (lane < nkept && j < a.rows) {
+        const uint32_t j = (kept_first + tsub * nwaves) * RPI + rsub;
+        if (tsub < nkept && j < a.rows) {
 #pragma unroll
             for (int t = 0; t < MT; t++) {
                 if (t > 0 && !full) break;
@@ -1066,17 +1075,17 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
     auto keep = [&](const float (&s)[MT], float (&kept)[MT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            const float total = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[t]), 63));
-            kept[t] = lane == nkept ? total : kept[t];
+            const float total = segment_total<SEG_LOG2>(s[t], lane);
+            kept[t] = tsub == nkept ? total : kept[t];
         }
     };
     // The sums of pass u's rows (s0) and, with PAIR, of the up rows (s1): kept, or stored.
     auto finish = [&](uint32_t u, const float (&s0)[MT], const float (&s1)[MT]) __attribute__((always_inline)) {
-        if (kKeep) {
+        if (KEEP) {
             keep(s0, kept0);
             if (PAIR) keep(s1, kept1);
             nkept++;
-            if (nkept == 64u) flush_kept();
+            if (nkept == SEG) flush_kept();
         } else {
             const uint32_t j = u * RPI + rsub;
             if (tsub == SEG - 1u && j < a.rows) {
@@ -1114,7 +1123,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
             reduce(s1);
             finish(u, s0, s1);
         }
-        if (kKeep) flush_kept();
+        if (KEEP) flush_kept();
         return;
     }
     // kRowDepth passes' loads stay in flight ahead of the one multiplied; a trip of
@@ -1133,7 +1142,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
         }
         if (done) break;
     }
-    if (kKeep) flush_kept();
+    if (KEEP) flush_kept();
 }
 
 // Steps of several tokens over rows too long for the tokens' inputs to fit the workgroup's LDS
@@ -1567,12 +1576,28 @@ static zhip_result run_slices(const Dispatch &d, const KArgs &q, uint32_t lds, u
 // Q3_K 13.1 / 9.3, and 2 x 14336 x 4096: Q4_K 20.2 / 20.4, Q3_K 21.7 / 21.7. One token
 // gains nothing from it (2 x 14336 x 4096 Q4_K 15.6 / 16.3, Q5_K 19.6 / 19.8).
 template <class P, int MT, bool PAIR, int SEG_LOG2> constexpr bool row_turns() { return PAIR && MT == 2 && !(P::PAIR2 && SEG_LOG2 == 6); }
-template <class P, int MT, bool PAIR, int SEG_LOG2>
-static zhip_result run_row_seg(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
-    constexpr auto kernel = matvec_quant_row_kernel<P, MT, PAIR, row_turns<P, MT, PAIR, SEG_LOG2>(), SEG_LOG2>;
+template <class P, int MT, bool PAIR, int SEG_LOG2, bool KEEP>
+static zhip_result run_row_kernel(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
+    constexpr auto kernel = matvec_quant_row_kernel<P, MT, PAIR, row_turns<P, MT, PAIR, SEG_LOG2>(), SEG_LOG2, KEEP>;
     if (lds > 65536u && !lds_opt_in<kernel, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
     hipLaunchKernelGGL(kernel, dim3(blocks, (q.mt + MT - 1u) / MT), dim3(256), lds, d.stream, q);
     return check_launch(d, P::name());
+}
+// Whether a wave's sums wait for one store in SEG passes (the stores go between the loads of the stream otherwise). A whole-wave
+// row's do wherever a wave has a second pass, and in the formats with KEEPS always, as it costs nothing there; several rows a pass from the
+// fourth pass on, and not a pair's (2 x 8192 x 2048 at two passes: level). us, stored pass by pass / kept: Q6_K 128256 x 4096 at
+// one / two tokens 80.3 91.8 / 77.5 80.2, 50257 x 2560 at two 36.2 / 30.9, 4096 x 4096 at four 10.4 / 8.7, 2 x 14336 x 4096 at two
+// 22.8 / 20.9; Q8_0 4096 x 4096 at one / two / four 6.0 7.3 10.0 / 5.6 6.6 8.0, 2 x 9728 x 2560 at two 15.1 / 13.6; four rows a pass,
+// 151936 x 1024, Q8_0 at eight 77 / 66, Q4_K at two 25.0 / 21.6, Q5_K at two / eight 29.2 86 / 25.2 73; two, 128256 x 2048 Q4_K at two 40.4 / 33.7; one token
+// over such rows 0 - 6 % (Q8_0 32000 x 2048 13.2 / 13.5). Launches of one pass a wave lose 2 - 5 % by it, a choice at run time costs all of them 3 %.
+template <class P, int MT, bool PAIR, int SEG_LOG2>
+static zhip_result run_row_seg(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
+    constexpr uint32_t RPI = 64u >> SEG_LOG2;
+    const uint32_t units = (q.a.rows + RPI - 1u) / RPI, nwaves = 4u * blocks;
+    if constexpr (SEG_LOG2 == 6 && P::KEEPS) return run_row_kernel<P, MT, PAIR, SEG_LOG2, true>(d, q, lds, blocks);
+    if constexpr (SEG_LOG2 == 6 || !PAIR)
+        if (units > (SEG_LOG2 == 6 ? 1u : 3u) * nwaves) return run_row_kernel<P, MT, PAIR, SEG_LOG2, true>(d, q, lds, blocks);
+    if constexpr (!(SEG_LOG2 == 6 && P::KEEPS)) return run_row_kernel<P, MT, PAIR, SEG_LOG2, false>(d, q, lds, blocks);
 }
 template <class P, int MT, bool PAIR>
 static zhip_result run_row(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
