@@ -224,6 +224,34 @@ def test_matvec_bf16_several_tokens_keep_token_bits(ctx, ctx_wide, wide, half):
     assert np.array_equal(run([5], 404, 4096)[0], whole[5, 404:])
 
 
+@pytest.mark.parametrize("half", HALVES)
+@pytest.mark.parametrize("k,n,pair", [(64, 135005, False), (1000, 12301, False), (1536, 7001, False), (2048, 6145, False), (512, 131080, True), (2048, 7001, True)])
+def test_matvec_half_rows_kept_for_one_store(ctx, half, k, n, pair):
+    """Outputs that wait for one store in several passes (32 of two rows, 64 of one): a matrix that repeats 1000
+    rows gives the bits that the 1000 rows alone give, which are stored pass by pass; with a
+    column offset, a padded stride, added to the outputs or not, one, two and five tokens."""
+    c, base, col0, stride = ctx, 1000, 3, n + 5
+    x = c.random(5 * k, 1).reshape(5, k)
+    bits, _ = random_half(c, (2 if pair else 1) * base * k, 1, half)
+    rows = np.asarray(bits).reshape(-1, base, k)
+    small, tall = c.upload(rows), c.upload(np.ascontiguousarray(rows[:, np.arange(n) % base]))
+    init, columns = c.random(5 * base, 2).reshape(5, base), np.arange(n) % base
+
+    def run(weights, count, outs, start, first, width, accumulate):
+        out = c.upload(start)
+        c.launcher().launch(Kernel["matvec_" + half], P.MatvecBf16(n=outs, k=k, col0=first, out_stride=width, eps=1e-6, accumulate=accumulate, silu_pair=pair, half=outs if pair else 0),
+                            [c.upload(x[:count]), weights, out, weights], (K.div_ceil(outs, K.matvec_rows), count, 1))
+        return c.read(out).reshape(count, width)
+
+    for count, accumulate in ((1, False), (2, not pair), (5, not pair), (5, False)):
+        want = run(small, count, base, init[:count], 0, base, accumulate)
+        start = np.full((count, stride), 7.0, np.float32)
+        start[:, col0 : col0 + n] = init[:count, columns]
+        got = run(tall, count, n, start, col0, stride, accumulate)
+        assert np.array_equal(got[:, col0 : col0 + n].view(np.uint32), want[:, columns].view(np.uint32)), (count, accumulate)
+        assert (got[:, :col0] == 7.0).all() and (got[:, col0 + n :] == 7.0).all()
+
+
 # Steps of one to eight tokens over short rows keep the inputs in registers; more than eight tokens
 # run in the general kernel, which adds in the same order: each token has its bits there.
 @pytest.mark.parametrize("k,n", [

@@ -41,8 +41,9 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// ROWS: weight rows a wave multiplies in a pass (with PAIR half of them gate rows, half up rows).
-template <class D, int MT, int ITERS, bool PAIR, int ROWS>
+// ROWS: weight rows a wave multiplies in a pass (with PAIR half of them gate rows, half up rows). KEEP: the
+// outputs of 64 / OUTS passes wait in the lanes for one store; see launch_iters.
+template <class D, int MT, int ITERS, bool PAIR, int ROWS, bool KEEP>
 __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
     extern __shared__ float4 xs4[];
     __shared__ float red[4 * MT];
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
                 p.q[r][it] = __builtin_amdgcn_raw_buffer_load_b128(PAIR && r >= OUTS ? up : gate, (it == ITERS - 1 ? last_at : at) + (uint32_t)(PAIR && r >= OUTS ? r - OUTS : r) * a.row_bytes + 1024u * it, 0, 0);
         const uint32_t j = u * OUTS + lane;
 #pragma unroll
-        for (int t = 0; t < MT; t++) p.before[t] = accumulate && (uint32_t)t < a.m && lane < (uint32_t)OUTS && j < a.rows ? a.out[(size_t)t * a.out_stride + a.col0 + j] : 0.f;
+        for (int t = 0; t < MT; t++) p.before[t] = !KEEP && accumulate && (uint32_t)t < a.m && lane < (uint32_t)OUTS && j < a.rows ? a.out[(size_t)t * a.out_stride + a.col0 + j] : 0.f;
         __builtin_amdgcn_sched_barrier(0);  // (the loads stay ahead of the multiply that follows them in the source)
     };
     Pass buf[2];
@@ -157,10 +158,28 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
             }
         }
 
-    auto multiply = [&](uint32_t u, const Pass &p) __attribute__((always_inline)) {
-        float v0[MT], v1[MT];  // lane o < OUTS: its output's (gate) sum, and with PAIR the up row's
+    // Lane o < OUTS: its output's (gate) sum, and with PAIR the up row's; KEEP: those of the pass numbered turn are lanes turn OUTS + o.
+    float v0[MT], v1[MT];
+    uint32_t turn = 0, kept_first = first;
 #pragma unroll
-        for (int t = 0; t < MT; t++) v0[t] = v1[t] = 0.f;
+    for (int t = 0; t < MT; t++) v0[t] = v1[t] = 0.f;
+    auto flush_kept = [&]() __attribute__((always_inline)) {
+        const uint32_t j = (kept_first + lane / OUTS * nwaves) * OUTS + lane % OUTS;
+        if (lane < turn * OUTS && j < a.rows) {
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                if ((uint32_t)t >= a.m) break;
+                float v = PAIR ? silu_f(v0[t]) * v1[t] : v0[t];
+                float *o = a.out + (size_t)t * a.out_stride + a.col0 + j;
+                if (accumulate) v += *o;
+                *o = v;
+            }
+        }
+        kept_first += turn * nwaves;
+        turn = 0;
+    };
+    auto multiply = [&](uint32_t u, const Pass &p) __attribute__((always_inline)) {
+        const uint32_t slot = KEEP ? turn * OUTS : 0u;
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
             float acc[MT];
@@ -182,9 +201,13 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
 #pragma unroll
             for (int t = 0; t < MT; t++) {
                 const float sum = wave_sum(acc[t]);
-                if (PAIR && r >= outs) v1[t] = lane == (uint32_t)(r - outs) ? sum : v1[t];
-                else v0[t] = lane == (uint32_t)r ? sum : v0[t];
+                if (PAIR && r >= outs) v1[t] = lane == slot + (uint32_t)(r - outs) ? sum : v1[t];
+                else v0[t] = lane == slot + (uint32_t)r ? sum : v0[t];
             }
+        }
+        if (KEEP) {
+            if (++turn == 64u / OUTS) flush_kept();
+            return;
         }
         const uint32_t j = u * OUTS + lane;
         if (lane < (uint32_t)OUTS && j < a.rows) {
@@ -205,6 +228,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
         multiply(u, buf[1]);
         if ((u += nwaves) >= passes) break;
     }
+    if (KEEP) flush_kept();
 }
 
 template <class D, int MT, int ITERS>
@@ -222,8 +246,20 @@ zhip_result launch_iters(const Dispatch &d, const MvArgs &a) {
     if (groups > 1u) blocks = want < cap ? (want + 7u) & ~7u : cap & ~7u;
     const dim3 grid(blocks ? blocks : 1u, groups);
     const uint32_t lds = MT * a.k * 4u;
-    if (pair) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2>), grid, dim3(256), lds, d.stream, a);
-    else hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS>), grid, dim3(256), lds, d.stream, a);
+    // Stores between the loads of the stream cost more than their bytes: from the fourth pass of a wave on (a pair's from the sixth: 2 x 4096
+    // x 2048 f16 at four tokens, four passes, 10.0 / 10.5 us, at eight, eight, 14.2 / 13.4) they wait in the lanes. us, stored pass by pass / kept, bf16: 151936 x 1024 at four / eight tokens 61.5 85.6 / 55.2 76.3, 50257 x 2560 61 88 / 57 76, 16384 x
+    // 2048 15.4 23.1 / 14.0 20.2, 2 x 8192 x 2048 15.8 22.6 / 14.8 21.4, at one token level (151936 x 1024 52.1 / 51.9). Not a pair's
+    // of longer rows: 2 x 9728 x 2560 at eight tokens 36.1 / 32.6, but at four 27.2 / 30.5.
+    constexpr bool PAIR_KEEPS = ITERS <= 4;
+    const bool keep = (a.rows + outs - 1u) / outs > (pair ? 20u : 12u) * blocks;
+    if constexpr (PAIR_KEEPS)
+        if (pair && keep) {
+            hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2, true>), grid, dim3(256), lds, d.stream, a);
+            return check_launch(d, D::name());
+        }
+    if (pair) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2, false>), grid, dim3(256), lds, d.stream, a);
+    else if (keep) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS, true>), grid, dim3(256), lds, d.stream, a);
+    else hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS, false>), grid, dim3(256), lds, d.stream, a);
     return check_launch(d, D::name());
 }
 
