@@ -388,6 +388,28 @@ def test_matvec_bf16_several_tokens_long_rows(ctx_wide, half, k, mb):
             assert np.array_equal(run([t], norm, accumulate)[0][rows], got[t][rows])
 
 
+@pytest.mark.parametrize("k", [6464, 6656])
+@pytest.mark.parametrize("over", [0, 1])
+def test_matvec_several_tokens_of_4_gib(ctx_wide, k, over):
+    """The largest matrix whose byte offsets, up to a tile past its last row, have 32 bits, and one row more, which
+    is the general kernel's: rows of whole 512s and of other lines, within 1e-5 of float64."""
+    c, base, m = ctx_wide, 1009, 2
+    n = -(-0xFFFFFFF0 // (2 * k)) - 65 + over
+    x = c.random(m * k, 1).reshape(m, k)
+    bits, values = random_half(c, base * k, k ** -0.5, "f16")
+    w, have = c.output(n * k // 2), base
+    c.rec.write_buffer(w.buffer, 0, bits.view(np.uint8))
+    while have < n:  # the base rows over and over
+        more = min(have, n - have)
+        c.rec.copy_buffer(w.buffer, 0, w.buffer, 2 * k * have, 2 * k * more)
+        have += more
+    out = c.output(m * n)
+    p = P.MatvecBf16(n=n, k=k, col0=0, out_stride=n, eps=1e-6)
+    c.launcher().launch(Kernel.matvec_f16, p, [c.upload(x), w, out, w], (K.div_ceil(n, K.matvec_rows), m, 1))
+    want = x.astype(np.float64) @ values.reshape(base, k).astype(np.float64).T
+    assert rel_err(c.read(out).reshape(m, n), want[:, np.arange(n) % base]) <= 1e-5
+
+
 @pytest.mark.parametrize("k", [1024, 1536, 2048, 2560, 3072, 3584, 4096])
 @pytest.mark.parametrize("half", HALVES)
 def test_matvec_bf16_several_tokens_norm_is_every_kernels(ctx, ctx_wide, half, k):

@@ -515,8 +515,10 @@ zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
 // wave, and rows of whole lines where the workgroups split the tokens of long ones themselves (`own` below); a gate / up pair only over rows that one workgroup takes whole.
 // (rows of more than 4096 weights are taken in stretches of columns: equal ones in one launch, workgroups sharing a
 // tile, with a launch for their sums; unequal ones behind the RMSNorm prologue a launch each; up to 16384: the split launch stages a token in 64 KB of LDS)
+// (32-bit byte offsets up to a tile past the last row: larger matrices are the general kernel's)
 bool matvec_bf16_mfma_stream_accepts(const MvArgs &a) {
-    if ((a.flags & FLAG_SILU_PAIR) && (a.k > 4096u || ((uint64_t)a.half + a.rows + 64u) * a.row_bytes >= 0xfffffff0ull)) return false;
+    const bool pair = a.flags & FLAG_SILU_PAIR;
+    if ((pair && a.k > 4096u) || ((pair ? (uint64_t)a.half : 0ull) + a.rows + 64u) * a.row_bytes >= 0xfffffff0ull) return false;
     return a.m >= 1 && a.k >= 1024u && a.k <= 16384u && (a.k % 512u == 0 || (a.k % 64u == 0 && a.k > 4096u && !(a.flags & FLAG_NORM))) && a.act_div == 0.f && a.rows >= 1 &&
            a.xr % 4u == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15u) == 0 && a.row_bytes == 2u * a.k;
 }
@@ -537,10 +539,8 @@ static zhip_result launch_for_k(const Dispatch &d, const StreamArgs &q, dim3 gri
 // f16: the weights are f16 (matvec_f16), bf16 otherwise.
 zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, uint64_t w_bytes, bool f16) {
     const char *name = f16 ? "matvec_f16" : "matvec_bf16";
-    // 32-bit byte offsets, a tile past the last row.
     const bool pair = a.flags & FLAG_SILU_PAIR;
     const uint64_t used = ((uint64_t)a.rows + (pair ? a.half : 0u)) * a.row_bytes;
-    if (used + 64ull * a.row_bytes >= 0xfffffff0ull) return fail(d, ZHIP_E_BAD_COMMAND, "%s: weights of 4 GiB or more", name);
     const uint32_t cus = (uint32_t)d.dev->compute_units;
     const uint32_t units = (a.rows + 7u) / 8u;
     const uint32_t groups = units < cus ? units : cus;
