@@ -23,21 +23,17 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
-#include <atomic>
-#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "common.h"
+#include "handover.h"
 
 #ifndef ZHIP_SOURCE_HASH
 #define ZHIP_SOURCE_HASH "dev"
@@ -227,92 +223,6 @@ constexpr uint32_t kFlaggedReads = 16, kMostPieces = 16, kFlags = kFlaggedReads 
 struct Signals {
     uint64_t begin, end;
     uint32_t flags[kFlags];
-};
-
-// A read on its way from its staging, which the GPU fills piece by piece, to its destination.
-struct Handover {
-    uint8_t *dst;
-    const uint8_t *src;
-    uint64_t size, piece;
-    const uint32_t *flags;
-    uint32_t ticket;
-};
-
-inline void pause_cpu() {
-#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
-    __builtin_ia32_pause();
-#endif
-}
-
-// A second thread for long reads: one copies 28 GB/s from pinned memory, the bus brings 54. Pieces
-// go to whichever of the two is free, in order; the thread sleeps but for the time between start()
-// and finish(), and looks at nothing of the context.
-class HandoverThread {
-  public:
-    // (no thread to be had: the caller copies alone)
-    void start(const Handover &job) {
-        std::lock_guard<std::mutex> hold(lock_);
-        job_ = job;
-        next_.store(0, std::memory_order_relaxed);
-        open_ = true;
-        if (!thread_.joinable()) {
-            try {
-                thread_ = std::thread([this] { run(); });
-            } catch (const std::system_error &) {
-            }
-        }
-        wake_.notify_one();
-    }
-    // The next piece that nobody has taken.
-    uint64_t take() { return next_.fetch_add(1, std::memory_order_relaxed); }
-    // When this returns the thread copies nothing any more. `failed`: what the GPU has not
-    // brought will not come.
-    void finish(bool failed) {
-        std::unique_lock<std::mutex> hold(lock_);
-        open_ = false;
-        give_up_.store(failed, std::memory_order_relaxed);
-        idle_.wait(hold, [this] { return !busy_; });
-        give_up_.store(false, std::memory_order_relaxed);
-    }
-    ~HandoverThread() {
-        {
-            std::lock_guard<std::mutex> hold(lock_);
-            stop_ = true;
-        }
-        wake_.notify_one();
-        if (thread_.joinable()) thread_.join();
-    }
-
-  private:
-    void run() {
-        std::unique_lock<std::mutex> hold(lock_);
-        for (;;) {
-            wake_.wait(hold, [this] { return stop_ || open_; });
-            if (stop_) return;
-            const Handover job = job_;
-            busy_ = true;
-            hold.unlock();
-            bool more = true;
-            while (more) {
-                const uint64_t p = take();
-                if (p * job.piece >= job.size) break;
-                while (__atomic_load_n(job.flags + p, __ATOMIC_ACQUIRE) != job.ticket && !give_up_.load(std::memory_order_relaxed)) pause_cpu();
-                more = !give_up_.load(std::memory_order_relaxed);
-                if (more) memcpy(job.dst + p * job.piece, job.src + p * job.piece, std::min(job.piece, job.size - p * job.piece));
-            }
-            hold.lock();
-            busy_ = false;
-            open_ = false;
-            idle_.notify_one();
-        }
-    }
-    std::mutex lock_;
-    std::condition_variable wake_, idle_;
-    std::thread thread_;
-    Handover job_{};
-    std::atomic<uint64_t> next_{0};
-    std::atomic<bool> give_up_{false};
-    bool open_ = false, busy_ = false, stop_ = false;
 };
 
 }  // namespace zhip
@@ -744,13 +654,13 @@ zhip_result hand_over(zhip_context *c, const Read &rd, uint32_t first_flag) {
     const bool shared = rd.size >= kSharedRead;
     if (shared) c->handover.start(job);
     zhip_result result = ZHIP_OK;
-    for (uint64_t next = 0; result == ZHIP_OK;) {
-        const uint64_t p = shared ? c->handover.take() : next++, at = p * job.piece;
-        if (at >= job.size) break;
+    for (uint32_t next = 0; result == ZHIP_OK;) {
+        const uint32_t p = shared ? c->handover.take() : next++;
+        if (p >= job.pieces()) break;
         result = wait_flag(c, flags + p);
-        if (result == ZHIP_OK) memcpy(job.dst + at, job.src + at, std::min(job.piece, job.size - at));
+        if (result == ZHIP_OK) job.copy(p);
     }
-    if (shared) c->handover.finish(result != ZHIP_OK);
+    if (shared) c->handover.finish();
     return result;
 }
 
