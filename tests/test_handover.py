@@ -20,9 +20,11 @@ static void check(bool ok, const char *what) {
 
 struct Job {
     std::vector<uint8_t> src, dst;
-    std::vector<uint32_t> flags;
+    std::vector<uint64_t> flags;
     Handover h;
-    Job(uint64_t size, uint64_t piece, uint32_t ticket) : src(size), dst(size, 0xee), flags((size + piece - 1) / piece, ticket - 1) {
+    // (what the flags hold from before differs from the ticket in the upper half alone)
+    Job(uint64_t size, uint64_t piece, uint64_t ticket) : src(size), dst(size, 0xee), flags((size + piece - 1) / piece, ticket) {
+        ticket += 1ull << 32;
         h = Handover{dst.data(), src.data(), size, piece, flags.data(), ticket};
     }
     // Piece p as the GPU leaves it.

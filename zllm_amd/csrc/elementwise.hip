@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256) void copy_kernel(T *dst, const T *src, uint64_
 // submit 5 us (the first one keeps the next kernel from starting), pieces as copies of the runtime's
 // with an event each up to 2 us of idle bus a piece.
 template <class T>
-__global__ __launch_bounds__(256) void read_kernel(T *dst, const T *src, uint64_t n, uint64_t piece, uint32_t *arrived, uint32_t *flags, uint32_t ticket, uint64_t *stamp) {
+__global__ __launch_bounds__(256) void read_kernel(T *dst, const T *src, uint64_t n, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *stamp) {
     for (uint64_t at = 0, p = 0; at < n; at += piece, p++) {
         const uint64_t end = at + piece < n ? at + piece : n;
         for (uint64_t i = at + (uint64_t)blockIdx.x * 256u + threadIdx.x; i < end; i += (uint64_t)gridDim.x * 256u) dst[i] = src[i];
@@ -383,7 +383,7 @@ zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t
 }
 
 // `piece` is a multiple of 16 bytes; one flag and one counter a piece.
-zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint32_t *flags, uint32_t ticket, uint64_t *stamp) {
+zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *stamp) {
     const bool wide = wide_copy(dst, src, bytes);
     const uint64_t unit = wide ? 16u : 4u, n = bytes / unit;
     const dim3 grid(blocks_for(std::min(n, piece / unit), 256, 128));

@@ -23,8 +23,8 @@ struct Handover {
     uint8_t *dst;
     const uint8_t *src;
     uint64_t size, piece;
-    const uint32_t *flags;
-    uint32_t ticket;
+    const uint64_t *flags;
+    uint64_t ticket;  // (of 64 bits: a process that submits for days would come round to one that a flag still holds)
     uint64_t pieces() const { return (size + piece - 1u) / piece; }
     bool arrived(uint64_t p) const { return __atomic_load_n(flags + p, __ATOMIC_ACQUIRE) == ticket; }
     void copy(uint64_t p) const { memcpy(dst + p * piece, src + p * piece, std::min(piece, size - p * piece)); }

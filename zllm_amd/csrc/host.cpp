@@ -222,7 +222,7 @@ constexpr uint32_t kFlaggedReads = 16, kMostPieces = 16, kFlags = kFlaggedReads 
 // Pinned, written by the GPU: its clock behind a submit's last staged write and behind its last read, a flag a piece.
 struct Signals {
     uint64_t begin, end;
-    uint32_t flags[kFlags];
+    uint64_t flags[kFlags];
 };
 
 }  // namespace zhip
@@ -276,7 +276,7 @@ struct zhip_context {
     uint64_t download_size = 0;
     Signals *signals = nullptr;   // pinned
     uint32_t *arrived = nullptr;  // on the device: kFlags counters of read_kernel's workgroups
-    uint32_t ticket = 0;          // of the last submit that waited for flags
+    uint64_t ticket = 0;          // of the last submit that waited for flags
     double tick_ns = 10.0;        // of the GPU's clock
     HandoverThread handover;
 
@@ -634,7 +634,7 @@ bool ends_in_flagged_reads(const zhip_context *c) {
 uint64_t piece_bytes(uint64_t size) { return std::max<uint64_t>(kReadPiece, (size / kMostPieces + 4096u) & ~4095ull); }
 
 // Waits for a piece. The stream is asked now and then, for what may keep a flag from being set.
-zhip_result wait_flag(zhip_context *c, const uint32_t *flag) {
+zhip_result wait_flag(zhip_context *c, const uint64_t *flag) {
     for (uint32_t spins = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != c->ticket; spins++) {
         pause_cpu();
         if (spins % 8192u != 0) continue;
@@ -648,7 +648,7 @@ zhip_result wait_flag(zhip_context *c, const uint32_t *flag) {
 
 // A read, from its staging to its destination, piece by piece as they arrive.
 zhip_result hand_over(zhip_context *c, const Read &rd, uint32_t first_flag) {
-    const uint32_t *flags = c->signals->flags + first_flag;
+    const uint64_t *flags = c->signals->flags + first_flag;
     const Handover job{rd.dst, c->download + rd.staging_offset, rd.size, piece_bytes(rd.size), flags, c->ticket};
     if (zhip_result r = wait_flag(c, flags)) return r;
     const bool shared = rd.size >= kSharedRead;
