@@ -45,8 +45,8 @@ def test_new_buffers_read_as_zero_and_round_trip(ctx):
 
 @pytest.mark.parametrize("words", [1, 3, 4, 16383, 16384, 16385, 131072, 131073, 262144, 2300000])
 def test_transfers_of_every_length(ctx, words):
-    """Short writes and reads go through pinned memory and long ones otherwise (64 KB), the longest
-    reads in pieces (512 KB; a sixteenth above 8 MB): every length and alignment arrives whole,
+    """Short writes go through pinned memory and long ones otherwise (64 KB), reads in pieces (128 KB; a
+    sixteenth above 2 MB): every length and alignment arrives whole,
     overlapping writes land in their order, and a batch without a submit has landed when it returns."""
     c = ctx
     old, new = c.random(words, 1), c.random(words, 1)
@@ -71,8 +71,8 @@ def test_transfers_of_every_length(ctx, words):
 
 
 def test_reads_into_one_destination_land_in_their_order(ctx):
-    """A long read arrives in pieces while others wait for the whole submit: where destinations
-    overlap, the read recorded last is the one that stays."""
+    """Reads are handed over in their order: where destinations
+    overlap, the one recorded last is the one that stays."""
     c = ctx
     words = 300000
     a, b = c.random(words, 1), c.random(words, 1)
@@ -241,8 +241,8 @@ def test_kernel_ranges_are_checked_before_launch(ctx):
 @pytest.mark.parametrize("size", [4, 131072 - 4, 131072, 131072 + 4, 786432 + 4, 2097152 + 4096 + 12])
 @pytest.mark.parametrize("reads", [1, 3, 17])
 def test_reads_arrive_whole_at_every_size(ctx, size, reads):
-    """A submit's reads, of whole buffers and from odd words on, over and over: in pieces behind flags,
-    or (more than sixteen reads) behind the stream's end."""
+    """A submit's reads, of whole buffers and from odd words on, over and over: sixteen at most in pieces behind flags,
+    others behind the stream's end."""
     c = ctx
     rng = np.random.default_rng(size + reads)
     data = rng.integers(0, 255, size + 16, dtype=np.uint8)
@@ -264,6 +264,46 @@ def test_reads_arrive_whole_at_every_size(ctx, size, reads):
         for i, o in enumerate(out):
             assert np.array_equal(o, data[4 * (i % 5) :][:size]), (turn, i)
         assert 0 < c.host.last_submit()[0] < 1e9
+
+
+@pytest.mark.parametrize("size", [4, 65536, 131072 + 4, 2097152 + 12])
+@pytest.mark.parametrize("reads,profile", [(1, False), (3, True), (16, False), (18, False)])
+@pytest.mark.parametrize("last", ["clear", "copy", "empty read"])
+def test_reads_ahead_of_other_work(ctx, size, reads, profile, last):
+    """Reads that do not end their submit see their buffer as it was when they were recorded, whatever
+    overwrites it behind them, and land in their order where destinations overlap."""
+    c = ctx
+    rng = np.random.default_rng(size + reads)
+    data, behind = rng.integers(1, 255, size, dtype=np.uint8), rng.integers(1, 255, size, dtype=np.uint8)
+    buf, other = c.upload(data), c.upload(behind)
+    c.flush()
+    if profile:
+        c.host.start_profile()
+    for turn in range(3):
+        c.rec.write_buffer(buf.buffer, 0, data)
+        out, both, over = [np.zeros(size, np.uint8) for _ in range(reads)], np.zeros(size, np.uint8), np.zeros(size, np.uint8)
+        c.rec.read_buffer(803, other.buffer, 0, over[:4])  # (short, and a long one over it)
+        c.rec.read_buffer(804, buf.buffer, 0, over)
+        for i, o in enumerate(out):
+            c.rec.read_buffer(700 + i, buf.buffer, 0, o)
+        c.rec.read_buffer(800, buf.buffer, 0, both)
+        c.rec.read_buffer(801, other.buffer, 0, both[: (size // 2) & ~3])
+        if last == "clear":
+            c.rec.clear_buffer(buf.buffer, 0, size)
+        elif last == "copy":
+            c.rec.copy_buffer(other.buffer, 0, buf.buffer, 0, size)
+        else:
+            c.rec.read_buffer(802, buf.buffer, 0, both[:0])
+        done = c.flush()
+        assert len(done) == reads + 5 + (last == "empty read")
+        assert all(np.array_equal(o, data) for o in out) and np.array_equal(over, data)
+        half = (size // 2) & ~3
+        assert np.array_equal(both[:half], behind[:half]) and np.array_equal(both[half:], data[half:])
+        assert 0 < c.host.last_submit()[0] < 1e9
+        want = {"clear": np.zeros(size, np.uint8), "copy": behind, "empty read": data}[last]
+        assert np.array_equal(c.read_bytes(buf)[:size], want)
+    if profile:
+        c.host.stop_profile()
 
 
 def test_reads_over_one_destination_leave_the_last_one(ctx):

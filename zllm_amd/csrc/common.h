@@ -167,7 +167,7 @@ zhip_result no_alloc_matmul_q8_0_float(int device, hipStream_t stream, const flo
 // also used instead of memset nodes so a captured stream stays replayable).
 zhip_result launch_fill(hipStream_t stream, void *dst, uint64_t words, uint32_t value);
 // Copies `bytes` (a multiple of 4; both ends 4-byte aligned) between device and pinned host memory.
-// (`stamp`, pinned, receives the GPU's clock; 0 bytes: that alone)
+// (`stamp`, pinned or null, receives the GPU's clock; 0 bytes: that alone)
 zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t *stamp);
 // Reads `bytes` to pinned memory in pieces: read_kernel, elementwise.hip.
 zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *stamp);
