@@ -306,6 +306,28 @@ def test_reads_ahead_of_other_work(ctx, size, reads, profile, last):
         c.host.stop_profile()
 
 
+@pytest.mark.parametrize("read", [True, False])
+def test_last_submit_has_no_host_work_in_it(ctx, read):
+    """What the host decodes between a staged write and the submit is no part of the submit's time: here bind
+    groups by the ten thousand, tens of milliseconds of them, for one short dispatch."""
+    c = ctx
+    width = 256
+    gu, act = c.upload(c.random(2 * width, 1)), c.output(width)
+    c.flush()
+    out = np.zeros(width, np.float32)
+    for turn in range(2):
+        new = c.random(2 * width, 1)
+        c.rec.write_buffer(gu.buffer, 0, new)
+        c.launcher().launch(Kernel.silu_mul, P.SiluMul(width, width), [gu, act], K.elementwise(width))
+        for i in range(40000):
+            c.rec.create_bind_group(c.set.pipelines[Kernel.silu_mul], 0, [cmd.Binding(1, gu.buffer, 0, gu.size), cmd.Binding(2, act.buffer, 0, act.size)])
+        if read:
+            c.rec.read_buffer(7, act.buffer, 0, out)
+        c.flush()
+        assert 0 < c.host.last_submit()[0] < 1e6
+        assert np.max(np.abs((out if read else c.read(act)) - silu_mul_want(new.reshape(1, -1), width)[0])) < 1e-5
+
+
 def test_reads_over_one_destination_leave_the_last_one(ctx):
     c = ctx
     rng = np.random.default_rng(7)

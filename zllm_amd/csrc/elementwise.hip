@@ -343,7 +343,7 @@ zhip_result launch_fill(hipStream_t stream, void *dst, uint64_t words, uint32_t 
 template <class T>
 __global__ __launch_bounds__(256) void copy_kernel(T *dst, const T *src, uint64_t n, uint64_t *stamp) {
     for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) dst[i] = src[i];
-    if (stamp && threadIdx.x == 0) __hip_atomic_store(stamp, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (stamp && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(stamp, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Reads: `n` units to pinned memory, piece after piece; the last workgroup to finish a piece

@@ -220,7 +220,7 @@ struct TimingTotal { uint64_t ns = 0, count = 0; };
 
 // Reads of a submit that the host waits for by their pieces' flags, and pieces of one.
 constexpr uint32_t kFlaggedReads = 16, kMostPieces = 16, kFlags = kFlaggedReads * kMostPieces;
-// Pinned, written by the GPU: its clock behind a submit's last staged write and behind its last read, a flag a piece.
+// Pinned, written by the GPU: its clock ahead of a submit's first op and behind its last read, a flag a piece.
 struct Signals {
     uint64_t begin, end;
     uint64_t flags[kFlags];
@@ -281,10 +281,11 @@ struct zhip_context {
     double tick_ns = 10.0;        // of the GPU's clock
     HandoverThread handover;
 
-    // Small writes wait here, pinned, for the copy kernel queued for each on the stream;
-    // upload_used bytes of it are taken, and nothing is in flight when that is 0.
+    // Small writes wait here, pinned, for the copy kernel queued for each on the stream (the
+    // last one's is launched with what comes behind it); upload_used bytes of it are taken, and nothing is in flight when that is 0.
     uint8_t *upload = nullptr;
     uint64_t upload_used = 0;
+    struct { uint8_t *dst; const uint8_t *src; uint64_t size; } last_write{};  // not launched yet, if of any size
     bool null_stream_work = false;  // a memset or copy on the null stream since it was last waited for
 
     const uint8_t *file = nullptr;
@@ -357,17 +358,27 @@ void drop_pending(zhip_context *c) {
 // A synchronous hipMemcpy of a step's token ids or of a lone projection's input costs 13 us,
 // a third of the shortest submit. Writes of up to kStagedWrite bytes are taken into pinned memory
 // as they are decoded and copied by a small kernel on the stream, ahead of whatever is
-// launched there later (2 us of host time). They never outlast the batch: zhip_execute and
+// launched there later (2 us of host time). The last one's kernel is launched when the submit's first op is, so that the
+// GPU's clock, which it leaves behind, has none of what the host does in between in it. They never outlast the batch: zhip_execute and
 // everything that does not order against the stream waits for them first.
 constexpr uint64_t kStagedWrite = 64u << 10, kUploadBytes = 4 * kStagedWrite;
 // Reads are a kernel's stores to pinned memory too. They arrive in pieces of at least this many
 // bytes, each handed to its destination while the next ones cross the bus, and from kSharedRead on by two threads.
 constexpr uint64_t kReadPiece = 128u << 10, kSharedRead = 768u << 10;
 
+zhip_result launch_last_write(zhip_context *c, uint64_t *stamp) {
+    const auto w = c->last_write;
+    c->last_write = {};
+    if (w.size == 0 && !stamp) return ZHIP_OK;
+    return launch_copy(c->stream, w.dst, w.src, w.size, stamp) == ZHIP_OK ? ZHIP_OK : set_error(c, ZHIP_E_GPU, "%s: launch failed", w.size ? "write_buffer" : "submit");
+}
+
 zhip_result finish_writes(zhip_context *c) {
     if (c->upload_used == 0) return ZHIP_OK;
+    const zhip_result r = launch_last_write(c, nullptr);
     c->upload_used = 0;
-    return hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    return r != ZHIP_OK ? r : hip_check(c, e, "hipStreamSynchronize");
 }
 
 // A new buffer's clearing and longer writes run on the null stream, which the context's stream
@@ -391,12 +402,11 @@ zhip_result write_device(zhip_context *c, uint8_t *dst, const void *src, uint64_
     }
     if (zhip_result r = finish_null_stream(c)) return r;
     const uint64_t room = (len + 15u) & ~15ull;
-    if (c->upload_used + room > kUploadBytes)
-        if (zhip_result r = finish_writes(c)) return r;
+    if (zhip_result r = c->upload_used + room > kUploadBytes ? finish_writes(c) : launch_last_write(c, nullptr)) return r;
     uint8_t *at = c->upload + c->upload_used;
     memcpy(at, src, len);
     c->upload_used += room;
-    if (launch_copy(c->stream, dst, at, len, &c->signals->begin) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "%s: launch failed", what);
+    c->last_write = {dst, at, len};
     return ZHIP_OK;
 }
 
@@ -413,6 +423,7 @@ zhip_result release_buffer(zhip_context *c, uint32_t id) {
 // (or if it is not a uniform-usage buffer and so was never shadowed).
 zhip_result refresh_shadow(zhip_context *c, Buffer &b) {
     if (b.shadowed && !b.shadow_stale) return ZHIP_OK;
+    if (zhip_result r = launch_last_write(c, nullptr)) return r;
     if (zhip_result r = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
     b.shadow.resize(b.size);
     if (zhip_result r = hip_check(c, hipMemcpy(b.shadow.data(), b.dev, b.size, hipMemcpyDeviceToHost), "hipMemcpy (params readback)")) return r;
@@ -703,12 +714,9 @@ zhip_result run_queue(zhip_context *c) {
     if (prefix > 0)
         if (zhip_result r = find_replay(c, prefix, &replay)) return r;
     c->ticket++;
-    if (ends_flagged) {
-        // The submit's staged writes have left the clock, or nothing is there to wait for.
-        if (c->upload_used == 0 && launch_copy(c->stream, c->signals, c->signals, 0, &c->signals->begin) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "submit: launch failed");
-    } else if (zhip_result r = hip_check(c, hipEventRecord(c->ev_begin, c->stream), "hipEventRecord")) {
-        return r;
-    }
+    if (zhip_result r = launch_last_write(c, ends_flagged ? &c->signals->begin : nullptr)) return r;
+    if (!ends_flagged)
+        if (zhip_result r = hip_check(c, hipEventRecord(c->ev_begin, c->stream), "hipEventRecord")) return r;
     bool replayed = false;
     if (replay) {
         if (hipGraphLaunch(replay->exec, c->stream) == hipSuccess) {
@@ -806,6 +814,7 @@ zhip_result submit(zhip_context *c) {
     std::string message;
     if (result != ZHIP_OK) {
         message = c->message;
+        (void)launch_last_write(c, nullptr);
         (void)hipStreamSynchronize(c->stream);
         (void)hipGetLastError();
         c->upload_used = 0;
