@@ -726,33 +726,36 @@ def test_quant_matvec_long_rows(ctx, t, k, pair, rows, n):
         assert got[tk].tobytes() == c.read(single).tobytes(), "a token's sums differ between a lone launch and a multi-token launch"
 
 
-@pytest.mark.parametrize("t,k,n", [
+@pytest.mark.parametrize("t,k,n,pair", [
     # One, two and four rows a wave's pass; a pass or two a wave, and more than the lanes of a row keep
-    # (sixteen passes, thirty-two), ragged in the last pass of either.
-    (TensorType.q8_0, 192, 139303), (TensorType.q4_k, 256, 139303), (TensorType.q6_k, 1024, 24579), (TensorType.q8_0, 1024, 25000),
-    (TensorType.q8_0, 1088, 135171), (TensorType.q6_k, 2048, 16385), (TensorType.q5_k, 1280, 17001),
-    (TensorType.q8_0, 2112, 2049), (TensorType.q6_k, 2304, 12301), (TensorType.q8_0, 4096, 4097), (TensorType.q6_k, 4096, 2048),
+    # (sixteen passes, thirty-two), ragged in the last pass of either; gate / up pairs that keep at
+    # two tokens (in turn) and more, and at one.
+    (TensorType.q8_0, 192, 139303, False), (TensorType.q4_k, 256, 139303, False), (TensorType.q6_k, 1024, 24579, False), (TensorType.q8_0, 1024, 25000, False),
+    (TensorType.q8_0, 1088, 135171, False), (TensorType.q6_k, 2048, 16385, False), (TensorType.q5_k, 1280, 17001, False), (TensorType.q5_k, 512, 14001, False),
+    (TensorType.q8_0, 2112, 2049, False), (TensorType.q6_k, 2304, 12301, False), (TensorType.q8_0, 4096, 4097, False), (TensorType.q6_k, 4096, 2048, False),
+    (TensorType.q8_0, 2560, 4099, True), (TensorType.q6_k, 2304, 6149, True), (TensorType.q6_k, 4096, 6200, True),
 ])
-def test_matvec_rows_kept_for_one_store(ctx, t, k, n):
+def test_matvec_rows_kept_for_one_store(ctx, t, k, n, pair):
     """Sums that wait for one store in several passes: a matrix that repeats 1000 rows gives the bits
     that the 1000 rows alone give, which are stored pass by pass; with a column offset, a padded
-    stride, added to the outputs or not, one, two and five tokens."""
-    c, base, col0, stride = ctx, 1000, 3, n + 5
+    stride, added to the outputs or not, one, two, three and five tokens."""
+    c, base, col0, stride, kinds = ctx, 1000, 3, n + 5, 2 if pair else 1
     x = c.random(5 * k, 1).reshape(5, k)
-    raw, _ = quant_rows(c, t, base, k)
-    row = np.ascontiguousarray(raw).reshape(-1).view(np.uint8).reshape(base, -1)
-    small, tall = c.gpu_weights(t, raw, k), c.gpu_weights(t, np.ascontiguousarray(np.resize(row, (n, row.shape[1]))), k)
-    init, columns = c.random(5 * base, 2).reshape(5, base), np.arange(n) % base
+    raw, _ = quant_rows(c, t, kinds * base, k)
+    columns = np.arange(n) % base
+    row = np.ascontiguousarray(raw).reshape(-1).view(np.uint8).reshape(kinds, base, -1)
+    small, tall = c.gpu_weights(t, raw, k), c.gpu_weights(t, np.ascontiguousarray(row[:, columns]).reshape(kinds * n, -1), k)
+    init = c.random(5 * base, 2).reshape(5, base)
     v = K.MatvecVariant()
     pipeline = c.set.matvec(c.rec, K.weight_kernel("matvec", t), v)
 
     def run(weights, count, rows, start, first, width, accumulate):
         out = c.upload(start)
-        c.launcher().launch_pipeline(pipeline, P.MatvecBf16(n=rows, k=k, col0=first, out_stride=width, eps=1e-6, accumulate=accumulate),
-                                     [c.upload(x[:count]), weights, out, weights], (K.div_ceil(rows, v.group_rows()), count, 1))
+        p = P.MatvecBf16(n=rows, k=k, col0=first, out_stride=width, eps=1e-6, accumulate=accumulate, silu_pair=pair, half=rows if pair else 0)
+        c.launcher().launch_pipeline(pipeline, p, [c.upload(x[:count]), weights, out, weights], (K.div_ceil(rows, v.group_rows()), count, 1))
         return c.read(out).reshape(count, width)
 
-    for count, accumulate in ((1, False), (1, True), (2, True), (2, False), (5, True)):
+    for count, accumulate in ((1, False), (1, not pair), (2, not pair), (2, False), (3, False), (5, not pair)):
         want = run(small, count, base, init[:count], 0, base, accumulate)
         start = np.full((count, stride), 7.0, np.float32)
         start[:, col0 : col0 + n] = init[:count, columns]

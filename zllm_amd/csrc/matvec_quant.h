@@ -164,6 +164,7 @@ struct KQ8 {
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool KEEPS = false;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
+    static constexpr int KEEPS_LONE = 0;  // a token a workgroup: never kept, kept in steps of one token, in any
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 4;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -239,6 +240,7 @@ struct KQ3 {
     static constexpr int NSUM = 4;
     static constexpr int STAGE2 = 0, STAGE4 = 2;  // tokens whose inputs are loaded at once, of two and of three or four
     static constexpr bool KEEPS = true;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
+    static constexpr int KEEPS_LONE = 1;  // a token a workgroup: never kept, kept in steps of one token, in any
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 3;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -329,6 +331,7 @@ struct KQ4 {
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool KEEPS = true;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
+    static constexpr int KEEPS_LONE = 1;  // a token a workgroup: never kept, kept in steps of one token, in any
     static constexpr bool PAIR2 = true;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 2;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -414,6 +417,7 @@ struct KQ5 {
     static constexpr int NSUM = 2;
     static constexpr int STAGE2 = 0, STAGE4 = 0;  // (rows of up to 4096 weights always have two tokens' inputs in registers)
     static constexpr bool KEEPS = true;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
+    static constexpr int KEEPS_LONE = 2;  // a token a workgroup: never kept, kept in steps of one token, in any
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     // The fifth bits leave the general kernel too few registers for three or more tokens' sums: rows
     // of up to 64 tasks always run two tokens a workgroup (four tokens, general / that: 9728 x 2560 21.7 /
@@ -510,6 +514,7 @@ struct KQ6 {
     static constexpr int NSUM = 4;
     static constexpr int STAGE2 = 2, STAGE4 = 1;  // tokens whose inputs are loaded at once
     static constexpr bool KEEPS = false;  // whole-wave rows keep their sums whatever the passes: see run_row_seg
+    static constexpr int KEEPS_LONE = 1;  // a token a workgroup: never kept, kept in steps of one token, in any
     static constexpr bool PAIR2 = false;  // a two-token gate / up step with the inputs in registers fits with both rows of a pair loaded
     static constexpr bool TWO = false;  // three and four tokens over rows of up to 64 tasks: always two a workgroup
     static constexpr uint32_t REG_SLICES = 4;  // three or more tokens over rows of two .. four slices of 64 tasks: see tokens_in_registers
@@ -1583,20 +1588,25 @@ static zhip_result run_row_kernel(const Dispatch &d, const KArgs &q, uint32_t ld
     hipLaunchKernelGGL(kernel, dim3(blocks, (q.mt + MT - 1u) / MT), dim3(256), lds, d.stream, q);
     return check_launch(d, P::name());
 }
-// Whether a wave's sums wait for one store in SEG passes (the stores go between the loads of the stream otherwise). A whole-wave
-// row's do wherever a wave has a second pass, and in the formats with KEEPS always, as it costs nothing there; several rows a pass from the
-// fourth pass on, and not a pair's (2 x 8192 x 2048 at two passes: level). us, stored pass by pass / kept: Q6_K 128256 x 4096 at
-// one / two tokens 80.3 91.8 / 77.5 80.2, 50257 x 2560 at two 36.2 / 30.9, 4096 x 4096 at four 10.4 / 8.7, 2 x 14336 x 4096 at two
-// 22.8 / 20.9; Q8_0 4096 x 4096 at one / two / four 6.0 7.3 10.0 / 5.6 6.6 8.0, 2 x 9728 x 2560 at two 15.1 / 13.6; four rows a pass,
-// 151936 x 1024, Q8_0 at eight 77 / 66, Q4_K at two 25.0 / 21.6, Q5_K at two / eight 29.2 86 / 25.2 73; two, 128256 x 2048 Q4_K at two 40.4 / 33.7; one token
-// over such rows 0 - 6 % (Q8_0 32000 x 2048 13.2 / 13.5). Launches of one pass a wave lose 2 - 5 % by it, a choice at run time costs all of them 3 %.
+// Whether a wave's sums wait for one store in SEG passes (the stores go between the loads of the stream otherwise), by the passes a wave has. Whole-wave
+// rows of the formats with KEEPS always, as it costs nothing there; other sums of two tokens a workgroup from more than one and a half passes on over such rows and from more than three where
+// a pass is of several rows, but not a pair's there (2 x 8192 x 2048 at two passes: level); of one token from more than three on, if KEEPS_LONE says so. Kept / stored, the mean over
+// launches of 1024 ... 16384 rows of 768 ... 4096 weights, weights from memory:
+//   two tokens, whole waves, in (1, 1.5], (1.5, 2], (4, 5] passes: Q6_K 1.01 1.00 0.91, Q8_0 1.00 0.99 0.92, pairs 1.02 0.99 0.96, 0.99 0.94 0.93
+//   two tokens, two or four rows a pass, in (1, 1.5], (2, 3], (3, 4]: Q3_K 1.00 1.00 0.94, Q4_K 1.00 0.95 0.93, Q5_K 1.00 0.93 0.91, Q6_K 1.01 0.95 0.93, Q8_0 1.02 0.94 0.95
+//     (of three to eight tokens, in (2, 3]: 1.02 0.99 0.96 1.01 0.98)
+//   one token, whole waves, in (1, 1.5], (1.5, 2], (3, 4], (4, 5]: Q6_K 1.03 1.02 0.98 0.97, Q8_0 1.02 1.01 1.00 0.99; several rows a pass, in (3, 4]: 0.98 0.93 0.93 0.98 1.00
+//   a token a workgroup in steps of several, in (3, 4]: Q3_K 1.01, Q4_K 1.00, Q5_K 0.97, Q6_K 1.01 (whole waves 1.02), Q8_0 1.00 (1.01)
+// us, stored / kept: Q6_K 128256 x 2304 at two tokens 81.4 / 67.2, 9728 x 4096 at two 10.9 / 9.7; Q8_0 9728 x 2560 at two 9.3 / 8.4, 2 x 9728 x 2560 15.9 / 14.2; four rows a
+// pass, 151936 x 1024, Q8_0 at eight 76 / 64, Q4_K at two 24.8 / 21.1, Q5_K at two / eight 28.9 86 / 24.8 72; two, 151936 x 2048 Q4_K at one / two 36.8 46.5 / 34.1 38.8;
+// one token, Q8_0 50257 x 1280 13.9 / 14.1, 151936 x 2048 56.6 / 57.7. (A choice within the kernel costs all launches 3 %.)
 template <class P, int MT, bool PAIR, int SEG_LOG2>
 static zhip_result run_row_seg(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     constexpr uint32_t RPI = 64u >> SEG_LOG2;
-    const uint32_t units = (q.a.rows + RPI - 1u) / RPI, nwaves = 4u * blocks;
+    const uint64_t units = (q.a.rows + RPI - 1u) / RPI, nwaves = 4u * blocks;
     if constexpr (SEG_LOG2 == 6 && P::KEEPS) return run_row_kernel<P, MT, PAIR, SEG_LOG2, true>(d, q, lds, blocks);
-    if constexpr (SEG_LOG2 == 6 || !PAIR)
-        if (units > (SEG_LOG2 == 6 ? 1u : 3u) * nwaves) return run_row_kernel<P, MT, PAIR, SEG_LOG2, true>(d, q, lds, blocks);
+    if constexpr ((SEG_LOG2 == 6 || !PAIR) && (MT == 2 || P::KEEPS_LONE > 0))
+        if ((MT == 2 || P::KEEPS_LONE == 2 || q.mt == 1u) && 2u * units > (SEG_LOG2 == 6 && MT == 2 ? 3u : 6u) * nwaves) return run_row_kernel<P, MT, PAIR, SEG_LOG2, true>(d, q, lds, blocks);
     if constexpr (!(SEG_LOG2 == 6 && P::KEEPS)) return run_row_kernel<P, MT, PAIR, SEG_LOG2, false>(d, q, lds, blocks);
 }
 template <class P, int MT, bool PAIR>
