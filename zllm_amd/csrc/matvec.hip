@@ -401,14 +401,23 @@ zhip_result launch_matvec_bf16_mfma_stream(const Dispatch &d, const MvArgs &a, u
 // and below the line, where only the default kernels run:
 //   4096 x 1024 (8 MB)           3.9 4.0 4.5 5.9
 //   2048 x 2048 (8 MB)           4.2 4.9 4.9 6.0
-// Long rows are past the registers of matvec_half_row.hip, and the general kernel takes them token by token:
-// without the prologue, this kernel / the general one at 1, 2, 4, 8 tokens, f16:
-//   768 x 6400 (9 MB)            9.1 9.2 9.3 9.4 / 7.4 10.3 18.2 32.8
-//   1024 x 7168                  10.6 10.8 10.9 11.4 / 9.7 12.1 20.3 36.4
-//   400 x 9600                   9.1 9.0 9.1 9.4 / 9.0 15.4 28.0 52.6
-//   2688 x 8064 (41 MB)          14.9 14.9 15.1 15.9 / 13.5 16.9 28.5 52.4
-//   3328 x 11520                 21.1 21.2 21.6 21.3 / 22.5 35.0 61 114
-// and below that line: 1024 x 6144 11.1 11.3 11.4 11.6 / 9.0 11.3 18.4 32.3, 3200 x 5248 (33 MB) 13.8 14.3 14.5 13.9 / 10.8 13.4 21.2 40.1.
+// Long rows are past the registers of matvec_half_row.hip, and the general kernel takes them two tokens a pass over the weights, above
+// 8192 weights one. Without the prologue, this kernel / the general one at 1, 2, 4 tokens, f16, weights from memory:
+//   344 x 6400 (4 MB)            9.8 9.9 10.0 / 7.2 9.7 16.6
+//   983 x 6400                   11.1 11.1 11.2 / 8.2 10.8 17.7
+//   3276 x 6400 (40 MB)          18.0 17.9 17.8 / 12.9 16.0 25.0
+//   5980 x 6400                  23.3 23.4 23.4 / 19.1 26.0 40.1
+//   273 x 8064 (4 MB)            9.0 9.0 9.0 / 7.8 10.7 18.8
+//   2600 x 8064 (40 MB)          15.7 15.7 15.5 / 13.7 17.1 27.3
+//   2184 x 9600                  17.8 17.9 17.9 / 15.3 23.6 40.9
+//   191 x 11520 (4 MB)           10.3 10.4 10.5 / 10.2 17.2 31.0
+//   1820 x 11520 (40 MB)         16.8 17.0 16.8 / 15.7 24.7 44.1
+//   1285 x 16320 (40 MB)         15.6 15.6 15.5 / 20.5 33.0 58.6
+// Over 160 matrices of 6400 ... 16320 weights a row, 4 ... 80 MB, three tokens take 0.4 - 0.8 of the general kernel's time, eight 0.2 - 0.4. Two are
+// level at 6400 in small matrices (0.8 - 1.1 below 7300, at the worst 1.17 at 40 MB; 0.4 - 1.0 from 7700 on) and below that line slower, 1024 x
+// 6144 11.3 / 11.3, 3200 x 5248 14.3 / 13.4: it lies where a step of two breaks even. One token pays 1.1 - 1.4 times the time up to
+// 7500 weights (fifteen lines of 512 columns, which the stretches do not divide evenly), 0.9 - 1.3 up to 13056, less than the general
+// kernel's from there on: less than it pays in the table above. Matrices of under 4 MB were not measured.
 // Shorter rows of no multiple of 512 stay with matvec_half_row.hip, which is the faster one at one and two tokens, at two by up to
 // 35 % (5376 x 1792 pair 13.3 / 9.5, 8064 x 2688 22.0 / 17.1; at eight 13.3 / 17.7, 22.5 / 31.6).
 constexpr uint64_t kBf16StreamBytes = kMatvecBf16StreamBytes, kBf16StreamLongBytes = 4ull << 20;

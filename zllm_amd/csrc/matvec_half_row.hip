@@ -249,7 +249,7 @@ zhip_result launch_iters(const Dispatch &d, const MvArgs &a) {
     // Stores between the loads of the stream cost more than their bytes: from the fourth pass of a wave on (a pair's from the sixth: 2 x 4096
     // x 2048 f16 at four tokens, four passes, 10.0 / 10.5 us, at eight, eight, 14.2 / 13.4) they wait in the lanes. us, stored pass by pass / kept, bf16: 151936 x 1024 at four / eight tokens 61.5 85.6 / 55.2 76.3, 50257 x 2560 61 88 / 57 76, 16384 x
     // 2048 15.4 23.1 / 14.0 20.2, 2 x 8192 x 2048 15.8 22.6 / 14.8 21.4, at one token level (151936 x 1024 52.1 / 51.9). Not a pair's
-    // of longer rows: 2 x 9728 x 2560 at eight tokens 36.1 / 32.6, but at four 27.2 / 30.5.
+    // of longer rows, at any number of tokens: 2 x 9728 x 2560 at four 27.2 / 30.5 (at eight 36.1 / 32.6).
     constexpr bool PAIR_KEEPS = ITERS <= 4;
     const bool keep = (a.rows + outs - 1u) / outs > (pair ? 20u : 12u) * blocks;
     if constexpr (PAIR_KEEPS)

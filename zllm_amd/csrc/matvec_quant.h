@@ -630,6 +630,16 @@ __device__ __forceinline__ float segment_sum(float v, uint32_t seg_log2) {
     return v;
 }
 
+// A segment's sum, which segment_sum leaves in its last lane (and in every lane of a segment of sixteen), in all of its lanes.
+template <int SEG_LOG2>
+__device__ __forceinline__ float segment_total(float v, uint32_t lane) {
+    if (SEG_LOG2 == 4) return v;
+    const float last = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
+    if (SEG_LOG2 == 6) return last;
+    const float first = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 31));
+    return lane < 32u ? first : last;
+}
+
 // Floats per task in the padded LDS copy: 64 inputs and one vector of padding,
 // so lanes reading the same offset of consecutive tasks hit different banks.
 constexpr uint32_t kTaskStride = 68;
@@ -897,16 +907,7 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
 // multiply turns into a sum of zero; no address arithmetic, clamp or branch per lane is left.
 // The staging of the inputs, a task's dot product and the lanes' reduction are the code of the
 // kernel above, so the results are its bits.
-// A segment's sum, which segment_sum leaves in its last lane (and in every lane of a segment of sixteen), in all of its lanes.
-template <int SEG_LOG2>
-__device__ __forceinline__ float segment_total(float v, uint32_t lane) {
-    if (SEG_LOG2 == 4) return v;
-    const float last = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
-    if (SEG_LOG2 == 6) return last;
-    const float first = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 31));
-    return lane < 32u ? first : last;
-}
-
+//
 // Passes whose loads are in flight ahead of the one multiplied. Measured on 14336 x 4096 Q4_K
 // (7.9 us with one): two or three passes ahead 8.6 / 9.8 us, and no better with fewer workgroups;
 // two passes asked for before the inputs are staged (instead of one) 8.7 us; the first pass
@@ -1040,10 +1041,10 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
     const bool accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
     auto out_at = [&](int t, uint32_t j) { return (size_t)(q.t0 + t) * a.out_stride + a.col0 + j; };
 
-    // With KEEP a pass's finished sums are kept in the rows' lanes of its number
-    // (the gate's and the up row's apart), and SEG passes' are finished and stored together:
-    // stores between the loads of the stream cost more than their bytes,
-    // and the activation runs once for 64 outputs instead of once a row. See run_row_seg.
+    // With KEEP a pass's finished sums wait in the lanes, the gate's and the up row's apart: lane tsub of
+    // row rsub's segment holds that row's of the wave's pass numbered tsub since the last store. SEG
+    // passes' (16, 32 or 64), 64 outputs, are finished and stored together: stores between the loads of the stream
+    // cost more than their bytes, and the activation runs once for them instead of once a row. Which launches: run_row_seg.
     float kept0[MT], kept1[MT];
 #pragma unroll
     for (int t = 0; t < MT; t++) kept0[t] = kept1[t] = 0.f;
