@@ -151,8 +151,9 @@ zhip_result zhip_profile_stop(zhip_context *context);
 zhip_result zhip_profile_read(zhip_context *context, zhip_timing *out, size_t capacity,
     size_t *out_count, uint64_t *out_untimed);
 /* GPU time of the last submit's recorded work (first op to last op: one event
- * pair on the host's stream, or, where it ends in reads, the GPU's clock read by kernels
- * launched ahead of the first op, not before, and behind the last read), in nanoseconds, and how many dispatches it ran:
+ * pair on the host's stream, or, where it ends in reads, by the GPU's clock from the copy of the
+ * last staged write, or a kernel ahead of the first op if there is none, to the last read, with no more than the
+ * host's clock from the first op's launch to the first piece read), in nanoseconds, and how many dispatches it ran:
  * the measurement a tuner's batched timing takes (src/tune/tune.zig:8-11). */
 zhip_result zhip_last_submit(zhip_context *context, uint64_t *out_ns, uint64_t *out_dispatches);
 /* How many submits so far ran their dispatches from a replayed graph (see

@@ -170,7 +170,7 @@ zhip_result launch_fill(hipStream_t stream, void *dst, uint64_t words, uint32_t 
 // (`stamp`, pinned or null, receives the GPU's clock; 0 bytes: that alone)
 zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t *stamp);
 // Reads `bytes` to pinned memory in pieces: read_kernel, elementwise.hip.
-zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *stamp);
+zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *first, uint64_t *last);
 
 // A launch's time by its workgroups, where two share a CU: a lone one's time, and a pair's, which is less than twice
 // that. An odd one out costs its CU a lone one's.

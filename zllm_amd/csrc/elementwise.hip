@@ -347,13 +347,13 @@ __global__ __launch_bounds__(256) void copy_kernel(T *dst, const T *src, uint64_
 }
 
 // Reads: `n` units to pinned memory, piece after piece; the last workgroup to finish a piece
-// leaves `ticket` in the piece's flag, where the host waits for it, and behind the last piece the
-// GPU's clock in `stamp`. `arrived` (a counter a piece) is zero before and after. An event and a stream
+// leaves `ticket` in the piece's flag, where the host waits for it, and behind the first piece and the last the
+// GPU's clock in `first`, if any, and `last`. `arrived` (a counter a piece) is zero before and after. An event and a stream
 // synchronization behind a read cost 2 us more than the flag, a pair of timing events around a
 // submit 5 us (the first one keeps the next kernel from starting), pieces as copies of the runtime's
 // with an event each up to 2 us of idle bus a piece.
 template <class T>
-__global__ __launch_bounds__(256) void read_kernel(T *dst, const T *src, uint64_t n, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *stamp) {
+__global__ __launch_bounds__(256) void read_kernel(T *dst, const T *src, uint64_t n, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *first, uint64_t *last) {
     for (uint64_t at = 0, p = 0; at < n; at += piece, p++) {
         const uint64_t end = at + piece < n ? at + piece : n;
         for (uint64_t i = at + (uint64_t)blockIdx.x * 256u + threadIdx.x; i < end; i += (uint64_t)gridDim.x * 256u) dst[i] = src[i];
@@ -363,7 +363,8 @@ __global__ __launch_bounds__(256) void read_kernel(T *dst, const T *src, uint64_
         if (threadIdx.x != 0) continue;
         if (__hip_atomic_fetch_add(arrived + p, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1u) continue;
         __hip_atomic_store(arrived + p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (end == n) __hip_atomic_store(stamp, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (at == 0 && first) __hip_atomic_store(first, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (end == n) __hip_atomic_store(last, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         __hip_atomic_store(flags + p, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
@@ -383,12 +384,12 @@ zhip_result launch_copy(hipStream_t stream, void *dst, const void *src, uint64_t
 }
 
 // `piece` is a multiple of 16 bytes; one flag and one counter a piece.
-zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *stamp) {
+zhip_result launch_read(hipStream_t stream, void *dst, const void *src, uint64_t bytes, uint64_t piece, uint32_t *arrived, uint64_t *flags, uint64_t ticket, uint64_t *first, uint64_t *last) {
     const bool wide = wide_copy(dst, src, bytes);
     const uint64_t unit = wide ? 16u : 4u, n = bytes / unit;
     const dim3 grid(blocks_for(std::min(n, piece / unit), 256, 128));
-    if (wide) hipLaunchKernelGGL(read_kernel<uint4>, grid, dim3(256), 0, stream, static_cast<uint4 *>(dst), static_cast<const uint4 *>(src), n, piece / unit, arrived, flags, ticket, stamp);
-    else hipLaunchKernelGGL(read_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), n, piece / unit, arrived, flags, ticket, stamp);
+    if (wide) hipLaunchKernelGGL(read_kernel<uint4>, grid, dim3(256), 0, stream, static_cast<uint4 *>(dst), static_cast<const uint4 *>(src), n, piece / unit, arrived, flags, ticket, first, last);
+    else hipLaunchKernelGGL(read_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), n, piece / unit, arrived, flags, ticket, first, last);
     return hipGetLastError() == hipSuccess ? ZHIP_OK : ZHIP_E_GPU;
 }
 

@@ -23,6 +23,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -220,9 +221,10 @@ struct TimingTotal { uint64_t ns = 0, count = 0; };
 
 // Reads of a submit that the host waits for by their pieces' flags, and pieces of one.
 constexpr uint32_t kFlaggedReads = 16, kMostPieces = 16, kFlags = kFlaggedReads * kMostPieces;
-// Pinned, written by the GPU: its clock ahead of a submit's first op and behind its last read, a flag a piece.
+// Pinned, written by the GPU: its clock behind a submit's last staged write (or ahead of its first op), behind the first piece read
+// and behind the last read, a flag a piece.
 struct Signals {
-    uint64_t begin, end;
+    uint64_t begin, first, end;
     uint64_t flags[kFlags];
 };
 
@@ -281,11 +283,10 @@ struct zhip_context {
     double tick_ns = 10.0;        // of the GPU's clock
     HandoverThread handover;
 
-    // Small writes wait here, pinned, for the copy kernel queued for each on the stream (the
-    // last one's is launched with what comes behind it); upload_used bytes of it are taken, and nothing is in flight when that is 0.
+    // Small writes wait here, pinned, for the copy kernel queued for each on the stream;
+    // upload_used bytes of it are taken, and nothing is in flight when that is 0.
     uint8_t *upload = nullptr;
     uint64_t upload_used = 0;
-    struct { uint8_t *dst; const uint8_t *src; uint64_t size; } last_write{};  // not launched yet, if of any size
     bool null_stream_work = false;  // a memset or copy on the null stream since it was last waited for
 
     const uint8_t *file = nullptr;
@@ -358,27 +359,17 @@ void drop_pending(zhip_context *c) {
 // A synchronous hipMemcpy of a step's token ids or of a lone projection's input costs 13 us,
 // a third of the shortest submit. Writes of up to kStagedWrite bytes are taken into pinned memory
 // as they are decoded and copied by a small kernel on the stream, ahead of whatever is
-// launched there later (2 us of host time). The last one's kernel is launched when the submit's first op is, so that the
-// GPU's clock, which it leaves behind, has none of what the host does in between in it. They never outlast the batch: zhip_execute and
+// launched there later (2 us of host time). They never outlast the batch: zhip_execute and
 // everything that does not order against the stream waits for them first.
 constexpr uint64_t kStagedWrite = 64u << 10, kUploadBytes = 4 * kStagedWrite;
 // Reads are a kernel's stores to pinned memory too. They arrive in pieces of at least this many
 // bytes, each handed to its destination while the next ones cross the bus, and from kSharedRead on by two threads.
 constexpr uint64_t kReadPiece = 128u << 10, kSharedRead = 768u << 10;
 
-zhip_result launch_last_write(zhip_context *c, uint64_t *stamp) {
-    const auto w = c->last_write;
-    c->last_write = {};
-    if (w.size == 0 && !stamp) return ZHIP_OK;
-    return launch_copy(c->stream, w.dst, w.src, w.size, stamp) == ZHIP_OK ? ZHIP_OK : set_error(c, ZHIP_E_GPU, "%s: launch failed", w.size ? "write_buffer" : "submit");
-}
-
 zhip_result finish_writes(zhip_context *c) {
     if (c->upload_used == 0) return ZHIP_OK;
-    const zhip_result r = launch_last_write(c, nullptr);
     c->upload_used = 0;
-    const hipError_t e = hipStreamSynchronize(c->stream);
-    return r != ZHIP_OK ? r : hip_check(c, e, "hipStreamSynchronize");
+    return hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 }
 
 // A new buffer's clearing and longer writes run on the null stream, which the context's stream
@@ -402,11 +393,12 @@ zhip_result write_device(zhip_context *c, uint8_t *dst, const void *src, uint64_
     }
     if (zhip_result r = finish_null_stream(c)) return r;
     const uint64_t room = (len + 15u) & ~15ull;
-    if (zhip_result r = c->upload_used + room > kUploadBytes ? finish_writes(c) : launch_last_write(c, nullptr)) return r;
+    if (c->upload_used + room > kUploadBytes)
+        if (zhip_result r = finish_writes(c)) return r;
     uint8_t *at = c->upload + c->upload_used;
     memcpy(at, src, len);
     c->upload_used += room;
-    c->last_write = {dst, at, len};
+    if (launch_copy(c->stream, dst, at, len, &c->signals->begin) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "%s: launch failed", what);
     return ZHIP_OK;
 }
 
@@ -423,7 +415,6 @@ zhip_result release_buffer(zhip_context *c, uint32_t id) {
 // (or if it is not a uniform-usage buffer and so was never shadowed).
 zhip_result refresh_shadow(zhip_context *c, Buffer &b) {
     if (b.shadowed && !b.shadow_stale) return ZHIP_OK;
-    if (zhip_result r = launch_last_write(c, nullptr)) return r;
     if (zhip_result r = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
     b.shadow.resize(b.size);
     if (zhip_result r = hip_check(c, hipMemcpy(b.shadow.data(), b.dev, b.size, hipMemcpyDeviceToHost), "hipMemcpy (params readback)")) return r;
@@ -714,9 +705,14 @@ zhip_result run_queue(zhip_context *c) {
     if (prefix > 0)
         if (zhip_result r = find_replay(c, prefix, &replay)) return r;
     c->ticket++;
-    if (zhip_result r = launch_last_write(c, ends_flagged ? &c->signals->begin : nullptr)) return r;
-    if (!ends_flagged)
-        if (zhip_result r = hip_check(c, hipEventRecord(c->ev_begin, c->stream), "hipEventRecord")) return r;
+    // What the host decoded behind the last staged write, looked up and captured is over: no part of the submit's time.
+    const auto started = std::chrono::steady_clock::now();
+    if (ends_flagged) {
+        // The submit's staged writes have left the GPU's clock, or nothing is there to wait for.
+        if (c->upload_used == 0 && launch_copy(c->stream, c->signals, c->signals, 0, &c->signals->begin) != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "submit: launch failed");
+    } else if (zhip_result r = hip_check(c, hipEventRecord(c->ev_begin, c->stream), "hipEventRecord")) {
+        return r;
+    }
     bool replayed = false;
     if (replay) {
         if (hipGraphLaunch(replay->exec, c->stream) == hipSuccess) {
@@ -766,7 +762,7 @@ zhip_result run_queue(zhip_context *c) {
             rd.flagged = ends_flagged || gets_flags(c, next_read - 1u, flagged);
             const uint32_t at_flags = flagged * kMostPieces;
             const zhip_result launched = !rd.flagged ? launch_copy(c->stream, to, from, rd.size, nullptr)
-                : launch_read(c->stream, to, from, rd.size, piece_bytes(rd.size), c->arrived + at_flags, c->signals->flags + at_flags, c->ticket, &c->signals->end);
+                : launch_read(c->stream, to, from, rd.size, piece_bytes(rd.size), c->arrived + at_flags, c->signals->flags + at_flags, c->ticket, flagged == 0 ? &c->signals->first : nullptr, &c->signals->end);
             if (launched != ZHIP_OK) return set_error(c, ZHIP_E_GPU, "read_buffer: launch failed");
             flagged += rd.flagged;
             break;
@@ -778,15 +774,24 @@ zhip_result run_queue(zhip_context *c) {
         if (zhip_result r = hip_check(c, hipEventRecord(c->ev_end, c->stream), "hipEventRecord")) return r;
     // The reads with flags while the stream runs on, the others behind its end.
     uint32_t next_flags = 0;
+    auto seen = started;  // the first piece
     for (const Read &rd : c->reads) {
         if (!rd.flagged) continue;
+        if (next_flags == 0) {
+            if (zhip_result r = wait_flag(c, c->signals->flags)) return r;
+            seen = std::chrono::steady_clock::now();
+        }
         if (zhip_result r = hand_over(c, rd, next_flags)) return r;
         next_flags += kMostPieces;
     }
     if (ends_flagged) {
         c->upload_used = 0;
-        const uint64_t begin = __atomic_load_n(&c->signals->begin, __ATOMIC_RELAXED), end = __atomic_load_n(&c->signals->end, __ATOMIC_RELAXED);
-        c->last_ns = end > begin ? (uint64_t)((double)(end - begin) * c->tick_ns) : 0;
+        // By the GPU's clock, but up to the first piece no more than the host's from the first op's launch on: begin may lie any
+        // time ahead of that. (A copy that is launched with the first op leaves the right time, but a replayed step waits 3 us for it.)
+        auto clock = [](const uint64_t &stamp) { return __atomic_load_n(&stamp, __ATOMIC_RELAXED); };
+        auto span = [&](uint64_t from, uint64_t to) { return to > from ? (uint64_t)((double)(to - from) * c->tick_ns) : 0ull; };
+        const uint64_t first = clock(c->signals->first), host_ns = (uint64_t)std::chrono::nanoseconds(seen - started).count();
+        c->last_ns = std::min<uint64_t>(span(clock(c->signals->begin), first), host_ns) + span(first, clock(c->signals->end));
         return ZHIP_OK;
     }
     if (zhip_result r = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
@@ -814,7 +819,6 @@ zhip_result submit(zhip_context *c) {
     std::string message;
     if (result != ZHIP_OK) {
         message = c->message;
-        (void)launch_last_write(c, nullptr);
         (void)hipStreamSynchronize(c->stream);
         (void)hipGetLastError();
         c->upload_used = 0;
