@@ -2211,6 +2211,31 @@ def test_matmul_kquant_int8_bits_do_not_depend_on_the_rows_of_a_launch(ctx, t, k
             assert rel_err(got[0], xs[:count].astype(np.float64) @ values.astype(np.float64).T + (init[:count] if accumulate else 0.0)) <= 1e-5
 
 
+@pytest.mark.parametrize("k", [256, 512, 768, 1280, 2304])
+@pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
+def test_matmul_kquant_int8_halves_of_k(ctx, t, k):
+    """Short steps over tall matrices, whose waves walk two parts of k each: the bits of the 90-row
+    matrix that the tall one is over and over, whose launches have a wave a part; one, two and three
+    blocks (parts of none), five and nine; rows that fill no tile, tokens short of one, two, four and six.
+    1e-5 against float64 over the rounded activations."""
+    c = ctx
+    rows, n, times = 190, 90, 273
+    x = c.random(rows * k, 1).reshape(rows, k)
+    raw, values = quant_rows(c, t, n, k)
+    small, large = c.gpu_weights(t, raw, k), c.gpu_weights(t, np.tile(raw.reshape(-1), times), k)
+    xs = oracle.round_like_llama(ORACLE_TYPE[t], x)
+    init = c.random(rows * n, 1).reshape(rows, n)
+    for accumulate, count in ((0, rows), (1, 126), (0, 62), (1, 62), (0, 30), (1, 3)):
+        act = quantize_x(c, t, c.upload(x[:count]), count, k)
+        got = []
+        for w, m in ((small, 1), (large, times)):
+            out = c.upload(np.tile(init[:count], (1, m)))
+            launch_int8(c, t, act, w, out, count, n * m, k, accumulate, None)
+            got.append(c.read(out).reshape(count, n * m))
+        assert np.array_equal(np.tile(got[0], (1, times)).view(np.uint32), got[1].view(np.uint32)), (accumulate, count)
+        assert rel_err(got[0], xs[:count].astype(np.float64) @ values.astype(np.float64).T + (init[:count] if accumulate else 0.0)) <= 1e-5
+
+
 @pytest.mark.parametrize("n", [1, 32, 77, 160])
 @pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
 def test_matmul_kquant_int8_lone_token_at_any_stride(ctx, t, n):

@@ -24,13 +24,17 @@
 // k is summed in four parts, blocks p * B / 4 .. of part p of B, each in its order, and the parts are
 // added as ((p0 + p1) + p2) + p3, whatever the matrix and the step: neither how a prompt is cut into
 // steps nor how a matrix is cut into launches changes an output's bits. A workgroup is S * RW waves.
-// Wave w walks part w % S of k (S = 4) or all four, closing each part's sums (S = 1), for rows 32 (w / S) .. + 31
+// Wave w walks part w % S of k (S = 4), two of them (S = 2) or all four, closing each part's sums (S = 1), for rows 32 (w / S) .. + 31
 // and the tile's 32 NT tokens, one 32-token tile of a block after the other with the block's
 // converted weights in registers (64 VGPRs). Every part has a ring of three token tiles in LDS, filled
 // two tiles ahead by whole-line direct loads that the part's RW waves share, and a wave's rows'
 // blocks arrive in a slot of its own a block ahead. One barrier a tile where RW > 1, which leaves the
 // loads in flight; the f32 end of a tile and block (five vector operations an output) is worked off
 // between the next tile's matrix instructions.
+//
+// With few tokens over a tall matrix there is one workgroup of four walking waves a CU, one a SIMD, and nobody issues while it
+// waits for an instruction's result; halving k gives every SIMD a second wave and leaves a wave's conversion its two token tiles: Q4_K 64 x
+// 28672 x 4096 29.6 -> 24.7 us, Q6_K 64 x 24576 x 3072 30.6 -> 25.1, 256 x 19456 x 2560 56.0 -> 47.6, Q3_K 32 x 28672 x 4096 20.1 -> 16.4.
 //
 // Measured (us, weights from HBM, against the predecessor): Q4_K 512 x 4096 x 4096 37.9 -> 28.2, 512 x 28672 x
 // 4096 232 -> 173, 512 x 4096 x 14336 115 -> 91, 128 x 4096 x 4096 17.3 -> 11.6, 64 x 4096 x 4096 9.7 -> 8.9;
@@ -285,6 +289,7 @@ template <class P> constexpr uint32_t wslot_bytes() { return (32u * (P::BLOCK / 
 template <class P, int RW, int S> constexpr uint32_t lds_bytes() { return S * part_bytes<P>() + S * RW * wslot_bytes<P>(); }
 // (the exchange of the parts' sums reuses the rings: 4 RW owners x 3 senders x NT KB)
 static_assert(4 * part_bytes<KqQ6>() >= 4 * 2 * 3 * 4 * 1024, "the exchange must fit the token rings");
+static_assert(lds_bytes<KqQ3, 4, 2>() >= 4 * 2 * 2 * 2 * 8 * 256 && lds_bytes<KqQ3, 2, 2>() >= 2 * 2 * 2 * 2 * 8 * 256, "nor may the one of two halves' pass the end");
 static_assert(lds_bytes<KqQ6, 2, 4>() <= 160 * 1024 && lds_bytes<KqQ5, 2, 4>() <= 160 * 1024, "rings and slots must fit the CU's LDS");
 
 template <class P, int NT, int RW, int S>
@@ -298,7 +303,7 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
     // The chip deals workgroups out to its eight dies in turn. Renumbered, those of a column of the matrix follow one
     // another on one die, whose L2 then has the column's weights for all but the first of them.
     uint32_t column = blockIdx.x, tokens = blockIdx.y;
-    if (S == 1 && a.by_die) {
+    if (S <= 2 && a.by_die) {
         const uint32_t id = tokens * gridDim.x + column, dealt = (gridDim.x & ~7u) * gridDim.y, turn = id >> 3;
         column = id < dealt ? (turn / gridDim.y << 3) + (id & 7u) : id / gridDim.y;
         tokens = (id < dealt ? turn : id) % gridDim.y;
@@ -349,13 +354,14 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[tt][e] = 0.f;
     // S = 1: the sums of the parts before this one, closed where a part ends. (A row of less than four
-    // blocks begins with an empty part, whose sum is a zero; -0 leaves the first part's as they are.)
-    float closed[S == 1 ? NT : 1][16];
-    if constexpr (S == 1) {
+    // blocks begins with an empty part, whose sum is a zero; -0 leaves the first part's as they are.) S = 2: the sum
+    // of the first of the wave's two parts.
+    float closed[S <= 2 ? NT : 1][16];
+    if constexpr (S <= 2) {
 #pragma unroll
         for (int tt = 0; tt < NT; tt++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) closed[tt][e] = blocks < 4u ? 0.f : -0.f;
+            for (int e = 0; e < 16; e++) closed[tt][e] = S == 2 || blocks < 4u ? 0.f : -0.f;
     }
     auto close = [&](int tt) __attribute__((always_inline)) {
 #pragma unroll
@@ -364,7 +370,7 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
             acc[tt][e] = 0.f;
         }
     };
-    uint32_t parts = 1, end = blocks / 4u;  // S = 1: where the part ends that block b is of
+    uint32_t parts = 1, end = S == 2 ? (2u * part + 1u) * blocks / 4u - first : blocks / 4u;  // S = 1: where the part ends that block b is of; S = 2: where the first ends
     bool closes = false;                    // the block of the last step's tile was its part's last
     u32x4 high[8], low[8];
     i32x16 total = {};  // the last tile's integer sums: finished during the next tile's matrix instructions
@@ -476,8 +482,8 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
                 if (RW == 2) *reinterpret_cast<uint2 *>(sums_at(count) + 8u * group) = uint2{s4.x, s4.y};
                 if (RW == 4) *reinterpret_cast<uint32_t *>(sums_at(count) + 4u * group) = s4.x;
             }
-            if (S == 1 && closes) close(prev);
-            if (S == 1 && tt == 0) closes = end == b + 1u;
+            if (S <= 2 && closes) close(prev);
+            if (S <= 2 && tt == 0) closes = end == b + 1u;
             if (tt == 0) P::factors(raw, d, dmin, mins);
 #pragma unroll
             for (int e = 0; e < 16; e++) total[e] = UNIT_SCALES ? __mul24(unit_scale(sc, 7), lsum[e]) + hsum[e] : P::PLANES == 2 ? (int)((uint32_t)hsum[e] << P::SHIFT) + lsum[e] : hsum[e];
@@ -502,19 +508,28 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
     }
     step_end<0, true>();  // nothing may still land in LDS during the exchange
 
-    // The parts of a row group meet in LDS: the wave of part p finishes sums 4 NT p .. + 4 NT - 1 of
-    // every lane's 16 NT and hands the rest to their owners.
+    // The parts of a row group meet in LDS: the wave of part p finishes sums 16 NT / S p .. + 16 NT / S - 1 of
+    // every lane's 16 NT and hands the rest to their owners (S = 2: of both its parts).
     float *inbox = reinterpret_cast<float *>(lds);
+    constexpr uint32_t OWN = 16 * NT / S, SENT = S == 4 ? 3 : 2;
     auto place = [&](uint32_t owner, uint32_t from, int i) __attribute__((always_inline)) {
-        return (((owner * RW + group) * 3u + ((from + 3u - owner) & 3u)) * (4 * NT) + i) * 64u + lane;
+        return (((owner * RW + group) * SENT + from) * OWN + i) * 64u + lane;
     };
+    auto sender = [](uint32_t owner, uint32_t from) __attribute__((always_inline)) { return (from + 3u - owner) & 3u; };
 #pragma unroll
-    for (int owner = 0; owner < (S == 4 ? 4 : 0); owner++) {
+    for (int owner = 0; owner < (S > 1 ? S : 0); owner++) {
         if (part == (uint32_t)owner) continue;
 #pragma unroll
-        for (int i = 0; i < 4 * NT; i++) inbox[place(owner, part, i)] = acc[(4 * NT * owner + i) / 16][(4 * NT * owner + i) % 16];
+        for (int i = 0; i < (int)OWN; i++) {
+            const int e = (int)OWN * owner + i;
+            if (S == 4) inbox[place(owner, sender(owner, part), i)] = acc[e / 16][e % 16];
+            if constexpr (S == 2) {
+                inbox[place(owner, 0, i)] = closed[e / 16][e % 16];
+                inbox[place(owner, 1, i)] = acc[e / 16][e % 16];
+            }
+        }
     }
-    if (S == 4) {
+    if (S > 1) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -540,8 +555,12 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
             if (S == 4) {
                 float v[4];
 #pragma unroll
-                for (int from = 0; from < 4; from++) v[from] = from == Q ? sum[i] : inbox[place(Q, from, i)];
+                for (int from = 0; from < 4; from++) v[from] = from == Q ? sum[i] : inbox[place(Q, sender(Q, from), i)];
                 sum[i] = ((v[0] + v[1]) + v[2]) + v[3];
+            }
+            if constexpr (S == 2) {
+                const float mine0 = closed[(base + i) / 16][(base + i) % 16], sent0 = inbox[place(Q / 2, 0, base + i - (int)OWN * (Q / 2))], sent1 = inbox[place(Q / 2, 1, base + i - (int)OWN * (Q / 2))];
+                sum[i] = Q < 2 ? ((mine0 + sum[i]) + sent0) + sent1 : ((sent0 + sent1) + mine0) + sum[i];
             }
         }
         if (a.accumulate) {
@@ -551,10 +570,10 @@ __global__ __launch_bounds__(64 * S * RW) __attribute__((amdgpu_waves_per_eu(NT 
 #pragma unroll
         for (int i = 0; i < 4 * NT; i++) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum[i]), obuf, offset(i), 0, 0);
     };
-    if (S == 1 || part == 0u) collect(std::integral_constant<int, 0>{});
-    if (S == 1 || part == 1u) collect(std::integral_constant<int, 1>{});
-    if (S == 1 || part == 2u) collect(std::integral_constant<int, 2>{});
-    if (S == 1 || part == 3u) collect(std::integral_constant<int, 3>{});
+    if (part == 0u) collect(std::integral_constant<int, 0>{});
+    if (part == (S == 4 ? 1u : 0u)) collect(std::integral_constant<int, 1>{});
+    if (part == (uint32_t)S / 2u) collect(std::integral_constant<int, 2>{});
+    if (part == (uint32_t)S - 1u) collect(std::integral_constant<int, 3>{});
 }
 
 template <class P, int NT, int RW, int S>
@@ -566,24 +585,27 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const KqArgs &a) {
     return check_launch(d, name);
 }
 
-// Which launch takes the step; the bits are the same. Workgroups that walk a part of k each (S = 4) have a CU to
-// themselves: a launch of w a CU takes w times one's time. Those that walk all of it (S = 1) share a CU two at a
-// time, and a pair takes less than twice a lone one's time: an odd one out costs `lone`, a pair `pair`. In k the
-// first kind's time grows like blocks + 3 (the exchange), the second's like blocks + 2. In units of such a
+// Which launch takes the step; the bits are the same. Workgroups that walk a part of k each (S = 4), or two with four row groups
+// (S = 2), have a CU to themselves: a launch of w a CU takes w times one's time. Those that walk all of it (S = 1), or half of it for
+// two row groups, share a CU two at a time, and a pair takes less than twice a lone one's time: an odd one out costs `lone`, a pair `pair`. In k the
+// first kinds' time grows like blocks + 3 (the exchange), the third's like blocks + 2. In units of such a
 // time, fitted to steps of 16 ... 512 tokens over sixteen matrices of 1024 x 3072 ... 28672 x 4096 and 4096 x 14336, every
-// launch of the list on each of them: the rule's launch is within 0.1 % (Q5_K 0.3 %, Q6_K 0.6 %) of the fastest one in the mean. (A line
+// launch of the list on each of them: the rule's launch is within 0.2 % (Q5_K 0.9 %, Q6_K 0.6 %) of the fastest one in the mean, and the launches
+// of S = 2 take 0.89 (Q3_K), 0.92, 0.92 and 0.91 of the time of those they came in place of. (A line
 // at a number of workgroups, as here before, lost 1.6 % / 6.2 % / 2.7 % / 1.8 % of Q4_K's / Q5_K's / Q6_K's / Q3_K's time, and where a
 // last round was nearly empty 30 - 80 %: 96 x 19456 x 2560 Q4_K 34.9 -> 20.5 us, Q5_K 40.6 -> 22.5, Q3_K 25.1 -> 19.0; Q5_K
 // 512 x 12288 x 2560 63.4 -> 55.9, 64 x 28672 x 4096 Q4_K 33.1 -> 31.6.)
 struct Costs {
-    uint32_t parts[5];  // token tiles x row groups: 1 x 1, 1 x 2, 2 x 1, 2 x 2, 4 x 2
-    SharedCu whole[3];      // of 1, 2 and 4 token tiles, four row groups (0: none; of two planes, four tiles' closed sums do not fit the registers)
-};
+    uint32_t parts[5];   // token tiles x row groups: 1 x 1, 1 x 2, 2 x 1, 2 x 2, 4 x 2
+    SharedCu whole[3];   // of 1, 2 and 4 token tiles, four row groups (of two planes, four tiles' closed sums do not fit the registers)
+    uint32_t halves[2];  // of 1 and 2 token tiles, four row groups
+    SharedCu halves2;    // of 2 token tiles, two row groups
+};  // (0: none, or never the cheapest)
 template <class P> constexpr Costs costs();
-template <> constexpr Costs costs<KqQ3>() { return {{19, 24, 22, 31, 42}, {{51, 73}, {67, 90}, {98, 118}}}; }
-template <> constexpr Costs costs<KqQ4>() { return {{14, 19, 18, 29, 39}, {{39, 56}, {50, 71}, {0, 0}}}; }
-template <> constexpr Costs costs<KqQ5>() { return {{13, 17, 19, 26, 40}, {{32, 47}, {51, 79}, {0, 0}}}; }
-template <> constexpr Costs costs<KqQ6>() { return {{17, 26, 21, 31, 43}, {{53, 74}, {66, 91}, {0, 0}}}; }
+template <> constexpr Costs costs<KqQ3>() { return {{19, 24, 22, 31, 42}, {{51, 73}, {67, 90}, {98, 118}}, {45, 0}, {32, 46}}; }
+template <> constexpr Costs costs<KqQ4>() { return {{14, 19, 18, 29, 0}, {{39, 56}, {50, 71}, {0, 0}}, {32, 38}, {0, 0}}; }
+template <> constexpr Costs costs<KqQ5>() { return {{13, 17, 19, 26, 40}, {{32, 47}, {51, 79}, {0, 0}}, {26, 41}, {0, 0}}; }
+template <> constexpr Costs costs<KqQ6>() { return {{17, 26, 21, 31, 43}, {{53, 74}, {66, 91}, {0, 0}}, {43, 0}, {40, 44}}; }
 
 template <class P>
 zhip_result launch_format(const Dispatch &d, const char *name, KqArgs a) {
@@ -593,11 +615,17 @@ zhip_result launch_format(const Dispatch &d, const char *name, KqArgs a) {
     constexpr uint32_t shapes[5][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {4, 2}};
     uint64_t least = ~0ull;
     int best = 0;
-    for (int i = 0; i < 8; i++) {
-        if (i >= 5 && c.whole[i - 5].lone == 0u) continue;
-        const uint64_t cost = i < 5 ? c.parts[i] * ((workgroups(shapes[i][0], shapes[i][1]) + cus - 1u) / cus) * (blocks + 3u) : c.whole[i - 5].of(workgroups(1u << (i - 5), 4u), cus) * (blocks + 2u);
+    auto consider = [&](int i, uint64_t cost) {
         if (cost < least) least = cost, best = i;
-    }
+    };
+    auto alone = [&](uint32_t each, uint32_t nt, uint32_t rw) { return each * ((workgroups(nt, rw) + cus - 1u) / cus) * (blocks + 3u); };
+    for (int i = 0; i < 5; i++)
+        if (c.parts[i] != 0u) consider(i, alone(c.parts[i], shapes[i][0], shapes[i][1]));
+    for (int i = 0; i < 3; i++)
+        if (c.whole[i].lone != 0u) consider(5 + i, c.whole[i].of(workgroups(1u << i, 4u), cus) * (blocks + 2u));
+    for (int i = 0; i < 2; i++)
+        if (c.halves[i] != 0u) consider(8 + i, alone(c.halves[i], 1u << i, 4u));
+    if (c.halves2.lone != 0u) consider(10, c.halves2.of(workgroups(2u, 2u), cus) * (blocks + 3u));
     // Matrices too large for the dies' L2s, several token tiles: 24576 x 3072 and 28672 x 4096 at 256 ... 512 tokens 1 - 8 % faster
     // column by column (two token tiles and one; four the same), matrices of up to 20 MB up to 4 % slower.
     a.by_die = (uint64_t)a.n * a.row_bytes >= (24u << 20);
@@ -606,12 +634,19 @@ zhip_result launch_format(const Dispatch &d, const char *name, KqArgs a) {
     case 1: return launch_tile<P, 1, 2, 4>(d, name, a);
     case 2: return launch_tile<P, 2, 1, 4>(d, name, a);
     case 3: return launch_tile<P, 2, 2, 4>(d, name, a);
-    case 4: return launch_tile<P, 4, 2, 4>(d, name, a);
     case 5: return launch_tile<P, 1, 4, 1>(d, name, a);
     case 6: return launch_tile<P, 2, 4, 1>(d, name, a);
+    case 8: return launch_tile<P, 1, 4, 2>(d, name, a);
     default: break;
     }
-    if constexpr (c.whole[2].lone != 0u) return launch_tile<P, 4, 4, 1>(d, name, a);
+    if constexpr (c.parts[4] != 0u)
+        if (best == 4) return launch_tile<P, 4, 2, 4>(d, name, a);
+    if constexpr (c.halves[1] != 0u)
+        if (best == 9) return launch_tile<P, 2, 4, 2>(d, name, a);
+    if constexpr (c.whole[2].lone != 0u)
+        if (best == 7) return launch_tile<P, 4, 4, 1>(d, name, a);
+    if constexpr (c.halves2.lone != 0u)
+        if (best == 10) return launch_tile<P, 2, 2, 2>(d, name, a);
     return fail(d, ZHIP_E_GPU, "%s: no launch", name);
 }
 
