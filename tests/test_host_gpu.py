@@ -43,6 +43,22 @@ def test_new_buffers_read_as_zero_and_round_trip(ctx):
     assert np.array_equal(got[100:110], data[:10]) and np.array_equal(got[:100], data[:100])
 
 
+def test_a_batch_of_many_completions(ctx):
+    """One completion per read and per submit, in their order, of more commands than the host keeps room for."""
+    c = ctx
+    data = c.random(16, 1)
+    buf, got = c.upload(data), np.zeros(16, np.float32)
+    done = []
+    for i in range(1500):
+        if i % 3 == 0:
+            c.rec.read_buffer(9000 + i, buf.buffer, 0, got)
+        c.rec.submit(i + 1)
+    c.host.execute(c.rec.batch(), done)
+    c.rec.clear()
+    want = [t for i in range(1500) for t in ([9000 + i] if i % 3 == 0 else []) + [i + 1]]
+    assert [d.token for d in done] == want and np.array_equal(got, data)
+
+
 @pytest.mark.parametrize("words", [1, 3, 4, 16383, 16384, 16385, 131072, 131073, 262144, 2300000])
 def test_transfers_of_every_length(ctx, words):
     """Short writes go through pinned memory and long ones otherwise (64 KB), reads in pieces (128 KB; a

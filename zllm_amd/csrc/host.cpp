@@ -307,6 +307,7 @@ struct zhip_context {
         uint64_t used = 0;
     };
     std::vector<Replay> replays;
+    std::vector<uint8_t> replay_scratch;  // the key of the submit at hand
     uint64_t replay_clock = 0;
     bool use_graphs = true;
     uint64_t replayed_submits = 0;
@@ -533,26 +534,35 @@ size_t replayable_prefix(zhip_context *c) {
 }
 
 zhip_result replay_key(zhip_context *c, size_t count, std::vector<uint8_t> &key) {
-    key.clear();
-    auto put_bytes = [&](const void *p, size_t n) { key.insert(key.end(), (const uint8_t *)p, (const uint8_t *)p + n); };
-    char err[384];
+    // A launch's function, variant, grid and bound device ranges, then its parameters.
+    struct Launch {
+        LaunchFn fn;
+        uint32_t variant, grid[3];
+        struct {
+            const uint8_t *ptr;
+            uint64_t size;
+        } bind[8];
+    };
     // Launchers may point kernels at the workspace: a graph captured with an allocation
     // that has since been replaced must never match again.
     const uint64_t work[2] = {(uint64_t)(uintptr_t)c->work.data, c->work.bytes};
-    put_bytes(work, sizeof work);
+    key.resize(sizeof work);
+    memcpy(key.data(), work, sizeof work);
+    char err[384];
     for (size_t i = 0; i < count; i++) {
         Dispatch d;
         Pipeline *pl = nullptr;
         if (zhip_result r = prepare_dispatch(c, c->ops[i], d, pl, err, sizeof err)) return r;
-        const LaunchFn fn = pl->launch;
-        put_bytes(&fn, sizeof fn);
-        put_bytes(&d.variant, sizeof d.variant);
-        put_bytes(d.grid, sizeof d.grid);
+        Launch l{pl->launch, d.variant, {d.grid[0], d.grid[1], d.grid[2]}, {}};
         for (uint32_t b = 0; b < 8; b++) {
-            const uint64_t range[3] = {d.bind[b].bound ? 1ull : 0ull, (uint64_t)(uintptr_t)d.bind[b].ptr, d.bind[b].size};
-            put_bytes(range, sizeof range);
+            // (a range that is not bound is no range's equal)
+            l.bind[b].ptr = d.bind[b].bound ? d.bind[b].ptr : nullptr;
+            l.bind[b].size = d.bind[b].bound ? d.bind[b].size : ~0ull;
         }
-        put_bytes(d.params, d.params_size);
+        const size_t at = key.size();
+        key.resize(at + sizeof l + d.params_size);
+        memcpy(key.data() + at, &l, sizeof l);
+        memcpy(key.data() + at + sizeof l, d.params, d.params_size);
     }
     return ZHIP_OK;
 }
@@ -594,7 +604,7 @@ zhip_result capture_replay(zhip_context *c, size_t count, hipGraphExec_t *out) {
 // one by one.
 zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **out) {
     *out = nullptr;
-    std::vector<uint8_t> key;
+    std::vector<uint8_t> &key = c->replay_scratch;
     if (zhip_result r = replay_key(c, count, key)) return r;
     zhip_context::Replay *entry = nullptr;
     for (auto &e : c->replays)
@@ -611,7 +621,7 @@ zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **ou
             if (entry->exec) (void)hipGraphExecDestroy(entry->exec);
             *entry = zhip_context::Replay();
         }
-        entry->key = std::move(key);
+        entry->key = key;
         entry->used = ++c->replay_clock;
         return ZHIP_OK;
     }
