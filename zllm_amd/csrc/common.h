@@ -86,6 +86,26 @@ struct Workspace {
     void release();
 };
 
+// Activations as a float rung's multiplies read them: two bytes a value, or two such planes (the rounded values and what each
+// rounding left). Such a multiply packs its f32 activations in a pass of its own, unless the dispatch right before it
+// wrote exactly those values: it has them in registers and stores them packed as well, the same roundings. A pass reads six bytes
+// a value from L2 and is a launch that the multiply waits for. us a step, passes / packed by the writers: six layers of 4096 x
+// 14336 with Q8_0 in bf16, 512 tokens, 2277 / 2187; twelve of 2048 x 6144 in f16, 128 tokens, 856 / 744; twelve of 1024 x 3072
+// in bf16, 17 tokens, 420 / 330; in two f16 planes, 100 tokens, 933 / 874.
+struct PackedCopy {
+    enum Kind : uint32_t { none, bf16, f16, f16_split };
+    static constexpr uint64_t kMost = 64u << 20;  // a writer packs up to here: 512 tokens of 65,536 values
+    const float *x = nullptr;  // rows x k values, dense
+    uint32_t rows = 0, k = 0;
+    Kind kind = none;
+    Workspace *room = nullptr;
+    uint8_t *data = nullptr;   // set once they have been written
+    uint64_t plane() const { return ((uint64_t)rows * k * 2u + 255u) & ~255ull; }
+    bool of(const float *p, uint32_t r, uint32_t c, Kind as) const { return kind == as && as != none && x == p && rows == r && k == c; }
+    // Where their writer puts them: null if they are too many or memory is short (the multiply then packs them itself).
+    uint8_t *reserve(const Dispatch &d) const;
+};
+
 // One resolved dispatch: binding 0's bytes come from the host's shadow copy of
 // the uniform buffer, so kernels take their parameters by value.
 struct Dispatch {
@@ -97,6 +117,9 @@ struct Dispatch {
     hipStream_t stream = nullptr;
     const DeviceInfo *dev = nullptr;
     Workspace *work = nullptr;
+    PackedCopy *wanted = nullptr;      // a float rung's multiply: nothing is launched, what it would pack is left there
+    PackedCopy *next = nullptr;        // what the dispatch behind this one would pack
+    const PackedCopy *have = nullptr;  // what the dispatch before this one has packed
     char *err = nullptr;  // message buffer for a failed launch
     size_t err_cap = 0;
 };

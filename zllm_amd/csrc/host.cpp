@@ -252,6 +252,13 @@ zhip_result Workspace::reserve(const Dispatch &d, uint64_t want) {
     return ZHIP_OK;
 }
 
+uint8_t *PackedCopy::reserve(const Dispatch &d) const {
+    const uint64_t want = kind == f16_split ? 2u * plane() : plane();
+    Dispatch quiet = d;
+    quiet.err_cap = 0;
+    return room && want <= kMost && room->reserve(quiet, want) == ZHIP_OK ? room->data : nullptr;
+}
+
 void Workspace::release() {
     if (data && !fixed) (void)hipFree(data);
     data = nullptr;
@@ -264,6 +271,9 @@ struct zhip_context {
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
     DeviceInfo info;
     Workspace work;
+    Workspace copies[2];       // packed activations: one is read while the next is written
+    uint32_t copies_made = 0;  // since the submit began
+    PackedCopy copy;           // that the last dispatch left, for the one behind it
     zhip_caps caps{};
     bool lost = false;
     std::string message;
@@ -461,13 +471,58 @@ zhip_result prepare_dispatch(zhip_context *c, const Op &op, Dispatch &d, Pipelin
     return ZHIP_OK;
 }
 
+bool is_float_rung(const Pipeline &pl) {
+    return pl.launch && pl.info && (pl.launch == pl.info->launch_bf16 || pl.launch == pl.info->launch_f16 || pl.launch == pl.info->launch_f16c);
+}
+
+// What the dispatch behind op number `at` would pack, if it is a float rung's multiply whose parameters the host holds.
+PackedCopy wanted_behind(zhip_context *c, size_t at) {
+    PackedCopy want;
+    if (at + 1 >= c->ops.size() || c->ops[at + 1].kind != Op::dispatch) return want;
+    const Op &op = c->ops[at + 1];
+    Pipeline *pl = get(c->pipelines, op.pipeline);
+    if (!pl || !is_float_rung(*pl)) return want;
+    const Buffer *ub = op.group.e[0].bound ? get(c->buffers, op.group.e[0].buffer) : nullptr;
+    if (!ub || !ub->shadowed || ub->shadow_stale) return want;
+    Dispatch d;
+    char err[384];
+    // What is wrong with it is reported when its turn comes.
+    std::string message = c->message;
+    const zhip_result r = prepare_dispatch(c, op, d, pl, err, sizeof err);
+    c->message = std::move(message);
+    d.wanted = &want;
+    if (r != ZHIP_OK || pl->launch(d) != ZHIP_OK) return PackedCopy{};
+    want.room = &c->copies[c->copies_made & 1u];
+    return want;
+}
+
+// Launches the dispatch that is op number `at`. What it packs for the one behind it holds for that one alone: whatever else
+// comes between may write there. (Under a profile every dispatch does its own work.)
+zhip_result launch_dispatch(zhip_context *c, size_t at, Dispatch &d, const Pipeline &pl) {
+    const PackedCopy have = c->copy;
+    PackedCopy next;
+    c->copy = PackedCopy{};
+    if (!c->profiling) {
+        if (pl.launch == launch_silu_mul || is_float_rung(pl)) next = wanted_behind(c, at);
+        d.have = &have;
+        d.next = &next;
+    }
+    const zhip_result r = pl.launch(d);
+    if (r == ZHIP_OK && next.data) {
+        c->copy = next;
+        c->copies_made++;
+    }
+    return r;
+}
+
 void mark_outputs(zhip_context *c, const Op &op, const Pipeline &pl) {
     for (uint32_t b = 1; b < 8; b++)
         if (op.group.e[b].bound && (pl.info->writes >> b & 1u))
             if (Buffer *buf = get(c->buffers, op.group.e[b].buffer)) mark_written(*buf);
 }
 
-zhip_result run_dispatch(zhip_context *c, const Op &op, size_t &timed) {
+zhip_result run_dispatch(zhip_context *c, size_t at, size_t &timed) {
+    const Op &op = c->ops[at];
     Dispatch d;
     Pipeline *pl = nullptr;
     char err[384] = "";
@@ -483,7 +538,7 @@ zhip_result run_dispatch(zhip_context *c, const Op &op, size_t &timed) {
         }
         if (zhip_result r = hip_check(c, hipEventRecord(c->events[2 * timed], c->stream), "hipEventRecord")) return r;
     }
-    const zhip_result r = pl->launch(d);
+    const zhip_result r = launch_dispatch(c, at, d, *pl);
     if (r != ZHIP_OK) {
         c->message = err[0] ? err : "kernel launch failed";
         return r;
@@ -543,9 +598,10 @@ zhip_result replay_key(zhip_context *c, size_t count, std::vector<uint8_t> &key)
             uint64_t size;
         } bind[8];
     };
-    // Launchers may point kernels at the workspace: a graph captured with an allocation
+    // Launchers may point kernels at the workspaces: a graph captured with an allocation
     // that has since been replaced must never match again.
-    const uint64_t work[2] = {(uint64_t)(uintptr_t)c->work.data, c->work.bytes};
+    const uint64_t work[6] = {(uint64_t)(uintptr_t)c->work.data, c->work.bytes, (uint64_t)(uintptr_t)c->copies[0].data, c->copies[0].bytes,
+        (uint64_t)(uintptr_t)c->copies[1].data, c->copies[1].bytes};
     key.resize(sizeof work);
     memcpy(key.data(), work, sizeof work);
     char err[384];
@@ -575,13 +631,16 @@ zhip_result capture_replay(zhip_context *c, size_t count, hipGraphExec_t *out) {
         return ZHIP_E_GPU;
     }
     zhip_result failed = ZHIP_OK;
+    c->copy = PackedCopy{};
+    c->copies_made = 0;
     char err[384];
     for (size_t i = 0; i < count && failed == ZHIP_OK; i++) {
         Dispatch d;
         Pipeline *pl = nullptr;
         failed = prepare_dispatch(c, c->ops[i], d, pl, err, sizeof err);
-        if (failed == ZHIP_OK) failed = pl->launch(d);
+        if (failed == ZHIP_OK) failed = launch_dispatch(c, i, d, *pl);
     }
+    c->copy = PackedCopy{};
     hipGraph_t graph = nullptr;
     const hipError_t ended = hipStreamEndCapture(c->stream, &graph);
     if (ended != hipSuccess || failed != ZHIP_OK || !graph) {
@@ -738,12 +797,15 @@ zhip_result run_queue(zhip_context *c) {
             replay->unusable = true;
         }
     }
+    c->copy = PackedCopy{};
+    c->copies_made = 0;
     for (size_t at = replayed ? prefix : 0; at < c->ops.size(); at++) {
         const Op &op = c->ops[at];
+        if (op.kind != Op::dispatch) c->copy = PackedCopy{};
         switch (op.kind) {
         case Op::dispatch: {
             const size_t before = timed;
-            if (zhip_result r = run_dispatch(c, op, timed)) return r;
+            if (zhip_result r = run_dispatch(c, at, timed)) return r;
             if (timed != before) keys.push_back(TimingKey{op.pipeline, {op.grid[0], op.grid[1], op.grid[2]}});
             dispatches++;
             break;
@@ -1162,6 +1224,7 @@ zhip_result zhip_destroy(zhip_context *c) {
     for (auto &e : c->replays)
         if (e.exec) (void)hipGraphExecDestroy(e.exec);
     c->work.release();
+    for (Workspace &w : c->copies) w.release();
     for (hipEvent_t ev : c->events) (void)hipEventDestroy(ev);
     if (c->arrived) (void)hipFree(c->arrived);
     if (c->signals) (void)hipHostFree(c->signals);

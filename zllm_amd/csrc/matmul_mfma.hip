@@ -84,6 +84,8 @@ struct MfmaArgs {
     uint32_t row_bytes;
     uint32_t x_bytes, w_bytes;  // bytes the kernel may read behind x and w
     uint32_t x_plane;           // compensated rung: bytes from the activations' f16 values to their residuals
+    uint8_t *copy;              // not null: the outputs packed, dense, for the next multiply (common.h, PackedCopy)
+    uint64_t copy_plane;
 };
 
 // Two floats to packed bf16, round to nearest even as the reference narrows
@@ -446,6 +448,14 @@ __global__ __launch_bounds__(THREADS) void matmul_mfma_kernel(MfmaArgs a) {
                     f32x4 *o4 = reinterpret_cast<f32x4 *>(o);
                     if (a.accumulate) v += *o4;
                     *o4 = v;
+                    if (a.copy) {
+                        uint8_t *to = a.copy + ((size_t)t * a.n + col) * 2u;
+                        const uint2 hi = {H::pack(v[0], v[1]), H::pack(v[2], v[3])};
+                        *reinterpret_cast<uint2 *>(to) = hi;
+                        if constexpr (COMP)
+                            *reinterpret_cast<uint2 *>(to + a.copy_plane) = uint2{H::pack(__fsub_rn(v[0], H::widen(hi.x & 0xffffu)), __fsub_rn(v[1], H::widen(hi.x >> 16))),
+                                H::pack(__fsub_rn(v[2], H::widen(hi.y & 0xffffu)), __fsub_rn(v[3], H::widen(hi.y >> 16)))};
+                    }
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; r++)
@@ -515,9 +525,9 @@ bool matmul_q8_bf16_accepts(uint32_t k, uint32_t k_slice, uint32_t slices);
 // The same for matrices with enough rows for 128-row tiles (matmul_q8_bf16_wide.hip).
 bool matmul_q8_bf16_wide_accepts(const Dispatch &d, uint32_t n);
 zhip_result launch_matmul_q8_bf16_wide(const Dispatch &d, const char *name, bool f16, const uint8_t *x, const uint8_t *w, float *out, uint32_t rows,
-    uint32_t n, uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes);
+    uint32_t n, uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes, uint8_t *copy);
 zhip_result launch_matmul_q8_bf16(const Dispatch &d, const char *name, bool f16, const uint8_t *x, const uint8_t *w, float *out, uint32_t rows, uint32_t n,
-    uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes);
+    uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes, uint8_t *copy);
 
 template <class W, class H, int MT, bool RAGGED, bool COMP = false>
 static zhip_result launch_kernel(const Dispatch &d, const char *name, const MfmaArgs &a, uint32_t slices) {
@@ -557,7 +567,20 @@ static zhip_result launch_mfma(const Dispatch &d, const char *name, bool sliced,
     if (x_bytes >= (1ull << 32) || w_bytes >= (1ull << 32)) return fail(d, ZHIP_E_BAD_COMMAND, "%s: operands of 4 GiB or more", name);
     a.x_bytes = (uint32_t)x_bytes;
     a.w_bytes = (uint32_t)w_bytes;
-    if (!XBF16) {
+    constexpr PackedCopy::Kind KIND = COMP ? PackedCopy::f16_split : std::is_same<H, F16>::value ? PackedCopy::f16 : PackedCopy::bf16;
+    const float *x32 = reinterpret_cast<const float *>(a.x);
+    if (d.wanted) {
+        if (!XBF16) *d.wanted = PackedCopy{x32, a.rows, a.k, KIND, nullptr, nullptr};
+        return ZHIP_OK;
+    }
+    if (!XBF16 && d.have && d.have->data && d.have->of(x32, a.rows, a.k, KIND)) {
+        // The dispatch that wrote the activations has packed them.
+        a.x = d.have->data;
+        if (COMP) {
+            a.x_plane = (uint32_t)d.have->plane();
+            a.x_bytes = (uint32_t)(d.have->plane() + x_bytes);
+        }
+    } else if (!XBF16) {
         // Narrow the step's activations once, into the workspace.
         if (!d.work) return fail(d, ZHIP_E_GPU, "%s: no workspace", name);
         const uint64_t plane = (x_bytes + 255u) & ~(uint64_t)255u;
@@ -592,25 +615,37 @@ static zhip_result launch_mfma(const Dispatch &d, const char *name, bool sliced,
     // the bytes cross from L2.
     if (kBf16Rung && slices == 1u && a.k_slice >= a.k && a.rows > kPlannerStepCap && (uint64_t)((a.rows + 255u) / 256u) * ((a.n + 127u) / 128u) >= (uint64_t)d.dev->compute_units)
         return launch_mfma_wide(d, name, q8_0, a.x, a.w, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate, a.row_bytes);
+    // Where the dispatch behind this one multiplies exactly the values stored here, they are packed as they are stored: every lane
+    // then stores four at a time.
+    uint8_t *copy = nullptr;
+    if (d.next && slices == 1u && a.col0 == 0u && a.out_stride == a.n && ((a.n | a.slice_stride) & 3u) == 0u && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0u &&
+        d.next->of(a.out, a.rows, a.n, KIND))
+        copy = d.next->reserve(d);
+    auto packed = [&](zhip_result r) {
+        if (r == ZHIP_OK && copy) d.next->data = copy;
+        return r;
+    };
     if constexpr (std::is_same<W, WQ8_0>::value && !COMP) {
         if (matmul_q8_bf16_accepts(a.k, a.k_slice, slices) && matmul_q8_bf16_wide_accepts(d, a.n))
-            return launch_matmul_q8_bf16_wide(d, name, std::is_same<H, F16>::value, a.x, a.w, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate,
-                a.row_bytes, a.x_bytes, a.w_bytes);
+            return packed(launch_matmul_q8_bf16_wide(d, name, std::is_same<H, F16>::value, a.x, a.w, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate,
+                a.row_bytes, a.x_bytes, a.w_bytes, copy));
         if (matmul_q8_bf16_accepts(a.k, a.k_slice, slices))
-            return launch_matmul_q8_bf16(d, name, std::is_same<H, F16>::value, a.x, a.w, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate, a.row_bytes,
-                a.x_bytes, a.w_bytes);
+            return packed(launch_matmul_q8_bf16(d, name, std::is_same<H, F16>::value, a.x, a.w, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate, a.row_bytes,
+                a.x_bytes, a.w_bytes, copy));
     }
     const bool ragged = a.k % BK != 0 || a.k_slice % BK != 0;
+    a.copy = copy;
+    a.copy_plane = copy ? d.next->plane() : 0u;
     if constexpr (COMP) {
         // Two planes of activations in LDS: 64-token tiles.
-        return ragged ? launch_kernel<W, H, 4, true, true>(d, name, a, slices) : launch_kernel<W, H, 4, false, true>(d, name, a, slices);
+        return packed(ragged ? launch_kernel<W, H, 4, true, true>(d, name, a, slices) : launch_kernel<W, H, 4, false, true>(d, name, a, slices));
     }
     // 128-token tiles unless those leave half of the CUs idle and 64-token tiles (which
     // convert every weight twice as often) still run in one round.
     const uint64_t tall = (uint64_t)((a.rows + 127u) / 128u) * ((a.n + BN - 1) / BN) * slices;
     if (a.rows > 64u && 2u * tall > (uint64_t)d.dev->compute_units)
-        return ragged ? launch_kernel<W, H, 8, true>(d, name, a, slices) : launch_kernel<W, H, 8, false>(d, name, a, slices);
-    return ragged ? launch_kernel<W, H, 4, true>(d, name, a, slices) : launch_kernel<W, H, 4, false>(d, name, a, slices);
+        return packed(ragged ? launch_kernel<W, H, 8, true>(d, name, a, slices) : launch_kernel<W, H, 8, false>(d, name, a, slices));
+    return packed(ragged ? launch_kernel<W, H, 4, true>(d, name, a, slices) : launch_kernel<W, H, 4, false>(d, name, a, slices));
 }
 
 // (matmul_q8_0_float with f32-bound activations on the bf16 rung: both tile heights, whole and ragged k)

@@ -256,6 +256,7 @@ __global__ __launch_bounds__((threads<RN>())) void matmul_q8_bf16_kernel(Q8Args 
                 f32x4 *o4 = reinterpret_cast<f32x4 *>(o);
                 if (a.accumulate) v += *o4;
                 *o4 = v;
+                if (a.copy) *reinterpret_cast<uint2 *>(a.copy + ((size_t)t * a.n + col) * 2u) = uint2{H::pack(v[0], v[1]), H::pack(v[2], v[3])};
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)
@@ -324,11 +325,11 @@ bool matmul_q8_bf16_accepts(uint32_t k, uint32_t k_slice, uint32_t slices) { ret
 
 // x: the activations packed two bytes a value, bf16 or (f16 = true) f16.
 zhip_result launch_matmul_q8_bf16(const Dispatch &d, const char *name, bool f16, const uint8_t *x, const uint8_t *w, float *out, uint32_t rows, uint32_t n,
-    uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes) {
+    uint32_t k, uint32_t col0, uint32_t out_stride, uint32_t accumulate, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes, uint8_t *copy) {
     Q8Args a{};
     a.x = x; a.w = w; a.out = out;
     a.rows = rows; a.n = n; a.k = k; a.col0 = col0; a.out_stride = out_stride; a.accumulate = accumulate;
-    a.row_bytes = row_bytes; a.x_bytes = x_bytes; a.w_bytes = w_bytes;
+    a.row_bytes = row_bytes; a.x_bytes = x_bytes; a.w_bytes = w_bytes; a.copy = copy;
     return f16 ? launch_as<AsF16>(d, name, a) : launch_as<AsBf16>(d, name, a);
 }
 

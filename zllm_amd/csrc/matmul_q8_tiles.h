@@ -29,6 +29,7 @@ struct Q8Args {
     float *out;
     uint32_t rows, n, k, col0, out_stride, accumulate, row_bytes;
     uint32_t x_bytes, w_bytes;  // bytes the kernel may read behind x and w
+    uint8_t *copy;              // not null: the outputs packed, dense, for the next multiply (common.h, PackedCopy)
 };
 
 // The operand type of a rung: two floats rounded into one word, and the matrix instruction.
