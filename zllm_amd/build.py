@@ -19,6 +19,8 @@ HEADERS = ["common.h", "decode.h", "handover.h", "matvec_common.h", "matvec_quan
 HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-ffp-contract=on",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # A kernel's first parameters in registers when its waves start (fourteen words of them, up to the first struct).
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-warning-option",
 ]
 

@@ -22,6 +22,22 @@ struct MvArgs {
     float act_div;       // > 0: inputs staged as silu(x / act_div)
 };
 
+// What a multiply's first loads are addressed by comes ahead of its other parameters, as parameters of their own: the first fourteen
+// words of those are in the wave's registers when it starts (the compiler's -amdgpu-kernarg-preload-count), a struct is
+// fetched from memory first: 0.2 - 0.3 us of a launch (2 MB read by 256 workgroups 3.03 -> 2.82 us behind the launch before). us a
+// token, 28 layers of 1024 x 3072 Q8_0 432 -> 391, bf16 486 -> 439; twelve of 2560 x 9728 Q5_K, two tokens, 513 -> 494. The outputs' stride gives its place to a gate / up step's `half`, and the count of tokens gives its to
+// eps where a workgroup has one token: those are fetched behind the first loads, and late is soon enough for them. (k and the flags
+// share a word: rows of 16 M weights and more have no kernel that takes its parameters so.)
+#define MV_FIRST const float *first_x, const uint8_t *first_w, const float *first_norm_w, float *first_out, uint32_t first_k, uint32_t first_rows, \
+    uint32_t first_row_bytes, uint32_t first_step, uint32_t first_xr, uint32_t first_m, float late_eps, float late_act_div, uint32_t late_out_stride
+#define MV_TAKE_FIRST(MT, PAIR)                                                                                                                           \
+    MvArgs { first_x, first_w, first_out, first_norm_w, 0u, first_k & 0xffffffu, 0u, PAIR ? late_out_stride : first_step,                                     \
+        MT == 1 ? __uint_as_float(first_m) : late_eps, first_k >> 24, first_step, first_xr, MT == 1 ? 1u : first_m, first_rows, first_row_bytes, late_act_div }
+// The tokens from t0 on.
+#define MV_GIVE_FIRST(MT, a, t0) (a).x + (size_t)(t0) * (a).xr, (a).w, (a).norm_w, (a).out + (size_t)(t0) * (a).out_stride + (a).col0, (a).k | (a).flags << 24, (a).rows, \
+    (a).row_bytes, (a).flags & FLAG_SILU_PAIR ? (a).half : (a).out_stride, (a).xr, MT == 1 ? __builtin_bit_cast(uint32_t, (a).eps) : (a).m - (t0), (a).eps, (a).act_div, \
+    (a).out_stride
+
 // The sum over a wave's lanes, in every lane: pairs 32, 16, 8, 4, 2 and 1 lanes apart, in that
 // order. Nothing goes through LDS: the halves and the rows of sixteen trade places
 // (v_permlane32_swap, v_permlane16_swap), the rest are DPP operands of the additions. A rotation

@@ -44,14 +44,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // ROWS: weight rows a wave multiplies in a pass (with PAIR half of them gate rows, half up rows). KEEP: the
 // outputs of 64 / OUTS passes wait in the lanes for one store; see launch_iters.
 template <class D, int MT, int ITERS, bool PAIR, int ROWS, bool KEEP>
-__global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
+__global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MV_FIRST) {
+    MvArgs a = MV_TAKE_FIRST(MT, PAIR);
     extern __shared__ float4 xs4[];
     __shared__ float red[4 * MT];
     constexpr int OUTS = PAIR ? ROWS / 2 : ROWS, XV = (ITERS + 1) / 2;
     // A step of more tokens than the registers hold: workgroups of their own for every MT of them.
     a.x += (size_t)(MT * blockIdx.y) * a.xr;
-    a.out += (size_t)(MT * blockIdx.y) * a.out_stride;
-    a.m -= MT * blockIdx.y;
+    if (MT > 1) a.m -= MT * blockIdx.y;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t k4 = a.k / 4u, tasks = a.k / 8u;
     const uint32_t passes = (a.rows + OUTS - 1u) / OUTS;
@@ -81,6 +81,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
         u32x4 q[ROWS][ITERS];
         float before[MT];
     };
+    auto out_at = [&](int t, uint32_t j) __attribute__((always_inline)) { return a.out + (size_t)(MT * blockIdx.y + t) * a.out_stride + j; };
     auto fetch = [&](uint32_t u, Pass &p) __attribute__((always_inline)) {
         const bool live = u < passes;
         const uint64_t off = live ? (uint64_t)u * OUTS * a.row_bytes : 0u;
@@ -92,10 +93,11 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
 #pragma unroll
             for (int it = 0; it < ITERS; it++)
                 p.q[r][it] = __builtin_amdgcn_raw_buffer_load_b128(PAIR && r >= OUTS ? up : gate, (it == ITERS - 1 ? last_at : at) + (uint32_t)(PAIR && r >= OUTS ? r - OUTS : r) * a.row_bytes + 1024u * it, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);  // (the loads stay ahead of the multiply that follows them in the source)
         const uint32_t j = u * OUTS + lane;
 #pragma unroll
-        for (int t = 0; t < MT; t++) p.before[t] = !KEEP && accumulate && (uint32_t)t < a.m && lane < (uint32_t)OUTS && j < a.rows ? a.out[(size_t)t * a.out_stride + a.col0 + j] : 0.f;
-        __builtin_amdgcn_sched_barrier(0);  // (the loads stay ahead of the multiply that follows them in the source)
+        for (int t = 0; t < MT; t++) p.before[t] = !KEEP && accumulate && (uint32_t)t < a.m && lane < (uint32_t)OUTS && j < a.rows ? *out_at(t, j) : 0.f;
+        __builtin_amdgcn_sched_barrier(0);
     };
     Pass buf[2];
     fetch(first, buf[0]);
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
             for (int t = 0; t < MT; t++) {
                 if ((uint32_t)t >= a.m) break;
                 float v = PAIR ? silu_f(v0[t]) * v1[t] : v0[t];
-                float *o = a.out + (size_t)t * a.out_stride + a.col0 + j;
+                float *o = out_at(t, j);
                 if (accumulate) v += *o;
                 *o = v;
             }
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MvArgs a) {
                 if ((uint32_t)t >= a.m) break;
                 float v = PAIR ? silu_f(v0[t]) * v1[t] : v0[t];
                 if (accumulate) v += p.before[t];
-                a.out[(size_t)t * a.out_stride + a.col0 + j] = v;
+                *out_at(t, j) = v;
             }
         }
     };
@@ -254,12 +256,12 @@ zhip_result launch_iters(const Dispatch &d, const MvArgs &a) {
     const bool keep = (a.rows + outs - 1u) / outs > (pair ? 20u : 12u) * blocks;
     if constexpr (PAIR_KEEPS)
         if (pair && keep) {
-            hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2, true>), grid, dim3(256), lds, d.stream, a);
+            hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2, true>), grid, dim3(256), lds, d.stream, MV_GIVE_FIRST(MT, a, 0));
             return check_launch(d, D::name());
         }
-    if (pair) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2, false>), grid, dim3(256), lds, d.stream, a);
-    else if (keep) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS, true>), grid, dim3(256), lds, d.stream, a);
-    else hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS, false>), grid, dim3(256), lds, d.stream, a);
+    if (pair) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, true, 2, false>), grid, dim3(256), lds, d.stream, MV_GIVE_FIRST(MT, a, 0));
+    else if (keep) hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS, true>), grid, dim3(256), lds, d.stream, MV_GIVE_FIRST(MT, a, 0));
+    else hipLaunchKernelGGL((matvec_half_row_kernel<D, MT, ITERS, false, ROWS, false>), grid, dim3(256), lds, d.stream, MV_GIVE_FIRST(MT, a, 0));
     return check_launch(d, D::name());
 }
 

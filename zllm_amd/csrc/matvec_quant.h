@@ -914,17 +914,17 @@ __global__ __launch_bounds__(256) void matvec_quant_kernel(KArgs q) {
 // asked for only once the inputs have arrived 8.0 us.
 constexpr int kRowDepth = 1;
 template <class P, int MT, bool PAIR, bool TURNS, int SEG_LOG2, bool KEEP>
-__global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
-    q.t0 += MT * blockIdx.y;  // (a step of more tokens: workgroups of their own for every MT of them)
-    const bool full = MT == 1 || q.t0 + MT <= q.a.m;  // (of two tokens the second may be absent: it runs as the first again and is not stored)
+__global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks nm) {
+    const MvArgs a = MV_TAKE_FIRST(MT, PAIR);
+    const uint32_t t0 = MT * blockIdx.y;  // (a step of more tokens: workgroups of their own for every MT of them)
+    const bool full = MT == 1 || t0 + MT <= a.m;  // (of two tokens the second may be absent: it runs as the first again and is not stored)
     static_assert(PAIR || !TURNS, "rows in turn are a pair's");
-    const MvArgs &a = q.a;
     extern __shared__ float4 lds4[];
     __shared__ float red[4 * MT];
     constexpr int NSUM = P::NSUM, RUN = 64 / NSUM, kRows = PAIR && !TURNS ? 2 : 1;
     constexpr uint32_t SEG = 1u << SEG_LOG2, RPI = 64u >> SEG_LOG2;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t tasks = q.tasks, k4 = a.k / 4u;
+    const uint32_t tasks = a.k / 64u, k4 = a.k / 4u;
     const uint32_t tok_stride4 = tasks * (kTaskStride / 4u);  // float4s per token
     const uint32_t tsub = lane & (SEG - 1u), rsub = lane >> SEG_LOG2;
     const uint32_t units = (a.rows + RPI - 1u) / RPI;
@@ -939,7 +939,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
         const uint32_t i = tid + 256u * j;
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            const float4 *xrow = reinterpret_cast<const float4 *>(a.x + (size_t)(q.t0 + (full ? t : 0)) * a.xr);
+            const float4 *xrow = reinterpret_cast<const float4 *>(a.x + (size_t)(t0 + (full ? t : 0)) * a.xr);
             xv[t][j] = i < k4 ? xrow[i] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
@@ -1036,10 +1036,9 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(KArgs q) {
             for (int e = 0; e < RUN; e++) xsum[t][s] += xr[t][s * RUN + e];
         }
     }
-    const Masks nm = q.nm;
     const typename P::Keys ch = P::keys(tsub & 3u);
     const bool accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
-    auto out_at = [&](int t, uint32_t j) { return (size_t)(q.t0 + t) * a.out_stride + a.col0 + j; };
+    auto out_at = [&](int t, uint32_t j) { return (size_t)(t0 + t) * a.out_stride + a.col0 + j; };
 
     // With KEEP a pass's finished sums wait in the lanes, the gate's and the up row's apart: lane tsub of
     // row rsub's segment holds that row's of the wave's pass numbered tsub since the last store. SEG
@@ -1379,10 +1378,10 @@ static zhip_result run_long(const Dispatch &d, const KArgs &q, uint32_t blocks) 
 // rows of the next round.
 // K4: the most vectors of four inputs a token has (4096: k <= 16384; 8192: k <= 32768).
 template <class P, int MT, bool PAIR, int R, int NW, int K4 = 4096>
-__global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
-    q.t0 += MT * blockIdx.y;
-    const bool full = MT == 1 || q.t0 + MT <= q.a.m;
-    const MvArgs &a = q.a;
+__global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(MV_FIRST, Masks nm) {
+    const MvArgs a = MV_TAKE_FIRST(MT, PAIR);
+    const uint32_t t0 = MT * blockIdx.y;
+    const bool full = MT == 1 || t0 + MT <= a.m;
     extern __shared__ float4 lds4[];  // the tokens in task order, padded per task; then the partial sums [parity][group][unit of the round][slice][row][token][lane]
     __shared__ float red[4 * MT];
     constexpr int NSUM = P::NSUM, RUN = 64 / NSUM, kRows = PAIR ? 2 : 1;
@@ -1391,7 +1390,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
     static_assert(R % 2 == 0, "the buffers alternate by name");
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t tasks = q.tasks, slices = (tasks + 63u) / 64u, k4 = a.k / 4u;
+    const uint32_t tasks = a.k / 64u, slices = (tasks + 63u) / 64u, k4 = a.k / 4u;
     const uint32_t tok_stride4 = tasks * (kTaskStride / 4u);  // float4s per token
     const uint32_t groups_here = (uint32_t)NW / slices;
     const uint32_t grp = wave / slices, slice = wave % slices;
@@ -1401,7 +1400,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
     const bool active = task < tasks;
     const bool norm = (a.flags & FLAG_NORM) != 0, accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
     const float4 *nw = reinterpret_cast<const float4 *>(a.norm_w);
-    auto token_row = [&](int t) { return reinterpret_cast<const float4 *>(a.x + (size_t)(q.t0 + (full ? t : 0)) * a.xr); };
+    auto token_row = [&](int t) { return reinterpret_cast<const float4 *>(a.x + (size_t)(t0 + (full ? t : 0)) * a.xr); };
 
     // Unit n of the group's walk: R consecutive units a round, the groups' rounds interleaved.
     auto unit_of = [&](uint32_t n) { return ((n / R) * groups + group) * R + n % R; };
@@ -1489,9 +1488,8 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
             for (int e = 0; e < RUN; e++) xsum[t][sr] += xr[t][sr * RUN + e];
         }
     }
-    const Masks nm = q.nm;
     const typename P::Keys ch = P::keys(task & 3u);
-    auto out_at = [&](int t, uint32_t j) { return (size_t)(q.t0 + t) * a.out_stride + a.col0 + j; };
+    auto out_at = [&](int t, uint32_t j) { return (size_t)(t0 + t) * a.out_stride + a.col0 + j; };
     // (the partial sums lie behind the tokens: no barrier between reading the one and writing the other)
     float *part = reinterpret_cast<float *>(lds4 + (size_t)MT * tok_stride4);
     constexpr uint32_t kMine = 2;  // units of a round a wave finishes, at most: R <= 4 over two or more slices
@@ -1569,7 +1567,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(KArgs q) {
 template <class P, int MT, bool PAIR, int R, int NW, int K4 = 4096>
 static zhip_result run_slices(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     if (!lds_opt_in<matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
-    hipLaunchKernelGGL((matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>), dim3(blocks, (q.a.m - q.t0 + MT - 1u) / MT), dim3(64 * NW), lds, d.stream, q);
+    hipLaunchKernelGGL((matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>), dim3(blocks, (q.a.m - q.t0 + MT - 1u) / MT), dim3(64 * NW), lds, d.stream, MV_GIVE_FIRST(MT, q.a, q.t0), q.nm);
     return check_launch(d, P::name());
 }
 
@@ -1586,7 +1584,7 @@ template <class P, int MT, bool PAIR, int SEG_LOG2, bool KEEP>
 static zhip_result run_row_kernel(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     constexpr auto kernel = matvec_quant_row_kernel<P, MT, PAIR, row_turns<P, MT, PAIR, SEG_LOG2>(), SEG_LOG2, KEEP>;
     if (lds > 65536u && !lds_opt_in<kernel, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
-    hipLaunchKernelGGL(kernel, dim3(blocks, (q.mt + MT - 1u) / MT), dim3(256), lds, d.stream, q);
+    hipLaunchKernelGGL(kernel, dim3(blocks, (q.mt + MT - 1u) / MT), dim3(256), lds, d.stream, MV_GIVE_FIRST(MT, q.a, q.t0), q.nm);
     return check_launch(d, P::name());
 }
 // Whether a wave's sums wait for one store in SEG passes (the stores go between the loads of the stream otherwise), by the passes a wave has. Whole-wave
