@@ -1428,6 +1428,33 @@ def test_repad_pads_blocks(ctx):
     assert np.array_equal(got[:, :src_bytes], raw) and not got[:, src_bytes:].any()
 
 
+@pytest.mark.parametrize("fmt,k", [("q8_0", 64), ("q4_k", 256), ("q8_0", 2112), ("q6_k", 3072), ("bf16", 128), ("f16", 1032)])
+@pytest.mark.parametrize("n", [1, 67, 8193, 140003])
+def test_matvec_adds_to_what_its_outputs_held(ctx, fmt, k, n):
+    """A step that adds asks for what its outputs hold ahead of the sums, a pass or a store of many passes at a time
+    (140003 rows: several such stores a wave). Exactly the step that does not add, plus what was there; one, two and three tokens."""
+    c = ctx
+    if n * k > 1 << 25:
+        n = (1 << 25) // k + 3
+    if fmt in ("bf16", "f16"):
+        wa, kernel = c.upload(random_half(c, n * k, 1, fmt)[0].reshape(n, k)), Kernel["matvec_" + fmt]
+    else:
+        wa, kernel = c.gpu_weights(TensorType[fmt], synth.random_blocks(c.rand, fmt, n, k), k), K.weight_kernel("matvec", TensorType[fmt])
+    grid_x, col0, stride = K.div_ceil(n, K.MatvecVariant().group_rows()), 3, n + 5
+    for m in (1, 2, 3):
+        xa, init = c.upload(c.random(m * k, 2)), c.random(m * stride, 4).reshape(m, stride)
+        got = {}
+        for accumulate in (False, True):
+            out = c.upload(init)
+            c.launcher().launch(kernel, P.MatvecBf16(n=n, k=k, col0=col0, out_stride=stride, eps=1e-6, accumulate=accumulate), [xa, wa, out, wa], (grid_x, m, 1))
+            got[accumulate] = c.read(out).reshape(m, stride)
+        sums = got[False][:, col0 : col0 + n]
+        assert np.isfinite(sums).all()
+        want = init.copy()
+        want[:, col0 : col0 + n] = sums + init[:, col0 : col0 + n]
+        assert np.array_equal(got[True].view(np.uint32), want.view(np.uint32))
+
+
 # ---- prefill multiplies: check.zig:288-325, 752-825 -------------------------------------
 
 def matmul_case(c, rows, n, k, split, accumulate, rung=K.Prefill.scalar_f32, half="bf16"):

@@ -38,6 +38,14 @@ struct MvArgs {
     (a).row_bytes, (a).flags & FLAG_SILU_PAIR ? (a).half : (a).out_stride, (a).xr, MT == 1 ? __builtin_bit_cast(uint32_t, (a).eps) : (a).m - (t0), (a).eps, (a).act_div, \
     (a).out_stride
 
+// What output j (below `rows`) of a token holds, for a step that adds to it: asked for with the rows it belongs to, since behind their
+// sums it is one more trip to memory (us a token, 28 layers of 1024 x 3072 bf16 439 -> 422; eight of 4096 x 14336 Q4_K 379 -> 375). One load whatever the step and the lane, out of the buffer's range where there is nothing to add
+// to: a load some waves leave out would have the others wait for one of the next rows' in its place.
+__device__ __forceinline__ float held_output(const float *out, uint32_t rows, bool accumulate, bool mine, uint32_t j) {
+    const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(out), 0, accumulate ? (int)(rows * 4u) : 0, 0x00020000);
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(buf, mine && j < rows ? 4u * j : 0x80000000u, 0, 0));
+}
+
 // The sum over a wave's lanes, in every lane: pairs 32, 16, 8, 4, 2 and 1 lanes apart, in that
 // order. Nothing goes through LDS: the halves and the rows of sixteen trade places
 // (v_permlane32_swap, v_permlane16_swap), the rest are DPP operands of the additions. A rotation

@@ -96,11 +96,20 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MV_FIRST) {
         __builtin_amdgcn_sched_barrier(0);  // (the loads stay ahead of the multiply that follows them in the source)
         const uint32_t j = u * OUTS + lane;
 #pragma unroll
-        for (int t = 0; t < MT; t++) p.before[t] = !KEEP && accumulate && (uint32_t)t < a.m && lane < (uint32_t)OUTS && j < a.rows ? *out_at(t, j) : 0.f;
+        for (int t = 0; t < MT; t++) p.before[t] = KEEP || PAIR ? 0.f : held_output(out_at(t, 0), a.rows, accumulate && (uint32_t)t < a.m, lane < (uint32_t)OUTS, j);
         __builtin_amdgcn_sched_barrier(0);
     };
     Pass buf[2];
     fetch(first, buf[0]);
+    // (KEEP: what the outputs of the lane's next store hold)
+    float held[MT];
+    auto ask_held = [&](uint32_t from) __attribute__((always_inline)) {
+        const uint32_t j = (from + lane / OUTS * nwaves) * OUTS + lane % OUTS;
+#pragma unroll
+        for (int t = 0; t < MT; t++) held[t] = held_output(out_at(t, 0), a.rows, accumulate && (uint32_t)t < a.m, true, j);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (KEEP && !PAIR) ask_held(first);
 
     float scale[MT];
 #pragma unroll
@@ -173,12 +182,13 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MV_FIRST) {
                 if ((uint32_t)t >= a.m) break;
                 float v = PAIR ? silu_f(v0[t]) * v1[t] : v0[t];
                 float *o = out_at(t, j);
-                if (accumulate) v += *o;
+                if (accumulate) v += PAIR ? *o : held[t];
                 *o = v;
             }
         }
         kept_first += turn * nwaves;
         turn = 0;
+        if (!PAIR) ask_held(kept_first);
     };
     auto multiply = [&](uint32_t u, const Pass &p) __attribute__((always_inline)) {
         const uint32_t slot = KEEP ? turn * OUTS : 0u;
@@ -217,7 +227,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MV_FIRST) {
             for (int t = 0; t < MT; t++) {
                 if ((uint32_t)t >= a.m) break;
                 float v = PAIR ? silu_f(v0[t]) * v1[t] : v0[t];
-                if (accumulate) v += p.before[t];
+                if (accumulate) v += PAIR ? *out_at(t, j) : p.before[t];
                 *out_at(t, j) = v;
             }
         }

@@ -965,6 +965,18 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
 #pragma unroll
     for (int dpt = 0; dpt < kRowDepth; dpt++) fetch(gwave + dpt * nwaves, 0u, buf[dpt]);
 
+    // What the outputs of a wave's next store hold: with KEEP those of SEG passes, the lane's by turn, otherwise a pass's. (A gate / up
+    // step hardly ever adds to anything: it reads them when it stores.)
+    const bool accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
+    float held[2][MT];
+    auto ask_held = [&](uint32_t u, float (&h)[MT]) __attribute__((always_inline)) {
+        const uint32_t j = (KEEP ? u + tsub * nwaves : u) * RPI + rsub;
+#pragma unroll
+        for (int t = 0; t < MT; t++) h[t] = held_output(a.out + (size_t)(t0 + t) * a.out_stride, a.rows, accumulate && (t == 0 || full), KEEP || tsub == SEG - 1u, j);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (!PAIR) ask_held(gwave, held[0]);
+
     // stage_token's arithmetic on the vectors already loaded, the tokens' sums of squares
     // meeting in LDS together.
     float scale[MT];
@@ -1037,7 +1049,6 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
         }
     }
     const typename P::Keys ch = P::keys(tsub & 3u);
-    const bool accumulate = (a.flags & FLAG_ACCUMULATE) != 0;
     auto out_at = [&](int t, uint32_t j) { return (size_t)(t0 + t) * a.out_stride + a.col0 + j; };
 
     // With KEEP a pass's finished sums wait in the lanes, the gate's and the up row's apart: lane tsub of
@@ -1055,12 +1066,13 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
             for (int t = 0; t < MT; t++) {
                 if (t > 0 && !full) break;
                 float r = PAIR ? silu_f(kept0[t]) * kept1[t] : kept0[t];
-                if (accumulate) r += a.out[out_at(t, j)];
+                if (accumulate) r += PAIR ? a.out[out_at(t, j)] : held[0][t];
                 a.out[out_at(t, j)] = r;
             }
         }
         kept_first += nkept * nwaves;
         nkept = 0;
+        if (!PAIR) ask_held(kept_first, held[0]);
     };
     // One row's sums over the wave, for every token.
     auto row_sums = [&](const typename P::Raw &row, float (&s)[MT]) __attribute__((always_inline)) {
@@ -1085,7 +1097,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
         }
     };
     // The sums of pass u's rows (s0) and, with PAIR, of the up rows (s1): kept, or stored.
-    auto finish = [&](uint32_t u, const float (&s0)[MT], const float (&s1)[MT]) __attribute__((always_inline)) {
+    auto finish = [&](uint32_t u, const float (&s0)[MT], const float (&s1)[MT], const float (&h)[MT]) __attribute__((always_inline)) {
         if (KEEP) {
             keep(s0, kept0);
             if (PAIR) keep(s1, kept1);
@@ -1098,7 +1110,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
                 for (int t = 0; t < MT; t++) {
                     if (t > 0 && !full) break;
                     float r = PAIR ? silu_f(s0[t]) * s1[t] : s0[t];
-                    if (accumulate) r += a.out[out_at(t, j)];
+                    if (accumulate) r += PAIR ? a.out[out_at(t, j)] : h[t];
                     a.out[out_at(t, j)] = r;
                 }
             }
@@ -1106,13 +1118,13 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
     };
     // (a row at a time: with the inputs in registers two rows share nothing, and one row's
     // sums and words are fewer registers than two rows')
-    auto multiply = [&](uint32_t u, const typename P::Raw (&rows)[kRows]) __attribute__((always_inline)) {
+    auto multiply = [&](uint32_t u, const typename P::Raw (&rows)[kRows], const float (&h)[MT]) __attribute__((always_inline)) {
         float s0[MT], s1[MT] = {};
         row_sums(rows[0], s0);
         if (PAIR) row_sums(rows[kRows - 1], s1);
         reduce(s0);
         if (PAIR) reduce(s1);
-        finish(u, s0, s1);
+        finish(u, s0, s1, h);
     };
 
     // Gate and up rows in turn: one row's loads in flight while the other is multiplied, so a
@@ -1126,7 +1138,7 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
             fetch(u + nwaves, 0u, buf[0]);
             row_sums(buf[1][0], s1);
             reduce(s1);
-            finish(u, s0, s1);
+            finish(u, s0, s1, held[0]);
         }
         if (KEEP) flush_kept();
         return;
@@ -1138,7 +1150,8 @@ __global__ __launch_bounds__(256) void matvec_quant_row_kernel(MV_FIRST, Masks n
 #pragma unroll
         for (int ph = 0; ph <= kRowDepth; ph++) {
             fetch(u + kRowDepth * nwaves, 0u, buf[(ph + kRowDepth) % (kRowDepth + 1)]);
-            multiply(u, buf[ph]);
+            if (!PAIR && !KEEP) ask_held(u + kRowDepth * nwaves, held[(ph + kRowDepth) % (kRowDepth + 1)]);
+            multiply(u, buf[ph], held[KEEP ? 0 : ph]);
             u += nwaves;
             if (u >= units) {
                 done = true;
