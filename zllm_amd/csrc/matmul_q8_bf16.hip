@@ -57,7 +57,10 @@ static_assert(lds_bytes<4, 2>() <= 160 * 1024, "three buffers must fit the CU's 
 static_assert(lds_bytes<4, 2>() >= 8 * 3 * 4 * 1024 && lds_bytes<2, 2>() >= 8 * 3 * 2 * 1024 && lds_bytes<1, 1>() >= 4 * 3 * 1024, "the exchange must fit the buffers");
 
 template <int TT, class H, int RN>
-__global__ __launch_bounds__((threads<RN>())) void matmul_q8_bf16_kernel(Q8Args a) {
+__global__ __launch_bounds__((threads<RN>())) void matmul_q8_bf16_kernel(
+    const uint8_t *x, const uint8_t *w, uint32_t k, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes, Q8Args a) {
+    // (what the first loads need are parameters of their own, ahead of the struct: those are in registers when the wave starts)
+    a.x = x, a.w = w, a.k = k, a.row_bytes = row_bytes, a.x_bytes = x_bytes, a.w_bytes = w_bytes;
     typedef typename H::vec opvec;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int BM = 32 * TT, BN = 32 * RN, CONSUMERS = 4 * RN, ABUF = abuf_bytes<TT>(), BUF = buf_bytes<TT, RN>();
@@ -289,7 +292,7 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const Q8Args &a) {
     // The kernel's 32-bit offsets also name the rows and tokens of partial tiles past the end.
     if ((uint64_t)grid.x * BN * a.row_bytes >= (1ull << 32) || (uint64_t)grid.y * (32 * TT) * a.k * 2u >= (1ull << 32))
         return fail(d, ZHIP_E_BAD_COMMAND, "%s: operands of 4 GiB or more", name);
-    hipLaunchKernelGGL(kernel, grid, dim3(threads<RN>()), bytes, d.stream, a);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads<RN>()), bytes, d.stream, a.x, a.w, a.k, a.row_bytes, a.x_bytes, a.w_bytes, a);
     return check_launch(d, name);
 }
 

@@ -43,7 +43,10 @@ static_assert(lds_bytes<4, 4>() <= 160 * 1024, "three buffers must fit the CU's 
 static_assert(lds_bytes<2, 2>() >= 4 * 2 * 4096 && lds_bytes<2, 4>() >= 8 * 2 * 4096, "the exchange must fit the buffers");
 
 template <int TT, class H, int RQ>
-__global__ __launch_bounds__(threads<RQ>()) void matmul_q8_bf16_wide_kernel(Q8Args a, uint32_t tiles_n) {
+__global__ __launch_bounds__(threads<RQ>()) void matmul_q8_bf16_wide_kernel(
+    const uint8_t *x, const uint8_t *w, uint32_t k, uint32_t row_bytes, uint32_t x_bytes, uint32_t w_bytes, uint32_t tiles_n, Q8Args a) {
+    // (what the first loads need are parameters of their own, ahead of the struct: those are in registers when the wave starts)
+    a.x = x, a.w = w, a.k = k, a.row_bytes = row_bytes, a.x_bytes = x_bytes, a.w_bytes = w_bytes;
     typedef typename H::vec opvec;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int BM = 32 * TT, BN = 32 * RQ, CONSUMERS = 2 * RQ, ABUF = abuf_bytes<TT>(), BUF = buf_bytes<TT, RQ>();
@@ -263,7 +266,7 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const Q8Args &a) {
     // The kernel's 32-bit offsets also name the rows and tokens of partial tiles past the end.
     if ((uint64_t)tiles_n * (32 * RQ) * a.row_bytes >= (1ull << 32) || tiles_t * (32 * TT) * a.k * 2u >= (1ull << 32))
         return fail(d, ZHIP_E_BAD_COMMAND, "%s: operands of 4 GiB or more", name);
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles), dim3(threads<RQ>()), bytes, d.stream, a, tiles_n);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles), dim3(threads<RQ>()), bytes, d.stream, a.x, a.w, a.k, a.row_bytes, a.x_bytes, a.w_bytes, tiles_n, a);
     return check_launch(d, name);
 }
 

@@ -97,7 +97,12 @@ __device__ __forceinline__ void sync_keeping_loads() {
 __device__ __forceinline__ uint32_t line_key(uint32_t row) { return (row & 7u) ^ ((row >> 3) & 1u); }
 
 template <int TW>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void matmul_q8_i8_kernel(Q8I8Args a) {
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void matmul_q8_i8_kernel(
+    const uint8_t *qx, const uint8_t *w_rows, const uint8_t *scales, uint32_t k, uint32_t row_bytes, uint32_t qx_bytes, uint32_t w_bytes, uint32_t dx_bytes, Q8I8Args a) {
+    // (What the first loads need are parameters of their own, ahead of the struct: those are in registers when the wave starts. A
+    // 512-token step over 28 layers of 1024 x 3072, quantize_q8 included: 1835 -> 1755 us. The struct's are on their way meanwhile: as
+    // parameters of their own the compiler fetches them where the outputs are stored, 0.5 % slower.)
+    a.qx = qx, a.w = w_rows, a.dx = scales, a.k = k, a.row_bytes = row_bytes, a.qx_bytes = qx_bytes, a.w_bytes = w_bytes, a.dx_bytes = dx_bytes;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef Tile<TW> T;
     constexpr uint32_t BUF = T::BUF, CHUNKS_AT = RING * BUF, CHUNK = T::CHUNK;
@@ -288,7 +293,7 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const Q8I8Args &a) 
     typedef Tile<TW> T;
     if (!lds_opt_in<matmul_q8_i8_kernel<TW>, T::LDS>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", name, T::LDS);
     const dim3 grid((a.n + BN - 1) / BN, (a.rows + T::BM - 1) / T::BM);
-    hipLaunchKernelGGL((matmul_q8_i8_kernel<TW>), grid, dim3(THREADS), T::LDS, d.stream, a);
+    hipLaunchKernelGGL((matmul_q8_i8_kernel<TW>), grid, dim3(THREADS), T::LDS, d.stream, a.qx, a.w, a.dx, a.k, a.row_bytes, a.qx_bytes, a.w_bytes, a.dx_bytes, a);
     return check_launch(d, name);
 }
 

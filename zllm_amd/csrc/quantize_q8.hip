@@ -132,7 +132,8 @@ __device__ __forceinline__ float norm_factor(const QuantizeQ8Params &p, double s
 // where it has the SIMD to itself. us, a row read twice by one workgroup (once for the sum) / this: 64 x 4096 4.6 / 2.5, 64 x 5120
 // 6.2 / 2.9, 128 x 4096 4.6 / 2.8, 201 x 2560 4.4 / 3.1, 512 x 1024 3.1 / 2.4, 512 x 4096 6.0 / 4.8.
 template <int J>
-__global__ __launch_bounds__(256) void quantize_q8_norm_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx, const float *nw) {
+__global__ __launch_bounds__(256) void quantize_q8_norm_kernel(const float *x, uint32_t *qx, float *dx, const float *nw, uint32_t k, uint32_t block, uint32_t mode, float eps) {
+    const QuantizeQ8Params p{k, block, mode, eps};
     __shared__ double squares[4];
     const uint32_t at = 4u * threadIdx.x;
     const size_t row = (size_t)blockIdx.y * p.k;
@@ -157,7 +158,8 @@ __global__ __launch_bounds__(256) void quantize_q8_norm_kernel(QuantizeQ8Params 
     }
 }
 // The same over rows of any length, read twice.
-__global__ __launch_bounds__(256) void quantize_q8_norm_long_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx, const float *nw) {
+__global__ __launch_bounds__(256) void quantize_q8_norm_long_kernel(const float *x, uint32_t *qx, float *dx, const float *nw, uint32_t k, uint32_t block, uint32_t mode, float eps) {
+    const QuantizeQ8Params p{k, block, mode, eps};
     __shared__ double squares[4];
     const uint32_t at = 4u * threadIdx.x;
     const size_t row = (size_t)blockIdx.y * p.k;
@@ -190,7 +192,8 @@ __global__ __launch_bounds__(256) void quantize_q8_norm_long_kernel(QuantizeQ8Pa
 }
 
 // Without the prologue: a chunk a wave.
-__global__ __launch_bounds__(256) void quantize_q8_kernel(QuantizeQ8Params p, const float *x, uint32_t *qx, float *dx) {
+__global__ __launch_bounds__(256) void quantize_q8_kernel(const float *x, uint32_t *qx, float *dx, uint32_t k, uint32_t block, uint32_t mode) {
+    const QuantizeQ8Params p{k, block, mode, 0.f};
     const uint32_t at = 1024u * blockIdx.x + 4u * threadIdx.x;
     const bool live = at < p.k;
     const size_t row = blockIdx.y;
@@ -223,7 +226,7 @@ static void launch_norm(const Dispatch &d, const QuantizeQ8Params &p, uint32_t s
     }
     const uint32_t rows = d.grid[1], cus = (uint32_t)d.dev->compute_units;
     const uint32_t each = cus / rows > 2u ? cus / rows : 2u, parts = rows > cus ? 1u : each < (uint32_t)J ? each : (uint32_t)J;
-    hipLaunchKernelGGL(quantize_q8_norm_kernel<J>, dim3(parts, rows), dim3(256), 0, d.stream, p, x, qx, dx, nw);
+    hipLaunchKernelGGL(quantize_q8_norm_kernel<J>, dim3(parts, rows), dim3(256), 0, d.stream, x, qx, dx, nw, p.k, p.block, p.mode, p.eps);
 }
 
 zhip_result launch_quantize_q8(const Dispatch &d) {
@@ -254,9 +257,9 @@ zhip_result launch_quantize_q8(const Dispatch &d) {
     // 13.9 / 13.8 / 15.9, 201 x 9728 with it 5.3 / 5.9 / 7.5; only 512 x 14336 without one is faster with
     // two, 8.9 / 8.6. (With the block's index shifted, not divided: 4.5, -, 13.1 and 5.5 us.)
     const uint32_t spans = (d.grid[0] + 3u) / 4u;
-    if (p.mode != 1u) hipLaunchKernelGGL(quantize_q8_kernel, dim3(spans, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx);
+    if (p.mode != 1u) hipLaunchKernelGGL(quantize_q8_kernel, dim3(spans, d.grid[1]), dim3(256), 0, d.stream, x, qx, dx, p.k, p.block, p.mode);
     else if (spans <= 8u) launch_norm<1>(d, p, spans, x, qx, dx, nw);
-    else hipLaunchKernelGGL(quantize_q8_norm_long_kernel, dim3(1, d.grid[1]), dim3(256), 0, d.stream, p, x, qx, dx, nw);
+    else hipLaunchKernelGGL(quantize_q8_norm_long_kernel, dim3(1, d.grid[1]), dim3(256), 0, d.stream, x, qx, dx, nw, p.k, p.block, p.mode, p.eps);
     return check_launch(d, "quantize_q8");
 }
 
