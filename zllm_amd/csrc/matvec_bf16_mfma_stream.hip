@@ -211,7 +211,12 @@ __device__ __forceinline__ void f16_pieces(const float4 &v, float scale, uint2 (
 // walker i / parts takes, and launch_matvec_parts_sum adds the stretches' sums. Without the RMSNorm prologue no
 // workgroup needs more of a token than its stretch (an F16 token's scale is then the stretch's own).
 template <int NP, bool SPLIT, bool F16, bool LONG, bool PAIR, bool WHOLE>
-__global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(StreamArgs q) {
+__global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(const float *first_x, const uint8_t *first_w, const float *first_norm_w, uint32_t k_flags, uint32_t xr, uint32_t row_bytes,
+    uint32_t rows, uint32_t half_at, uint32_t w_bytes, uint32_t rounds_walkers, uint32_t counts, StreamArgs q) {
+    // (what the first loads are addressed by is in registers when the wave starts: see MV_FIRST. Some share a word: launch_blocks)
+    q.a.x = first_x, q.a.w = first_w, q.a.norm_w = first_norm_w, q.a.k = k_flags & 0xffffffu, q.a.flags = k_flags >> 24, q.a.xr = xr, q.a.row_bytes = row_bytes, q.a.rows = rows;
+    q.a.half = half_at, q.w_bytes = w_bytes, q.rounds = rounds_walkers & 0xffffu, q.tail_rem = counts & 0xffffu, q.tail_base = counts >> 16 & 15u, q.a.m = counts >> 20 & 15u, q.by_die = counts >> 24 & 1u;
+    q.parts = counts >> 25;
     static_assert(!PAIR || !LONG, "gate / up steps take whole rows");
     constexpr uint32_t PER = PAIR ? 2u : 1u;  // weight tiles an output tile
     constexpr uint32_t PIECES = pieces_of(F16, WHOLE);
@@ -233,7 +238,7 @@ __global__ __launch_bounds__(THREADS) void matvec_bf16_mfma_stream_kernel(Stream
     // die's workgroups take neighbouring tiles (one die then reads a contiguous eighth of every
     // round's stretch of the matrix: 55 us against 58 us for four tokens over 151936 x 1024).
     const uint32_t kpart = LONG ? blockIdx.x % q.parts : 0u, walker = LONG ? blockIdx.x / q.parts : blockIdx.x;
-    const uint32_t G = LONG ? gridDim.x / q.parts : gridDim.x;
+    const uint32_t G = rounds_walkers >> 16;
     const uint32_t b = q.by_die ? (walker & 7u) * (G >> 3) + (walker >> 3) : walker;
     const uint32_t tail_units = q.tail_base + (b < q.tail_rem ? 1u : 0u);
     const uint32_t tail_row = 32u * q.rounds * G + 8u * (b * q.tail_base + (b < q.tail_rem ? b : q.tail_rem));
@@ -505,7 +510,10 @@ zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
         }
         configured = true;
     }
-    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), LDS_BYTES, d.stream, q);
+    const uint32_t walkers = grid.x / q.parts;
+    if ((q.rounds | walkers) > 0xffffu || q.tail_base > 15u) return fail(d, ZHIP_E_GPU, "%s: %u rounds of %u workgroups", F16 ? "matvec_f16" : "matvec_bf16", q.rounds, walkers);
+    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), LDS_BYTES, d.stream, q.a.x, q.a.w, q.a.norm_w, q.a.k | q.a.flags << 24, q.a.xr, q.a.row_bytes, q.a.rows, q.a.half, q.w_bytes,
+        q.rounds | walkers << 16, q.tail_rem | q.tail_base << 16 | q.a.m << 20 | q.by_die << 24 | q.parts << 25, q);
     return check_launch(d, F16 ? "matvec_f16" : "matvec_bf16");
 }
 

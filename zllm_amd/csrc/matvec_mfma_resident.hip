@@ -166,7 +166,11 @@ __device__ __forceinline__ rf16x8 nibbles(ru32x2 w, ru32x2 fifth, uint32_t mask,
 // workgroup b multiplies columns 2048 (b % parts) .. (part `kpart`) of the tiles that walker b / parts takes, and
 // matvec_kquant_mfma_parts_sum_kernel adds the parts in their order and applies the epilogue.
 template <class F, bool PAIR, bool LONG>
-__global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(ResArgs q) {
+__global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(const float *first_x, const uint8_t *first_w, const float *first_norm_w, uint32_t w_bytes, uint32_t xr, uint32_t row_bytes,
+    uint32_t half_at, uint32_t rounds, uint32_t walkers, uint32_t left_flags, uint32_t counts, ResArgs q) {
+    // (what the first loads are addressed by is in registers when the wave starts: see MV_FIRST)
+    q.a.x = first_x, q.a.w = first_w, q.a.norm_w = first_norm_w, q.w_bytes = w_bytes, q.a.xr = xr, q.a.row_bytes = row_bytes, q.a.half = half_at, q.rounds = rounds;
+    q.left = left_flags & 0xffffffu, q.a.flags = left_flags >> 24, q.a.m = counts & 15u, q.split = counts >> 4 & 1u, q.parts = counts >> 8;
     static_assert(!LONG || !PAIR, "pairs over long rows are matvec_mfma_rows.hip's");
     constexpr int DEPTH = LONG ? kLongDepth : kDepth;
     const MvArgs &a = q.a;
@@ -176,13 +180,11 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
     __shared__ float lds_part[2][WAVES][128];     // [tile parity][wave][2 lane + token of the lane's two]
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, l16 = lane & 15u, g = lane >> 4;
     const __amdgpu_buffer_rsrc_t wbuf = make_buffer(a.w, q.w_bytes), nobuf = make_buffer(a.w, 0);
-    uint32_t sixteen = q.sixteen;
-    asm volatile("" : "+v"(sixteen));
 
     // The workgroup's weight tiles: output tiles b, b + G, ...; with SILU_PAIR the gate tile
     // and then the up tile of each. Tile p of the run starts at matrix row:
     const uint32_t per = PAIR ? 2u : 1u;
-    const uint32_t kpart = LONG ? blockIdx.x % q.parts : 0u, walker = LONG ? blockIdx.x / q.parts : blockIdx.x, walkers = LONG ? gridDim.x / q.parts : gridDim.x;
+    const uint32_t kpart = LONG ? blockIdx.x % q.parts : 0u, walker = LONG ? blockIdx.x / q.parts : blockIdx.x;
     // When the output tiles left over after whole rounds are at most half as many as the
     // workgroups, two workgroups share each, eight rows apiece: a whole tile more on half of
     // the CUs would be the launch's tail.
@@ -255,6 +257,8 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
         if (LONG) ready = q.scales[tsrc];
     }
     load_tile(0, 0);
+    uint32_t sixteen = q.sixteen;
+    asm volatile("" : "+v"(sixteen));
     if (norm) {
         float rs;
         if (LONG) {
@@ -445,13 +449,13 @@ __global__ __launch_bounds__(THREADS) void matvec_kquant_mfma_resident_kernel(Re
 // The outputs of a step over long rows: the parts' sums added in the order of their columns,
 // then the SILU_PAIR / ACCUMULATE epilogue. One thread an output.
 template <bool PAIR>
-__global__ __launch_bounds__(256) void matvec_kquant_mfma_parts_sum_kernel(MvArgs a, const float *partial, uint32_t parts) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x, row = i % a.rows, t = i / a.rows;
-    if (t >= a.m) return;
+__global__ __launch_bounds__(256) void matvec_kquant_mfma_parts_sum_kernel(const float *partial, float *out, uint32_t rows, uint32_t m, uint32_t out_stride, uint32_t accumulate, uint32_t parts) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, row = i % rows, t = i / rows;
+    if (t >= m) return;
     constexpr uint32_t per = PAIR ? 2u : 1u;
-    const float *src = partial + (size_t)t * a.rows + row;
-    const size_t plane = (size_t)8u * a.rows;
-    float *o = a.out + (size_t)t * a.out_stride + a.col0 + row;
+    const float *src = partial + (size_t)t * rows + row;
+    const size_t plane = (size_t)8u * rows;
+    float *o = out + (size_t)t * out_stride + row;
     // Every load first: the parts were written by other workgroups and come from memory.
     float first[kMatvecMaxParts], second[kMatvecMaxParts];
 #pragma unroll
@@ -459,7 +463,7 @@ __global__ __launch_bounds__(256) void matvec_kquant_mfma_parts_sum_kernel(MvArg
         first[p] = p < parts ? src[per * p * plane] : 0.f;
         second[p] = (PAIR && p < parts) ? src[(per * p + 1u) * plane] : 0.f;
     }
-    const float before = (a.flags & FLAG_ACCUMULATE) ? *o : 0.f;
+    const float before = accumulate ? *o : 0.f;
     float sum = first[0], up = second[0];
 #pragma unroll
     for (uint32_t p = 1; p < kMatvecMaxParts; p++) {
@@ -469,7 +473,7 @@ __global__ __launch_bounds__(256) void matvec_kquant_mfma_parts_sum_kernel(MvArg
         }
     }
     const float v = PAIR ? silu_f(sum) * up : sum;
-    *o = (a.flags & FLAG_ACCUMULATE) ? before + v : v;
+    *o = accumulate ? before + v : v;
 }
 
 }  // namespace
@@ -498,8 +502,8 @@ zhip_result launch_matvec_parts_scales(const Dispatch &d, const char *name, cons
 
 zhip_result launch_matvec_parts_sum(const Dispatch &d, const char *name, const MvArgs &a, const float *partial, uint32_t parts) {
     const dim3 sums((a.rows * a.m + 255u) / 256u);
-    if (a.flags & FLAG_SILU_PAIR) hipLaunchKernelGGL(matvec_kquant_mfma_parts_sum_kernel<true>, sums, dim3(256), 0, d.stream, a, partial, parts);
-    else hipLaunchKernelGGL(matvec_kquant_mfma_parts_sum_kernel<false>, sums, dim3(256), 0, d.stream, a, partial, parts);
+    if (a.flags & FLAG_SILU_PAIR) hipLaunchKernelGGL(matvec_kquant_mfma_parts_sum_kernel<true>, sums, dim3(256), 0, d.stream, partial, a.out + a.col0, a.rows, a.m, a.out_stride, a.flags & FLAG_ACCUMULATE, parts);
+    else hipLaunchKernelGGL(matvec_kquant_mfma_parts_sum_kernel<false>, sums, dim3(256), 0, d.stream, partial, a.out + a.col0, a.rows, a.m, a.out_stride, a.flags & FLAG_ACCUMULATE, parts);
     return check_launch(d, name);
 }
 
@@ -528,6 +532,10 @@ static zhip_result launch_resident(const Dispatch &d, const MvArgs &a, uint64_t 
     const uint32_t left = halves ? tiles : tiles % groups;
     ResArgs q{a, (uint32_t)w_bytes, mask, bias_bits, halves ? 0u : tiles / groups, left, (halves || 2u * left <= groups) ? 1u : 0u, parts, nullptr, nullptr};
     const dim3 grid(groups * parts);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(THREADS), 0, d.stream, q.a.x, q.a.w, q.a.norm_w, q.w_bytes, q.a.xr, q.a.row_bytes, q.a.half, q.rounds, groups, q.left | q.a.flags << 24,
+            q.a.m | q.split << 4 | q.parts << 8, q);
+    };
     if (parts > 1u) {
         const uint64_t bytes = (uint64_t)parts * 8u * a.rows * sizeof(float);
         if (!d.work) return fail(d, ZHIP_E_GPU, "%s: no workspace", F::name());
@@ -537,12 +545,12 @@ static zhip_result launch_resident(const Dispatch &d, const MvArgs &a, uint64_t 
             q.scales = reinterpret_cast<const float *>(d.work->data);
             if (zhip_result r = launch_matvec_parts_scales(d, F::name(), a, reinterpret_cast<float *>(d.work->data))) return r;
         }
-        hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, true>), grid, dim3(THREADS), 0, d.stream, q);
+        launch(matvec_kquant_mfma_resident_kernel<F, false, true>);
         if (zhip_result r = check_launch(d, F::name())) return r;
         return launch_matvec_parts_sum(d, F::name(), a, q.partial, parts);
     }
-    if (pair) hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, true, false>), grid, dim3(THREADS), 0, d.stream, q);
-    else hipLaunchKernelGGL((matvec_kquant_mfma_resident_kernel<F, false, false>), grid, dim3(THREADS), 0, d.stream, q);
+    if (pair) launch(matvec_kquant_mfma_resident_kernel<F, true, false>);
+    else launch(matvec_kquant_mfma_resident_kernel<F, false, false>);
     return check_launch(d, F::name());
 }
 

@@ -40,6 +40,7 @@
 // every 256th input a thousand times the others 1.44 - 3.34e-7 / 1.04 - 1.59e-7.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -314,7 +315,14 @@ template <class F> constexpr uint32_t wave_bytes() { return shared_bytes<F>() + 
 // NB: the most blocks of 256 weights a wave takes of a row. LONG: q.parts workgroups share a tile, each over
 // its share of the row's blocks, and leave their sums in q.partial.
 template <class F, int NB, int TEAMS, bool ACT, bool LONG>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void matvec_mfma_rows_kernel(RowsArgs q) {
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void matvec_mfma_rows_kernel(const float *first_x, const uint8_t *first_w, const float *first_norm_w,
+    uint32_t k_flags, uint32_t xr, uint32_t row_bytes, uint32_t rows, uint32_t half_at, uint32_t groups_left, uint32_t whole_rounds, uint32_t counts, RowsArgs q) {
+    // (ahead of the struct, in registers when the wave starts: what the first loads of inputs and weights are addressed by; see
+    // MV_FIRST. Some share a word: launch_nb. With the other matrix-core kernels' and the sums', four tokens through eight layers of
+    // 4096 x 14336 Q4_K, 597 -> 582 us a step.)
+    q.a.x = first_x, q.a.w = first_w, q.a.norm_w = first_norm_w, q.a.k = k_flags & 0xffffffu, q.a.flags = k_flags >> 24, q.a.xr = xr, q.a.row_bytes = row_bytes;
+    q.a.rows = rows, q.a.half = half_at, q.groups = groups_left & 0xffffu, q.left = groups_left >> 16, q.rounds = whole_rounds;
+    q.a.m = counts & 15u, q.split = counts >> 4 & 1u, q.parts = counts >> 8 & 255u, q.blocks = counts >> 16;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ float lds_part[2][WAVES][128];  // [round parity][wave][2 lane + token of the lane's two]
     __shared__ float lds_ss[WAVES][8];
@@ -651,13 +659,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 // The outputs of a step over rows in parts: the parts' sums in the order of their blocks, the norm's
 // factor, the SILU_PAIR / ACCUMULATE epilogue. One thread an output.
 template <bool PAIR>
-__global__ __launch_bounds__(256) void matvec_mfma_rows_sum_kernel(MvArgs a, const float *partial, uint32_t parts, uint32_t norm) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x, row = i % a.rows, t = i / a.rows;
-    if (t >= a.m) return;
+__global__ __launch_bounds__(256) void matvec_mfma_rows_sum_kernel(const float *partial, float *out, uint32_t rows, uint32_t m, uint32_t out_stride, uint32_t accumulate, uint32_t parts, uint32_t norm, uint32_t k, float eps) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, row = i % rows, t = i / rows;
+    if (t >= m) return;
     constexpr uint32_t per = PAIR ? 2u : 1u;
-    const float *src = partial + kSums + (size_t)t * a.rows + row;
-    const size_t plane = (size_t)8u * a.rows;
-    float *o = a.out + (size_t)t * a.out_stride + a.col0 + row;
+    const float *src = partial + kSums + (size_t)t * rows + row;
+    const size_t plane = (size_t)8u * rows;
+    float *o = out + (size_t)t * out_stride + row;
     // Every load first: the parts were written by other workgroups and come from memory.
     float first[kMaxParts], second[kMaxParts], squares[kMaxParts];
 #pragma unroll
@@ -666,7 +674,7 @@ __global__ __launch_bounds__(256) void matvec_mfma_rows_sum_kernel(MvArgs a, con
         second[p] = (PAIR && p < parts) ? src[(per * p + 1u) * plane] : 0.f;
         squares[p] = (norm && p < parts) ? partial[8u * p + t] : 0.f;
     }
-    const float before = (a.flags & FLAG_ACCUMULATE) ? *o : 0.f;
+    const float before = accumulate ? *o : 0.f;
     float sum = first[0], up = second[0], ss = squares[0];
 #pragma unroll
     for (uint32_t p = 1; p < kMaxParts; p++) {
@@ -675,19 +683,20 @@ __global__ __launch_bounds__(256) void matvec_mfma_rows_sum_kernel(MvArgs a, con
         ss += squares[p];
     }
     if (norm) {
-        const float scale = 1.0f / sqrtf(ss / (float)a.k + a.eps);
+        const float scale = 1.0f / sqrtf(ss / (float)k + eps);
         sum *= scale;
         up *= scale;
     }
     const float v = PAIR ? silu_f(sum) * up : sum;
-    *o = (a.flags & FLAG_ACCUMULATE) ? before + v : v;
+    *o = accumulate ? before + v : v;
 }
 
 template <class F, int NB, int TEAMS, bool ACT, bool LONG>
 zhip_result launch_nb(const Dispatch &d, const RowsArgs &q) {
     constexpr int bytes = (int)(WAVES * wave_bytes<F>());
     if (!lds_opt_in<matvec_mfma_rows_kernel<F, NB, TEAMS, ACT, LONG>, bytes>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", F::name(), bytes);
-    hipLaunchKernelGGL((matvec_mfma_rows_kernel<F, NB, TEAMS, ACT, LONG>), dim3(q.groups * q.parts), dim3(THREADS), bytes, d.stream, q);
+    hipLaunchKernelGGL((matvec_mfma_rows_kernel<F, NB, TEAMS, ACT, LONG>), dim3(q.groups * q.parts), dim3(THREADS), bytes, d.stream, q.a.x, q.a.w, q.a.norm_w, q.a.k | q.a.flags << 24, q.a.xr,
+        q.a.row_bytes, q.a.rows, q.a.half, q.groups | q.left << 16, q.rounds, q.a.m | q.split << 4 | q.parts << 8 | q.blocks << 16, q);
     return check_launch(d, F::name());
 }
 
@@ -701,7 +710,7 @@ zhip_result launch_format(const Dispatch &d, const MvArgs &a) {
     const bool pair = (a.flags & FLAG_SILU_PAIR) != 0, norm = (a.flags & FLAG_NORM) != 0;
     const uint32_t blocks = (a.k + 255u) / 256u, tiles = (a.rows + 15u) / 16u;
     const uint32_t parts = blocks > F::MOST * WAVES ? (blocks + WAVES - 1u) / WAVES : 1u;
-    const uint32_t most = (uint32_t)d.dev->compute_units / parts;
+    const uint32_t most = std::min((uint32_t)d.dev->compute_units, 0xffffu) / parts;  // (the count has half a word of the kernel's parameters)
     if (most == 0u) return fail(d, ZHIP_E_GPU, "%s: %d compute units for %u parts of a row", F::name(), d.dev->compute_units, parts);
     const uint32_t groups = tiles < most ? (2u * tiles <= most ? 2u * tiles : tiles) : most;
     const bool halves = tiles < groups;  // every workgroup takes eight outputs of one tile
@@ -717,8 +726,8 @@ zhip_result launch_format(const Dispatch &d, const MvArgs &a) {
         }
         if (zhip_result r = launch_act<F, 1, 1, true>(d, q)) return r;
         const dim3 sums((a.rows * a.m + 255u) / 256u);
-        if (pair) hipLaunchKernelGGL(matvec_mfma_rows_sum_kernel<true>, sums, dim3(256), 0, d.stream, a, q.partial, parts, norm && a.act_div <= 0.f);
-        else hipLaunchKernelGGL(matvec_mfma_rows_sum_kernel<false>, sums, dim3(256), 0, d.stream, a, q.partial, parts, norm && a.act_div <= 0.f);
+        if (pair) hipLaunchKernelGGL(matvec_mfma_rows_sum_kernel<true>, sums, dim3(256), 0, d.stream, q.partial, a.out + a.col0, a.rows, a.m, a.out_stride, a.flags & FLAG_ACCUMULATE, parts, norm && a.act_div <= 0.f, a.k, a.eps);
+        else hipLaunchKernelGGL(matvec_mfma_rows_sum_kernel<false>, sums, dim3(256), 0, d.stream, q.partial, a.out + a.col0, a.rows, a.m, a.out_stride, a.flags & FLAG_ACCUMULATE, parts, norm && a.act_div <= 0.f, a.k, a.eps);
         return check_launch(d, F::name());
     }
     if constexpr (F::MOST > 1u) {
