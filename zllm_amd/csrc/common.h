@@ -106,6 +106,29 @@ struct PackedCopy {
     uint8_t *reserve(const Dispatch &d) const;
 };
 
+// Activations as an int8 Q8_0 multiply reads them, rounded to 8-bit blocks of 32 by a quantize_q8 dispatch. Where such a multiply
+// writes them, that dispatch is the next and another such multiply the one behind it, the first rounds what it stores, into a
+// place aside (it may still be reading the last rounding where the next one belongs), the quantize_q8 launch is left out, and the
+// second multiplies from there and puts the rounding where the caller has it. Two launches fewer a layer, and a SiLU pair's values are not
+// read back. See matmul_q8_i8.hip for what it measured.
+struct RoundedCopy {
+    static constexpr uint64_t kMost = 64u << 20;  // 512 tokens of 116,000 values
+    const float *x = nullptr;  // rows x k values, dense (mode 2: rows x 2 k)
+    uint32_t rows = 0, k = 0, mode = 0;
+    uint8_t *q = nullptr, *d = nullptr;  // the caller's values and scales
+    Workspace *room = nullptr;
+    uint8_t *data = nullptr;  // set once they have been rounded: the values, and scales_at() behind them the scales
+    uint64_t scales_at() const { return ((uint64_t)rows * k + 255u) & ~255ull; }
+    uint64_t scales_bytes() const { return (uint64_t)rows * (k / 32u) * 4u; }
+    uint8_t *reserve(const Dispatch &d) const;
+};
+// What an int8 Q8_0 multiply's launch touches, where it is one that can read them so.
+struct RoundedRead {
+    const uint8_t *q = nullptr, *d = nullptr, *w = nullptr, *out = nullptr;
+    uint32_t rows = 0, k = 0;
+    uint64_t w_bytes = 0, out_bytes = 0;
+};
+
 // One resolved dispatch: binding 0's bytes come from the host's shadow copy of
 // the uniform buffer, so kernels take their parameters by value.
 struct Dispatch {
@@ -120,6 +143,10 @@ struct Dispatch {
     PackedCopy *wanted = nullptr;      // a float rung's multiply: nothing is launched, what it would pack is left there
     PackedCopy *next = nullptr;        // what the dispatch behind this one would pack
     const PackedCopy *have = nullptr;  // what the dispatch before this one has packed
+    RoundedCopy *rounds = nullptr;         // quantize_q8: nothing is launched, what it would round is left there
+    RoundedRead *reads = nullptr;          // matmul_q8_0: the same
+    RoundedCopy *rounded_out = nullptr;    // what the quantize_q8 behind this dispatch would round
+    const RoundedCopy *rounded_in = nullptr;  // what the multiply before the last dispatch has rounded
     char *err = nullptr;  // message buffer for a failed launch
     size_t err_cap = 0;
 };

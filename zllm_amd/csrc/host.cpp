@@ -259,6 +259,13 @@ uint8_t *PackedCopy::reserve(const Dispatch &d) const {
     return room && want <= kMost && room->reserve(quiet, want) == ZHIP_OK ? room->data : nullptr;
 }
 
+uint8_t *RoundedCopy::reserve(const Dispatch &d) const {
+    const uint64_t want = scales_at() + scales_bytes();
+    Dispatch quiet = d;
+    quiet.err_cap = 0;
+    return room && want <= kMost && room->reserve(quiet, want) == ZHIP_OK ? room->data : nullptr;
+}
+
 void Workspace::release() {
     if (data && !fixed) (void)hipFree(data);
     data = nullptr;
@@ -274,6 +281,8 @@ struct zhip_context {
     Workspace copies[2];       // packed activations: one is read while the next is written
     uint32_t copies_made = 0;  // since the submit began
     PackedCopy copy;           // that the last dispatch left, for the one behind it
+    RoundedCopy rounded;       // the last rounding that a multiply made,
+    size_t rounded_at = SIZE_MAX;  // and the number of the op that it stands for (the multiply that reads it is the next)
     zhip_caps caps{};
     bool lost = false;
     std::string message;
@@ -475,41 +484,95 @@ bool is_float_rung(const Pipeline &pl) {
     return pl.launch && pl.info && (pl.launch == pl.info->launch_bf16 || pl.launch == pl.info->launch_f16 || pl.launch == pl.info->launch_f16c);
 }
 
-// What the dispatch behind op number `at` would pack, if it is a float rung's multiply whose parameters the host holds.
-PackedCopy wanted_behind(zhip_context *c, size_t at) {
-    PackedCopy want;
-    if (at + 1 >= c->ops.size() || c->ops[at + 1].kind != Op::dispatch) return want;
-    const Op &op = c->ops[at + 1];
-    Pipeline *pl = get(c->pipelines, op.pipeline);
-    if (!pl || !is_float_rung(*pl)) return want;
+// The pipeline of op number `at`, if it is a dispatch and before `end`.
+Pipeline *dispatched(zhip_context *c, size_t at, size_t end) { return at < end && c->ops[at].kind == Op::dispatch ? get(c->pipelines, c->ops[at].pipeline) : nullptr; }
+
+// Resolves a dispatch ahead of its turn, if the host holds its parameters. What is wrong with it is reported when its turn comes.
+bool foresee(zhip_context *c, size_t at, Dispatch &d, char *err, size_t err_cap) {
+    const Op &op = c->ops[at];
     const Buffer *ub = op.group.e[0].bound ? get(c->buffers, op.group.e[0].buffer) : nullptr;
-    if (!ub || !ub->shadowed || ub->shadow_stale) return want;
+    if (!ub || !ub->shadowed || ub->shadow_stale) return false;
+    Pipeline *pl = nullptr;
+    std::string message = c->message;
+    const zhip_result r = prepare_dispatch(c, op, d, pl, err, err_cap);
+    c->message = std::move(message);
+    return r == ZHIP_OK;
+}
+
+// What the dispatch behind op number `at` would pack, if it is a float rung's multiply whose parameters the host holds.
+PackedCopy wanted_behind(zhip_context *c, size_t at, size_t end) {
+    PackedCopy want;
+    Pipeline *pl = dispatched(c, at + 1, end);
     Dispatch d;
     char err[384];
-    // What is wrong with it is reported when its turn comes.
-    std::string message = c->message;
-    const zhip_result r = prepare_dispatch(c, op, d, pl, err, sizeof err);
-    c->message = std::move(message);
+    if (!pl || !is_float_rung(*pl) || !foresee(c, at + 1, d, err, sizeof err)) return want;
     d.wanted = &want;
-    if (r != ZHIP_OK || pl->launch(d) != ZHIP_OK) return PackedCopy{};
+    if (pl->launch(d) != ZHIP_OK) return PackedCopy{};
     want.room = &c->copies[c->copies_made & 1u];
     return want;
 }
 
+bool apart(const uint8_t *p, uint64_t p_bytes, const uint8_t *q, uint64_t q_bytes) { return p + p_bytes <= q || q + q_bytes <= p; }
+
+// What the quantize_q8 behind op number `at`, an int8 Q8_0 multiply, would round, if the op behind that is such a multiply too and
+// multiplies exactly that. The first multiply can then round what it stores, and the second put the rounding where it
+// belongs (common.h, RoundedCopy): not where the two write or read anything else of what the rounding overwrites, nor
+// where one of them writes the next one's parameters.
+RoundedCopy rounding_behind(zhip_context *c, size_t at, size_t end, const Dispatch &first) {
+    RoundedCopy made;
+    Pipeline *quantize = dispatched(c, at + 1, end), *second = dispatched(c, at + 2, end);
+    if (!quantize || !second || quantize->launch != launch_quantize_q8 || second->launch != launch_matmul_q8_0) return made;
+    const Group &mid = c->ops[at + 1].group, &last = c->ops[at + 2].group;
+    for (const uint32_t writes : {c->ops[at].group.e[3].buffer, mid.e[2].buffer, mid.e[3].buffer})
+        if (writes == mid.e[0].buffer || writes == last.e[0].buffer) return made;
+    Dispatch d;
+    char err[384];
+    RoundedRead before, behind;
+    if (!foresee(c, at + 1, d, err, sizeof err)) return made;
+    d.rounds = &made;
+    if (quantize->launch(d) != ZHIP_OK || made.rows == 0u || made.mode == 1u) return RoundedCopy{};
+    d = first;
+    d.reads = &before;
+    if (launch_matmul_q8_0(d) != ZHIP_OK || before.rows == 0u) return RoundedCopy{};
+    d = Dispatch{};
+    if (!foresee(c, at + 2, d, err, sizeof err)) return RoundedCopy{};
+    d.reads = &behind;
+    if (launch_matmul_q8_0(d) != ZHIP_OK || behind.q != made.q || behind.d != made.d || behind.rows != made.rows || behind.k != made.k) return RoundedCopy{};
+    const uint64_t values = (uint64_t)made.rows * made.k, scales = made.scales_bytes();
+    for (const RoundedRead &r : {before, behind})
+        if (!apart(made.q, values, r.out, r.out_bytes) || !apart(made.d, scales, r.out, r.out_bytes) || !apart(made.q, values, r.w, r.w_bytes) || !apart(made.d, scales, r.w, r.w_bytes)) return RoundedCopy{};
+    if (!apart(made.q, values, made.d, scales) || ((uintptr_t)made.d & 15u)) return RoundedCopy{};
+    made.room = &c->copies[c->copies_made & 1u];
+    return made;
+}
+
 // Launches the dispatch that is op number `at`. What it packs for the one behind it holds for that one alone: whatever else
-// comes between may write there. (Under a profile every dispatch does its own work.)
-zhip_result launch_dispatch(zhip_context *c, size_t at, Dispatch &d, const Pipeline &pl) {
+// comes between may write there. What it rounds stands for the dispatch behind it and is read by the one after that. (Under a profile every
+// dispatch does its own work.)
+zhip_result launch_dispatch(zhip_context *c, size_t at, size_t end, Dispatch &d, const Pipeline &pl) {
+    if (at == c->rounded_at) return ZHIP_OK;
+    const RoundedCopy rounded = c->rounded;
+    RoundedCopy rounds;
+    if (c->rounded_at != SIZE_MAX && at == c->rounded_at + 1u) d.rounded_in = &rounded;
+    c->rounded_at = SIZE_MAX;
     const PackedCopy have = c->copy;
     PackedCopy next;
     c->copy = PackedCopy{};
     if (!c->profiling) {
-        if (pl.launch == launch_silu_mul || is_float_rung(pl)) next = wanted_behind(c, at);
+        if (pl.launch == launch_silu_mul || is_float_rung(pl)) next = wanted_behind(c, at, end);
+        if (pl.launch == launch_matmul_q8_0) rounds = rounding_behind(c, at, end, d);
+        if (rounds.room) d.rounded_out = &rounds;
         d.have = &have;
         d.next = &next;
     }
     const zhip_result r = pl.launch(d);
     if (r == ZHIP_OK && next.data) {
         c->copy = next;
+        c->copies_made++;
+    }
+    if (r == ZHIP_OK && rounds.data) {
+        c->rounded = rounds;
+        c->rounded_at = at + 1u;
         c->copies_made++;
     }
     return r;
@@ -538,7 +601,7 @@ zhip_result run_dispatch(zhip_context *c, size_t at, size_t &timed) {
         }
         if (zhip_result r = hip_check(c, hipEventRecord(c->events[2 * timed], c->stream), "hipEventRecord")) return r;
     }
-    const zhip_result r = launch_dispatch(c, at, d, *pl);
+    const zhip_result r = launch_dispatch(c, at, c->ops.size(), d, *pl);
     if (r != ZHIP_OK) {
         c->message = err[0] ? err : "kernel launch failed";
         return r;
@@ -633,12 +696,13 @@ zhip_result capture_replay(zhip_context *c, size_t count, hipGraphExec_t *out) {
     zhip_result failed = ZHIP_OK;
     c->copy = PackedCopy{};
     c->copies_made = 0;
+    c->rounded_at = SIZE_MAX;
     char err[384];
     for (size_t i = 0; i < count && failed == ZHIP_OK; i++) {
         Dispatch d;
         Pipeline *pl = nullptr;
         failed = prepare_dispatch(c, c->ops[i], d, pl, err, sizeof err);
-        if (failed == ZHIP_OK) failed = launch_dispatch(c, i, d, *pl);
+        if (failed == ZHIP_OK) failed = launch_dispatch(c, i, count, d, *pl);
     }
     c->copy = PackedCopy{};
     hipGraph_t graph = nullptr;
@@ -799,6 +863,7 @@ zhip_result run_queue(zhip_context *c) {
     }
     c->copy = PackedCopy{};
     c->copies_made = 0;
+    c->rounded_at = SIZE_MAX;
     for (size_t at = replayed ? prefix : 0; at < c->ops.size(); at++) {
         const Op &op = c->ops[at];
         if (op.kind != Op::dispatch) c->copy = PackedCopy{};

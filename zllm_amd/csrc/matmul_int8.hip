@@ -581,7 +581,12 @@ static zhip_result launch_int8(const Dispatch &d, const char *name, int type) {
     a.rows = (uint32_t)rows; a.n = (uint32_t)n; a.k = p.k; a.col0 = p.col0; a.out_stride = p.out_stride;
     a.accumulate = p.accumulate; a.k_slice = p.k_slice; a.slice_stride = p.slice_stride; a.row_bytes = (uint32_t)row_bytes;
     a.qx_bytes = (uint32_t)x_need; a.w_bytes = (uint32_t)w_need; a.dx_bytes = (uint32_t)d_need;
-    if (type == 8 && matmul_q8_i8_accepts(p.k, p.k_slice, (uint32_t)slices))
+    const bool tiled = type == 8 && matmul_q8_i8_accepts(p.k, p.k_slice, (uint32_t)slices);
+    if (d.reads) {
+        if (tiled) *d.reads = RoundedRead{a.qx, a.dx, a.w, d.bind[3].ptr, a.rows, a.k, w_need, o_need};
+        return ZHIP_OK;
+    }
+    if (tiled)
         return launch_matmul_q8_i8(d, name, a.qx, a.w, a.dx, a.out, a.rows, a.n, a.k, a.col0, a.out_stride, a.accumulate, a.row_bytes, a.qx_bytes,
             a.w_bytes, a.dx_bytes);
     const dim3 grid((uint32_t)tiles_n, (uint32_t)tiles_t, (uint32_t)slices);

@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "round_q8.h"
 
 namespace zhip {
 
@@ -58,6 +59,9 @@ struct Tile {
     // The rings, or the exchange of the four units' sums that reuses them (8 waves x 3 inboxes x TW KB).
     static constexpr int RINGS = RING * BUF + 2 * CHUNK, EXCHANGE = WAVES * 3 * TW * 1024, LDS = RINGS > EXCHANGE ? RINGS : EXCHANGE;
     static_assert(2 * LDS <= 160 * 1024, "two workgroups' buffers must fit the CU's LDS");
+    // The finished tile behind the exchange, for its rounding: a token's 64 outputs, and four to keep the tokens' out of one another's banks.
+    static constexpr int LINE = 68, DONE = EXCHANGE;
+    static_assert(DONE + BM * LINE * 4 <= LDS, "the finished tile must fit behind the exchange");
 };
 
 struct Q8I8Args {
@@ -67,6 +71,9 @@ struct Q8I8Args {
     float *out;
     uint32_t rows, n, k, col0, out_stride, accumulate, row_bytes;
     uint32_t qx_bytes, w_bytes, dx_bytes;  // bytes the kernel may read behind the pointers
+    uint8_t *home_qx, *home_dx;  // not null: qx and dx are a multiply's rounding, and belong there too
+    uint8_t *next_qx;            // ROUND: the rounded outputs and their scales
+    float *next_dx;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_buffer(const uint8_t *base, uint32_t bytes) {
@@ -96,9 +103,14 @@ __device__ __forceinline__ void sync_keeping_loads() {
 // at the LDS's full rate.
 __device__ __forceinline__ uint32_t line_key(uint32_t row) { return (row & 7u) ^ ((row >> 3) & 1u); }
 
-template <int TW>
+// ROUND: what is stored is also rounded for the multiply after the next dispatch, as that dispatch would (RoundedCopy): 1, the outputs; 2,
+// silu(gate) * up of outputs j and n / 2 + j, for which a workgroup's tile is 32 gate rows and their 32 up rows.
+// A quantize_q8 launch is bound by its start and end, and the SiLU pair's reads 8 bytes a value back. us a step, with the launches of quantize_q8 /
+// without those that follow a multiply: 28 layers of 1024 x 3072 at 9 / 64 / 512 tokens 1083 / 1165 / 1729 -> 1031 / 1100 / 1634, eight of 2560 x 9728 at
+// 128 tokens 845 -> 812, four of 4096 x 14336 at 512 1661 -> 1631.
+template <int TW, int ROUND>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void matmul_q8_i8_kernel(
-    const uint8_t *qx, const uint8_t *w_rows, const uint8_t *scales, uint32_t k, uint32_t row_bytes, uint32_t qx_bytes, uint32_t w_bytes, uint32_t dx_bytes, Q8I8Args a) {
+    const uint8_t *qx, const uint8_t *w_rows, const uint8_t *scales, uint32_t k, uint32_t row_bytes, uint32_t qx_bytes, uint32_t w_bytes, uint32_t dx_bytes, uint32_t skip, Q8I8Args a) {
     // (What the first loads need are parameters of their own, ahead of the struct: those are in registers when the wave starts. A
     // 512-token step over 28 layers of 1024 x 3072, quantize_q8 included: 1835 -> 1755 us. The struct's are on their way meanwhile: as
     // parameters of their own the compiler fetches them where the outputs are stored, 0.5 % slower.)
@@ -112,7 +124,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     constexpr int PER_STEP = 2, DL = XROWS / 4, PER_CHUNK = DL + 1;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t j0 = blockIdx.x * BN, t0 = blockIdx.y * T::BM;
+    // The tile's rows 0 .. 31 are the matrix's from j0 on, its rows 32 .. 63 `skip` further than that.
+    const uint32_t j0 = blockIdx.x * (ROUND == 2 ? BN / 2u : BN), t0 = blockIdx.y * T::BM;
+    if (ROUND != 2) skip = 0u;
     const uint32_t steps = a.k / BK;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
 
@@ -122,7 +136,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     const uint32_t xrow = XROWS * wave + (lane >> 3);
     const uint32_t xoff = (t0 + xrow) * a.k + 16u * ((lane & 7u) ^ line_key(xrow));
     const uint32_t wrow = WROWS * wave + (lane >> 3);
-    const uint32_t woff = (j0 + wrow) * a.row_bytes + 16u * ((lane & 7u) ^ line_key(wrow));
+    const uint32_t first_row = j0 + (wave >= WAVES / 2u ? skip : 0u);  // (of the wave's lines, less their place in the tile)
+    const uint32_t woff = (first_row + wrow) * a.row_bytes + 16u * ((lane & 7u) ^ line_key(wrow));
     // (A step past the end of k is asked for like the rest, so that every wait counts the same loads,
     // but as the last one: nothing reads it.)
     auto fetch = [&](uint32_t buf, uint32_t step) __attribute__((always_inline)) {
@@ -142,7 +157,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
 #pragma unroll
         for (uint32_t i = 0; i < (uint32_t)DL; i++)
             load_lds_b32(dbuf, base + 64u * (XROWS * wave + 4u * i), first + i * (a.k / 2u) + 4u * ((l & 15u) ^ (4u * ((XROWS / 4u * wave + i) & 3u))), 0);
-        load_lds_b32(wbuf, base + T::DBUF + 32u * WROWS * wave, (j0 + WROWS * wave + (l >> 3)) * a.row_bytes + a.k + 32u * chunk + 4u * (l & 7u), 0);
+        load_lds_b32(wbuf, base + T::DBUF + 32u * WROWS * wave, (first_row + WROWS * wave + (l >> 3)) * a.row_bytes + a.k + 32u * chunk + 4u * (l & 7u), 0);
     };
 
     // ---- this wave's fragments: rows 32 wn .. + 31, the TW token tiles, unit kq of a step
@@ -232,6 +247,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 
+    // The rounding this launch reads, to where the caller has it: sixteen bytes a thread, the first on their way during the exchange.
+    const uint32_t pieces = a.home_qx ? (a.qx_bytes + a.dx_bytes) / 16u : 0u, values = a.qx_bytes / 16u;
+    const uint32_t piece0 = a.home_qx ? (blockIdx.y * gridDim.x + blockIdx.x) * THREADS + tid : 0u;
+    auto piece = [&](uint32_t i) __attribute__((always_inline)) { return i < values ? reinterpret_cast<const uint4 *>(a.qx)[i] : reinterpret_cast<const uint4 *>(a.dx)[i - values]; };
+    auto settle = [&](uint32_t i, const uint4 &v) __attribute__((always_inline)) { (i < values ? reinterpret_cast<uint4 *>(a.home_qx)[i] : reinterpret_cast<uint4 *>(a.home_dx)[i - values]) = v; };
+    uint4 moved = {};
+    if (piece0 < pieces) moved = piece(piece0);
+
     // The four units of a tile meet in LDS: a row half's 4 TW quarters of tiles (quarter p of tile tt: the
     // lane's sums 4 p .. + 3) are shared out, quarter i to the wave of unit i / TW, and each wave hands the
     // others' to their owners.
@@ -249,11 +272,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     const bool aligned = ((a.out_stride | a.col0) & 3u) == 0u && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0u;
     // In each 32 x 32 tile the lane holds rows 8 p + 4 (lane / 32) .. + 3, p < 4, of token
     // lane % 32: sixteen contiguous bytes of the token's output row per quarter.
+    float *done = reinterpret_cast<float *>(lds + T::DONE);
     auto collect = [&](auto quarter) __attribute__((always_inline)) {
         constexpr int Q = decltype(quarter)::value;
 #pragma unroll
         for (int i = Q * TW; i < (Q + 1) * TW; i++) {
-            const uint32_t t = t0 + 32u * (i / 4) + lrow, col = j0 + 32u * wn + 8u * (i % 4) + 4u * h;
+            const uint32_t t = t0 + 32u * (i / 4) + lrow, col = j0 + 32u * wn + (wn ? skip : 0u) + 8u * (i % 4) + 4u * h;
             f32x4 part[4];
 #pragma unroll
             for (int from = 0; from < 4; from++) part[from] = from == Q ? mine(i) : inbox[slot(Q, from, i % TW)];
@@ -264,6 +288,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
                 f32x4 *o4 = reinterpret_cast<f32x4 *>(o);
                 if (a.accumulate) v += *o4;
                 *o4 = v;
+                if (ROUND) *reinterpret_cast<f32x4 *>(done + (32u * (i / 4) + lrow) * T::LINE + 32u * wn + 8u * (i % 4) + 4u * h) = v;
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)
@@ -286,15 +311,48 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     case 2: collect(std::integral_constant<int, 2>{}); break;
     default: collect(std::integral_constant<int, 3>{}); break;
     }
+    if (piece0 < pieces) settle(piece0, moved);
+    if (pieces > THREADS * gridDim.x * gridDim.y)
+        for (uint32_t i = piece0 + THREADS * gridDim.x * gridDim.y; i < pieces; i += THREADS * gridDim.x * gridDim.y) settle(i, piece(i));
+
+    // Eight lanes a 32-value block, four values each, as quantize_q8 has them.
+    if constexpr (ROUND != 0) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        constexpr uint32_t LANES = ROUND == 2 ? 8u : 16u;  // a token
+        const uint32_t width = ROUND == 2 ? a.n / 2u : a.n;
+#pragma unroll
+        for (uint32_t i = 0; i < (T::BM * LANES + THREADS - 1u) / THREADS; i++) {
+            const uint32_t at = tid + THREADS * i, token = at / LANES, c = 4u * (at % LANES);
+            if (T::BM * LANES % THREADS != 0u && at >= T::BM * LANES) break;  // (whole waves)
+            const qf32x4 *line = reinterpret_cast<const qf32x4 *>(done + token * T::LINE + c);
+            qf32x4 v = line[0];
+            if (ROUND == 2) v = silu_pair(v, line[8]);
+            float mag = fabsf(v[0]);
+#pragma unroll
+            for (int e = 1; e < 4; e++) mag = fabsf(v[e]) > mag ? fabsf(v[e]) : mag;
+            int q[4];
+            const float d = round_block(v, max_of_eight(mag), q);
+            if (t0 + token >= a.rows || j0 + c >= width) continue;
+            const size_t to = (size_t)(t0 + token) * width + j0 + c;
+            reinterpret_cast<uint32_t *>(a.next_qx)[to / 4u] = four_bytes(q);
+            if (at % 8u == 0u) a.next_dx[to / 32u] = d;
+        }
+    }
 }
 
-template <int TW>
+template <int TW, int ROUND>
 zhip_result launch_tile(const Dispatch &d, const char *name, const Q8I8Args &a) {
     typedef Tile<TW> T;
-    if (!lds_opt_in<matmul_q8_i8_kernel<TW>, T::LDS>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", name, T::LDS);
+    if (!lds_opt_in<matmul_q8_i8_kernel<TW, ROUND>, T::LDS>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", name, T::LDS);
     const dim3 grid((a.n + BN - 1) / BN, (a.rows + T::BM - 1) / T::BM);
-    hipLaunchKernelGGL((matmul_q8_i8_kernel<TW>), grid, dim3(THREADS), T::LDS, d.stream, a.qx, a.w, a.dx, a.k, a.row_bytes, a.qx_bytes, a.w_bytes, a.dx_bytes, a);
+    hipLaunchKernelGGL((matmul_q8_i8_kernel<TW, ROUND>), grid, dim3(THREADS), T::LDS, d.stream, a.qx, a.w, a.dx, a.k, a.row_bytes, a.qx_bytes, a.w_bytes, a.dx_bytes, a.n / 2u - BN / 2u, a);
     return check_launch(d, name);
+}
+template <int TW>
+zhip_result launch_round(const Dispatch &d, const char *name, const Q8I8Args &a, uint32_t round) {
+    return round == 0u ? launch_tile<TW, 0>(d, name, a) : round == 1u ? launch_tile<TW, 1>(d, name, a) : launch_tile<TW, 2>(d, name, a);
 }
 
 }  // namespace
@@ -310,6 +368,18 @@ zhip_result launch_matmul_q8_i8(const Dispatch &d, const char *name, const uint8
     a.qx = qx; a.w = w; a.dx = dx; a.out = out;
     a.rows = rows; a.n = n; a.k = k; a.col0 = col0; a.out_stride = out_stride; a.accumulate = accumulate;
     a.row_bytes = row_bytes; a.qx_bytes = qx_bytes; a.w_bytes = w_bytes; a.dx_bytes = dx_bytes;
+    if (d.rounded_in && d.rounded_in->data && d.rounded_in->q == qx && d.rounded_in->d == dx && d.rounded_in->rows == rows && d.rounded_in->k == k) {
+        a.home_qx = d.rounded_in->q; a.home_dx = d.rounded_in->d;
+        a.qx = d.rounded_in->data; a.dx = a.qx + d.rounded_in->scales_at();
+    }
+    uint32_t round = 0;
+    RoundedCopy *next = d.rounded_out;
+    if (next && next->x == out && next->rows == rows && col0 == 0u && out_stride == n && n == (next->mode == 2u ? 2u * next->k : next->k) && (reinterpret_cast<uintptr_t>(out) & 15u) == 0u) {
+        if (uint8_t *to = next->reserve(d)) {
+            round = next->mode == 2u ? 2u : 1u;
+            a.next_qx = to; a.next_dx = reinterpret_cast<float *>(to + next->scales_at());
+        }
+    }
     // The tile whose workgroups, two a CU, take least: costs fitted to both tiles' times at 16 ... 512 tokens over sixteen
     // matrices of 1024 x 3072 ... 28672 x 4096, where the rule's tile is the faster one but for 0.01 % of the time in the mean (64-token tiles
     // wherever they kept half of the CUs busy, as here before, 0.6 %). us, 64 / 32: 512 x 1024 x 2048 (256 workgroups of 64
@@ -317,8 +387,9 @@ zhip_result launch_matmul_q8_i8(const Dispatch &d, const char *name, const uint8
     // 3072 x 1024 (144) 7.2 / 5.6, 512 x 2048 x 1024 (128) 10.7 / 8.6, 64 x 4096 x 4096 (64) 18.0 / 13.8.
     constexpr SharedCu tall{52, 85}, flat{40, 60};
     const uint64_t columns = (n + BN - 1) / BN, cus = (uint64_t)d.dev->compute_units;
-    if (tall.of((rows + 63u) / 64u * columns, cus) < flat.of((rows + 31u) / 32u * columns, cus)) return launch_tile<2>(d, name, a);
-    return launch_tile<1>(d, name, a);
+    const zhip_result r = tall.of((rows + 63u) / 64u * columns, cus) < flat.of((rows + 31u) / 32u * columns, cus) ? launch_round<2>(d, name, a, round) : launch_round<1>(d, name, a, round);
+    if (r == ZHIP_OK && round != 0u) next->data = a.next_qx;
+    return r;
 }
 
 }  // namespace zhip

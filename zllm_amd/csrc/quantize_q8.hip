@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "round_q8.h"
 
 namespace zhip {
 
@@ -25,24 +26,7 @@ struct QuantizeQ8Params {  // params.QuantizeQ8 (src/kernels/kernels.zig:495-501
 };
 static_assert(sizeof(QuantizeQ8Params) == 16, "params.QuantizeQ8 is 16 bytes");
 
-typedef float qf32x4 __attribute__((ext_vector_type(4)));
-
-// ggml's nearest_int: adding 1.5 * 2^23 rounds the f32 to an integer, ties to even.
-__device__ __forceinline__ int nearest_int(float y) {
-    return __float_as_int(__fadd_rn(y, 12582912.0f)) - 0x4b400000;
-}
-
-// max over lane pairs, quads, groups of eight and rows of sixteen: every lane of the group ends
-// with the group's maximum.
-template <int CTRL>
-__device__ __forceinline__ float max_with(float v) {
-    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false)));
-}
-__device__ __forceinline__ float max_of_eight(float v) {
-    v = max_with<0xB1>(v);   // quad_perm [1, 0, 3, 2]
-    v = max_with<0x4E>(v);   // quad_perm [2, 3, 0, 1]
-    return max_with<0x141>(v);  // row_half_mirror: the other quad of the eight
-}
+// The same over a wave.
 __device__ __forceinline__ float max_of_wave(float v) {
     v = max_with<0x140>(max_of_eight(v));  // row_mirror: the other eight of the row
     const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)), b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
@@ -78,17 +62,10 @@ __device__ __forceinline__ void round_chunk(const QuantizeQ8Params &p, const qf3
             for (int e = 0; e < 4; e++) q[e] = min(127, nearest_int(__fmul_rn(iscale, v[e])));
         }
     } else {
-        const float amax = max_of_eight(mag);
-        if (amax != 0.f) {
-            const float d32 = __fdiv_rn(amax, 127.0f);
-            const float id = __fdiv_rn(127.0f, amax);
-            d = (float)(_Float16)d32;
-#pragma unroll
-            for (int e = 0; e < 4; e++) q[e] = nearest_int(__fmul_rn(v[e], id));
-        }
+        d = round_block(v, max_of_eight(mag), q);
     }
     if (!live) return;
-    qx[base / 4u] = ((uint32_t)q[0] & 0xffu) | (((uint32_t)q[1] & 0xffu) << 8) | (((uint32_t)q[2] & 0xffu) << 16) | (((uint32_t)q[3] & 0xffu) << 24);
+    qx[base / 4u] = four_bytes(q);
     if (((4u * lane) & (p.block - 1u)) == 0u) dx[base >> (p.block == 256u ? 8 : 5)] = d;  // (a division by the block would be one of 64 bits)
 }
 
@@ -208,8 +185,7 @@ __global__ __launch_bounds__(256) void quantize_q8_kernel(const float *x, uint32
             gate[i] = live ? gate[i] : 0.f;
             up[i] = live ? up[i] : 0.f;
         }
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = gate[i] / (1.0f + expf(-gate[i])) * up[i];
+        v = silu_pair(gate, up);
     } else if (live) {
         v = *reinterpret_cast<const qf32x4 *>(x + row * p.k + at);
     }
@@ -249,6 +225,10 @@ zhip_result launch_quantize_q8(const Dispatch &d) {
         return fail(d, ZHIP_E_BAD_COMMAND, "quantize_q8: bound ranges too small");
     if (((uintptr_t)d.bind[1].ptr | (p.mode == 1u ? (uintptr_t)d.bind[4].ptr : 0)) & 15u) return fail(d, ZHIP_E_BAD_COMMAND, "quantize_q8: x and norm weights must be 16-byte aligned");
     if (((uintptr_t)d.bind[2].ptr | (uintptr_t)d.bind[3].ptr) & 3u) return fail(d, ZHIP_E_BAD_COMMAND, "quantize_q8: outputs must be 4-byte aligned");
+    if (d.rounds) {
+        if (p.block == 32u) *d.rounds = RoundedCopy{reinterpret_cast<const float *>(d.bind[1].ptr), (uint32_t)rows, p.k, p.mode, d.bind[2].ptr, d.bind[3].ptr, nullptr, nullptr};
+        return ZHIP_OK;
+    }
     const float *x = reinterpret_cast<const float *>(d.bind[1].ptr), *nw = reinterpret_cast<const float *>(d.bind[4].ptr);
     uint32_t *qx = reinterpret_cast<uint32_t *>(d.bind[2].ptr);
     float *dx = reinterpret_cast<float *>(d.bind[3].ptr);
