@@ -34,8 +34,9 @@ struct MvArgs {
     MvArgs { first_x, first_w, first_out, first_norm_w, 0u, first_k & 0xffffffu, 0u, PAIR ? late_out_stride : first_step,                                     \
         MT == 1 ? __uint_as_float(first_m) : late_eps, first_k >> 24, first_step, first_xr, MT == 1 ? 1u : first_m, first_rows, first_row_bytes, late_act_div }
 // The tokens from t0 on.
-#define MV_GIVE_FIRST(MT, a, t0) (a).x + (size_t)(t0) * (a).xr, (a).w, (a).norm_w, (a).out + (size_t)(t0) * (a).out_stride + (a).col0, (a).k | (a).flags << 24, (a).rows, \
-    (a).row_bytes, (a).flags & FLAG_SILU_PAIR ? (a).half : (a).out_stride, (a).xr, MT == 1 ? __builtin_bit_cast(uint32_t, (a).eps) : (a).m - (t0), (a).eps, (a).act_div, \
+#define MV_GIVE_FIRST(MT, a, t0) MV_GIVE_FIRST_AS(a, t0, MT == 1 ? __builtin_bit_cast(uint32_t, (a).eps) : (a).m - (t0))
+#define MV_GIVE_FIRST_AS(a, t0, last) (a).x + (size_t)(t0) * (a).xr, (a).w, (a).norm_w, (a).out + (size_t)(t0) * (a).out_stride + (a).col0, (a).k | (a).flags << 24, (a).rows, \
+    (a).row_bytes, (a).flags & FLAG_SILU_PAIR ? (a).half : (a).out_stride, (a).xr, last, (a).eps, (a).act_div, \
     (a).out_stride
 
 // What output j (below `rows`) of a token holds, for a step that adds to it: asked for with the rows it belongs to, since behind their
