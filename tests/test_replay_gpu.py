@@ -11,6 +11,7 @@ import pytest
 
 import oracle
 from gpucheck import Ctx, rel_err
+from test_rounded_activations_gpu import Chain
 from zllm_amd import Device, synth
 from zllm_amd import kernels as K
 from zllm_amd.kernels import Kernel, TensorType, params as P
@@ -247,6 +248,32 @@ def test_a_regrown_workspace_retires_the_graphs_that_pointed_into_it():
     finally:
         for d in devs:
             d.deinit()
+
+
+def test_plans_whose_activations_are_rounded_by_their_writers_leave_the_others_their_graphs(pair):
+    """The place such activations are kept in grows with the first plan that uses it and again with a longer
+    one: each is replayed from its second pass on, a decode step that does not use it goes on being replayed,
+    and the shorter plan runs launch by launch once more, since its graph points into the place it had."""
+    replaying, eager = pair
+    count = replaying.c.host.replayed_submits
+
+    def decode(seed):
+        x = synth.activations(synth.rng(seed), 2, KDIM)
+        assert np.array_equal(replaying.step(x), eager.step(x))
+
+    def prefill(chains, seed):
+        x = synth.activations(synth.rng(seed), chains[0].rows, chains[0].dim) * np.float32(0.1)
+        assert chains[0].run(x, False) == chains[1].run(x, False)
+
+    short, long = ([Chain(s.c, *shape, "") for s in pair] for shape in ((19, 256, 384, 640), (4500, 2048, 128, 256)))  # 9.2 MB where 8 are kept at first
+    seen = []
+    for i, step in enumerate((decode, decode, decode, lambda j: prefill(short, j), lambda j: prefill(short, j), decode, lambda j: prefill(long, j), lambda j: prefill(long, j),
+                              decode, lambda j: prefill(short, j), lambda j: prefill(short, j), lambda j: prefill(long, j), decode)):
+        before = count()
+        step(0x1A00 + i)
+        seen.append(count() - before)
+    assert seen == [0, 1, 1, 0, 1, 1, 0, 1, 1, 0, 1, 1, 1]
+    assert eager.c.host.replayed_submits() == 0
 
 
 def test_a_parameter_block_written_by_a_kernel_of_the_step_is_not_replayed():

@@ -17,7 +17,7 @@ class Chain:
     once more from the last rounding."""
 
     def __init__(self, c: Ctx, rows, dim, attn, ffn, change):
-        self.c = c
+        self.c, self.rows, self.dim = c, rows, dim
         b = K.Builder(c.rec, c.set)
         self.launches = []
         self.x, self.a, self.gu, self.out, self.more = (c.output(rows * n + 8) for n in (dim, attn + 4, 2 * ffn, 96, 40))

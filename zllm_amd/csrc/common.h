@@ -81,6 +81,7 @@ struct Workspace {
     uint8_t *data = nullptr;
     uint64_t bytes = 0;
     bool fixed = false;  // memory the workspace does not own: never grown, never freed
+    bool used = false;   // asked for since this was last cleared
     // Makes at least `want` bytes available (fails on a fixed workspace that is too small).
     zhip_result reserve(const Dispatch &d, uint64_t want);
     void release();

@@ -235,6 +235,7 @@ using namespace zhip;
 // Growing replaces the allocation, so earlier dispatches that may still be
 // running with the old one are waited for first.
 zhip_result Workspace::reserve(const Dispatch &d, uint64_t want) {
+    used = true;
     if (want <= bytes) return ZHIP_OK;
     if (fixed) return fail(d, ZHIP_E_BAD_COMMAND, "workspace: %llu bytes wanted, the fixed scratch holds %llu", (unsigned long long)want, (unsigned long long)bytes);
     const uint64_t size = (want + (8u << 20) - 1) & ~(uint64_t)((8u << 20) - 1);
@@ -323,6 +324,13 @@ struct zhip_context {
         std::vector<uint8_t> key;   // every launch's function, grid, bound ranges and parameter bytes
         hipGraphExec_t exec = nullptr;
         bool unusable = false;      // capturing it failed once: stay eager
+        bool ran = false;           // launch by launch, to its end
+        // Of the two places for packed activations, those its launches used, as they were when it last ran launch by launch. (Not in the
+        // key: most submits use neither, and one that made them grow would never find itself again.)
+        struct {
+            const uint8_t *data = nullptr;
+            uint64_t bytes = 0;
+        } places[2];
         uint64_t used = 0;
     };
     std::vector<Replay> replays;
@@ -661,10 +669,9 @@ zhip_result replay_key(zhip_context *c, size_t count, std::vector<uint8_t> &key)
             uint64_t size;
         } bind[8];
     };
-    // Launchers may point kernels at the workspaces: a graph captured with an allocation
+    // Launchers may point kernels at the workspace: a graph captured with an allocation
     // that has since been replaced must never match again.
-    const uint64_t work[6] = {(uint64_t)(uintptr_t)c->work.data, c->work.bytes, (uint64_t)(uintptr_t)c->copies[0].data, c->copies[0].bytes,
-        (uint64_t)(uintptr_t)c->copies[1].data, c->copies[1].bytes};
+    const uint64_t work[2] = {(uint64_t)(uintptr_t)c->work.data, c->work.bytes};
     key.resize(sizeof work);
     memcpy(key.data(), work, sizeof work);
     char err[384];
@@ -722,11 +729,18 @@ zhip_result capture_replay(zhip_context *c, size_t count, hipGraphExec_t *out) {
     return ZHIP_OK;
 }
 
+// Whether the places for packed activations that an entry's launches used are still the same ones.
+bool in_place(const zhip_context *c, const zhip_context::Replay &e) {
+    for (int i = 0; i < 2; i++)
+        if (e.places[i].data && (e.places[i].data != c->copies[i].data || e.places[i].bytes != c->copies[i].bytes)) return false;
+    return true;
+}
+
 // The graph of the queue's first `count` dispatches if this exact sequence has been seen
 // before (captured now if this is the second time), else null: the caller then runs them
-// one by one.
-zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **out) {
-    *out = nullptr;
+// one by one, and notes in `first` what they used.
+zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **out, zhip_context::Replay **first) {
+    *out = *first = nullptr;
     std::vector<uint8_t> &key = c->replay_scratch;
     if (zhip_result r = replay_key(c, count, key)) return r;
     zhip_context::Replay *entry = nullptr;
@@ -746,9 +760,17 @@ zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **ou
         }
         entry->key = key;
         entry->used = ++c->replay_clock;
+        *first = entry;
         return ZHIP_OK;
     }
     entry->used = ++c->replay_clock;
+    if (!entry->ran || !in_place(c, *entry)) {
+        if (entry->exec) (void)hipGraphExecDestroy(entry->exec);
+        entry->exec = nullptr;
+        entry->unusable = entry->ran = false;
+        *first = entry;
+        return ZHIP_OK;
+    }
     if (entry->unusable) return ZHIP_OK;
     if (!entry->exec && capture_replay(c, count, &entry->exec) != ZHIP_OK) {
         entry->unusable = true;
@@ -834,9 +856,9 @@ zhip_result run_queue(zhip_context *c) {
     // Parameter blocks the GPU wrote are read back while resolving the launches: before the
     // timed region and before any capture.
     const size_t prefix = (c->use_graphs && !c->profiling) ? replayable_prefix(c) : 0;
-    zhip_context::Replay *replay = nullptr;
+    zhip_context::Replay *replay = nullptr, *first_seen = nullptr;
     if (prefix > 0)
-        if (zhip_result r = find_replay(c, prefix, &replay)) return r;
+        if (zhip_result r = find_replay(c, prefix, &replay, &first_seen)) return r;
     c->ticket++;
     // What the host decoded behind the last staged write, looked up and captured is over: no part of the submit's time.
     const auto started = std::chrono::steady_clock::now();
@@ -864,6 +886,7 @@ zhip_result run_queue(zhip_context *c) {
     c->copy = PackedCopy{};
     c->copies_made = 0;
     c->rounded_at = SIZE_MAX;
+    for (Workspace &w : c->copies) w.used = false;
     for (size_t at = replayed ? prefix : 0; at < c->ops.size(); at++) {
         const Op &op = c->ops[at];
         if (op.kind != Op::dispatch) c->copy = PackedCopy{};
@@ -907,6 +930,10 @@ zhip_result run_queue(zhip_context *c) {
         }
     }
     c->last_dispatches = dispatches;
+    if (first_seen) {
+        first_seen->ran = true;
+        for (int i = 0; i < 2; i++) first_seen->places[i] = {c->copies[i].used ? c->copies[i].data : nullptr, c->copies[i].used ? c->copies[i].bytes : 0u};
+    }
     if (!ends_flagged)
         if (zhip_result r = hip_check(c, hipEventRecord(c->ev_end, c->stream), "hipEventRecord")) return r;
     // The reads with flags while the stream runs on, the others behind its end.
