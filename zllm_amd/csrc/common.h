@@ -82,8 +82,13 @@ struct Workspace {
     uint64_t bytes = 0;
     bool fixed = false;  // memory the workspace does not own: never grown, never freed
     bool used = false;   // asked for since this was last cleared
+    bool kept = false;   // as it is: growing waits for the stream, which would end the capture of a graph
+    uint64_t refused = ~0ull;  // reserve_quietly: the least that has not been there since this was last cleared
     // Makes at least `want` bytes available (fails on a fixed workspace that is too small).
     zhip_result reserve(const Dispatch &d, uint64_t want);
+    // The same for what a launch can do without: null, and no message, if memory is short. Asked for once, not by every launch of a
+    // step: growing waits for the launches before it.
+    uint8_t *reserve_quietly(const Dispatch &d, uint64_t want);
     void release();
 };
 

@@ -232,47 +232,6 @@ struct Signals {
 
 using namespace zhip;
 
-// Growing replaces the allocation, so earlier dispatches that may still be
-// running with the old one are waited for first.
-zhip_result Workspace::reserve(const Dispatch &d, uint64_t want) {
-    used = true;
-    if (want <= bytes) return ZHIP_OK;
-    if (fixed) return fail(d, ZHIP_E_BAD_COMMAND, "workspace: %llu bytes wanted, the fixed scratch holds %llu", (unsigned long long)want, (unsigned long long)bytes);
-    const uint64_t size = (want + (8u << 20) - 1) & ~(uint64_t)((8u << 20) - 1);
-    if (hipStreamSynchronize(d.stream) != hipSuccess) return fail(d, ZHIP_E_GPU, "workspace: stream synchronisation failed");
-    if (data) (void)hipFree(data);
-    data = nullptr;
-    bytes = 0;
-    const hipError_t e = hipMalloc(reinterpret_cast<void **>(&data), size);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        data = nullptr;
-        return fail(d, e == hipErrorOutOfMemory ? ZHIP_E_OUT_OF_MEMORY : ZHIP_E_GPU, "workspace: cannot allocate %llu bytes", (unsigned long long)size);
-    }
-    bytes = size;
-    return ZHIP_OK;
-}
-
-uint8_t *PackedCopy::reserve(const Dispatch &d) const {
-    const uint64_t want = kind == f16_split ? 2u * plane() : plane();
-    Dispatch quiet = d;
-    quiet.err_cap = 0;
-    return room && want <= kMost && room->reserve(quiet, want) == ZHIP_OK ? room->data : nullptr;
-}
-
-uint8_t *RoundedCopy::reserve(const Dispatch &d) const {
-    const uint64_t want = scales_at() + scales_bytes();
-    Dispatch quiet = d;
-    quiet.err_cap = 0;
-    return room && want <= kMost && room->reserve(quiet, want) == ZHIP_OK ? room->data : nullptr;
-}
-
-void Workspace::release() {
-    if (data && !fixed) (void)hipFree(data);
-    data = nullptr;
-    bytes = 0;
-}
-
 struct zhip_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -693,9 +652,30 @@ zhip_result replay_key(zhip_context *c, size_t count, std::vector<uint8_t> &key)
     return ZHIP_OK;
 }
 
-// Captures the queue's first `count` dispatches into an executable graph. Nothing runs.
-zhip_result capture_replay(zhip_context *c, size_t count, hipGraphExec_t *out) {
+// Captures an entry's launches, the queue's first `count` dispatches, into an executable graph. Nothing runs. What they get of the workspaces
+// is what they got launch by launch: none of them grows, and a place that was not to be had then is not to be had now, so
+// that every launch is one whose set-up has been done.
+struct KeptWorkspaces {
+    zhip_context *c;
+    Workspace aside[2];
+    KeptWorkspaces(zhip_context *c, const zhip_context::Replay &e) : c(c) {
+        c->work.kept = true;
+        for (int i = 0; i < 2; i++) {
+            if (!e.places[i].data) std::swap(aside[i], c->copies[i]);
+            c->copies[i].kept = true;
+        }
+    }
+    ~KeptWorkspaces() {
+        c->work.kept = false;
+        for (int i = 0; i < 2; i++) {
+            if (aside[i].data) c->copies[i] = aside[i];
+            c->copies[i].kept = false;
+        }
+    }
+};
+zhip_result capture_replay(zhip_context *c, size_t count, const zhip_context::Replay &entry, hipGraphExec_t *out) {
     *out = nullptr;
+    const KeptWorkspaces kept(c, entry);
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
         (void)hipGetLastError();
         return ZHIP_E_GPU;
@@ -772,7 +752,7 @@ zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **ou
         return ZHIP_OK;
     }
     if (entry->unusable) return ZHIP_OK;
-    if (!entry->exec && capture_replay(c, count, &entry->exec) != ZHIP_OK) {
+    if (!entry->exec && capture_replay(c, count, *entry, &entry->exec) != ZHIP_OK) {
         entry->unusable = true;
         entry->exec = nullptr;
         return ZHIP_OK;
@@ -886,7 +866,7 @@ zhip_result run_queue(zhip_context *c) {
     c->copy = PackedCopy{};
     c->copies_made = 0;
     c->rounded_at = SIZE_MAX;
-    for (Workspace &w : c->copies) w.used = false;
+    for (Workspace &w : c->copies) w.used = false, w.refused = ~0ull;
     for (size_t at = replayed ? prefix : 0; at < c->ops.size(); at++) {
         const Op &op = c->ops[at];
         if (op.kind != Op::dispatch) c->copy = PackedCopy{};
