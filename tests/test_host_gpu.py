@@ -59,6 +59,30 @@ def test_a_batch_of_many_completions(ctx):
     assert [d.token for d in done] == want and np.array_equal(got, data)
 
 
+@pytest.mark.parametrize("reads", [1, 1023, 1024, 3000])
+def test_reads_of_earlier_batches_complete_with_the_next_submit(ctx, reads):
+    """Reads recorded without a submit wait for one: all of them complete with the batch that has nothing else, however many."""
+    c = ctx
+    data = c.random(16, 1)
+    buf, got = c.upload(data), np.zeros(16, np.float32)
+    done = []
+    for first in range(0, reads, 1000):
+        for i in range(first, min(first + 1000, reads)):
+            c.rec.read_buffer(9000 + i, buf.buffer, 0, got)
+        c.host.execute(c.rec.batch(), done)
+        c.rec.clear()
+    assert done == []
+    c.rec.submit(7)
+    c.host.execute(c.rec.batch(), done)
+    c.rec.clear()
+    assert [d.token for d in done] == [9000 + i for i in range(reads)] + [7] and np.array_equal(got, data)
+    with pytest.raises(host.BadCommand):  # (another error is not taken for it)
+        c.rec.read_buffer(1, buf.buffer, 4, got)
+        c.rec.submit(8)
+        c.host.execute(c.rec.batch(), done)
+    c.rec.clear()
+
+
 @pytest.mark.parametrize("words", [1, 3, 4, 16383, 16384, 16385, 131072, 131073, 262144, 2300000])
 def test_transfers_of_every_length(ctx, words):
     """Short writes go through pinned memory and long ones otherwise (64 KB), reads in pieces (128 KB; a

@@ -6,6 +6,7 @@ reference's error set (src/agility/host.zig:38).
 from __future__ import annotations
 
 import ctypes as C
+import re
 from dataclasses import dataclass
 
 import numpy as np
@@ -60,6 +61,7 @@ _ERRORS = {
     -1: GpuError, -2: DeviceLost, -3: BadCommand, -4: BadId, -5: Truncated, -6: BadLength, -7: UnsupportedKernel,
     -8: UnsupportedPrefill, -9: OutOfMemory, -10: NoDevice, -11: ValueError,
 }
+_NO_ROOM = -11  # (among the reasons of ZHIP_E_INVALID_ARGUMENT)
 
 
 @dataclass(frozen=True)
@@ -178,16 +180,23 @@ class Host:
     def execute(self, words, completions: list) -> None:
         """Runs one batch, appending one completion per submit and per read."""
         words = np.ascontiguousarray(words, dtype=np.uint32)
-        # Room for what no batch of so many words exceeds: looking for the commands that complete took as long as the library's own
-        # decoding, ahead of the first launch (a lone projection's step 22.5 -> 19.1 us).
-        cap = words.size + 64
-        if cap > len(self._out):
-            self._out = (_lib.CCompletion * (2 * cap))()
-        out, n = self._out, C.c_size_t(0)
-        r = _lib.lib.zhip_execute(self.d.ctx, words.__array_interface__["data"][0], words.size, out, cap, C.byref(n))
+        # Room for what a batch of so many words completes by itself: looking for the commands that complete took as long as the
+        # library's own decoding, ahead of the first launch (a lone projection's step 22.5 -> 19.1 us). Reads that earlier
+        # batches left without a submit come on top: the library counts those and refuses the batch, before any of it has run.
+        if words.size > len(self._out):
+            self._out = (_lib.CCompletion * (2 * words.size))()
+        n = C.c_size_t(0)
+        r = self._execute(words, n)
+        if r == _NO_ROOM and (need := re.match(r"the batch completes (\d+) tokens", self.d.error_message())):
+            self._out = (_lib.CCompletion * int(need[1]))()
+            r = self._execute(words, n)
+        out = self._out
         for i in range(n.value):
             completions.append(Completion(out[i].token, out[i].status))
         self.d.check(r)
+
+    def _execute(self, words: np.ndarray, n: C.c_size_t) -> int:
+        return _lib.lib.zhip_execute(self.d.ctx, words.__array_interface__["data"][0], words.size, self._out, len(self._out), C.byref(n))
 
     def set_file(self, data: np.ndarray | None) -> None:
         self._file = None if data is None else np.ascontiguousarray(data).view(np.uint8)
