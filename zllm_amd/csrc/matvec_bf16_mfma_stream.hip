@@ -511,7 +511,7 @@ zhip_result launch_blocks(const Dispatch &d, const StreamArgs &q, dim3 grid) {
         configured = true;
     }
     const uint32_t walkers = grid.x / q.parts;
-    if ((q.rounds | walkers) > 0xffffu || q.tail_base > 15u) return fail(d, ZHIP_E_GPU, "%s: %u rounds of %u workgroups", F16 ? "matvec_f16" : "matvec_bf16", q.rounds, walkers);
+    if (!MV_HOLDS(q.a) || (q.rounds | walkers | q.tail_rem) > 0xffffu || (q.tail_base | q.a.m) > 15u || q.parts > 127u) return fail(d, ZHIP_E_GPU, "%s: %u rounds of %u workgroups", F16 ? "matvec_f16" : "matvec_bf16", q.rounds, walkers);
     hipLaunchKernelGGL(kernel, grid, dim3(THREADS), LDS_BYTES, d.stream, q.a.x, q.a.w, q.a.norm_w, q.a.k | q.a.flags << 24, q.a.xr, q.a.row_bytes, q.a.rows, q.a.half, q.w_bytes,
         q.rounds | walkers << 16, q.tail_rem | q.tail_base << 16 | q.a.m << 20 | q.by_die << 24 | q.parts << 25, q);
     return check_launch(d, F16 ? "matvec_f16" : "matvec_bf16");

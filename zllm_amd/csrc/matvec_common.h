@@ -26,8 +26,8 @@ struct MvArgs {
 // words of those are in the wave's registers when it starts (the compiler's -amdgpu-kernarg-preload-count), a struct is
 // fetched from memory first: 0.2 - 0.3 us of a launch (2 MB read by 256 workgroups 3.03 -> 2.82 us behind the launch before). us a
 // token, 28 layers of 1024 x 3072 Q8_0 432 -> 391, bf16 486 -> 439; twelve of 2560 x 9728 Q5_K, two tokens, 513 -> 494. The outputs' stride gives its place to a gate / up step's `half`, and the count of tokens gives its to
-// eps where a workgroup has one token: those are fetched behind the first loads, and late is soon enough for them. (k and the flags
-// share a word: rows of 16 M weights and more have no kernel that takes its parameters so.)
+// eps where a workgroup has one token: those are fetched behind the first loads, and late is soon enough for them. k and the flags
+// share a word: rows of 16 M weights and more have no kernel that takes its parameters so, and each launch of one makes sure of it (MV_HOLDS).
 #define MV_FIRST const float *first_x, const uint8_t *first_w, const float *first_norm_w, float *first_out, uint32_t first_k, uint32_t first_rows, \
     uint32_t first_row_bytes, uint32_t first_step, uint32_t first_xr, uint32_t first_m, float late_eps, float late_act_div, uint32_t late_out_stride
 #define MV_TAKE_FIRST(MT, PAIR)                                                                                                                           \
@@ -38,6 +38,9 @@ struct MvArgs {
 #define MV_GIVE_FIRST_AS(a, t0, last) (a).x + (size_t)(t0) * (a).xr, (a).w, (a).norm_w, (a).out + (size_t)(t0) * (a).out_stride + (a).col0, (a).k | (a).flags << 24, (a).rows, \
     (a).row_bytes, (a).flags & FLAG_SILU_PAIR ? (a).half : (a).out_stride, (a).xr, last, (a).eps, (a).act_div, \
     (a).out_stride
+
+// What shares a word keeps to its part of it.
+#define MV_HOLDS(a) ((a).k < 1u << 24 && (a).flags < 1u << 8)
 
 // What output j (below `rows`) of a token holds, for a step that adds to it: asked for with the rows it belongs to, since behind their
 // sums it is one more trip to memory (us a token, 28 layers of 1024 x 3072 bf16 439 -> 422; eight of 4096 x 14336 Q4_K 379 -> 375). One load whatever the step and the lane, out of the buffer's range where there is nothing to add

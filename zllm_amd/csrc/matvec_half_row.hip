@@ -245,6 +245,7 @@ __global__ __launch_bounds__(256, 2) void matvec_half_row_kernel(MV_FIRST) {
 
 template <class D, int MT, int ITERS>
 zhip_result launch_iters(const Dispatch &d, const MvArgs &a) {
+    if (!MV_HOLDS(a)) return fail(d, ZHIP_E_GPU, "%s: k = %u", D::name(), a.k);
     // (Groups of tokens: blocks a multiple of the eight dies, so that the groups' workgroups of the same rows
     // share an L2; at three groups of 170 blocks 2 x 4096 x 2048 took 17.6 us instead of 12.4.)
     // Two workgroups a CU (three and more measured slower everywhere but on gate / up pairs of 200 MB:

@@ -532,6 +532,7 @@ static zhip_result launch_resident(const Dispatch &d, const MvArgs &a, uint64_t 
     const uint32_t left = halves ? tiles : tiles % groups;
     ResArgs q{a, (uint32_t)w_bytes, mask, bias_bits, halves ? 0u : tiles / groups, left, (halves || 2u * left <= groups) ? 1u : 0u, parts, nullptr, nullptr};
     const dim3 grid(groups * parts);
+    if (a.flags > 255u || left >= 1u << 24 || a.m > 15u || parts >= 1u << 24) return fail(d, ZHIP_E_GPU, "%s: %u tokens, %u parts, %u tiles left", F::name(), a.m, parts, left);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(THREADS), 0, d.stream, q.a.x, q.a.w, q.a.norm_w, q.w_bytes, q.a.xr, q.a.row_bytes, q.a.half, q.rounds, groups, q.left | q.a.flags << 24,
             q.a.m | q.split << 4 | q.parts << 8, q);

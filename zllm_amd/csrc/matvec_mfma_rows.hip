@@ -695,6 +695,8 @@ template <class F, int NB, int TEAMS, bool ACT, bool LONG>
 zhip_result launch_nb(const Dispatch &d, const RowsArgs &q) {
     constexpr int bytes = (int)(WAVES * wave_bytes<F>());
     if (!lds_opt_in<matvec_mfma_rows_kernel<F, NB, TEAMS, ACT, LONG>, bytes>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %d bytes of LDS", F::name(), bytes);
+    if (!MV_HOLDS(q.a) || q.a.m > 15u || q.parts > 255u || (q.blocks | q.groups | q.left) > 0xffffu)
+        return fail(d, ZHIP_E_GPU, "%s: %u tokens, %u blocks in %u parts, %u workgroups, %u tiles left", F::name(), q.a.m, q.blocks, q.parts, q.groups, q.left);
     hipLaunchKernelGGL((matvec_mfma_rows_kernel<F, NB, TEAMS, ACT, LONG>), dim3(q.groups * q.parts), dim3(THREADS), bytes, d.stream, q.a.x, q.a.w, q.a.norm_w, q.a.k | q.a.flags << 24, q.a.xr,
         q.a.row_bytes, q.a.rows, q.a.half, q.groups | q.left << 16, q.rounds, q.a.m | q.split << 4 | q.parts << 8 | q.blocks << 16, q);
     return check_launch(d, F::name());

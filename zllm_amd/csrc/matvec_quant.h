@@ -1595,6 +1595,7 @@ __global__ __launch_bounds__(64 * NW) void matvec_quant_slices_kernel(MV_FIRST, 
 
 template <class P, int MT, bool PAIR, int R, int NW, int K4 = 4096>
 static zhip_result run_slices(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
+    if (!MV_HOLDS(q.a)) return fail(d, ZHIP_E_GPU, "%s: k = %u", P::name(), q.a.k);
     if (!lds_opt_in<matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
     hipLaunchKernelGGL((matvec_quant_slices_kernel<P, MT, PAIR, R, NW, K4>), dim3(blocks, (q.a.m - q.t0 + MT - 1u) / MT), dim3(64 * NW), lds, d.stream, MV_GIVE_FIRST_AS(q.a, q.t0, MT == 1 ? blocks : q.a.m - q.t0), q.nm);
     return check_launch(d, P::name());
@@ -1612,6 +1613,7 @@ template <class P, int MT, bool PAIR, int SEG_LOG2> constexpr bool row_turns() {
 template <class P, int MT, bool PAIR, int SEG_LOG2, bool KEEP>
 static zhip_result run_row_kernel(const Dispatch &d, const KArgs &q, uint32_t lds, uint32_t blocks) {
     constexpr auto kernel = matvec_quant_row_kernel<P, MT, PAIR, row_turns<P, MT, PAIR, SEG_LOG2>(), SEG_LOG2, KEEP>;
+    if (!MV_HOLDS(q.a)) return fail(d, ZHIP_E_GPU, "%s: k = %u", P::name(), q.a.k);
     if (lds > 65536u && !lds_opt_in<kernel, 160 * 1024 - 64>()) return fail(d, ZHIP_E_GPU, "%s: cannot reserve %u bytes of LDS", P::name(), lds);
     hipLaunchKernelGGL(kernel, dim3(blocks, (q.mt + MT - 1u) / MT), dim3(256), lds, d.stream, MV_GIVE_FIRST(MT, q.a, q.t0), q.nm);
     return check_launch(d, P::name());
