@@ -144,7 +144,9 @@ zhip_result zhip_execute(zhip_context *context, const uint32_t *words, size_t n_
 
 /* Replaces Host.startProfile/stopProfile/timings (src/gpu/host.zig:167-190):
  * while profiling every dispatch is bracketed by its own event pair, which
- * serialises dispatches as both reference hosts do. zhip_profile_read copies
+ * serialises dispatches as both reference hosts do, and none leaves its
+ * activations to another (zhip_handed_over): the times of a profile are those
+ * of every dispatch by itself, not a step's. zhip_profile_read copies
  * up to `capacity` rows and reports the row count and the untimed dispatches. */
 zhip_result zhip_profile_start(zhip_context *context);
 zhip_result zhip_profile_stop(zhip_context *context);
@@ -159,6 +161,12 @@ zhip_result zhip_last_submit(zhip_context *context, uint64_t *out_ns, uint64_t *
 /* How many submits so far ran their dispatches from a replayed graph (see
  * ZHIP_OPTION_NO_REPLAY). No counterpart in the reference; for tests and reports. */
 zhip_result zhip_replayed_submits(zhip_context *context, uint64_t *out_count);
+/* How many dispatches so far left their activations to the one that wrote them:
+ * multiplies on a float rung that found them packed, and quantize_q8 dispatches
+ * between two int8 matmul_q8_0 whose rounding the first of those made (the
+ * buffers hold what they would hold otherwise). No counterpart in the
+ * reference; for tests and reports. */
+zhip_result zhip_handed_over(zhip_context *context, uint64_t *out_packed, uint64_t *out_rounded);
 
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that

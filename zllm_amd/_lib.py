@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(HERE, "libzllm_hip.so")
 # Every entry point include/zllm_hip.h declares.
 EXPORTS = (
     "zhip_create", "zhip_destroy", "zhip_get_caps", "zhip_supports_prefill", "zhip_set_file", "zhip_execute",
-    "zhip_profile_start", "zhip_profile_stop", "zhip_profile_read", "zhip_last_submit", "zhip_replayed_submits", "zhip_last_error",
+    "zhip_profile_start", "zhip_profile_stop", "zhip_profile_read", "zhip_last_submit", "zhip_replayed_submits", "zhip_handed_over", "zhip_last_error",
     "zhip_force_loss", "zhip_kernel_artifact", "zhip_backend_source", "zhip_kernel_ordinal",
     "zhip_matmul_q8_0_float_no_alloc", "zhip_no_alloc_capacity",
 )
@@ -66,6 +66,8 @@ def _load() -> C.CDLL:
     lib.zhip_last_submit.argtypes = [ctx, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]
     lib.zhip_replayed_submits.restype = C.c_int32
     lib.zhip_replayed_submits.argtypes = [ctx, C.POINTER(C.c_uint64)]
+    lib.zhip_handed_over.restype = C.c_int32
+    lib.zhip_handed_over.argtypes = [ctx, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]
     lib.zhip_last_error.restype = C.c_size_t
     lib.zhip_last_error.argtypes = [ctx, C.c_char_p, C.c_size_t]
     lib.zhip_force_loss.restype = C.c_int32

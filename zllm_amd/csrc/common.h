@@ -100,7 +100,7 @@ struct Workspace {
 // in bf16, 17 tokens, 420 / 330; in two f16 planes, 100 tokens, 933 / 874.
 struct PackedCopy {
     enum Kind : uint32_t { none, bf16, f16, f16_split };
-    static constexpr uint64_t kMost = 64u << 20;  // a writer packs up to here: 512 tokens of 65,536 values
+    static constexpr uint64_t kMost = 64u << 20;  // a writer packs up to here: 512 tokens of 65,536 values, in two planes 32,768
     const float *x = nullptr;  // rows x k values, dense
     uint32_t rows = 0, k = 0;
     Kind kind = none;

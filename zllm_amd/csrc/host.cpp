@@ -232,6 +232,11 @@ struct Signals {
 
 using namespace zhip;
 
+// Dispatches whose activations the one that wrote them has packed, or rounded.
+struct HandOvers {
+    uint64_t packed = 0, rounded = 0;
+};
+
 struct zhip_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -290,6 +295,7 @@ struct zhip_context {
             const uint8_t *data = nullptr;
             uint64_t bytes = 0;
         } places[2];
+        HandOvers handed;  // that its graph makes
         uint64_t used = 0;
     };
     std::vector<Replay> replays;
@@ -297,6 +303,7 @@ struct zhip_context {
     uint64_t replay_clock = 0;
     bool use_graphs = true;
     uint64_t replayed_submits = 0;
+    HandOvers handed;
 };
 
 namespace {
@@ -536,11 +543,13 @@ zhip_result launch_dispatch(zhip_context *c, size_t at, size_t end, Dispatch &d,
     if (r == ZHIP_OK && next.data) {
         c->copy = next;
         c->copies_made++;
+        c->handed.packed++;
     }
     if (r == ZHIP_OK && rounds.data) {
         c->rounded = rounds;
         c->rounded_at = at + 1u;
         c->copies_made++;
+        c->handed.rounded++;
     }
     return r;
 }
@@ -673,9 +682,9 @@ struct KeptWorkspaces {
         }
     }
 };
-zhip_result capture_replay(zhip_context *c, size_t count, const zhip_context::Replay &entry, hipGraphExec_t *out) {
-    *out = nullptr;
+zhip_result capture_replay(zhip_context *c, size_t count, zhip_context::Replay &entry) {
     const KeptWorkspaces kept(c, entry);
+    const HandOvers before = c->handed;
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
         (void)hipGetLastError();
         return ZHIP_E_GPU;
@@ -692,6 +701,8 @@ zhip_result capture_replay(zhip_context *c, size_t count, const zhip_context::Re
         if (failed == ZHIP_OK) failed = launch_dispatch(c, i, count, d, *pl);
     }
     c->copy = PackedCopy{};
+    entry.handed = HandOvers{c->handed.packed - before.packed, c->handed.rounded - before.rounded};
+    c->handed = before;
     hipGraph_t graph = nullptr;
     const hipError_t ended = hipStreamEndCapture(c->stream, &graph);
     if (ended != hipSuccess || failed != ZHIP_OK || !graph) {
@@ -699,11 +710,11 @@ zhip_result capture_replay(zhip_context *c, size_t count, const zhip_context::Re
         if (graph) (void)hipGraphDestroy(graph);
         return failed != ZHIP_OK ? failed : ZHIP_E_GPU;
     }
-    const hipError_t made = hipGraphInstantiate(out, graph, nullptr, nullptr, 0);
+    const hipError_t made = hipGraphInstantiate(&entry.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (made != hipSuccess) {
         (void)hipGetLastError();
-        *out = nullptr;
+        entry.exec = nullptr;
         return ZHIP_E_GPU;
     }
     return ZHIP_OK;
@@ -752,9 +763,8 @@ zhip_result find_replay(zhip_context *c, size_t count, zhip_context::Replay **ou
         return ZHIP_OK;
     }
     if (entry->unusable) return ZHIP_OK;
-    if (!entry->exec && capture_replay(c, count, *entry, &entry->exec) != ZHIP_OK) {
+    if (!entry->exec && capture_replay(c, count, *entry) != ZHIP_OK) {
         entry->unusable = true;
-        entry->exec = nullptr;
         return ZHIP_OK;
     }
     *out = entry;
@@ -854,6 +864,8 @@ zhip_result run_queue(zhip_context *c) {
             for (size_t i = 0; i < prefix; i++)
                 if (Pipeline *pl = get(c->pipelines, c->ops[i].pipeline)) mark_outputs(c, c->ops[i], *pl);
             c->replayed_submits++;
+            c->handed.packed += replay->handed.packed;
+            c->handed.rounded += replay->handed.rounded;
             dispatches = prefix;
             replayed = true;
         } else {
@@ -1408,6 +1420,13 @@ zhip_result zhip_profile_read(zhip_context *c, zhip_timing *out, size_t capacity
 zhip_result zhip_replayed_submits(zhip_context *c, uint64_t *out) {
     if (!c || !out) return ZHIP_E_INVALID_ARGUMENT;
     *out = c->replayed_submits;
+    return ZHIP_OK;
+}
+
+zhip_result zhip_handed_over(zhip_context *c, uint64_t *out_packed, uint64_t *out_rounded) {
+    if (!c || !out_packed || !out_rounded) return ZHIP_E_INVALID_ARGUMENT;
+    *out_packed = c->handed.packed;
+    *out_rounded = c->handed.rounded;
     return ZHIP_OK;
 }
 

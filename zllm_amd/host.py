@@ -230,6 +230,12 @@ class Host:
         self.d.check(_lib.lib.zhip_replayed_submits(self.d.ctx, C.byref(n)))
         return n.value
 
+    def handed_over(self) -> tuple[int, int]:
+        """Dispatches so far whose activations the one that wrote them packed, and rounded."""
+        packed, rounded = C.c_uint64(0), C.c_uint64(0)
+        self.d.check(_lib.lib.zhip_handed_over(self.d.ctx, C.byref(packed), C.byref(rounded)))
+        return packed.value, rounded.value
+
     def last_submit(self) -> tuple[int, int]:
         """GPU nanoseconds and dispatch count of the last submit's work."""
         ns, count = C.c_uint64(0), C.c_uint64(0)
