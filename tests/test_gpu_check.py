@@ -2238,21 +2238,25 @@ def test_matmul_kquant_int8_bits_do_not_depend_on_the_rows_of_a_launch(ctx, t, k
             assert rel_err(got[0], xs[:count].astype(np.float64) @ values.astype(np.float64).T + (init[:count] if accumulate else 0.0)) <= 1e-5
 
 
-@pytest.mark.parametrize("k", [256, 512, 768, 1280, 2304])
+# Rows of a matrix, how often a tall one has them over, the blocks of a row, (accumulate, tokens): test_kquant_launch.py has the launches they take.
+KQUANT_HALVES = (90, 273, (1, 2, 3, 5, 9), ((0, 190), (1, 126), (0, 62), (1, 62), (0, 30), (1, 3)))
+
+
+@pytest.mark.parametrize("blocks", KQUANT_HALVES[2])
 @pytest.mark.parametrize("t", [TensorType.q3_k, TensorType.q4_k, TensorType.q5_k, TensorType.q6_k])
-def test_matmul_kquant_int8_halves_of_k(ctx, t, k):
-    """Short steps over tall matrices, whose waves walk two parts of k each: the bits of the 90-row
-    matrix that the tall one is over and over, whose launches have a wave a part; one, two and three
-    blocks (parts of none), five and nine; rows that fill no tile, tokens short of one, two, four and six.
+def test_matmul_kquant_int8_halves_of_k(ctx, t, blocks):
+    """Short steps over tall matrices: the bits of the 90-row matrix that the tall one is over and over, whose launches have a wave a
+    part of k where the tall one's waves walk two parts or all of them. Every launch of two parts, in rows of every one of these numbers of blocks that
+    the rule gives it (in three or less some parts have none); rows that fill no tile, tokens short of one, two, four and six.
     1e-5 against float64 over the rounded activations."""
     c = ctx
-    rows, n, times = 190, 90, 273
+    (n, times, _, steps), k, rows = KQUANT_HALVES, 256 * blocks, max(count for _, count in KQUANT_HALVES[3])
     x = c.random(rows * k, 1).reshape(rows, k)
     raw, values = quant_rows(c, t, n, k)
     small, large = c.gpu_weights(t, raw, k), c.gpu_weights(t, np.tile(raw.reshape(-1), times), k)
     xs = oracle.round_like_llama(ORACLE_TYPE[t], x)
     init = c.random(rows * n, 1).reshape(rows, n)
-    for accumulate, count in ((0, rows), (1, 126), (0, 62), (1, 62), (0, 30), (1, 3)):
+    for accumulate, count in steps:
         act = quantize_x(c, t, c.upload(x[:count]), count, k)
         got = []
         for w, m in ((small, 1), (large, times)):

@@ -23,7 +23,8 @@
 //
 // k is summed in four parts, blocks p * B / 4 .. of part p of B, each in its order, and the parts are
 // added as ((p0 + p1) + p2) + p3, whatever the matrix and the step: neither how a prompt is cut into
-// steps nor how a matrix is cut into launches changes an output's bits. A workgroup is S * RW waves.
+// steps nor how a matrix is cut into launches changes an output's bits (but for the sign of a sum that is too small for a
+// float: a wave with fewer steps than its workgroup adds zeros to it). A workgroup is S * RW waves.
 // Wave w walks part w % S of k (S = 4), two of them (S = 2) or all four, closing each part's sums (S = 1), for rows 32 (w / S) .. + 31
 // and the tile's 32 NT tokens, one 32-token tile of a block after the other with the block's
 // converted weights in registers (64 VGPRs). Every part has a ring of three token tiles in LDS, filled
@@ -46,6 +47,7 @@
 
 #include "common.h"
 #include "decode.h"
+#include "matmul_kquant_launch.h"
 
 namespace zhip {
 
@@ -119,6 +121,7 @@ __device__ __forceinline__ uint32_t low_bytes(uint32_t even, uint32_t odd) { ret
 // A format: BLOCK bytes; Raw, the bytes lane (row, h) reads of a block, positions 16 h .. + 15 of
 // each of the eight 32-weight units; Scales, what is unpacked once a block; unit(): unit u's planes.
 struct KqQ4 {
+    static constexpr int TYPE = 4;
     static constexpr uint32_t BLOCK = 144;
     static constexpr int PLANES = 2, SHIFT = 3;
     static constexpr bool PERMUTED = false;
@@ -166,6 +169,7 @@ struct KqQ4 {
 };
 
 struct KqQ5 {
+    static constexpr int TYPE = 5;
     static constexpr uint32_t BLOCK = 176;
     static constexpr int PLANES = 2, SHIFT = 8;
     static constexpr bool PERMUTED = false;
@@ -204,6 +208,7 @@ struct KqQ5 {
 };
 
 struct KqQ6 {
+    static constexpr int TYPE = 6;
     static constexpr uint32_t BLOCK = 224;  // padded from 210 at load
     static constexpr int PLANES = 2, SHIFT = 8;
     static constexpr bool PERMUTED = false;
@@ -252,6 +257,7 @@ struct KqQ6 {
 };
 
 struct KqQ3 {
+    static constexpr int TYPE = 3;
     static constexpr uint32_t BLOCK = 128;  // repacked at load: eight 16-byte units
     static constexpr int PLANES = 1, SHIFT = 0;
     static constexpr bool PERMUTED = true;
@@ -590,69 +596,24 @@ zhip_result launch_tile(const Dispatch &d, const char *name, const KqArgs &a) {
     return check_launch(d, name);
 }
 
-// Which launch takes the step; the bits are the same. Workgroups that walk a part of k each (S = 4), or two with four row groups
-// (S = 2), have a CU to themselves: a launch of w a CU takes w times one's time. Those that walk all of it (S = 1), or half of it for
-// two row groups, share a CU two at a time, and a pair takes less than twice a lone one's time: an odd one out costs `lone`, a pair `pair`. In k the
-// first kinds' time grows like blocks + 3 (the exchange), the third's like blocks + 2. In units of such a
-// time, fitted to steps of 16 ... 512 tokens over sixteen matrices of 1024 x 3072 ... 28672 x 4096 and 4096 x 14336, every
-// launch of the list on each of them: the rule's launch is within 0.2 % (Q5_K 0.9 %, Q6_K 0.6 %) of the fastest one in the mean, and the launches
-// of S = 2 take 0.89 (Q3_K), 0.92, 0.92 and 0.91 of the time of those they came in place of. (A line
-// at a number of workgroups, as here before, lost 1.6 % / 6.2 % / 2.7 % / 1.8 % of Q4_K's / Q5_K's / Q6_K's / Q3_K's time, and where a
-// last round was nearly empty 30 - 80 %: 96 x 19456 x 2560 Q4_K 34.9 -> 20.5 us, Q5_K 40.6 -> 22.5, Q3_K 25.1 -> 19.0; Q5_K
-// 512 x 12288 x 2560 63.4 -> 55.9, 64 x 28672 x 4096 Q4_K 33.1 -> 31.6.)
-struct Costs {
-    uint32_t parts[5];   // token tiles x row groups: 1 x 1, 1 x 2, 2 x 1, 2 x 2, 4 x 2
-    SharedCu whole[3];   // of 1, 2 and 4 token tiles, four row groups (of two planes, four tiles' closed sums do not fit the registers)
-    uint32_t halves[2];  // of 1 and 2 token tiles, four row groups
-    SharedCu halves2;    // of 2 token tiles, two row groups
-};  // (0: none, or never the cheapest)
-template <class P> constexpr Costs costs();
-template <> constexpr Costs costs<KqQ3>() { return {{19, 24, 22, 31, 42}, {{51, 73}, {67, 90}, {98, 118}}, {45, 0}, {32, 46}}; }
-template <> constexpr Costs costs<KqQ4>() { return {{14, 19, 18, 29, 0}, {{39, 56}, {50, 71}, {0, 0}}, {32, 38}, {0, 0}}; }
-template <> constexpr Costs costs<KqQ5>() { return {{13, 17, 19, 26, 40}, {{32, 47}, {51, 79}, {0, 0}}, {26, 41}, {0, 0}}; }
-template <> constexpr Costs costs<KqQ6>() { return {{17, 26, 21, 31, 43}, {{53, 74}, {66, 91}, {0, 0}}, {43, 0}, {40, 44}}; }
+// The launch of that number in kKquantLaunches, if the format's costs have it.
+template <class P, int I>
+zhip_result launch_one(const Dispatch &d, const char *name, const KqArgs &a, int best) {
+    constexpr KquantLaunch l = kKquantLaunches[I];
+    if constexpr (kquant_costs(P::TYPE).has(I))
+        if (best == I) return launch_tile<P, (int)l.tiles, (int)l.groups, (int)l.split>(d, name, a);
+    if constexpr (I + 1 < kKquantLaunchCount) return launch_one<P, I + 1>(d, name, a, best);
+    return fail(d, ZHIP_E_GPU, "%s: no launch", name);
+}
 
 template <class P>
 zhip_result launch_format(const Dispatch &d, const char *name, KqArgs a) {
-    constexpr Costs c = costs<P>();
-    const uint64_t cus = (uint64_t)d.dev->compute_units, groups = (a.n + 31u) / 32u, blocks = a.k / 256u;
-    auto workgroups = [&](uint32_t nt, uint32_t rw) { return (groups + rw - 1u) / rw * ((a.rows + 32u * nt - 1u) / (32u * nt)); };
-    constexpr uint32_t shapes[5][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {4, 2}};
-    uint64_t least = ~0ull;
-    int best = 0;
-    auto consider = [&](int i, uint64_t cost) {
-        if (cost < least) least = cost, best = i;
-    };
-    auto alone = [&](uint32_t each, uint32_t nt, uint32_t rw) { return each * ((workgroups(nt, rw) + cus - 1u) / cus) * (blocks + 3u); };
-    for (int i = 0; i < 5; i++)
-        if (c.parts[i] != 0u) consider(i, alone(c.parts[i], shapes[i][0], shapes[i][1]));
-    for (int i = 0; i < 3; i++)
-        if (c.whole[i].lone != 0u) consider(5 + i, c.whole[i].of(workgroups(1u << i, 4u), cus) * (blocks + 2u));
-    for (int i = 0; i < 2; i++)
-        if (c.halves[i] != 0u) consider(8 + i, alone(c.halves[i], 1u << i, 4u));
-    if (c.halves2.lone != 0u) consider(10, c.halves2.of(workgroups(2u, 2u), cus) * (blocks + 3u));
+    constexpr KquantCosts c = kquant_costs(P::TYPE);
+    const int best = kquant_launch(c, a.rows, a.n, a.k, (uint32_t)d.dev->compute_units);
     // Matrices too large for the dies' L2s, several token tiles: 24576 x 3072 and 28672 x 4096 at 256 ... 512 tokens 1 - 8 % faster
     // column by column (two token tiles and one; four the same), matrices of up to 20 MB up to 4 % slower.
     a.by_die = (uint64_t)a.n * a.row_bytes >= (24u << 20);
-    switch (best) {
-    case 0: return launch_tile<P, 1, 1, 4>(d, name, a);
-    case 1: return launch_tile<P, 1, 2, 4>(d, name, a);
-    case 2: return launch_tile<P, 2, 1, 4>(d, name, a);
-    case 3: return launch_tile<P, 2, 2, 4>(d, name, a);
-    case 5: return launch_tile<P, 1, 4, 1>(d, name, a);
-    case 6: return launch_tile<P, 2, 4, 1>(d, name, a);
-    case 8: return launch_tile<P, 1, 4, 2>(d, name, a);
-    default: break;
-    }
-    if constexpr (c.parts[4] != 0u)
-        if (best == 4) return launch_tile<P, 4, 2, 4>(d, name, a);
-    if constexpr (c.halves[1] != 0u)
-        if (best == 9) return launch_tile<P, 2, 4, 2>(d, name, a);
-    if constexpr (c.whole[2].lone != 0u)
-        if (best == 7) return launch_tile<P, 4, 4, 1>(d, name, a);
-    if constexpr (c.halves2.lone != 0u)
-        if (best == 10) return launch_tile<P, 2, 2, 2>(d, name, a);
-    return fail(d, ZHIP_E_GPU, "%s: no launch", name);
+    return launch_one<P, 0>(d, name, a, best);
 }
 
 }  // namespace
