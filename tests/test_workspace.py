@@ -9,17 +9,19 @@ PROGRAM = r"""
 #include "common.h"
 #include <cstdio>
 #include <cstdlib>
+#include <functional>
 #include <string>
 using namespace zhip;
 
 static std::string calls;  // s: synchronised, m: allocated, x: refused, f: freed
 static uint64_t most = ~0ull;
+static std::function<uint64_t()> held_by;
 static uintptr_t next_address = 1u << 20;
 extern "C" hipError_t hipStreamSynchronize(hipStream_t) { calls += 's'; return hipSuccess; }
 extern "C" hipError_t hipFree(void *) { calls += 'f'; return hipSuccess; }
 extern "C" hipError_t hipGetLastError() { return hipSuccess; }
 extern "C" hipError_t hipMalloc(void **p, size_t size) {
-    if (size > most) { calls += 'x'; return hipErrorOutOfMemory; }
+    if (size > most || (held_by && size > held_by())) { calls += 'x'; return hipErrorOutOfMemory; }
     calls += 'm';
     *p = reinterpret_cast<void *>(next_address);
     next_address += size;
@@ -98,6 +100,25 @@ int main() {
     rounded.room = nullptr;
     rounded.k = 32;
     check(!rounded.reserve(d) && called(""), "no place");
+
+    // Short of memory for a workspace or a buffer: what the places hold is given back for it, as much as it takes.
+    most = 1ull << 40;
+    Workspace places[kSpareWorkspaces], work;
+    work.spare = places;
+    for (Workspace &p : places) check(p.reserve(d, 64 * MB) == ZHIP_OK && called("sm"), "places");
+    const uint64_t all = 100 * MB;
+    held_by = [&] { return all - places[0].bytes / 2 - places[1].bytes / 2; };  // (what hipMalloc has left)
+    void *p = nullptr;
+    check(allocate(&p, 30 * MB, nullptr, places) == hipSuccess && p && called("m"), "room enough");
+    check(allocate(&p, 60 * MB, nullptr, places) == hipSuccess && called("xsfm") && !places[0].data && places[1].bytes == 64 * MB, "one given back");
+    check(places[0].reserve(d, 64 * MB) == ZHIP_OK && called("sm"), "there again");
+    check(allocate(&p, 101 * MB, nullptr, places) == hipErrorOutOfMemory && called("xsfxsfx") && !places[0].data && !places[1].data, "both, and not enough");
+    check(allocate(&p, 101 * MB, nullptr, places) == hipErrorOutOfMemory && called("x"), "nothing to give");
+    check(places[1].reserve(d, 64 * MB) == ZHIP_OK && called("sm") && work.reserve(d, 90 * MB) == ZHIP_OK && called("sxsfm") && !places[1].data, "a workspace");
+    check(allocate(&p, 101 * MB, nullptr, nullptr) == hipErrorOutOfMemory && called("x"), "without any");
+    held_by = nullptr;
+    work.release();
+    calls.clear();
 
     w.release();
     check(!w.data && w.bytes == 0 && called("f"), "given back");

@@ -83,6 +83,7 @@ struct Workspace {
     bool fixed = false;  // memory the workspace does not own: never grown, never freed
     bool used = false;   // asked for since this was last cleared
     bool kept = false;   // as it is: growing waits for the stream, which would end the capture of a graph
+    Workspace *spare = nullptr;  // kSpareWorkspaces that are given up where memory is short of what this one needs
     uint64_t refused = ~0ull;  // reserve_quietly: the least that has not been there since this was last cleared
     // Makes at least `want` bytes available (fails on a fixed workspace that is too small).
     zhip_result reserve(const Dispatch &d, uint64_t want);
@@ -91,6 +92,11 @@ struct Workspace {
     uint8_t *reserve_quietly(const Dispatch &d, uint64_t want);
     void release();
 };
+// The places of packed activations: two, one is read while the next is written. Nobody needs them where memory is short: a dispatch that asks for
+// the workspace reads from neither, and between submits nothing is in them.
+constexpr int kSpareWorkspaces = 2;
+// hipMalloc, with what `spare` (kSpareWorkspaces of them, or null) hold where memory is short.
+hipError_t allocate(void **p, uint64_t size, hipStream_t stream, Workspace *spare);
 
 // Activations as a float rung's multiplies read them: two bytes a value, or two such planes (the rounded values and what each
 // rounding left). Such a multiply packs its f32 activations in a pass of its own, unless the dispatch right before it

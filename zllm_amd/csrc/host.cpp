@@ -243,7 +243,7 @@ struct zhip_context {
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
     DeviceInfo info;
     Workspace work;
-    Workspace copies[2];       // packed activations: one is read while the next is written
+    Workspace copies[kSpareWorkspaces];  // packed activations
     uint32_t copies_made = 0;  // since the submit began
     PackedCopy copy;           // that the last dispatch left, for the one behind it
     RoundedCopy rounded;       // the last rounding that a multiply made,
@@ -294,7 +294,7 @@ struct zhip_context {
         struct {
             const uint8_t *data = nullptr;
             uint64_t bytes = 0;
-        } places[2];
+        } places[kSpareWorkspaces];
         HandOvers handed;  // that its graph makes
         uint64_t used = 0;
     };
@@ -666,17 +666,17 @@ zhip_result replay_key(zhip_context *c, size_t count, std::vector<uint8_t> &key)
 // that every launch is one whose set-up has been done.
 struct KeptWorkspaces {
     zhip_context *c;
-    Workspace aside[2];
+    Workspace aside[kSpareWorkspaces];
     KeptWorkspaces(zhip_context *c, const zhip_context::Replay &e) : c(c) {
         c->work.kept = true;
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < kSpareWorkspaces; i++) {
             if (!e.places[i].data) std::swap(aside[i], c->copies[i]);
             c->copies[i].kept = true;
         }
     }
     ~KeptWorkspaces() {
         c->work.kept = false;
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < kSpareWorkspaces; i++) {
             if (aside[i].data) c->copies[i] = aside[i];
             c->copies[i].kept = false;
         }
@@ -722,7 +722,7 @@ zhip_result capture_replay(zhip_context *c, size_t count, zhip_context::Replay &
 
 // Whether the places for packed activations that an entry's launches used are still the same ones.
 bool in_place(const zhip_context *c, const zhip_context::Replay &e) {
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < kSpareWorkspaces; i++)
         if (e.places[i].data && (e.places[i].data != c->copies[i].data || e.places[i].bytes != c->copies[i].bytes)) return false;
     return true;
 }
@@ -924,7 +924,7 @@ zhip_result run_queue(zhip_context *c) {
     c->last_dispatches = dispatches;
     if (first_seen) {
         first_seen->ran = true;
-        for (int i = 0; i < 2; i++) first_seen->places[i] = {c->copies[i].used ? c->copies[i].data : nullptr, c->copies[i].used ? c->copies[i].bytes : 0u};
+        for (int i = 0; i < kSpareWorkspaces; i++) first_seen->places[i] = {c->copies[i].used ? c->copies[i].data : nullptr, c->copies[i].used ? c->copies[i].bytes : 0u};
     }
     if (!ends_flagged)
         if (zhip_result r = hip_check(c, hipEventRecord(c->ev_end, c->stream), "hipEventRecord")) return r;
@@ -1061,7 +1061,7 @@ zhip_result run_command(zhip_context *c, const Command &cmd, zhip_completion *ou
         b.size = size;
         b.usage = a[3];
         const uint64_t alloc = std::max<uint64_t>((size + 255u) & ~255ull, 256u);
-        if (zhip_result r = hip_check(c, hipMalloc(reinterpret_cast<void **>(&b.dev), alloc), "hipMalloc")) return r;
+        if (zhip_result r = hip_check(c, allocate(reinterpret_cast<void **>(&b.dev), alloc, c->stream, c->copies), "hipMalloc")) return r;
         // New buffers read as zero, as WebGPU's do.
         c->null_stream_work = true;
         if (zhip_result r = hip_check(c, hipMemset(b.dev, 0, alloc), "hipMemset")) { (void)hipFree(b.dev); return r; }
@@ -1254,6 +1254,7 @@ zhip_result zhip_create(const zhip_options *options, zhip_context **out_context)
     if (!c) return ZHIP_E_OUT_OF_MEMORY;
     c->device = index;
     c->use_graphs = !(options && (options->flags & ZHIP_OPTION_NO_REPLAY)) && !getenv("ZHIP_NO_REPLAY");
+    c->work.spare = c->copies;
     c->info.compute_units = prop.multiProcessorCount;
     c->info.max_lds = (int)prop.sharedMemPerBlock;
     c->info.wide_decode = options && (options->flags & ZHIP_OPTION_WIDE_DECODE);

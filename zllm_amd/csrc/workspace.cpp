@@ -3,6 +3,17 @@
 
 namespace zhip {
 
+hipError_t allocate(void **p, uint64_t size, hipStream_t stream, Workspace *spare) {
+    hipError_t e = hipMalloc(p, size);
+    for (int i = 0; spare && i < kSpareWorkspaces && e == hipErrorOutOfMemory; i++) {
+        if (!spare[i].data || hipStreamSynchronize(stream) != hipSuccess) continue;
+        (void)hipGetLastError();
+        spare[i].release();
+        e = hipMalloc(p, size);
+    }
+    return e;
+}
+
 // Growing replaces the allocation, so earlier dispatches that may still be
 // running with the old one are waited for first.
 zhip_result Workspace::reserve(const Dispatch &d, uint64_t want) {
@@ -15,7 +26,7 @@ zhip_result Workspace::reserve(const Dispatch &d, uint64_t want) {
     if (data) (void)hipFree(data);
     data = nullptr;
     bytes = 0;
-    const hipError_t e = hipMalloc(reinterpret_cast<void **>(&data), size);
+    const hipError_t e = allocate(reinterpret_cast<void **>(&data), size, d.stream, spare);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         data = nullptr;
