@@ -183,20 +183,16 @@ class Host:
         # Room for what a batch of so many words completes by itself: looking for the commands that complete took as long as the
         # library's own decoding, ahead of the first launch (a lone projection's step 22.5 -> 19.1 us). Reads that earlier
         # batches left without a submit come on top: the library counts those and refuses the batch, before any of it has run.
-        if words.size > len(self._out):
-            self._out = (_lib.CCompletion * (2 * words.size))()
-        n = C.c_size_t(0)
-        r = self._execute(words, n)
+        out, n = self._out, C.c_size_t(0)
+        if words.size > len(out):
+            out = self._out = (_lib.CCompletion * (2 * words.size))()
+        r = _lib.lib.zhip_execute(self.d.ctx, words.__array_interface__["data"][0], words.size, out, len(out), C.byref(n))
         if r == _NO_ROOM and (need := re.match(r"the batch completes (\d+) tokens", self.d.error_message())):
-            self._out = (_lib.CCompletion * int(need[1]))()
-            r = self._execute(words, n)
-        out = self._out
+            out = self._out = (_lib.CCompletion * int(need[1]))()
+            r = _lib.lib.zhip_execute(self.d.ctx, words.__array_interface__["data"][0], words.size, out, len(out), C.byref(n))
         for i in range(n.value):
             completions.append(Completion(out[i].token, out[i].status))
         self.d.check(r)
-
-    def _execute(self, words: np.ndarray, n: C.c_size_t) -> int:
-        return _lib.lib.zhip_execute(self.d.ctx, words.__array_interface__["data"][0], words.size, self._out, len(self._out), C.byref(n))
 
     def set_file(self, data: np.ndarray | None) -> None:
         self._file = None if data is None else np.ascontiguousarray(data).view(np.uint8)
